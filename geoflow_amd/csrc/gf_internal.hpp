@@ -134,6 +134,7 @@ int gf_grefderiv_t(gf_mesh *m, int idir, int trans, const double *u, double *du,
 int gf_mul_t(gf_mesh *m, const double *a, const double *b, double *out);
 int gf_dot_t(gf_mesh *m, const double *a, const double *b, size_t n, double *result);
 int gf_axpy_t(gf_mesh *m, double a, const double *x, double *y);
+int gf_grad3c(gf_mesh *m, const double *u, double *const *du, const double *edx);
 int gf_helm3c(gf_mesh *m, double p, const double *pf, const double *qf, double qs,
               const double *u, double *uo);
 

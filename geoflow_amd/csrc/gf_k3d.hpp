@@ -201,6 +201,106 @@ void k_burgers_stage3p(
   }
 }
 
+// First derivatives of a field on regular 3-D elements in one pass, the
+// element in the pencil layout of pen_op3 (z derivative in the column's
+// registers, x and y through LDS):
+//   ADV false  o0, o1, o2 = d_x p, d_y p, d_z p (GMTK::grad, gmtk.ipp:2883-2892;
+//              edx NULL: reference-space derivatives, compute_grefderivs)
+//   ADV true   o0 = M (((d_x p) v0 + (d_y p) v1) + (d_z p) v2), GAdvect::apply
+//              (gadvect.ipp:57-99); a missing velocity component is zero
+// Memory bound: four fields for the gradient, five for the advection (the
+// composed advection moved 23).  At 24^3, p = 7: gradient 34 us against 43 of
+// the LDS form k_grad, advection 41.5 us (6.8 TB/s) against 242 composed; at
+// 21x17x13, p = 5: 8.1 against 9.7 us and 8.5 against 51 us.
+template <int N, bool ADV>
+__global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_grad3p(
+    const double *__restrict__ p, const double *__restrict__ v0, const double *__restrict__ v1,
+    const double *__restrict__ v2, double *__restrict__ o0, double *__restrict__ o1,
+    double *__restrict__ o2, const double *__restrict__ W, const double *__restrict__ edx,
+    const double *__restrict__ ejac, size_t nelems) {
+  using S = gf::Pen3<N>;
+  constexpr int NV = ADV ? N : 1;
+  __shared__ double su[S::EPB][S::SZ], sd[S::EPB][S::SZ];
+  ColIdx<N> t(nelems);
+  const size_t col = t.e * S::NN + t.r;
+  double rp[N], vx[NV], vy[NV], vz[NV];
+#pragma unroll
+  for (int k = 0; k < N; k++) rp[k] = p[col + k * S::N2];
+  // the velocities' loads are in flight while p is differentiated
+  if constexpr (ADV) {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const size_t g = col + k * S::N2;
+      vx[k] = v0 ? v0[g] : 0.0;
+      vy[k] = v1 ? v1[g] : 0.0;
+      vz[k] = v2 ? v2[g] : 0.0;
+    }
+  }
+  const double rx = edx ? edx[t.e * 3] : 1.0, ry = edx ? edx[t.e * 3 + 1] : 1.0,
+               rz = edx ? edx[t.e * 3 + 2] : 1.0;
+  double *u = su[t.el], *d = sd[t.el];
+#pragma unroll
+  for (int k = 0; k < N; k++) u[S::at(t.i, t.j, k)] = rp[k];
+  double dz[N], x[N], y[N];
+  gf::gll_apply<N, false>(rp, dz);
+  __syncthreads();
+  // x pencil (j, k) = (t.i, t.j) to sd, y pencil (i, k) back into su
+#pragma unroll
+  for (int m = 0; m < N; m++) x[m] = u[S::at(m, t.i, t.j)];
+  gf::gll_apply<N, false>(x, y);
+#pragma unroll
+  for (int m = 0; m < N; m++) d[S::at(m, t.i, t.j)] = y[m];
+#pragma unroll
+  for (int m = 0; m < N; m++) x[m] = u[S::at(t.i, m, t.j)];
+  gf::gll_apply<N, false>(x, y);
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < N; m++) u[S::at(t.i, m, t.j)] = y[m];
+  __syncthreads();
+  if (!t.active) return;
+  if constexpr (ADV) {
+    const double jac = ejac[t.e], wi = W[t.i], wj = W[t.j];
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int q = S::at(t.i, t.j, k);
+      double a = (d[q] * rx) * vx[k];
+      a += (u[q] * ry) * vy[k];
+      a += (dz[k] * rz) * vz[k];
+      o0[col + k * S::N2] = a * (((W[k] * wj) * wi) * jac);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const int q = S::at(t.i, t.j, k);
+      const size_t g = col + k * S::N2;
+      o0[g] = d[q] * rx;
+      o1[g] = u[q] * ry;
+      o2[g] = dz[k] * rz;
+    }
+  }
+}
+
+template <int N>
+int launch_advect3p(gf_mesh *m, const double *p, const double *const *v, double *po) {
+  using S = gf::Pen3<N>;
+  const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
+  hipLaunchKernelGGL((k_grad3p<N, true>), dim3(nb), dim3(S::THREADS), 0, m->ctx->stream, p, v[0],
+                     v[1], v[2], po, (double *)nullptr, (double *)nullptr, m->W[0], m->edx, m->ejac,
+                     m->nelems);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+template <int N>
+int launch_grad3p(gf_mesh *m, const double *p, double *const *o, const double *edx) {
+  using S = gf::Pen3<N>;
+  const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
+  hipLaunchKernelGGL((k_grad3p<N, false>), dim3(nb), dim3(S::THREADS), 0, m->ctx->stream, p,
+                     (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, o[0],
+                     o[1], o[2], m->W[0], edx, m->ejac, m->nelems);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+
 template <int N>
 int launch_stage3p(gf_mesh *m, const StageArgs &a) {
   using S = gf::Pen3<N>;
@@ -990,6 +1090,8 @@ int launch_update_box_n(gf_mesh *m, CGVecs<T> &v, double *part) {
 
 #define GF_K3D_INSTANTIATE(N)                                                                \
   template int launch_stage3p<N>(gf_mesh *, const StageArgs &);                              \
+  template int launch_advect3p<N>(gf_mesh *, const double *, const double *const *, double *); \
+  template int launch_grad3p<N>(gf_mesh *, const double *, double *const *, const double *);  \
   template int launch_stage3b<N>(gf_mesh *, double *const *, double *const *, double *const *, \
                                  double *const *, double, double, double, int, int);         \
   template int launch_rk_out_box<N>(gf_mesh *, double *const *, double *const *,              \

@@ -1189,6 +1189,7 @@ int gf_grefderivs(gf_mesh *m, int dotrans, const double *u, double *const *du) {
   if (!dotrans && m->Niso) {
     for (int k = 0; k < m->dim; k++)
       if (!du[k]) return GF_ERR_ARG;
+    if (m->dim == 3 && m->dconst) return gf_grad3c(m, u, du, nullptr);
     return GF_DISPATCH_N(m->dim, m->Niso, gfl::launch_grad, m, u, du[0], du[1],
                          m->dim == 3 ? du[2] : nullptr, (const double *)nullptr);
   }
@@ -1239,6 +1240,7 @@ int gf_grad(gf_mesh *m, const double *u, double *const *du) {
   if (m->gtype == GF_GE_REGULAR && m->Niso) {
     for (int k = 0; k < m->dim; k++)
       if (!du[k]) return GF_ERR_ARG;
+    if (m->dim == 3 && m->dconst) return gf_grad3c(m, u, du, m->edx);
     return GF_DISPATCH_N(m->dim, m->Niso, gfl::launch_grad, m, u, du[0], du[1],
                          m->dim == 3 ? du[2] : nullptr, (const double *)m->edx);
   }

@@ -76,6 +76,24 @@ __device__ __forceinline__ void gll_apply_eo(const T (&x)[N], T (&y)[N]) {
   }
 }
 
+// y = D x (TR false) or D^T x (TR true) for a pencil in registers: the
+// even/odd form at even N, ascending sums (the reference's dmxm) at odd N.
+template <int N, bool TR, typename T>
+__device__ __forceinline__ void gll_apply(const T (&x)[N], T (&y)[N]) {
+  if constexpr (N % 2 == 0) {
+    gll_apply_eo<N, TR, T>(x, y);
+  } else {
+#pragma unroll
+    for (int l = 0; l < N; l++) {
+      T s = T(0);
+#pragma unroll
+      for (int m = 0; m < N; m++)
+        s = fma((T)(TR ? GllD<N>::at(m, l) : GllD<N>::at(l, m)), x[m], s);
+      y[l] = s;
+    }
+  }
+}
+
 template <int N>
 struct Pen3 {
   // Each pass reads D through its own copy (rows contiguous for the gradient,

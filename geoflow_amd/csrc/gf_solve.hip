@@ -859,6 +859,10 @@ int gf_helm3c(gf_mesh *m, double p, const double *pf, const double *qf, double q
   return GF_DISPATCH_N3(m->Niso, helm3c_d, m, p, pf, qf, qs, u, uo);
 }
 
+int gf_grad3c(gf_mesh *m, const double *u, double *const *du, const double *edx) {
+  return GF_DISPATCH_N3(m->Niso, launch_grad3p, m, u, du, edx);
+}
+
 int gf_axpy_t(gf_mesh *m, double a, const double *x, double *y) {
   hipLaunchKernelGGL(k_axpy, dim3(nblocks(m->ndof)), dim3(kThreads), 0, m->ctx->stream, y, a, x,
                      m->ndof);
@@ -884,6 +888,31 @@ static int copy(gf_mesh *m, double *y, const double *x) {
     if (_rc) return _rc; \
   } while (0)
 
+// The Burgers right-hand side of every component in one kernel: the RK stage
+// kernels with no previous stage.
+static int rhs_fused(gf_mesh *m, double nu, const double *const *u, double *const *dudt) {
+  if (m->dim == 3) {
+    double *in[3] = {const_cast<double *>(u[0]), const_cast<double *>(u[1]),
+                     const_cast<double *>(u[2])};
+    return GF_DISPATCH_N3(m->Niso, launch_stage3b, m, in, (double *const *)nullptr,
+                          (double *const *)nullptr, dudt, 0.0, 0.0, nu, 0, 0);
+  }
+  StageArgs a;
+  memset(&a, 0, sizeof(a));
+  for (int k = 0; k < m->dim; k++) {
+    a.uin[k] = u[k];
+    a.kout[k] = dudt[k];
+  }
+  a.D = m->D[0];
+  a.W = m->W[0];
+  a.edx = m->edx;
+  a.ejac = m->ejac;
+  a.imass = m->imass;
+  a.nu = nu;
+  a.nelems = m->nelems;
+  return GF_DISPATCH_N(m->dim, m->Niso, launch_stage, m, a);
+}
+
 extern "C" {
 
 int gf_helmholtz_apply_f32(gf_mesh *m, float p_scalar, float q_scalar, const float *q_field,
@@ -900,6 +929,12 @@ int gf_helmholtz_apply_f32(gf_mesh *m, float p_scalar, float q_scalar, const flo
 // po *= mass.
 int gf_advect(gf_mesh *m, const double *p, int nvel, const double *const *u, double *po) {
   if (!m || !p || !u || !po || nvel < 1) return GF_ERR_ARG;
+  // one pass over the element where the constant-D pencils serve the mesh
+  // (24^3, p = 7: 41.5 us, 6.8 TB/s of its five fields, against 242 composed)
+  if (m->dim == 3 && m->dconst && nvel <= 3) {
+    const double *v[3] = {u[0], nvel > 1 ? u[1] : nullptr, nvel > 2 ? u[2] : nullptr};
+    return GF_DISPATCH_N3(m->Niso, launch_advect3p, m, p, v, po);
+  }
   double *t = (double *)gf_ws(m, WS_TMP2, m->ndof * sizeof(double));
   if (!t) return gf_set_err(m->ctx, GF_ERR_ALLOC, "workspace");
   if (u[0]) {
@@ -925,6 +960,13 @@ int gf_burgers_rhs(gf_mesh *m, int mode, double nu, int nstate, const double *co
     if (!u[k]) return gf_set_err(m->ctx, GF_ERR_ARG, "NULL state component");
   for (int k = 0; k < (mode == 1 ? 1 : nstate); k++)
     if (!dudt[k]) return gf_set_err(m->ctx, GF_ERR_ARG, "NULL output component");
+  // nonlinear on regular meshes: the fused stage kernel without a previous
+  // stage is the right-hand side (2 dim field passes; composed, every
+  // component took dim + 1 element kernels and 2 dim + 3 pointwise ones:
+  // 24^3, p = 7: 94 us against 978)
+  if (mode == 0 && nstate == m->dim && m->gtype == GF_GE_REGULAR && m->Niso &&
+      (m->dim == 2 || m->dconst))
+    return rhs_fused(m, nu, u, dudt);
   double *urhs = (double *)gf_ws(m, WS_TMP3, m->ndof * sizeof(double));
   if (!urhs) return gf_set_err(m->ctx, GF_ERR_ALLOC, "workspace");
   if (mode == 2) {

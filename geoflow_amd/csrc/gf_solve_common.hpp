@@ -243,6 +243,10 @@ struct CGVecs {
 template <int N>
 int launch_stage3p(gf_mesh *m, const StageArgs &a);
 template <int N>
+int launch_advect3p(gf_mesh *m, const double *p, const double *const *v, double *po);
+template <int N>
+int launch_grad3p(gf_mesh *m, const double *p, double *const *o, const double *edx);
+template <int N>
 int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
                    double *const *kout, double bh, double ch, double nu, int acc_mode,
                    int smooth_v);

@@ -1,0 +1,61 @@
+"""Fused right-hand side, advection and gradient kernels of regular meshes
+against the oracle, at every element order and at element counts that leave
+the last workgroup partly empty."""
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+import geoflow_amd as ga
+import oracle
+
+pytestmark = [pytest.mark.gpu,
+              pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")]
+
+# FP64 sums of at most 3 (p + 1) products per node and their transposes: the
+# parity tests' 1e-12 of the largest value
+TOL = 1e-12
+
+
+def _rel(a, b):
+    return float(np.abs(a.cpu().numpy() - b).max() / np.abs(b).max())
+
+
+def _dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+@pytest.mark.parametrize("dim,p,ne", [(3, 1, [3, 2, 1]), (3, 2, [5, 1, 3]), (3, 3, [2, 3, 2]),
+                                      (3, 4, [3, 1, 1]), (3, 5, [1, 1, 1]), (3, 6, [3, 2, 1]),
+                                      (3, 7, [2, 1, 3]), (3, 8, [2, 2, 1]), (3, 9, [1, 3, 1]),
+                                      (2, 3, [5, 3]), (2, 11, [2, 1])])
+def test_fused_operators(dim, p, ne):
+    from geoflow_amd.device import Context, Mesh
+    P1 = [1.3, 0.8, 2.1][:dim]
+    bdy = [ga.GF_BDY_DIRICHLET] * (2 * dim)
+    bg, og = ga.BoxGrid(dim, p, ne, P1=P1, bdy=bdy), oracle.Grid.box(dim, p, ne, P1=P1, bdy=bdy)
+    m = Mesh(Context(0), bg)
+    rng = np.random.default_rng(p)
+    us = [rng.standard_normal(bg.ndof) for _ in range(dim)]
+    q = rng.standard_normal(bg.ndof)
+    dus, dq = [_dev(u) for u in us], _dev(q)
+    for nu in (1.0, 0.03):
+        for a, b in zip(m.burgers_rhs(dus, nu), og.burgers_rhs(us, nu)):
+            assert _rel(a, b) <= TOL
+    assert _rel(m.advect(dq, dus), og.advect(q, us)) <= TOL
+    for d, g in enumerate(m.grad(dq)):
+        assert _rel(g, og.deriv(q, d + 1)) <= TOL
+    for d, g in enumerate(m.grefderivs(dq)):
+        assert _rel(g, og.grefderiv(q, d + 1)) <= TOL
+    # a missing component is a zero velocity
+    if dim == 3:
+        import ctypes
+        from geoflow_amd._capi import lib
+        from geoflow_amd.device import _ptr
+        vp = ctypes.c_void_p
+        out = m.new()
+        v = (vp * 3)(None, dus[1].data_ptr(), None)
+        m._c(lib().gf_advect(m.h, _ptr(dq), 3, v, _ptr(out)))
+        z = np.zeros(bg.ndof)
+        assert _rel(out, og.advect(q, [z, us[1], z])) <= TOL
+        # fewer components than directions
+        assert _rel(m.advect(dq, dus[:2]), og.advect(q, us[:2] + [z])) <= TOL
