@@ -221,26 +221,10 @@ __host__ __device__ __forceinline__ double box_inv(int n) {
   return n == 1 ? 1.0 : (n == 2 ? 0.5 : (n == 4 ? 0.25 : 0.125));
 }
 
-// True when node (i,j,k) can have partners (lies on its element's boundary).
-template <int N>
-__device__ __forceinline__ bool on_elem_boundary(int i, int j, int k) {
-  return i == 0 || i == N - 1 || j == 0 || j == N - 1 || k == 0 || k == N - 1;
-}
-
-// Loads u at the 8 member slots of a group (slots past the count re-read the
-// node itself), unconditionally: the loads are independent and issue back to
-// back, instead of one conditional, waited-for load per member.
-template <typename I, typename T>
-__device__ __forceinline__ void box_load8(const T *__restrict__ u, const I (&g)[8], int n,
-                                          I gself, T (&v)[8]) {
-#pragma unroll
-  for (int m = 0; m < 8; m++) v[m] = u[m < n ? g[m] : gself];
-}
-
-// As box_load8, but absent slots are not read (their lanes are masked off
-// and the slot is set to 0), which saves address and cache work when most
-// nodes of a wave have small groups.  Slot 0 (the smallest member) is always
-// read.
+// Loads u at the member slots of a group; absent slots are not read (their
+// lanes are masked off and the slot is set to 0), which saves address and
+// cache work when most nodes of a wave have small groups.  Slot 0 (the
+// smallest member) is always read.
 template <typename I, typename T>
 __device__ __forceinline__ void box_load8m(const T *__restrict__ u, const I (&g)[8], int n,
                                            T (&v)[8]) {
@@ -253,18 +237,10 @@ __device__ __forceinline__ void box_load8m(const T *__restrict__ u, const I (&g)
   }
 }
 
-// 0 + v[0] + v[1] + ... + v[n-1] in that order; n == 1 returns v[0]
-// unchanged (singleton groups are not reduced).
-template <typename T>
-__device__ __forceinline__ T box_sum8(const T (&v)[8], int n) {
-  T s = T(0);
-#pragma unroll
-  for (int m = 0; m < 8; m++) s = m < n ? s + v[m] : s;
-  return n == 1 ? v[0] : s;
-}
-
-// box_sum8 for slots filled by box_load8m (absent slots hold +0): adding
-// them changes nothing, because a sum that starts from +0 is never -0 (in
+// 0 + v[0] + v[1] + ... over the members in that order (n == 1 returns v[0]
+// unchanged: singleton groups are not reduced), for slots filled by box_load8m.
+// Absent slots hold +0 and adding them changes nothing, because a sum that
+// starts from +0 is never -0 (in
 // round-to-nearest x + y is -0 only when both are -0), and s + (+0) == s for
 // every other s.  Same result bit for bit, without a select per slot.
 template <typename T>
@@ -275,43 +251,34 @@ __device__ __forceinline__ T box_sum8z(const T (&v)[8], int n) {
   return n == 1 ? v[0] : s;
 }
 
-// GGFX Sum of u at node (i,j,k) (global index gself) from the element's
-// partner offsets, over the ascending group.  *cnt_out receives the group
-// size.
-template <int N, typename I, typename T>
-__device__ __forceinline__ T box_gather_sum(const BoxElemDeltas &d, const T *__restrict__ u,
-                                            I gself, int i, int j, int k, int *cnt_out) {
-  I g[8];
-  const int n = box_members<I>(d, N, gself, i, j, k, g);
-  *cnt_out = n;
-  T v[8];
-  box_load8<I, T>(u, g, n, gself, v);
-  return box_sum8<T>(v, n);
-}
-
 // ---------------------------------------------------------------------------
-// Element halo in LDS for a gather Smooth at N = 8 (one wave of 64 lanes per
-// element, lane = a + 8 b owning the column (a, b, .)).  Instead of each node
-// loading its group members from global memory -- loads under per-lane
-// conditions, each waited for in turn -- the wave loads the element's own
-// values and every partner value it can need with 17 unconditional loads
-// per lane, all in flight together, and the group sums read LDS.
-// Layout (doubles):
-//   own values       [0, 512)     i + 8 j + 64 k
-//   faces            [512, 896)   512 + 64 f + p + 8 q, f = 2 d + s (d the
-//                                 face direction, s = 1 for the upper face),
-//                                 (p, q) the node's other two indices in
-//                                 increasing direction order
-//   edges            [896, 992)   896 + 8 e + r, e = 4 pd + 2 s1 + s2 for the
-//                                 direction pair pd (0: xy, 1: xz, 2: yz) with
-//                                 sides s1, s2, r the node's third index
-//   corners          [992, 1000)  992 + sx + 2 sy + 4 sz
-//   zero             1000         +0, read for absent partners
+// Element halo in LDS for a gather Smooth (N^2 threads per element, thread
+// l = a + N b owning the column (a, b, .)).  Instead of each node loading its
+// group members from global memory -- loads under per-lane conditions, each
+// waited for in turn -- the element's threads load its own values and every
+// partner value it can need with unconditional loads, all in flight
+// together, and the group sums read LDS.  Layout (values of T):
+//   own values       [0, N^3)     i + N j + N^2 k
+//   faces            FACE + N^2 f + p + N q, f = 2 d + s (d the face
+//                    direction, s = 1 for the upper face), (p, q) the node's
+//                    other two indices in increasing direction order
+//   edges            EDGE + N e + r, e = 4 pd + 2 s1 + s2 for the direction
+//                    pair pd (0: xy, 1: xz, 2: yz) with sides s1, s2, r the
+//                    node's third index
+//   corners          CORNER + sx + 2 sy + 4 sz
+//   zero             ZERO: +0, read for absent partners
 // A halo slot holds the value at the partner node across that face, edge
 // or corner (the offsets of box_elem_deltas added up); where the element has
 // no partner the offset is 0, the slot holds an own value and is never read.
 // ---------------------------------------------------------------------------
-constexpr int kHalo8 = 1001;
+template <int N>
+struct Halo {
+  static constexpr int N2 = N * N, FACE = N * N * N, EDGE = FACE + 6 * N2,
+                       CORNER = EDGE + 12 * N, ZERO = CORNER + 8, SIZE = ZERO + 1;
+  static constexpr int ER = (12 * N + N2 - 1) / N2;  // edge rounds per thread
+  static constexpr int CR = (8 + N2 - 1) / N2;       // corner rounds
+  static constexpr int RQ = 6 + ER + CR;             // partner loads per thread
+};
 
 // f(std::integral_constant<int, B>), ..., f(std::integral_constant<int, E-1>):
 // a loop whose index is a compile-time constant in the body.
@@ -322,25 +289,27 @@ __host__ __device__ __forceinline__ void static_for(F &&f) {
     static_for<B + 1, E>(f);
   }
 }
-constexpr int kHalo8Zero = 1000;
 
-__device__ __forceinline__ int64_t halo8_delta(const BoxElemDeltas &de, int d, int s) {
+__device__ __forceinline__ int64_t halo_delta(const BoxElemDeltas &de, int d, int s) {
   return s ? de.hi[d] : de.lo[d];
 }
 
-// Offset from the element's first node read by load q (0..8) of lane `lane`
-// and the LDS slot it fills (-1: the lane has nothing to load in this round;
-// it reads the element's first node instead, so every load is
+// Offset from the element's first node read by load q (0 .. RQ-1) of thread
+// l and the LDS slot it fills (-1: the thread has nothing to load in this
+// round; it reads the element's first node instead, so every load is
 // unconditional and in bounds).
-__device__ __forceinline__ int64_t halo8_src(const BoxElemDeltas &de, int lane, int q, int *slot) {
-  if (q < 6) {  // faces: the node's own offset is a lane function per face
-    const int d = q >> 1, s = q & 1, p = lane & 7, r = lane >> 3;
-    const int own = d == 0 ? 8 * lane + 7 * s : (d == 1 ? p + 64 * r + 56 * s : lane + 448 * s);
-    *slot = 512 + 64 * q + lane;
-    return own + halo8_delta(de, d, s);
+template <int N>
+__device__ __forceinline__ int64_t halo_src(const BoxElemDeltas &de, int l, int q, int *slot) {
+  using H = Halo<N>;
+  if (q < 6) {  // faces: the node's own offset is a function of l per face
+    const int d = q >> 1, s = q & 1, p = l % N, r = l / N;
+    const int own = d == 0 ? N * l + (N - 1) * s
+                           : (d == 1 ? p + H::N2 * r + N * (N - 1) * s : l + H::N2 * (N - 1) * s);
+    *slot = H::FACE + H::N2 * q + l;
+    return own + halo_delta(de, d, s);
   }
-  if (q < 8) {  // edges: 12 x 8 values over two rounds
-    const int e = (q - 6) * 8 + (lane >> 3), r = lane & 7;
+  if (q < 6 + H::ER) {  // edges
+    const int x = (q - 6) * H::N2 + l, e = x / N, r = x - e * N;
     if (e >= 12) {
       *slot = -1;
       return 0;
@@ -348,54 +317,56 @@ __device__ __forceinline__ int64_t halo8_src(const BoxElemDeltas &de, int lane, 
     // pair pd: 0 (x, y), 1 (x, z), 2 (y, z), sides s1, s2; selects only,
     // so no array is indexed by a lane-dependent value
     const int pd = e >> 2, s1 = (e >> 1) & 1, s2 = e & 1;
-    const int e1 = s1 ? 7 : 0, e2 = s2 ? 7 : 0;
+    const int e1 = s1 ? N - 1 : 0, e2 = s2 ? N - 1 : 0;
     const int c0 = pd == 2 ? r : e1;
     const int c1 = pd == 0 ? e2 : (pd == 1 ? r : e1);
     const int c2 = pd == 0 ? r : e2;
-    const int64_t dx = halo8_delta(de, 0, s1), dy1 = halo8_delta(de, 1, s1),
-                  dy2 = halo8_delta(de, 1, s2), dz = halo8_delta(de, 2, s2);
-    *slot = 896 + 8 * e + r;
-    return c0 + 8 * c1 + 64 * c2 + (pd == 0 ? dx + dy2 : (pd == 1 ? dx + dz : dy1 + dz));
+    const int64_t dx = halo_delta(de, 0, s1), dy1 = halo_delta(de, 1, s1),
+                  dy2 = halo_delta(de, 1, s2), dz = halo_delta(de, 2, s2);
+    *slot = H::EDGE + x;
+    return c0 + N * c1 + H::N2 * c2 + (pd == 0 ? dx + dy2 : (pd == 1 ? dx + dz : dy1 + dz));
   }
-  if (lane >= 8) {  // corners
+  const int c = (q - 6 - H::ER) * H::N2 + l;
+  if (c >= 8) {  // corners
     *slot = -1;
     return 0;
   }
-  const int sx = lane & 1, sy = (lane >> 1) & 1, sz = lane >> 2;
-  *slot = 992 + lane;
-  return 7 * sx + 56 * sy + 448 * sz + halo8_delta(de, 0, sx) + halo8_delta(de, 1, sy) +
-         halo8_delta(de, 2, sz);
+  const int sx = c & 1, sy = (c >> 1) & 1, sz = c >> 2;
+  *slot = H::CORNER + c;
+  return (N - 1) * (sx + N * sy + H::N2 * sz) + halo_delta(de, 0, sx) + halo_delta(de, 1, sy) +
+         halo_delta(de, 2, sz);
 }
 
-// The partner values of field u for the element at ebase: 9 loads per lane
-// into registers (halo8_src), then their LDS slots in the halo hl (kHalo8
-// values) and the zero slot; the element's own values, hl[0, 512), are
-// copied separately (one 4 KB block in the element's layout).
-template <typename T>
-struct Halo8Rim {
-  T hv[9];
-  int slot[9];
+// The partner values of field u for the element at ebase: RQ loads per
+// thread into registers (halo_src), then their LDS slots in the halo hl and
+// the zero slot; the element's own values, hl[0, N^3), are copied separately.
+template <int N, typename T>
+struct HaloRim {
+  static constexpr int RQ = Halo<N>::RQ;
+  T hv[RQ];
+  int slot[RQ];
   __device__ __forceinline__ void issue(const T *__restrict__ u, const BoxElemDeltas &de,
-                                        int64_t ebase, int lane) {
+                                        int64_t ebase, int l) {
 #pragma unroll
-    for (int q = 0; q < 9; q++) hv[q] = u[ebase + halo8_src(de, lane, q, &slot[q])];
+    for (int q = 0; q < RQ; q++) hv[q] = u[ebase + halo_src<N>(de, l, q, &slot[q])];
   }
-  __device__ __forceinline__ void store(T *hl, int lane) const {
+  __device__ __forceinline__ void store(T *hl, int l) const {
 #pragma unroll
-    for (int q = 0; q < 9; q++)
+    for (int q = 0; q < RQ; q++)
       if (slot[q] >= 0) hl[slot[q]] = hv[q];
-    if (lane == 0) hl[kHalo8Zero] = T(0);
+    if (l == 0) hl[Halo<N>::ZERO] = T(0);
   }
 };
 
-// True when halo8_order's canonical order is GGFX's on this box at N = 8:
-// every partner offset in x smaller than every one in y, and the x and y ones
-// together smaller than every z one (superincreasing in x, y, z).  An offset
-// is the element stride less 7 node strides between neighbours, (ne - 1)
-// element strides plus 7 node strides across a periodic wrap, and 7 node
-// strides within an element that is its own periodic neighbour (ne = 1).
-__host__ __device__ __forceinline__ bool box_halo8_ok(const BoxTopo &t) {
-  const int64_t NN = 512, ns[3] = {1, 8, 64};
+// True when halo_order's canonical order is GGFX's on this box at N nodes
+// per direction: every partner offset in x smaller than every one in y, and
+// the x and y ones together smaller than every z one (superincreasing in x,
+// y, z).  An offset is the element stride less N - 1 node strides between
+// neighbours, (ne - 1) element strides plus N - 1 node strides across a
+// periodic wrap, and N - 1 node strides within an element that is its own
+// periodic neighbour (ne = 1).
+__host__ __device__ __forceinline__ bool box_halo_ok(const BoxTopo &t, int N) {
+  const int64_t NN = (int64_t)N * N * N, ns[3] = {1, N, (int64_t)N * N};
   const int64_t es[3] = {NN, (int64_t)t.ne[0] * NN, (int64_t)t.ne[0] * t.ne[1] * NN};
   int64_t below = 0;  // sum of the largest offsets of the lower directions
   bool ok = true;
@@ -403,10 +374,10 @@ __host__ __device__ __forceinline__ bool box_halo8_ok(const BoxTopo &t) {
     int64_t mn, mx;
     if (t.ne[d] == 1) {
       if (!t.per[d]) continue;  // no partners in this direction
-      mn = mx = 7 * ns[d];
+      mn = mx = (N - 1) * ns[d];
     } else {
-      mn = es[d] - 7 * ns[d];
-      mx = t.per[d] ? (int64_t)(t.ne[d] - 1) * es[d] + 7 * ns[d] : mn;
+      mn = es[d] - (N - 1) * ns[d];
+      mx = t.per[d] ? (int64_t)(t.ne[d] - 1) * es[d] + (N - 1) * ns[d] : mn;
     }
     ok = ok && below < mn;
     below += mx;
@@ -414,54 +385,57 @@ __host__ __device__ __forceinline__ bool box_halo8_ok(const BoxTopo &t) {
   return ok;
 }
 
-// Per-lane constants of the group sums of the column (i, j, .): which x and
+// Per-thread constants of the group sums of the column (i, j, .): which x and
 // y partners exist, whether they lie below, and the k-independent parts of
 // their halo addresses (the zero slot where a partner is absent).
-struct Halo8Col {
+template <int N>
+struct HaloCol {
+  using H = Halo<N>;
   int i, j, xon, yon, nx, ny;
-  int ax0, ay0, axy0;  // + k * (8 xon), + k * (8 yon), + k * (xon & yon)
-  __device__ __forceinline__ Halo8Col(const BoxElemDeltas &de, int i_, int j_) : i(i_), j(j_) {
-    const int sx = i == 7, sy = j == 7;
-    const int64_t dx = i == 0 ? de.lo[0] : (i == 7 ? de.hi[0] : 0);
-    const int64_t dy = j == 0 ? de.lo[1] : (j == 7 ? de.hi[1] : 0);
+  int ax0, ay0, axy0;  // + k * (N xon), + k * (N yon), + k * (xon & yon)
+  __device__ __forceinline__ HaloCol(const BoxElemDeltas &de, int i_, int j_) : i(i_), j(j_) {
+    const int sx = i == N - 1, sy = j == N - 1;
+    const int64_t dx = i == 0 ? de.lo[0] : (i == N - 1 ? de.hi[0] : 0);
+    const int64_t dy = j == 0 ? de.lo[1] : (j == N - 1 ? de.hi[1] : 0);
     xon = dx != 0;
     yon = dy != 0;
     nx = dx < 0;
     ny = dy < 0;
-    ax0 = xon ? 512 + 64 * sx + j : kHalo8Zero;
-    ay0 = yon ? 640 + 64 * sy + i : kHalo8Zero;
-    axy0 = (xon & yon) ? 896 + 16 * sx + 8 * sy : kHalo8Zero;
+    ax0 = xon ? H::FACE + H::N2 * sx + j : H::ZERO;
+    ay0 = yon ? H::FACE + H::N2 * (2 + sy) + i : H::ZERO;
+    axy0 = (xon & yon) ? H::EDGE + N * (2 * sx + sy) : H::ZERO;
   }
 };
 
-// The group of node (i, j, K) as halo addresses in GGFX order: the partner
-// offsets' magnitudes are superincreasing x < y < z for N = 8 (an element
-// has 512 nodes, more than any in-element offset), so ascending global
-// index is the canonical order -- lower side first in z, then in y, then in
-// x -- over the 2 x 2 (x 2 on the z faces) crossings, an absent partner's
-// terms reading the zero slot, which adds +0 and leaves every sum as it is
-// (box_sum8z).  Returns the count of the group.
-template <int K>
-__device__ __forceinline__ int halo8_order(const Halo8Col &c, const BoxElemDeltas &de,
-                                           int (&a)[8]) {
-  const int own = c.i + 8 * c.j + 64 * K;
-  const int ax = c.ax0 + K * 8 * c.xon, ay = c.ay0 + K * 8 * c.yon;
+// The group of node (i, j, K) as halo addresses in canonical order -- lower
+// side first in z, then in y, then in x, the lower side of a direction being
+// the copy with the smaller global index -- over the 2 x 2 (x 2 on the z
+// faces) crossings, an absent partner's terms reading the zero slot, which
+// adds +0 and leaves every sum as it is (box_sum8z).  Every copy of a node
+// has the same order.  Where box_halo_ok holds it is ascending global index,
+// GGFX's order.  Returns the count of the group.
+template <int N, int K>
+__device__ __forceinline__ int halo_order(const HaloCol<N> &c, const BoxElemDeltas &de,
+                                          int (&a)[8]) {
+  using H = Halo<N>;
+  const int own = c.i + N * c.j + H::N2 * K;
+  const int ax = c.ax0 + K * N * c.xon, ay = c.ay0 + K * N * c.yon;
   const int axy = c.axy0 + K * (c.xon & c.yon);
   // within a y row, lower x first; then lower y row first
   const int l0 = c.nx ? ax : own, u0 = c.nx ? own : ax;
   const int l1 = c.nx ? axy : ay, u1 = c.nx ? ay : axy;
   int p[4] = {c.ny ? l1 : l0, c.ny ? u1 : u0, c.ny ? l0 : l1, c.ny ? u0 : u1};
   int zon = 0, nz = 0;
-  int q[4] = {kHalo8Zero, kHalo8Zero, kHalo8Zero, kHalo8Zero};
-  if (K == 0 || K == 7) {
+  int q[4] = {H::ZERO, H::ZERO, H::ZERO, H::ZERO};
+  if (K == 0 || K == N - 1) {
     const int64_t dz = K == 0 ? de.lo[2] : de.hi[2];
     zon = dz != 0;
     nz = dz < 0;
-    const int sz = K == 7, sx = c.i == 7, sy = c.j == 7;
-    const int bz = zon ? 768 + 64 * sz + c.i + 8 * c.j : kHalo8Zero;
-    const int bxz = (zon & c.xon) ? 928 + 16 * sx + 8 * sz + c.j : kHalo8Zero;
-    const int byz = (zon & c.yon) ? 960 + 16 * sy + 8 * sz + c.i : kHalo8Zero;
-    const int bxyz = (zon & c.xon & c.yon) ? 992 + sx + 2 * sy + 4 * sz : kHalo8Zero;
+    const int sz = K == N - 1, sx = c.i == N - 1, sy = c.j == N - 1;
+    const int bz = zon ? H::FACE + H::N2 * (4 + sz) + c.i + N * c.j : H::ZERO;
+    const int bxz = (zon & c.xon) ? H::EDGE + N * (4 + 2 * sx + sz) + c.j : H::ZERO;
+    const int byz = (zon & c.yon) ? H::EDGE + N * (8 + 2 * sy + sz) + c.i : H::ZERO;
+    const int bxyz = (zon & c.xon & c.yon) ? H::CORNER + sx + 2 * sy + 4 * sz : H::ZERO;
     const int m0 = c.nx ? bxz : bz, n0 = c.nx ? bz : bxz;
     const int m1 = c.nx ? bxyz : byz, n1 = c.nx ? byz : bxyz;
     q[0] = c.ny ? m1 : m0;
@@ -475,6 +449,21 @@ __device__ __forceinline__ int halo8_order(const Halo8Col &c, const BoxElemDelta
     a[4 + m] = nz ? p[m] : q[m];
   }
   return (1 + c.xon) * (1 + c.yon) * (1 + zon);
+}
+
+// The N = 8 instances under their own names.
+constexpr int kHalo8 = Halo<8>::SIZE;
+constexpr int kHalo8Zero = Halo<8>::ZERO;
+template <typename T>
+using Halo8Rim = HaloRim<8, T>;
+using Halo8Col = HaloCol<8>;
+__host__ __device__ __forceinline__ bool box_halo8_ok(const BoxTopo &t) {
+  return box_halo_ok(t, 8);
+}
+template <int K>
+__device__ __forceinline__ int halo8_order(const Halo8Col &c, const BoxElemDeltas &de,
+                                           int (&a)[8]) {
+  return halo_order<8, K>(c, de, a);
 }
 
 }  // namespace gf

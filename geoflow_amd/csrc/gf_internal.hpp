@@ -78,8 +78,7 @@ struct gf_mesh_s {
   // kernels may form it from the node position instead of reading it.
   bool has_box_mask = false;
   // halo8: N = 8 structured box whose partner offsets are superincreasing in
-  // the order x < y < z, so the stage kernels gather through the LDS halo
-  // (gf::halo8_order's canonical order is GGFX's)
+  // the order x < y < z (gf::halo8_order's canonical order is GGFX's)
   bool halo8 = false;
   // reusable device workspace; ws_frozen: gf_mesh_reserve(GF_RESERVE_FREEZE)
   // was called, so gf_ws hands out only what is already allocated

@@ -312,201 +312,158 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 }
 
 // ---------------------------------------------------------------------------
-// Burgers RK on a structured box (mesh->has_box): the GGFX Smooth of each
-// stage derivative, of the final-stage input and of the step output is formed
-// by gather in the kernels that consume them (gf_boxdss.hpp), in the GGFX
-// summation order, instead of separate DSS passes.  Stage derivatives are
-// stored unsmoothed.
-//   kp       previous stage derivative K_{s-1} (unsmoothed) or NULL (stage 1)
-//   acc_mode 0: no accumulator; 1: acc = Smooth(uin) + Ks*ch; 2: acc += Ks*ch
-//            (step_b accumulates from uin and smooths the output at the end;
-//            starting from Smooth(uin) keeps the accumulator continuous, so
-//            the final Smooth is the identity up to rounding and the output
-//            kernel needs only the last stage derivative's group sums)
-//   smooth_v the stage input is the final-stage input of step_b, which is
-//            smoothed: v = Smooth(uin + bh*Ks) (gexrk_stepper.ipp:300-318)
-//   acc_mode 3: the previous step's output fused with this step's first
-//            stage: uin is the previous accumulator, bh the last weight c h,
-//            and v = acc + c h Smooth(K_last) -- the output kernel's value,
-//            in the same operations -- is stored through `acc` (the state)
-//            and is this stage's input
+// Burgers RK on a structured box (mesh->has_box): the GGFX Smooth S of the
+// stage derivatives, of the final-stage input and of the step output is
+// formed by gather in the kernels that consume them (gf_boxdss.hpp) instead
+// of separate DSS passes.  Stage derivatives are stored unsmoothed.
+//
+// S is linear, so step_b's output S(uin + sum_s c_s h S(K_s))
+// (gexrk_stepper.ipp:251-341) is S(uin + sum_s c_s h K_s) with the
+// unsmoothed own K_s, and one gather at the end serves the whole sum.  A
+// stage has its own K_s in registers and the previous one in its halo, so
+// the accumulator is touched in every second stage only.
+//   IN  stage input
+//     0  v = uin                        (first stage from a state)
+//     1  v = uin + bh S(kp)
+//     2  v = S(uin + bh S(kp))          (step_b's smoothed final-stage input,
+//                                        for a state that may be discontinuous)
+//     3  v = S(kp), kp the finished accumulator of the previous step: the
+//        step output, stored to `acc` (the state), is this stage's input
+//   ACC  accumulation after the operator
+//     0  none                           K -> kout
+//     1  acc = uin + ca kp + cb K       K -> kout
+//     2  acc = uin + ca kp + cb K       (last stage: K is not stored)
+//     3  acc = acc + ca kp + cb K       (last stage)
+// Group sums are pairwise (x, then y, then z), exact for equal members of
+// groups of 2, 4 and 8, so S leaves a continuous state as it is and IN 1 and
+// IN 2 agree bit for bit on it.
+//
+// Bound by memory: at 32^3, p = 7 an RK4 step moves 42 fields of 134 MB; the
+// form whose every stage smoothed into the accumulator moved 54 and gathered
+// uin too in the last one.  Stages (IN, ACC) = (3,0) 358, (1,1) 424, (1,0)
+// 338, (1,3) 399 us, 3.6-3.8 TB/s where a copy of this size has 4.7; before,
+// 392 + 543 + 459 + 601 us.  19x14x11, p = 5 (RK3): 27 + 27 + 22 us against
+// 39 + 41 + 27, where the members were loaded node by node.
 // ---------------------------------------------------------------------------
-template <int N, bool KP, int ACC, bool SMV, bool HL>
-__global__ __launch_bounds__(gf::Pen3<N>::THREADS) __attribute__((amdgpu_waves_per_eu(N == 8 ? 4 : 1)))
-void k_burgers_stage3b(const double *__restrict__ ui0, const double *__restrict__ ui1,
-                       const double *__restrict__ ui2, const double *__restrict__ kp0,
-                       const double *__restrict__ kp1, const double *__restrict__ kp2,
-                       double *__restrict__ ac0, double *__restrict__ ac1, double *__restrict__ ac2,
-                       double *__restrict__ ko0, double *__restrict__ ko1, double *__restrict__ ko2,
-                       const double *__restrict__ imass, const double *__restrict__ W,
-                       const double *__restrict__ edx, const double *__restrict__ ejac,
-                       gf::PenD<double> Dp, double bh, double ch, double nu, gf::BoxTopo topo,
-                       size_t nelems, size_t imstride) {
+template <int N, int IN, int ACC>
+__global__ __launch_bounds__(gf::Pen3<N>::THREADS) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))
+void k_burgers_stage3b(
+    const double *__restrict__ ui0, const double *__restrict__ ui1, const double *__restrict__ ui2,
+    const double *__restrict__ kp0, const double *__restrict__ kp1, const double *__restrict__ kp2,
+    double *ac0, double *ac1, double *ac2, double *__restrict__ ko0, double *__restrict__ ko1,
+    double *__restrict__ ko2, const double *__restrict__ imass, const double *__restrict__ W,
+    const double *__restrict__ edx, const double *__restrict__ ejac, gf::PenD<double> Dp,
+    double bh, double ca, double cb, double nu, gf::BoxTopo topo, size_t nelems, size_t imstride) {
   using S = gf::Pen3<N>;
-  // N = 8 with a previous stage: the three LDS element buffers share memory
-  // with the halos of the gather (lds_copy512, gf::Halo8Rim; the kernel is
-  // held to two waves per SIMD by its registers, so 16 KB of LDS per wave
-  // costs nothing)
-  constexpr bool HALO = N == 8 && KP && HL;
-  constexpr bool GU = SMV || ACC == 1;  // the stage reads uin's group sums
-  // halo path: K's halo, uin's halo or own values, and (without uin's halo)
-  // the accumulator's own values, one after the other
-  constexpr int NHL = GU ? 2 * gf::kHalo8 : gf::kHalo8 + 512 + (ACC == 2 ? 512 : 0);
-  constexpr int NSL = HALO && NHL > 3 * S::SZ ? NHL : 3 * S::EPB * S::SZ;
-  static_assert(!HALO || 3 * S::SZ <= NSL, "element buffers fit the halo area");
-  __shared__ double sl[NSL];
-  double(*su)[S::SZ] = (double(*)[S::SZ])sl;
-  double(*sd)[S::SZ] = (double(*)[S::SZ])(sl + S::EPB * S::SZ);
-  double(*sx)[S::SZ] = (double(*)[S::SZ])(sl + 2 * S::EPB * S::SZ);
+  using H = gf::Halo<N>;
+  constexpr bool KP = IN != 0, GU = IN == 2, UIN = IN != 3;
+  static_assert(KP || ACC == 0, "the first stage accumulates nothing");
+  static_assert(IN != 3 || ACC == 0, "an output stage is a first stage");
+  // N = 8: an element is one wave and its own values go straight to LDS
+  // (lds_copy512), behind kp's halo; else they pass through registers
+  constexpr bool L8 = N == 8;
+  constexpr int UOFF = H::SIZE, AOFF = UOFF + 512;
+  constexpr int HL = !KP ? 0
+                         : (GU ? 2 * H::SIZE
+                               : H::SIZE + (L8 && UIN ? 512 : 0)) + (L8 && ACC == 3 ? 512 : 0);
+  // per element: the halos, then (the same memory) the three element buffers
+  constexpr int NSL = HL > 3 * S::SZ ? HL : 3 * S::SZ;
+  __shared__ double sl[S::EPB * NSL];
   const double *uin[3] = {ui0, ui1, ui2};
   const double *kp[3] = {kp0, kp1, kp2};
   double *acc[3] = {ac0, ac1, ac2};
   double *kout[3] = {ko0, ko1, ko2};
   ColIdx<N> t(nelems);
   const size_t col = t.e * S::NN + t.r;
-  gf::BoxElemDeltas de = {{0, 0, 0}, {0, 0, 0}};
-  if (KP) {
+  double *hk = sl + t.el * NSL;
+  double im[N];
+#pragma unroll
+  for (int k = 0; k < N; k++) im[k] = imass[t.e * imstride + t.r + (size_t)k * S::N2];
+  double ru[3][N], ra[ACC ? 3 : 1][ACC ? N : 1];
+  if constexpr (KP) {
     int ec[3];
     gf::box_elem_coords(topo, t.e, ec);
-    de = gf::box_elem_deltas(topo, N, ec);
-  }
-  // The inverse mass of the column, read once for all components (through
-  // LDS on the halo path).
-  double im[N];
-  if constexpr (HALO) {
-    lds_copy512(imass + t.e * imstride, sl, (int)threadIdx.x);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < N; k++) im[k] = sl[threadIdx.x + 64 * k];
-  } else {
-#pragma unroll
-    for (int k = 0; k < N; k++) im[k] = imass[t.e * imstride + t.r + (size_t)k * S::N2];
-  }
-  double ru[3][N];
-  if constexpr (HALO) {
-    // Per component: every load of the previous stage derivative (and of
-    // uin's halo where its group sums are needed) is issued at once -- the
-    // element's own values copied straight to LDS, the partner values
-    // through registers -- and each node sums its group from LDS in GGFX
-    // order (halo8_order): the operations and order of the gather path
-    // below, so the same result bit for bit.
-    const int lane = (int)threadIdx.x;
-    const int64_t ebase = (int64_t)t.e * 512;
-    // K's halo; uin's halo (GU) or own values; the accumulator's own values
-    double *hk = sl, *hu = sl + gf::kHalo8, *ha = sl + gf::kHalo8 + 512;
-    const gf::Halo8Col hc(de, t.i, t.j);
+    const gf::BoxElemDeltas de = gf::box_elem_deltas(topo, N, ec);
+    const int l = t.r;
+    const int64_t ebase = (int64_t)t.e * S::NN;
+    double *hu = hk + UOFF;
+    double *ha = hk + (GU ? 2 * H::SIZE : AOFF);
+    const gf::HaloCol<N> hc(de, t.i, t.j);
     gf::static_for<0, 3>([&](auto cc) {
       constexpr int c = decltype(cc)::value;
       __syncthreads();  // the previous component's group sums have read LDS
-      // the element's own values straight to LDS, the partner values
-      // through registers
-      lds_copy512(kp[c] + ebase, hk, lane);
-      lds_copy512(uin[c] + ebase, hu, lane);
-      if (ACC == 2 && !GU) lds_copy512(acc[c] + ebase, ha, lane);
-      gf::Halo8Rim<double> Lk, Lu;
-      Lk.issue(kp[c], de, ebase, lane);
-      if (GU) Lu.issue(uin[c], de, ebase, lane);
-      double ao[8];
+      // every load of the component is issued before the first LDS store
+      double ko[N], uo[N], ao[N];
+      if constexpr (L8) {
+        lds_copy512(kp[c] + ebase, hk, l);
+        if (UIN) lds_copy512(uin[c] + ebase, hu, l);
+        if (ACC == 3) lds_copy512(acc[c] + ebase, ha, l);
+      } else {
 #pragma unroll
-      for (int k = 0; k < 8; k++) ao[k] = ACC == 2 && GU ? acc[c][col + (size_t)k * 64] : 0.0;
-      Lk.store(hk, lane);
-      if (GU) Lu.store(hu, lane);
+        for (int k = 0; k < N; k++) ko[k] = kp[c][col + (size_t)k * S::N2];
+        if (UIN) {
+#pragma unroll
+          for (int k = 0; k < N; k++) uo[k] = uin[c][col + (size_t)k * S::N2];
+        }
+        if (ACC == 3) {
+#pragma unroll
+          for (int k = 0; k < N; k++) ao[k] = acc[c][col + (size_t)k * S::N2];
+        }
+      }
+      gf::HaloRim<N, double> Lk, Lu;
+      Lk.issue(kp[c], de, ebase, l);
+      if (GU) Lu.issue(uin[c], de, ebase, l);
+      Lk.store(hk, l);
+      if (GU) Lu.store(hu, l);
+      if constexpr (!L8) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+          hk[l + S::N2 * k] = ko[k];
+          if (GU) hu[l + S::N2 * k] = uo[k];
+        }
+      }
       __syncthreads();
-      gf::static_for<0, 8>([&](auto kc) {
+      gf::static_for<0, N>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
-        constexpr int NT = (k == 0 || k == 7) ? 8 : 4;  // terms that can be non-zero
-        const int own = lane + 64 * k;
+        constexpr bool ZF = k == 0 || k == N - 1;  // groups of up to 8, else 4
+        const int own = l + S::N2 * k;
         int ad[8];
-        const int cnt = gf::halo8_order<k>(hc, de, ad);
-        double sk = 0.0;
-#pragma unroll
-        for (int m = 0; m < NT; m++) sk = sk + hk[ad[m]];
-        // GGFX Smooth: Sum / count (an exact multiply for counts 1, 2, 4, 8)
-        const double ks = cnt == 1 ? hk[own] : sk * gf::box_inv(cnt);
-        const double uo = hu[own];
-        double v = uo + bh * ks;
-        double av = 0.0;
-        if (ACC == 2) av = (GU ? ao[k] : ha[own]) + ks * ch;
-        if (ACC == 3) av = v;
-        if (ACC == 1) {
-          // the accumulator starts from Smooth(uin), so it stays continuous
-          double su1 = 0.0;
-#pragma unroll
-          for (int m = 0; m < NT; m++) su1 = su1 + hu[ad[m]];
-          const double us = cnt == 1 ? uo : su1 * gf::box_inv(cnt);
-          av = us + ks * ch;
-        }
-        if (SMV && cnt > 1) {
+        const int cnt = gf::halo_order<N, k>(hc, de, ad);
+        const double inv = gf::box_inv(cnt);  // Smooth: Sum / count, exact
+        auto sum = [&](auto &&val) {
+          double s = (val(ad[0]) + val(ad[1])) + (val(ad[2]) + val(ad[3]));
+          if (ZF) s = s + ((val(ad[4]) + val(ad[5])) + (val(ad[6]) + val(ad[7])));
+          return s * inv;
+        };
+        const double kown = L8 ? hk[own] : ko[k];
+        const double ks = sum([&](int q) { return hk[q]; });
+        double v;
+        if constexpr (IN == 3) {
+          v = ks;
+          if (t.active) acc[c][col + (size_t)k * S::N2] = v;
+        } else {
+          const double u = L8 ? hu[own] : uo[k];
+          v = fma(bh, ks, u);
           // the members only: an absent partner's zero slot would add bh ks
-          double sv = 0.0;
-#pragma unroll
-          for (int m = 0; m < NT; m++)
-            if (ad[m] != gf::kHalo8Zero) sv = sv + (hu[ad[m]] + bh * ks);
-          v = sv * gf::box_inv(cnt);
+          if (GU) v = sum([&](int q) { return q == H::ZERO ? 0.0 : fma(bh, ks, hu[q]); });
+          if constexpr (ACC == 1 || ACC == 2) ra[c][k] = fma(ca, kown, u);
+          if constexpr (ACC == 3) ra[c][k] = fma(ca, kown, L8 ? ha[own] : ao[k]);
         }
-        if (ACC && t.active) acc[c][col + (size_t)k * 64] = av;
+        // the value is formed here, node by node: without this the compiler
+        // interleaves the sums of many nodes and keeps their operands live
+        // (354 registers instead of 154 at N = 8, IN 1, ACC 0)
+        asm volatile("" : "+v"(v));
         ru[c][k] = v;
       });
     });
     __syncthreads();  // the element buffers below reuse the halo area
   } else {
-  // Stage input (and accumulator) per node; all loads are issued before any
-  // store, the accumulator stores follow the loop.  Absent group members are
-  // not read (box_load8m).
-  double av[ACC ? 3 : 1][ACC ? N : 1];
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const size_t g = col + (size_t)k * S::N2;
-    if (!KP) {
-#pragma unroll
-      for (int c = 0; c < 3; c++) ru[c][k] = uin[c][g];
-      continue;
-    }
-    int64_t mem[8];
-    int own;
-    const int cnt = gf::box_members_own<int64_t>(de, N, (int64_t)g, t.i, t.j, k, mem, &own);
-#pragma unroll
-    for (int c = 0; c < 3; c++) {
-      double kv[8];
-      gf::box_load8m<int64_t, double>(kp[c], mem, cnt, kv);
-      const double ao = ACC == 2 ? acc[c][g] : 0.0;
-      double uv[8];
-      double ui;
-      if (GU) gf::box_load8m<int64_t, double>(uin[c], mem, cnt, uv);
-      if (SMV) {
-        // the node's own value is one of the gathered slots (picking it
-        // there measured faster than a separate load in this form only)
-        ui = uv[0];
-#pragma unroll
-        for (int m = 1; m < 8; m++) ui = own == m ? uv[m] : ui;
-      } else {
-        ui = uin[c][g];
-      }
-      // GGFX Smooth: Sum / count (an exact multiply for counts 1, 2, 4, 8)
-      const double ks = cnt == 1 ? kv[0] : gf::box_sum8z<double>(kv, cnt) * gf::box_inv(cnt);
-      double v = ui + bh * ks;
-      if (ACC == 2) av[c][k] = ao + ks * ch;
-      if (ACC == 3) av[c][k] = v;
-      if (ACC == 1) {
-        // the accumulator starts from Smooth(uin), so it stays continuous
-        const double us = cnt == 1 ? uv[0] : gf::box_sum8z<double>(uv, cnt) * gf::box_inv(cnt);
-        av[c][k] = us + ks * ch;
-      }
-      if (SMV) {
-#pragma unroll
-        for (int q = 0; q < 8; q++) uv[q] = uv[q] + bh * ks;
-        if (cnt > 1) v = gf::box_sum8<double>(uv, cnt) * gf::box_inv(cnt);
-      }
-      ru[c][k] = v;
-    }
-  }
-  if (ACC && t.active) {
 #pragma unroll
     for (int c = 0; c < 3; c++)
 #pragma unroll
-      for (int k = 0; k < N; k++) acc[c][col + (size_t)k * S::N2] = av[ACC ? c : 0][ACC ? k : 0];
+      for (int k = 0; k < N; k++) ru[c][k] = uin[c][col + (size_t)k * S::N2];
   }
-  }
+  double *su = hk, *sd = hk + S::SZ, *sx = hk + 2 * S::SZ;
   const double jac = ejac[t.e];
   const double wa = W[t.i], wb = W[t.j];
   const double rx = edx[t.e * 3], ry = edx[t.e * 3 + 1], rz = edx[t.e * 3 + 2];
@@ -517,221 +474,114 @@ void k_burgers_stage3b(const double *__restrict__ ui0, const double *__restrict_
     auto zcb = [&](int k, double uz, double) { uzs[k] = uz; };
     auto xcb = [&](int, double ux, double) { return ux * rx; };
     auto ycb = [&](int, double uy, double) { return uy * ry; };
-    double *ko = kout[c];
+    double *ko = kout[c], *ac = acc[c];
     auto post = [&](int k, double L, double M, double hx, double hy) {
       if (!t.active) return;
       const size_t g = col + k * S::N2;
-      const double uz = uzs[k];
-      double po = hx * ru[0][k];
-      po += hy * ru[1][k];
-      po += (uz * rz) * ru[2][k];
-      const double adv = po * M;
+      // contractions written out: every form of the stage rounds alike
+      const double po =
+          fma(uzs[k] * rz, ru[2][k], fma(hy, ru[1][k], hx * ru[0][k]));
       if (nu != 1.0) L *= nu;
-      const double urhs = -1.0 * L + -1.0 * adv;
-      ko[g] = im[k] * urhs;
+      const double urhs = fma(-po, M, -L);
+      const double K = im[k] * urhs;
+      if (ACC < 2) ko[g] = K;
+      if (ACC) ac[g] = fma(cb, K, ra[ACC ? c : 0][ACC ? k : 0]);
     };
-    gf::pen_op3<N, double, true>(ru[c], su[t.el], sd[t.el], sx[t.el], Dp, W, t.i, t.j, wa, wb, jac,
-                                 rx * rx, ry * ry, rz * rz, (const double *)nullptr, xcb, ycb, zcb,
-                                 post);
+    gf::pen_op3<N, double, true>(ru[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,
+                                 rz * rz, (const double *)nullptr, xcb, ycb, zcb, post);
     __syncthreads();  // the next component reuses the LDS buffers
   }
 }
 
-// Step output on a structured box: u = acc + cl*Smooth(K), the smooth by
-// gather.  step_b forms Smooth(acc + cl*Smooth(K)) (its last update and GGFX
-// Smooth); the accumulator here is continuous (it starts from Smooth(uin)
-// and adds smoothed stage derivatives), so that final Smooth is the identity
-// up to rounding and is not formed.
-template <int N, typename I>
-__global__ __launch_bounds__(kThreads) void k_rk_out_box(
-    double *__restrict__ u0, double *__restrict__ u1, double *__restrict__ u2,
-    const double *__restrict__ a0, const double *__restrict__ a1, const double *__restrict__ a2,
-    const double *__restrict__ k0, const double *__restrict__ k1, const double *__restrict__ k2,
-    double cl, gf::BoxTopo topo, size_t nelems) {
-  constexpr int NN = N * N * N;
-  constexpr int CE = NN >= kThreads ? 1 : kThreads / NN;
-  constexpr int CN = CE * NN;
-  double *u[3] = {u0, u1, u2};
-  const double *acc[3] = {a0, a1, a2};
-  const double *kf[3] = {k0, k1, k2};
-  const size_t nchunks = (nelems + CE - 1) / CE;
-  const size_t cpb = (nchunks + gridDim.x - 1) / gridDim.x;
-  const size_t c0 = xcd_block() * cpb, c1 = c0 + cpb < nchunks ? c0 + cpb : nchunks;
-  int ecw[3] = {0, 0, 0};
-  if (CE == 1) gf::box_elem_coords(topo, c0, ecw);
-  for (size_t ch = c0; ch < c1; ch++) {
-    int ec0[3];
-    if (CE == 1) {
-      ec0[0] = ecw[0];
-      ec0[1] = ecw[1];
-      ec0[2] = ecw[2];
-      gf::box_elem_next(topo, ecw);
-    } else {
-      gf::box_elem_coords(topo, ch * CE, ec0);
-    }
-    const gf::BoxElemDeltas d0 = gf::box_elem_deltas(topo, N, ec0);
-#pragma unroll
-    for (int q0 = 0; q0 < CN; q0 += kThreads) {
-      const int q = q0 + (int)threadIdx.x;
-      if (q >= CN) break;
-      const int el = CE == 1 ? 0 : q / NN;
-      const int rr = CE == 1 ? q : q - el * NN;
-      const size_t e = ch * CE + el;
-      if (e >= nelems) break;
-      gf::BoxElemDeltas de = d0;
-      if (CE > 1 && el) {
-        int ec[3];
-        gf::box_elem_coords(topo, e, ec);
-        de = gf::box_elem_deltas(topo, N, ec);
-      }
-      const int i = rr % N, j = (rr / N) % N, k = rr / (N * N);
-      const I g = (I)(e * NN + rr);
-      I mem[8];
-      const int cnt = gf::box_members<I>(de, N, g, i, j, k, mem);
-      // every load of the node (all components) before the first store;
-      // absent group members are not read
-      double kv[3][8], av[3];
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        gf::box_load8m<I, double>(kf[c], mem, cnt, kv[c]);
-        av[c] = acc[c][g];
-      }
-#pragma unroll
-      for (int c = 0; c < 3; c++) {
-        const double ks =
-            cnt == 1 ? kv[c][0] : gf::box_sum8z<double>(kv[c], cnt) * gf::box_inv(cnt);
-        u[c][g] = 1.0 * av[c] + cl * ks;
-      }
-    }
-  }
-}
-
-// Step output on an N = 8 box through the LDS halo: one element per
-// 64-thread block; per component the element's K and accumulator are copied
-// to LDS (lds_copy512) while its partner values are loaded into
-// registers (gf::Halo8Rim), and each node sums its group from LDS in canonical order
-// (gf::halo8_order) -- k_rk_out_box's operations, the same result bit for
-// bit, with every K value fetched once instead of once per group copy.
+// Step output on a structured box: u = S(acc), the Smooth by gather through
+// the LDS halo, with the operations of the fused form (IN 3 above).
 template <int N>
-__global__ __launch_bounds__(64) void k_rk_out_halo8(
+__global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_rk_out_halo(
     double *__restrict__ u0, double *__restrict__ u1, double *__restrict__ u2,
     const double *__restrict__ a0, const double *__restrict__ a1, const double *__restrict__ a2,
-    const double *__restrict__ k0, const double *__restrict__ k1, const double *__restrict__ k2,
-    double cl, gf::BoxTopo topo, size_t nelems) {
-  // K's halo, then the accumulator's own values
-  __shared__ double sl[gf::kHalo8 + 512];
-  double *hk = sl, *ha = sl + gf::kHalo8;
+    gf::BoxTopo topo, size_t nelems) {
+  using S = gf::Pen3<N>;
+  using H = gf::Halo<N>;
+  __shared__ double sl[S::EPB * H::SIZE];
   double *u[3] = {u0, u1, u2};
   const double *acc[3] = {a0, a1, a2};
-  const double *kf[3] = {k0, k1, k2};
-  const size_t e = xcd_block();
-  if (e >= nelems) return;  // the whole block
-  const int lane = (int)threadIdx.x;
+  ColIdx<N> t(nelems);
+  double *hk = sl + t.el * H::SIZE;
+  const int l = t.r;
+  const int64_t ebase = (int64_t)t.e * S::NN;
   int ec[3];
-  gf::box_elem_coords(topo, e, ec);
-  static_assert(N == 8, "the LDS halo serves N = 8");
-  const gf::BoxElemDeltas de = gf::box_elem_deltas(topo, 8, ec);
-  const gf::Halo8Col hc(de, lane & 7, lane >> 3);
-  const int64_t ebase = (int64_t)e * 512;
+  gf::box_elem_coords(topo, t.e, ec);
+  const gf::BoxElemDeltas de = gf::box_elem_deltas(topo, N, ec);
+  const gf::HaloCol<N> hc(de, t.i, t.j);
   gf::static_for<0, 3>([&](auto cc) {
     constexpr int c = decltype(cc)::value;
     __syncthreads();  // the previous component's sums have read LDS
-    // own values straight to LDS, the partner values through registers
-    lds_copy512(kf[c] + ebase, hk, lane);
-    lds_copy512(acc[c] + ebase, ha, lane);
-    gf::Halo8Rim<double> L;
-    L.issue(kf[c], de, ebase, lane);
-    L.store(hk, lane);
-    __syncthreads();
-    gf::static_for<0, 8>([&](auto kc) {
-      constexpr int k = decltype(kc)::value;
-      constexpr int NT = (k == 0 || k == 7) ? 8 : 4;  // terms that can be non-zero
-      const int own = lane + 64 * k;
-      int ad[8];
-      const int cnt = gf::halo8_order<k>(hc, de, ad);
-      double sk = 0.0;
+    gf::HaloRim<N, double> L;
+    if constexpr (N == 8) {
+      lds_copy512(acc[c] + ebase, hk, l);
+      L.issue(acc[c], de, ebase, l);
+    } else {
+      double ao[N];
 #pragma unroll
-      for (int m = 0; m < NT; m++) sk = sk + hk[ad[m]];
-      const double ks = cnt == 1 ? hk[own] : sk * gf::box_inv(cnt);
-      u[c][ebase + own] = 1.0 * ha[own] + cl * ks;
+      for (int k = 0; k < N; k++) ao[k] = acc[c][ebase + l + S::N2 * k];
+      L.issue(acc[c], de, ebase, l);
+#pragma unroll
+      for (int k = 0; k < N; k++) hk[l + S::N2 * k] = ao[k];
+    }
+    L.store(hk, l);
+    __syncthreads();
+    gf::static_for<0, N>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      constexpr bool ZF = k == 0 || k == N - 1;
+      int ad[8];
+      const int cnt = gf::halo_order<N, k>(hc, de, ad);
+      double s = (hk[ad[0]] + hk[ad[1]]) + (hk[ad[2]] + hk[ad[3]]);
+      if (ZF) s = s + ((hk[ad[4]] + hk[ad[5]]) + (hk[ad[6]] + hk[ad[7]]));
+      if (t.active) u[c][ebase + l + S::N2 * k] = s * gf::box_inv(cnt);
     });
   });
 }
 
-template <int N, bool KP, int ACC, bool SMV, bool HL>
-void launch_stage3b_h(gf_mesh *m, int nb, double *const *uin, double *const *kp,
-                      double *const *acc, double *const *kout, double bh, double ch, double nu) {
+template <int N, int IN, int ACC>
+int launch_stage3b_h(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
+                     double *const *kout, double bh, double ca, double cb, double nu) {
   using S = gf::Pen3<N>;
-  hipLaunchKernelGGL((k_burgers_stage3b<N, KP, ACC, SMV, HL>), dim3(nb), dim3(S::THREADS), 0,
-                     m->ctx->stream, uin[0], uin[1], uin[2], kp ? kp[0] : nullptr,
-                     kp ? kp[1] : nullptr, kp ? kp[2] : nullptr, acc ? acc[0] : nullptr,
-                     acc ? acc[1] : nullptr, acc ? acc[2] : nullptr, kout[0], kout[1], kout[2],
-                     m->imass_el ? m->imass_el : m->imass, m->W[0], m->edx, m->ejac, pend_d(m),
-                     bh, ch, nu, m->box, m->nelems, m->imass_el ? (size_t)0 : (size_t)S::NN);
-}
-
-// The N = 8 gather through the LDS halo where the box's partner offsets
-// order x < y < z (gf_mesh::halo8), else the per-node gather.
-template <int N, bool KP, int ACC, bool SMV>
-void launch_stage3b_v(gf_mesh *m, int nb, double *const *uin, double *const *kp,
-                      double *const *acc, double *const *kout, double bh, double ch, double nu) {
-  if constexpr (N == 8 && KP) {
-    if (m->halo8) {
-      launch_stage3b_h<N, KP, ACC, SMV, true>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-      return;
-    }
-  }
-  launch_stage3b_h<N, KP, ACC, SMV, false>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-}
-
-template <int N>
-int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
-                   double *const *kout, double bh, double ch, double nu, int acc_mode,
-                   int smooth_v) {
-  using S = gf::Pen3<N>;
-  int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
-  if (!kp)
-    launch_stage3b_v<N, false, 0, false>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-  else if (acc_mode == 1 && !smooth_v)
-    launch_stage3b_v<N, true, 1, false>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-  else if (acc_mode == 2 && !smooth_v)
-    launch_stage3b_v<N, true, 2, false>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-  else if (acc_mode == 1 && smooth_v)
-    launch_stage3b_v<N, true, 1, true>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-  else if (acc_mode == 2 && smooth_v)
-    launch_stage3b_v<N, true, 2, true>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-  else if (acc_mode == 3 && !smooth_v)
-    launch_stage3b_v<N, true, 3, false>(m, nb, uin, kp, acc, kout, bh, ch, nu);
-  else
-    return gf_set_err(m->ctx, GF_ERR_ARG, "stage3b: unsupported stage form");
+  const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
+  auto at = [](double *const *p, int c) { return p ? p[c] : nullptr; };
+  hipLaunchKernelGGL((k_burgers_stage3b<N, IN, ACC>), dim3(nb), dim3(S::THREADS), 0,
+                     m->ctx->stream, at(uin, 0), at(uin, 1), at(uin, 2), at(kp, 0), at(kp, 1),
+                     at(kp, 2), at(acc, 0), at(acc, 1), at(acc, 2), at(kout, 0), at(kout, 1),
+                     at(kout, 2), m->imass_el ? m->imass_el : m->imass, m->W[0], m->edx, m->ejac,
+                     pend_d(m), bh, ca, cb, nu, m->box, m->nelems,
+                     m->imass_el ? (size_t)0 : (size_t)S::NN);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
 
 template <int N>
-int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc, double *const *kf,
-                      double cl) {
-  if constexpr (N == 8) {
-    if (m->halo8) {
-      hipLaunchKernelGGL(k_rk_out_halo8<N>, dim3(xcd_grid(m->nelems)), dim3(64), 0, m->ctx->stream,
-                         u[0], u[1], u[2], acc[0], acc[1], acc[2], kf[0], kf[1], kf[2], cl,
-                         m->box, m->nelems);
-      GF_LAUNCH_CHECK(m->ctx);
-      return GF_OK;
-    }
-  }
-  constexpr int NN = N * N * N;
-  constexpr int CE = NN >= kThreads ? 1 : kThreads / NN;
-  size_t nchunks = (m->nelems + CE - 1) / CE;
-  int nb = xcd_grid(std::min<size_t>(nchunks, 8192));
-  if (m->ndof < ((size_t)1 << 31))
-    hipLaunchKernelGGL((k_rk_out_box<N, int32_t>), dim3(nb), dim3(kThreads), 0, m->ctx->stream,
-                       u[0], u[1], u[2], acc[0], acc[1], acc[2], kf[0], kf[1], kf[2], cl, m->box,
-                       m->nelems);
-  else
-    hipLaunchKernelGGL((k_rk_out_box<N, int64_t>), dim3(nb), dim3(kThreads), 0, m->ctx->stream,
-                       u[0], u[1], u[2], acc[0], acc[1], acc[2], kf[0], kf[1], kf[2], cl, m->box,
-                       m->nelems);
+int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
+                   double *const *kout, double bh, double ca, double cb, double nu, int in,
+                   int accm) {
+#define GF_STAGE(I, A) \
+  if (in == I && accm == A) return launch_stage3b_h<N, I, A>(m, uin, kp, acc, kout, bh, ca, cb, nu)
+  GF_STAGE(0, 0);
+  GF_STAGE(3, 0);
+  GF_STAGE(1, 0);
+  GF_STAGE(1, 1);
+  GF_STAGE(1, 2);
+  GF_STAGE(1, 3);
+  GF_STAGE(2, 2);
+  GF_STAGE(2, 3);
+#undef GF_STAGE
+  return gf_set_err(m->ctx, GF_ERR_ARG, "stage3b: unsupported stage form");
+}
+
+template <int N>
+int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc) {
+  using S = gf::Pen3<N>;
+  hipLaunchKernelGGL(k_rk_out_halo<N>, dim3(xcd_grid((m->nelems + S::EPB - 1) / S::EPB)),
+                     dim3(S::THREADS), 0, m->ctx->stream, u[0], u[1], u[2], acc[0], acc[1], acc[2],
+                     m->box, m->nelems);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
@@ -1093,9 +943,8 @@ int launch_update_box_n(gf_mesh *m, CGVecs<T> &v, double *part) {
   template int launch_advect3p<N>(gf_mesh *, const double *, const double *const *, double *); \
   template int launch_grad3p<N>(gf_mesh *, const double *, double *const *, const double *);  \
   template int launch_stage3b<N>(gf_mesh *, double *const *, double *const *, double *const *, \
-                                 double *const *, double, double, double, int, int);         \
-  template int launch_rk_out_box<N>(gf_mesh *, double *const *, double *const *,              \
-                                    double *const *, double);                                \
+                                 double *const *, double, double, double, double, int, int); \
+  template int launch_rk_out_box<N>(gf_mesh *, double *const *, double *const *);             \
   template int helm3c_d<N>(gf_mesh *, double, const double *, const double *, double,         \
                            const double *, double *);                                        \
   template int helm3c_f<N>(gf_mesh *, float, const float *, float, const float *, float *);   \

@@ -1031,7 +1031,7 @@ int gf_mesh_create(gf_ctx *ctx, const gf_mesh_desc *d, gf_mesh **out) {
     m->has_box = ok;
     m->has_box_mask = ok && mask_ok;
   }
-  // the LDS-halo gather of the N = 8 stage kernels (gf::box_halo8_ok)
+  // whether the halo's canonical order is GGFX's (gf::box_halo8_ok)
   m->halo8 = m->has_box && m->Niso == 8 && gf::box_halo8_ok(m->box);
   m->red_cap = gf_red_need(m->nelems);
   GF_HIP(ctx, hipMalloc((void **)&m->red, m->red_cap * sizeof(double)));

@@ -58,10 +58,15 @@ __device__ __forceinline__ void gll_apply_eo(const T (&x)[N], T (&y)[N]) {
   constexpr int H = N / 2;
   auto A = [](int l, int m) { return TR ? GllD<N>::at(m, l) : GllD<N>::at(l, m); };
   T e[H], o[H];
+  {
+    // x may be products: a sum of two products has two contracted forms that
+    // round differently, and the choice may vary from kernel to kernel
+#pragma clang fp contract(off)
 #pragma unroll
-  for (int m = 0; m < H; m++) {
-    e[m] = x[m] + x[N - 1 - m];
-    o[m] = x[m] - x[N - 1 - m];
+    for (int m = 0; m < H; m++) {
+      e[m] = x[m] + x[N - 1 - m];
+      o[m] = x[m] - x[N - 1 - m];
+    }
   }
 #pragma unroll
   for (int l = 0; l < H; l++) {

@@ -895,7 +895,7 @@ static int rhs_fused(gf_mesh *m, double nu, const double *const *u, double *cons
     double *in[3] = {const_cast<double *>(u[0]), const_cast<double *>(u[1]),
                      const_cast<double *>(u[2])};
     return GF_DISPATCH_N3(m->Niso, launch_stage3b, m, in, (double *const *)nullptr,
-                          (double *const *)nullptr, dudt, 0.0, 0.0, nu, 0, 0);
+                          (double *const *)nullptr, dudt, 0.0, 0.0, 0.0, nu, 0, 0);
   }
   StageArgs a;
   memset(&a, 0, sizeof(a));
@@ -1114,14 +1114,16 @@ int rk_step_fused(gf_mesh *m, double nu, int order, double dt, double *const *u)
   return GF_OK;
 }
 
-// RK steps on a structured box (order >= 2): the same arithmetic as
-// rk_step_fused, with every Smooth done by gather inside the stage kernels
-// and the output kernel.  Per step: `order` stage kernels and one output
-// kernel, no DSS passes.  Between consecutive steps the output kernel and the
-// next step's first stage are one kernel (acc_mode 3), which computes the
-// output value with the output kernel's operations, stores it and continues
-// with it as the stage input, so n steps give the same bits as n single
-// steps.
+// RK steps on a structured box (order >= 2): step_b with every Smooth formed
+// by gather inside the stage kernels (k_burgers_stage3b) and the output
+// kernel, no DSS passes.  The accumulator uin + sum_s c_s h K_s is advanced
+// by two stage derivatives at a time, in the stages 1, 3 (and the last one);
+// its Smooth, the step output, is formed by the output kernel or, between
+// consecutive steps, by the next step's first stage with the same
+// operations, so n steps give the same bits as n single steps.  The state
+// the caller passes may be discontinuous, so the first step smooths its
+// final-stage input as step_b does; from then on the state is continuous,
+// that Smooth is the identity bit for bit and is not formed.
 int rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps, double *const *u) {
   size_t bytes = m->ndof * sizeof(double);
   double alpha[4], beta[16], c[4];
@@ -1134,30 +1136,25 @@ int rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps, double
   }
   const double h = dt;
   const int ns = order;
-  int kb = 0;  // buffer of the current step's first stage derivative
-  bool have_k0 = false;
+  double *const *none = nullptr;
   for (int n = 0; n < nsteps; n++) {
-    // stage 1 from the state itself (unless the previous step's output
-    // kernel formed it)
-    if (!have_k0)
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, u, (double *const *)nullptr,
-                        (double *const *)nullptr, K[kb], 0.0, 0.0, nu, 0, 0));
-    // middle stages and the final stage (whose input is smoothed)
+    // stage 0: from the state, or from the previous step's accumulator
+    // (whose Smooth is stored as the state)
+    if (n == 0)
+      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, u, none, none, K[0], 0.0, 0.0, 0.0, nu, 0, 0));
+    else
+      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, none, acc, u, K[0], 0.0, 0.0, 0.0, nu, 3, 0));
     for (int s = 1; s < ns; s++) {
       const bool last = s == ns - 1;
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, u, K[(kb + s - 1) % 2], acc, K[(kb + s) % 2],
-                        beta[s * 4 + (s - 1)] * h, c[s - 1] * h, nu, s == 1 ? 1 : 2, last ? 1 : 0));
-    }
-    const int kl = (kb + ns - 1) % 2;
-    if (n + 1 < nsteps) {
-      kb = (kl + 1) % 2;
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, acc, K[kl], u, K[kb], c[ns - 1] * h, 0.0, nu,
-                        3, 0));
-      have_k0 = true;
-    } else {
-      RC(GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, u, acc, K[kl], c[ns - 1] * h));
+      // accumulate K_{s-1} and K_s at odd s; a last stage at even s adds K_s
+      const bool odd = s % 2 == 1;
+      const int accm = last ? (s == 1 ? 2 : 3) : (s == 1 ? 1 : 0);
+      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, u, K[(s - 1) % 2], acc, K[s % 2],
+                        beta[s * 4 + (s - 1)] * h, odd ? c[s - 1] * h : 0.0, c[s] * h, nu,
+                        last && n == 0 ? 2 : 1, accm));
     }
   }
+  if (nsteps > 0) RC(GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, u, acc));
   return GF_OK;
 }
 
@@ -2559,20 +2556,20 @@ extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *a
     else
       launch = [&]() { return GF_DISPATCH_N3(m->Niso, cgapply3c_d, m, ca3); };
   } else if (w == "rk_out_box") {
-    // structured-box step output: reads acc and K (both gathered), writes u
+    // structured-box step output: reads acc (gathered), writes u
     if (m->dim != 3 || !m->has_box)
       return gf_set_err(m->ctx, GF_ERR_UNSUPPORTED, "rk_out_box timing: structured 3-D boxes");
     launch = [&]() {
-      return GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, buf, buf + 6, buf + 9, 1e-5 / 6.0);
+      return GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, buf, buf + 6);
     };
   } else if (w == "burgers_stage_box") {
-    // structured-box stage, middle-stage form: reads uin, K_prev (gathered),
-    // acc; writes acc, K (5 fields per component)
+    // structured-box stage, second-stage form: reads uin, K_prev (gathered);
+    // writes acc, K (4 fields per component)
     if (m->dim != 3 || !m->has_box)
       return gf_set_err(m->ctx, GF_ERR_UNSUPPORTED, "burgers_stage_box timing: structured 3-D boxes");
     launch = [&]() {
       return GF_DISPATCH_N3(m->Niso, launch_stage3b, m, buf, buf + 3, buf + 6, buf + 9, 0.5e-5,
-                            1e-5 / 3.0, 0.02, 2, 0);
+                            1e-5 / 6.0, 1e-5 / 3.0, 0.02, 1, 1);
     };
   } else if (w == "cg_update" || w == "cg_update_f32") {
     // CG update with the Jacobi preconditioner: x, w, r, q (the diagonal

@@ -248,11 +248,10 @@ template <int N>
 int launch_grad3p(gf_mesh *m, const double *p, double *const *o, const double *edx);
 template <int N>
 int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
-                   double *const *kout, double bh, double ch, double nu, int acc_mode,
-                   int smooth_v);
+                   double *const *kout, double bh, double ca, double cb, double nu, int in,
+                   int accm);
 template <int N>
-int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc, double *const *kf,
-                      double cl);
+int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc);
 template <int N>
 int helm3c_d(gf_mesh *m, double p, const double *pf, const double *qf, double qs, const double *u,
              double *uo);

@@ -242,9 +242,9 @@ size_t gf_mesh_ndof(const gf_mesh *mesh);
  * GF_MESH_BOX_MASK    the boundary mask is formed from the box faces;
  * GF_MESH_CONST_D     3-D regular mesh whose D is the standard GLL matrix, so the
  *                     pencil kernels (D as compile-time constants) are used;
- * GF_MESH_BOX_HALO    p = 7 structured box whose RK stages gather the previous
- *                     stage derivative through an LDS halo of each element
- *                     (same results as the per-node gather);
+ * GF_MESH_BOX_HALO    p = 7 structured box on which the order of the group sums
+ *                     formed from an element's LDS halo (lower side first in
+ *                     z, y, x) is GGFX's member order;
  * GF_MESH_IMASS_ELEM  3-D regular mesh whose inverse mass is the same at every
  *                     element bit for bit (uniform periodic boxes), so the RK
  *                     stages read one element's values. */
