@@ -97,6 +97,11 @@ struct gf_mesh_s {
   std::vector<int> h_seg_boff;      // nseg+1 update-block offsets (host)
   int64_t *seg_eoff = nullptr;      // device copies of the two
   int *seg_boff = nullptr;
+  // the members' boxes when the members are the boxes of box_list (then the
+  // CG update gathers), and the boxes as given at creation (host)
+  gf::BoxTopo *seg_topo = nullptr;
+  std::vector<gf::BoxTopo> h_boxes;
+  double cg_epoch = 0.0;            // number of the CG loop (done flags in the mirrors)
   double *sscal = nullptr;          // per-member solver scalars (device)
   double *hsscal = nullptr, *hsscal_dev = nullptr;  // mapped host mirror of sscal
   std::vector<int> seg_iters;       // last solve: iterations per member
@@ -158,7 +163,3 @@ enum {
   WS_ADJ_BEGIN = 96,        // adjoint stage states and cotangents (up to 36 slots)
   WS_ADJ_CKPT = 160         // adjoint checkpoints and segment states
 };
-
-// Reduction partials a mesh needs: one per apply block (at most one block
-// per element) plus the update kernels' pairs.
-size_t gf_red_need(size_t nelems);

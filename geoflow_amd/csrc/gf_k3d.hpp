@@ -49,94 +49,118 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_helm3p(
                            gf::NoPenCB(), gf::NoPenCB(), gf::NoPenCB(), post);
 }
 
-template <int N, typename T>
-__global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_cg_apply3p(
-    const T *__restrict__ r, const T *__restrict__ dinv, T *__restrict__ w, T *__restrict__ qv,
-    gf::PenD<T> Dp, const T *__restrict__ W, const T *__restrict__ edx,
-    const T *__restrict__ ejac, const T *__restrict__ qf, T qs, const T *__restrict__ mask, double pd,
-    const double *__restrict__ scal, double *__restrict__ part, size_t nelems, gf::BoxTopo topo,
-    int tmask, const int64_t *__restrict__ seg_eoff, int nseg, const double *__restrict__ sscal,
-    const T *__restrict__ dtab, const unsigned char *__restrict__ deq) {
+// CG apply (see CGCtl), 3-D pencil form: x += alpha w, w = z + beta w, then
+// q = A w on the element (unassembled) and the partial sums of w.q.  Because
+// w is continuous and zero where masked, sum_j w_j (DSS q)_j imult_j equals
+// sum_j w_j q_j over local nodes, so the dot product of gcg.ipp:307-308 is
+// formed before the assembly; the Dirichlet mask is applied to q here (it is
+// constant over each coincidence group, so DSS(q) mask = DSS(q mask)).
+// NT: x and w, which this kernel alone reads and writes, bypass the caches
+// (see launch_cg_apply3p).
+template <int N, typename T, bool NT>
+__global__ __launch_bounds__(kThreads) void k_cg_apply3p(CGApply3Args a) {
   using S = gf::Pen3<N>;
-  __shared__ T su[S::EPB][S::SZ], sd[S::EPB][S::SZ];
-  __shared__ double sred[S::THREADS > 64 ? S::THREADS : 64];
-  ColIdx<N> t(nelems);
-  // batched mesh: each element's member scalars; an element of a member
-  // that has converged computes nothing it stores, and the partial sums are
-  // kept per element so that each member's are one contiguous range
-  if (nseg > 0) {
-    scal = sscal + kSegScal * seg_of(seg_eoff, nseg, t.e);
-    if (scal[S_DONE] != 0.0) {
-      if (S::EPB == 1) return;  // the whole workgroup
-      t.active = false;
+  using C = CGShape<N>;
+  __shared__ T sl[C::EPB][2][S::SZ];
+  __shared__ double sred[2 * (kThreads / 64)];
+  const CGBlock b(a.c, (int)xcd_block(), a.c.nbA);
+  if (!b.ok) return;
+  const T *__restrict__ r = (const T *)a.r, *__restrict__ dinv = (const T *)a.dinv;
+  const T *__restrict__ dtab = (const T *)a.dtab, *__restrict__ W = (const T *)a.W;
+  const T *__restrict__ edx = (const T *)a.edx, *__restrict__ ejac = (const T *)a.ejac;
+  const T *__restrict__ qf = (const T *)a.qf, *__restrict__ mask = (const T *)a.mask;
+  T *__restrict__ x = (T *)a.x, *__restrict__ w = (T *)a.w, *__restrict__ qv = (T *)a.q;
+  const C t;
+  const T p = (T)a.p, qs = (T)a.qs;
+  CGHead h(a.c, b);
+  T rv[N], dv[N], wv[N], xv[N], jac, f0, f1, f2;
+  size_t e, col;
+  bool act;
+  // the element of a chunk: all its loads; the Jacobi values from the table
+  // where the element's equal it
+  auto load = [&](int64_t c) {
+    const size_t eg = b.e0 + (size_t)c * C::EPB + t.el;
+    act = t.own() && eg < b.e1;
+    e = eg < b.e1 ? eg : b.e1 - 1;
+    col = e * S::NN + t.r;
+    const T *dsrc = dinv ? ((dtab && a.deq[e]) ? dtab + t.r : dinv + col) : nullptr;
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+      const size_t g = col + q * S::N2;
+      rv[q] = r[g];
+      wv[q] = NT ? __builtin_nontemporal_load(w + g) : w[g];
+      xv[q] = NT ? __builtin_nontemporal_load(x + g) : x[g];
     }
-  } else if (scal[S_DONE] != 0.0) {
-    return;
-  }
-  const bool first = scal[S_FIRST] != 0.0;
-  const T beta = (T)scal[S_BETA];
-  const size_t col = t.e * S::NN + t.r;
-  const T jac = ejac[t.e];
-  const T f0 = edx[t.e * 3], f1 = edx[t.e * 3 + 1], f2 = edx[t.e * 3 + 2];
-  // all loads of the column first, then the stores of w; the Jacobi values
-  // from the table where the element's equal it
-  const T *dsrc = dinv ? ((dtab && deq[t.e]) ? dtab + t.r : dinv + col) : nullptr;
-  T ru[N], dv[N], wv[N];
 #pragma unroll
-  for (int k = 0; k < N; k++) {
-    const size_t g = col + k * S::N2;
-    ru[k] = r[g];
-    dv[k] = dsrc ? dsrc[k * S::N2] : T(1);
-    wv[k] = first ? T(0) : w[g];
-  }
-#pragma unroll
-  for (int k = 0; k < N; k++) {
-    const T z = dinv ? dv[k] * ru[k] : ru[k];
-    ru[k] = first ? z : beta * wv[k] + T(1) * z;
-  }
-  if (t.active) {
-#pragma unroll
-    for (int k = 0; k < N; k++) w[col + k * S::N2] = ru[k];
-  }
-  double dot = 0.0;
-  const T p = (T)pd;
-  int ec[3] = {0, 0, 0};
-  if (tmask) gf::box_elem_coords(topo, t.e, ec);
-  auto post = [&](int k, T Lu, T M, T, T) {
-    if (!t.active) return;
-    const size_t g = col + k * S::N2;
-    T acc = Lu;
-    if (p != T(1)) acc *= p;
-    if (qf) {
-      T tq = M * ru[k];
-      tq *= qf[g];
-      acc += tq;
-    } else if (qs != T(0)) {
-      T tq = M * ru[k];
-      if (qs != T(1)) tq *= qs;
-      acc += tq;
-    }
-    if (mask) acc *= mask[g];
-    else if (tmask && gf::box_masked(topo, N, ec, t.i, t.j, k)) acc *= T(0);
-    qv[g] = acc;
-    dot += (double)ru[k] * (double)acc;
+    for (int q = 0; q < N; q++) dv[q] = dsrc ? dsrc[q * S::N2] : T(1);
+    jac = ejac[e];
+    f0 = edx[e * 3];
+    f1 = edx[e * 3 + 1];
+    f2 = edx[e * 3 + 2];
   };
-  gf::pen_op3<N, T, false>(ru, su[t.el], sd[t.el], (T *)nullptr, Dp, W, t.i, t.j, W[t.i],
-                           W[t.j], jac, f0 * f0, f1 * f1, f2 * f2, (const T *)nullptr,
-                           gf::NoPenCB(), gf::NoPenCB(), gf::NoPenCB(), post);
-  if (nseg > 0) {
-    // per-element partials: the element's lanes, summed in lane order
-    sred[threadIdx.x] = dot;
-    __syncthreads();
-    if (t.r == 0 && t.active) {
-      double v = 0.0;
-      for (int q2 = 0; q2 < S::N2; q2++) v += sred[t.el * S::N2 + q2];
-      part[t.e] = v;
+  CGWalk k(a.c, b, C::EPB, false);
+  if (k.in()) load(k.c);
+  const T wi = W[t.i], wj = W[t.j];
+  h.finish(a.c, b, sred);
+  if (!h.run) return;
+  const T beta = (T)h.beta, alpha = (T)h.alpha;
+  double dot = 0.0;
+  while (k.in()) {
+    T ru[N];
+    const size_t ce = e, cc = col;
+    const bool ca = act;
+    const T cj = jac, c0 = f0 * f0, c1 = f1 * f1, c2 = f2 * f2;
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+      const T z = dinv ? dv[q] * rv[q] : rv[q];
+      ru[q] = h.first ? z : beta * wv[q] + z;
     }
-    return;
+    if (ca) {
+#pragma unroll
+      for (int q = 0; q < N; q++) {
+        const size_t g = cc + q * S::N2;
+        const T xn = xv[q] + alpha * wv[q];
+        if (!a.c.init) {
+          if (NT) __builtin_nontemporal_store(xn, x + g);
+          else x[g] = xn;
+        }
+        if (!h.xonly) {
+          if (NT) __builtin_nontemporal_store(ru[q], w + g);
+          else w[g] = ru[q];
+        }
+      }
+    }
+    k.next();
+    if (k.in()) load(k.c);  // in flight while this element is worked
+    if (h.xonly) continue;
+    int ec[3] = {0, 0, 0};
+    if (a.tmask) gf::box_elem_coords(a.topo, ce, ec);
+    auto post = [&](int q, T Lu, T M, T, T) {
+      if (!ca) return;
+      const size_t g = cc + q * S::N2;
+      T acc = Lu;
+      if (p != T(1)) acc *= p;
+      if (qf) {
+        T tq = M * ru[q];
+        tq *= qf[g];
+        acc += tq;
+      } else if (qs != T(0)) {
+        T tq = M * ru[q];
+        if (qs != T(1)) tq *= qs;
+        acc += tq;
+      }
+      if (mask) acc *= mask[g];
+      else if (a.tmask && gf::box_masked(a.topo, N, ec, t.i, t.j, q)) acc *= T(0);
+      qv[g] = acc;
+      dot += (double)ru[q] * (double)acc;
+    };
+    gf::pen_op3<N, T, false, C::WAVE>(ru, sl[t.el][0], sl[t.el][1], (T *)nullptr, gf::PenD<T>(), W,
+                                      t.i, t.j, wi, wj, cj, c0, c1, c2, (const T *)nullptr,
+                                      gf::NoPenCB(), gf::NoPenCB(), gf::NoPenCB(), post, t.own());
   }
-  double bs = gf::block_reduce<false>(dot, sred);
-  if (threadIdx.x == 0) part[blockIdx.x] = bs;
+  if (h.xonly) return;
+  const double bs = gf::block_reduce<false>(dot, sred);
+  if (threadIdx.x == 0) a.c.partA[b.b0 + b.lb] = bs;
 }
 
 // Fused Burgers stage, 3-D pencil form (see k_burgers_stage for the contract).
@@ -597,25 +621,30 @@ int launch_helm3p(gf_mesh *m, T p, const T *pf, const T *qf, T qs, const T *u, T
   return GF_OK;
 }
 
+// Blocks of the 3-D CG kernels: as many as are resident at once (FP64 8
+// waves a CU by registers, FP32 16).  Twice as many in FP64: 20^3, p = 6
+// 76 us an iteration against 71, 16^3, p = 7 50 against 43.
+template <typename T, int N>
+int cg_blocks3(size_t nelems) {
+  constexpr int EPB = CGShape<N>::EPB;
+  return loop_blocks((nelems + EPB - 1) / EPB, sizeof(T) == 8 ? 512 : 1024);
+}
+
+// stream: the solve's vectors do not fit the 256 MB Infinity Cache.  Then x
+// and w, read and written by this kernel only, are marked non-temporal, so
+// that the cache keeps r and q for the update kernel (which walks backwards).
 template <int N, typename T>
 int launch_cg_apply3p(gf_mesh *m, const CGApply3Args &a) {
-  using S = gf::Pen3<N>;
-  int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
-  gf::PenD<T> Dp;
-  for (int c = 0; c < 3; c++) {
-    Dp.R[c] = (const T *)a.DR[c];
-    Dp.C[c] = (const T *)a.DC[c];
-  }
-  hipLaunchKernelGGL((k_cg_apply3p<N, T>), dim3(nb), dim3(S::THREADS), 0, m->ctx->stream,
-                     (const T *)a.r, (const T *)a.dinv, (T *)a.w, (T *)a.q, Dp, (const T *)a.W,
-                     (const T *)a.edx, (const T *)a.ejac, (const T *)a.qf, (T)a.qs, (const T *)a.mask, a.p,
-                     (const double *)a.scal, a.part, a.nelems, a.topo, a.tmask, a.seg_eoff, a.nseg,
-                     (const double *)a.sscal, (const T *)a.dtab, a.deq);
+  if (a.c.stream)
+    hipLaunchKernelGGL((k_cg_apply3p<N, T, true>), dim3(a.c.nbA), dim3(kThreads), 0, m->ctx->stream,
+                       a);
+  else
+    hipLaunchKernelGGL((k_cg_apply3p<N, T, false>), dim3(a.c.nbA), dim3(kThreads), 0,
+                       m->ctx->stream, a);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
 
-// Number of workgroups (= partial sums) the 3-D column apply launches.
 template <int N>
 int helm3c_d(gf_mesh *m, double p, const double *pf, const double *qf, double qs, const double *u,
              double *uo) {
@@ -631,312 +660,105 @@ int cgapply3c_d(gf_mesh *m, const CGApply3Args &a) { return launch_cg_apply3p<N,
 template <int N>
 int cgapply3c_f(gf_mesh *m, const CGApply3Args &a) { return launch_cg_apply3p<N, float>(m, a); }
 
-// u3 = uin + bh*k ; acc = accsrc + ch*k   (final-stage input of step_b, :315-320)
-
-// k_cg_update on a structured box: q arrives unassembled (straight from the
-// apply) and is assembled here by gather (gf_boxdss.hpp), in the GGFX order,
-// so no DSS pass runs between the apply and the update.  The multiplicity
-// weight is 1/(group size), which equals GGFX::get_imult.  Work is split in
-// chunks of whole elements so that an element's box coordinates are formed
-// once per chunk (and are wave-uniform when a chunk is one element).
-template <typename T, int NORM, int N, typename I>
-__global__ __launch_bounds__(kThreads) void k_cg_update_box(
-    T *__restrict__ x, const T *__restrict__ w, T *__restrict__ r, const T *__restrict__ qv,
-    const T *__restrict__ dinv, const double *__restrict__ mass, gf::BoxTopo topo, double *scal,
-    double *__restrict__ part, size_t nelems) {
-  constexpr int NN = N * N * N;
-  constexpr int CE = NN >= kThreads ? 1 : kThreads / NN;  // elements per chunk
-  constexpr int CN = CE * NN;                              // nodes per chunk
-  constexpr int QPC = (CN + kThreads - 1) / kThreads;      // nodes per thread per chunk
-  // chunks per batch: every load of a batch is issued before its first
-  // store, so a batch should keep enough bytes in flight (FP32 takes two)
-  constexpr int BC = (sizeof(T) == 4 && QPC <= 2) ? 2 : 1;
-  constexpr int NQ = BC * QPC;
-  __shared__ double sred[kThreads / 64];
-  if (scal[S_DONE] != 0.0) return;
-  const T alpha = (T)scal[S_ALPHA];
-  double rho = 0.0, nrm = 0.0;
-  // each (XCD-renumbered) block walks a contiguous range of chunks
-  const size_t nchunks = (nelems + CE - 1) / CE;
-  const size_t cpb = (nchunks + gridDim.x - 1) / gridDim.x;
-  const size_t c0 = xcd_block() * cpb, c1 = c0 + cpb < nchunks ? c0 + cpb : nchunks;
-  // box coordinates of the walk's next element (chunks of one element)
-  int ecw[3] = {0, 0, 0};
-  if (CE == 1) gf::box_elem_coords(topo, c0, ecw);
-  for (size_t c = c0; c < c1; c += BC) {
-    I gs[NQ];
-    T dv[NQ], xo[NQ], wo[NQ], ro[NQ], qm[NQ][8];
-    int cnt[NQ];
-    bool ok[NQ];
-#pragma unroll
-    for (int bc = 0; bc < BC; bc++) {
-      const size_t cc = c + bc;
-      int ec0[3];
-      if (CE == 1) {
-        ec0[0] = ecw[0];
-        ec0[1] = ecw[1];
-        ec0[2] = ecw[2];
-        gf::box_elem_next(topo, ecw);
-      } else {
-        gf::box_elem_coords(topo, cc * CE, ec0);
-      }
-      const gf::BoxElemDeltas d0 = gf::box_elem_deltas(topo, N, ec0);  // uniform when CE == 1
-#pragma unroll
-      for (int qq = 0; qq < QPC; qq++) {
-        const int s = bc * QPC + qq;
-        const int q = qq * kThreads + (int)threadIdx.x;
-        const int el = CE == 1 ? 0 : q / NN;
-        const int rr = CE == 1 ? q : q - el * NN;
-        const size_t e = cc * CE + el;
-        ok[s] = cc < c1 && q < CN && e < nelems;
-        gf::BoxElemDeltas de = d0;
-        if (CE > 1 && el) {
-          int ec[3];
-          gf::box_elem_coords(topo, e, ec);
-          de = gf::box_elem_deltas(topo, N, ec);
-        }
-        const int i = rr % N, j = (rr / N) % N, k = rr / (N * N);
-        // out-of-range slots read node 0 (always valid) and are not stored
-        const I g = ok[s] ? (I)(e * NN + rr) : (I)0;
-        gs[s] = g;
-        I mem[8];
-        if (ok[s]) {
-          cnt[s] = gf::box_members<I>(de, N, g, i, j, k, mem);
-        } else {
-          cnt[s] = 1;
-#pragma unroll
-          for (int m2 = 0; m2 < 8; m2++) mem[m2] = (I)0;
-        }
-        dv[s] = dinv ? dinv[g] : T(1);
-        xo[s] = x[g];
-        wo[s] = w[g];
-        ro[s] = r[g];
-        gf::box_load8m<I, T>(qv, mem, cnt[s], qm[s]);
-      }
-    }
-#pragma unroll
-    for (int s = 0; s < NQ; s++) {
-      if (!ok[s]) continue;
-      const I g = gs[s];
-      const T qa = gf::box_sum8z<T>(qm[s], cnt[s]);
-      const T xv = (T)1 * xo[s] + alpha * wo[s];
-      x[g] = xv;
-      const T rv = (T)1 * ro[s] + (-alpha) * qa;
-      r[g] = rv;
-      const T z = dinv ? dv[s] * rv : rv;
-      const double im = gf::box_inv(cnt[s]);
-      rho += (double)rv * (double)z * im;
-      const double rd = (double)rv;
-      if (NORM == GF_NORM_INF) nrm = fmax(nrm, fabs(rd));
-      else if (NORM == GF_NORM_EUC) nrm += rd * rd;
-      else if (NORM == GF_NORM_L2) nrm += mass[g] * rd * rd;
-      else if (NORM == GF_NORM_L1) nrm += mass[g] * fabs(rd);
-      else nrm += rd * rd * im;
-    }
-  }
-  double a = gf::block_reduce<false>(rho, sred);
-  double b = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
-                                 : gf::block_reduce<false>(nrm, sred);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = a;
-    part[2 * blockIdx.x + 1] = b;
-  }
-}
-
-// 16-byte vector of T (4 floats or 2 doubles).
-template <typename T>
-struct Vec16;
-template <>
-struct Vec16<float> {
-  using V = float4;
-  static constexpr int R = 4;
-  __device__ static float get(const V &v, int n) {
-    return n == 0 ? v.x : (n == 1 ? v.y : (n == 2 ? v.z : v.w));
-  }
-  __device__ static void set(V &v, int n, float a) {
-    if (n == 0) v.x = a;
-    else if (n == 1) v.y = a;
-    else if (n == 2) v.z = a;
-    else v.w = a;
-  }
-};
-template <>
-struct Vec16<double> {
-  using V = double2;
-  static constexpr int R = 2;
-  __device__ static double get(const V &v, int n) { return n == 0 ? v.x : v.y; }
-  __device__ static void set(V &v, int n, double a) {
-    if (n == 0) v.x = a;
-    else v.y = a;
-  }
-};
-
-// True when k_cg_update_boxv handles order N in precision T: a node row
-// splits into at least two 16-byte runs and a workgroup holds whole elements.
-template <typename T, int N>
-constexpr bool boxv_ok() {
-  return N % Vec16<T>::R == 0 && N > Vec16<T>::R &&
-         kThreads % (N * N * N / Vec16<T>::R) == 0;
-}
-
-// k_cg_update_box with each lane working a run of R = 16/sizeof(T)
-// consecutive nodes along x (one 16-byte load or store per vector), so the
-// wave issues a quarter (FP32) or half (FP64) of the memory instructions.
-// The group of a node is the product of its partner choices per direction:
-// the run's y, z and yz partners are runs of the neighbouring elements at the
-// same x offset (16-byte loads), and only the run's first or last node can
-// have an x partner (scalar loads).  Members are summed in the order
-// (z side, y side, x side), lower side first, where the lower side of a
-// direction is the copy with the smaller global index; because the element
-// index dominates the global index, that order is the ascending order of the
-// group's global indices, GGFX's summation order (ggfx.hpp:346-443), so the
-// result equals k_cg_update_box's bit for bit.
-template <typename T, int NORM, int N, typename I>
-__global__ __launch_bounds__(kThreads) void k_cg_update_boxv(
-    T *__restrict__ x, const T *__restrict__ w, T *__restrict__ r, const T *__restrict__ qv,
-    const T *__restrict__ dinv, const double *__restrict__ mass, gf::BoxTopo topo, double *scal,
-    double *__restrict__ part, size_t nelems, const T *__restrict__ dtab,
-    const unsigned char *__restrict__ deq) {
-  using VT = Vec16<T>;
-  using V = typename VT::V;
-  constexpr int R = VT::R;
-  constexpr int NN = N * N * N;
-  constexpr int RPR = N / R;           // runs per node row
-  constexpr int RPE = NN / R;          // runs per element
-  constexpr int EPP = kThreads / RPE;  // elements per workgroup pass
-  __shared__ double sred[kThreads / 64];
-  if (scal[S_DONE] != 0.0) return;
-  const T alpha = (T)scal[S_ALPHA];
-  double rho = 0.0, nrm = 0.0;
-  const int el = (int)threadIdx.x / RPE, rr = (int)threadIdx.x - el * RPE;
-  const int ir = rr % RPR, j = (rr / RPR) % N, k = rr / (RPR * N);
-  const int i0 = ir * R;
-  // the run node that can have an x partner: the row's first or last node
-  const int xn = ir == 0 ? 0 : (ir == RPR - 1 ? R - 1 : -1);
-  const size_t npass = (nelems + EPP - 1) / EPP;
-  const size_t ppb = (npass + gridDim.x - 1) / gridDim.x;
-  const size_t c0 = xcd_block() * ppb, c1 = c0 + ppb < npass ? c0 + ppb : npass;
-  for (size_t c = c0; c < c1; c++) {
-    const size_t e = c * EPP + el;
-    if (e >= nelems) continue;
+// CG update on structured boxes (see CGCtl): q arrives unassembled, straight
+// from the apply, and is assembled here through the LDS halo of each element
+// (gf_boxdss.hpp), so no DSS pass runs in between; r -= alpha DSS(q), and the
+// partial sums of r.z / (group size) and of the norm.  All copies of a node
+// sum its group in the same order, so r stays continuous bit for bit.  topos:
+// the box of each system of a batched mesh.
+template <typename T, int NORM, int N>
+__global__ __launch_bounds__(kThreads) void k_cg_update_halo(
+    CGCtl c, T *__restrict__ r, const T *__restrict__ qv, const T *__restrict__ dinv,
+    const double *__restrict__ mass, gf::BoxTopo topo1, const gf::BoxTopo *__restrict__ topos,
+    const T *__restrict__ dtab, const unsigned char *__restrict__ deq) {
+  using S = gf::Pen3<N>;
+  using C = CGShape<N>;
+  using H = gf::Halo<N>;
+  __shared__ T sl[C::EPB][H::SIZE];
+  __shared__ double sred[2 * (kThreads / 64)];
+  const CGBlock b(c, (int)xcd_block(), c.nbU);
+  if (!b.ok) return;
+  CGAlphaHead h(c, b);
+  const gf::BoxTopo topo = topos ? topos[b.s] : topo1;
+  const C t;
+  T *hl = sl[t.el];
+  T qo[N], ro[N], dv[N];
+  gf::HaloRim<N, T> L;
+  gf::BoxElemDeltas de;
+  size_t col;
+  bool act;
+  auto load = [&](int64_t ch) {
+    const size_t el = (size_t)ch * C::EPB + t.el, nel = b.e1 - b.e0;
+    act = t.own() && el < nel;
+    const size_t le = el < nel ? el : nel - 1, e = b.e0 + le;
+    col = e * S::NN + t.r;
     int ec[3];
-    gf::box_elem_coords(topo, e, ec);
-    const gf::BoxElemDeltas d = gf::box_elem_deltas(topo, N, ec);
-    const I g0 = (I)(e * NN) + (I)(k * N * N + j * N + i0);
-    const I dy = j == 0 ? (I)d.lo[1] : (j == N - 1 ? (I)d.hi[1] : (I)0);
-    const I dz = k == 0 ? (I)d.lo[2] : (k == N - 1 ? (I)d.hi[2] : (I)0);
-    const I dx = xn == 0 ? (I)d.lo[0] : (xn == R - 1 ? (I)d.hi[0] : (I)0);
-    const bool py = dy != 0, pz = dz != 0, px = dx != 0;
-    // every load of the run before its first store
-    const V xo = *(const V *)(x + g0);
-    const V wo = *(const V *)(w + g0);
-    const V ro = *(const V *)(r + g0);
-    V dv;
-    if (dinv)  // the Jacobi values from the table where the element's equal it
-      dv = (dtab && deq[e]) ? *(const V *)(dtab + (g0 - (I)(e * NN))) : *(const V *)(dinv + g0);
-    const V q0 = *(const V *)(qv + g0);
-    V qy = {}, qz = {}, qyz = {};
-    if (py) qy = *(const V *)(qv + g0 + dy);
-    if (pz) qz = *(const V *)(qv + g0 + dz);
-    if (py && pz) qyz = *(const V *)(qv + g0 + dy + dz);
-    T sx = T(0), sxy = T(0), sxz = T(0), sxyz = T(0);
-    if (px) {
-      const I gx = g0 + (I)xn + dx;
-      sx = qv[gx];
-      if (py) sxy = qv[gx + dy];
-      if (pz) sxz = qv[gx + dz];
-      if (py && pz) sxyz = qv[gx + dy + dz];
-    }
-    // the partner side is the lower one when its offset is negative
-    const bool ysw = dy < 0, zsw = dz < 0, xsw = dx < 0;
-    V xv, rv;
+    gf::box_elem_coords(topo, le, ec);
+    de = gf::box_elem_deltas(topo, N, ec);
+    const T *dsrc = dinv ? ((dtab && deq[e]) ? dtab + t.r : dinv + col) : nullptr;
 #pragma unroll
-    for (int n = 0; n < R; n++) {
-      // t[side z][side y][side x], side 0 = own copy, 1 = partner
-      T t[2][2][2];
-      t[0][0][0] = VT::get(q0, n);
-      t[0][1][0] = VT::get(qy, n);
-      t[1][0][0] = VT::get(qz, n);
-      t[1][1][0] = VT::get(qyz, n);
-      const bool hx = (n == 0 || n == R - 1) && n == xn && px;
-      t[0][0][1] = hx ? sx : T(0);
-      t[0][1][1] = hx ? sxy : T(0);
-      t[1][0][1] = hx ? sxz : T(0);
-      t[1][1][1] = hx ? sxyz : T(0);
-      const bool xs = hx && xsw;
-      // canonical order: lower side first in z, then y, then x; absent
-      // partners contribute +0 (see box_sum8z)
-      T sum = T(0);
+    for (int q = 0; q < N; q++) qo[q] = qv[col + q * S::N2];
+    L.issue(qv, de, (int64_t)(e * S::NN), t.r);
 #pragma unroll
-      for (int cz = 0; cz < 2; cz++)
+    for (int q = 0; q < N; q++) ro[q] = r[col + q * S::N2];
 #pragma unroll
-        for (int cy = 0; cy < 2; cy++)
+    for (int q = 0; q < N; q++) dv[q] = dsrc ? dsrc[q * S::N2] : T(1);
+  };
+  CGWalk k(c, b, C::EPB, true);
+  if (k.in()) load(k.c);
+  double alpha64;
+  if (!h.finish(b, sred, alpha64)) return;
+  const T alpha = (T)alpha64;
+  double rho = 0.0, nrm = 0.0;
+  while (k.in()) {
+    gf::elem_sync<C::WAVE>();  // the previous element's sums have read LDS
 #pragma unroll
-          for (int cx = 0; cx < 2; cx++) {
-            const int sz = cz ^ (int)zsw, sy = cy ^ (int)ysw, sxi = cx ^ (int)xs;
-            sum = sum + t[sz][sy][sxi];
-          }
-      const int cnt = (1 + (int)py) * (1 + (int)pz) * (1 + (int)hx);
-      const T qa = cnt == 1 ? t[0][0][0] : sum;
-      const T xn1 = (T)1 * VT::get(xo, n) + alpha * VT::get(wo, n);
-      VT::set(xv, n, xn1);
-      const T rn1 = (T)1 * VT::get(ro, n) + (-alpha) * qa;
-      VT::set(rv, n, rn1);
-      const T z = dinv ? VT::get(dv, n) * rn1 : rn1;
-      const double im = gf::box_inv(cnt);
-      rho += (double)rn1 * (double)z * im;
-      const double rd = (double)rn1;
-      if (NORM == GF_NORM_INF) nrm = fmax(nrm, fabs(rd));
-      else if (NORM == GF_NORM_EUC) nrm += rd * rd;
-      else if (NORM == GF_NORM_L2) nrm += mass[g0 + n] * rd * rd;
-      else if (NORM == GF_NORM_L1) nrm += mass[g0 + n] * fabs(rd);
-      else nrm += rd * rd * im;
-    }
-    *(V *)(x + g0) = xv;
-    *(V *)(r + g0) = rv;
+    for (int q = 0; q < N; q++)
+      if (t.own()) hl[t.r + S::N2 * q] = qo[q];
+    if (t.own()) L.store(hl, t.r);
+    gf::elem_sync<C::WAVE>();
+    const gf::HaloCol<N> hc(de, t.i, t.j);
+    gf::static_for<0, N>([&](auto kc) {
+      constexpr int q = decltype(kc)::value;
+      int ad[8];
+      const int cnt = gf::halo_order<N, q>(hc, de, ad);
+      T s = (hl[ad[0]] + hl[ad[1]]) + (hl[ad[2]] + hl[ad[3]]);
+      if (q == 0 || q == N - 1) s = s + ((hl[ad[4]] + hl[ad[5]]) + (hl[ad[6]] + hl[ad[7]]));
+      T rn = ro[q] + (-alpha) * s;
+      asm volatile("" : "+v"(rn));  // node by node (see k_burgers_stage3b)
+      const size_t g = col + q * S::N2;
+      if (act) {
+        r[g] = rn;
+        cg_accum<NORM>((double)rn, dinv ? (double)(dv[q] * rn) : (double)rn, gf::box_inv(cnt), mass,
+                       g, rho, nrm);
+      }
+    });
+    k.next();
+    if (k.in()) load(k.c);
   }
-  double a = gf::block_reduce<false>(rho, sred);
-  double b = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
-                                 : gf::block_reduce<false>(nrm, sred);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = a;
-    part[2 * blockIdx.x + 1] = b;
-  }
+  const double ra = gf::block_reduce<false>(rho, sred);
+  const double rb = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
+                                        : gf::block_reduce<false>(nrm, sred);
+  if (threadIdx.x == 0) ((double2 *)c.partU)[b.b0 + b.lb] = make_double2(ra, rb);
 }
 
 template <typename T, int NORM, int N>
-int launch_update_box_n(gf_mesh *m, CGVecs<T> &v, double *part) {
-  if constexpr (boxv_ok<T, N>()) {
-    if (m->ndof < ((size_t)1 << 31))
-      hipLaunchKernelGGL((k_cg_update_boxv<T, NORM, N, int32_t>), dim3(kUpdBlocks), dim3(kThreads),
-                         0, m->ctx->stream, v.x, v.w, v.r, v.q, v.dinv, m->mass, m->box, m->scal,
-                         part, m->nelems, v.dtab, v.deq);
-    else
-      hipLaunchKernelGGL((k_cg_update_boxv<T, NORM, N, int64_t>), dim3(kUpdBlocks), dim3(kThreads),
-                         0, m->ctx->stream, v.x, v.w, v.r, v.q, v.dinv, m->mass, m->box, m->scal,
-                         part, m->nelems, v.dtab, v.deq);
-    return GF_OK;
-  }
-  // 32-bit node indices whenever every index of the mesh fits
-  if (m->ndof < ((size_t)1 << 31))
-    hipLaunchKernelGGL((k_cg_update_box<T, NORM, N, int32_t>), dim3(kUpdBlocks), dim3(kThreads), 0,
-                       m->ctx->stream, v.x, v.w, v.r, v.q, v.dinv, m->mass, m->box, m->scal, part,
-                       m->nelems);
-  else
-    hipLaunchKernelGGL((k_cg_update_box<T, NORM, N, int64_t>), dim3(kUpdBlocks), dim3(kThreads), 0,
-                       m->ctx->stream, v.x, v.w, v.r, v.q, v.dinv, m->mass, m->box, m->scal, part,
-                       m->nelems);
+int launch_update_box_n(gf_mesh *m, const CGCtl &c, const CGVecs<T> &v) {
+  hipLaunchKernelGGL((k_cg_update_halo<T, NORM, N>), dim3(c.nbU), dim3(kThreads), 0,
+                     m->ctx->stream, c, v.r, v.q, v.dinv, m->mass, m->box, v.topos, v.dtab, v.deq);
+  GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
 
 }  // namespace gfs
 
-#define GF_K3D_UPD(T, N)                                                              \
-  template int launch_update_box_n<T, GF_NORM_INF, N>(gf_mesh *, CGVecs<T> &, double *); \
-  template int launch_update_box_n<T, GF_NORM_EUC, N>(gf_mesh *, CGVecs<T> &, double *); \
-  template int launch_update_box_n<T, GF_NORM_L2, N>(gf_mesh *, CGVecs<T> &, double *);  \
-  template int launch_update_box_n<T, GF_NORM_L1, N>(gf_mesh *, CGVecs<T> &, double *);  \
-  template int launch_update_box_n<T, GF_NORM_ASSEMBLED_L2, N>(gf_mesh *, CGVecs<T> &, double *);
+#define GF_K3D_UPD(T, N) \
+  template int cg_blocks3<T, N>(size_t); \
+  template int launch_update_box_n<T, GF_NORM_INF, N>(gf_mesh *, const CGCtl &, const CGVecs<T> &); \
+  template int launch_update_box_n<T, GF_NORM_EUC, N>(gf_mesh *, const CGCtl &, const CGVecs<T> &); \
+  template int launch_update_box_n<T, GF_NORM_L2, N>(gf_mesh *, const CGCtl &, const CGVecs<T> &); \
+  template int launch_update_box_n<T, GF_NORM_L1, N>(gf_mesh *, const CGCtl &, const CGVecs<T> &); \
+  template int launch_update_box_n<T, GF_NORM_ASSEMBLED_L2, N>(gf_mesh *, const CGCtl &, const CGVecs<T> &);
 
 #define GF_K3D_INSTANTIATE(N)                                                                \
   template int launch_stage3p<N>(gf_mesh *, const StageArgs &);                              \

@@ -39,14 +39,6 @@ int gf_check_hip(gf_ctx *ctx, hipError_t e, const char *what) {
   return e == hipErrorOutOfMemory ? GF_ERR_ALLOC : GF_ERR_HIP;
 }
 
-size_t gf_red_need(size_t nelems) {
-  // apply partials (one per block, at most one block per element) at the
-  // front, then the update kernels' (rho, norm) pairs and the set-up slots
-  const size_t need = nelems + 64 + 2 * 1024 + 128;
-  const size_t base = (size_t)GF_RED_MAX_BLOCKS * 8;
-  return need > base ? need : base;
-}
-
 void *gf_ws(gf_mesh *m, int slot, size_t bytes) {
   if ((int)m->ws.size() <= slot) {
     if (m->ws_frozen) return nullptr;
@@ -977,6 +969,41 @@ int gf_mesh_create(gf_ctx *ctx, const gf_mesh_desc *d, gf_mesh **out) {
     UP(m->goff, goff.data(), goff.size());
     UP(m->gmem, gmem.data(), std::max<size_t>(gmem.size(), 1));
   }
+  // Boxes in sequence: kept where every node's group is the one its box
+  // implies (device-built groups are, by construction).
+  if (d->box_count >= 1 && d->box_list && d->dim == 3 && d->gtype == GF_GE_REGULAR && m->Niso) {
+    size_t e0 = 0;
+    bool ok = true;
+    for (int b = 0; ok && b < d->box_count; b++) {
+      gf::BoxTopo t = {};
+      size_t nb = 1;
+      for (int c = 0; c < 3; c++) {
+        t.ne[c] = d->box_list[6 * b + c];
+        t.per[c] = d->box_list[6 * b + 3 + c] ? 1 : 0;
+        ok = ok && t.ne[c] >= 1;
+        nb *= (size_t)std::max(t.ne[c], 1);
+      }
+      ok = ok && nb <= m->nelems - e0;
+      const int Nn = m->Niso;
+      for (size_t le = 0; ok && !devmaps && le < nb; le++) {
+        int ec[3];
+        gf::box_elem_coords(t, le, ec);
+        const gf::BoxElemDeltas de = gf::box_elem_deltas(t, Nn, ec);
+        for (size_t r = 0; ok && r < m->nn; r++) {
+          const size_t q = (e0 + le) * m->nn + r;
+          int64_t g[8];
+          const int c = gf::box_members<int64_t>(de, Nn, (int64_t)q, (int)(r % Nn),
+                                                 (int)((r / Nn) % Nn), (int)(r / (Nn * Nn)), g);
+          const int64_t o = d->ggfx_offs[q];
+          ok = d->ggfx_offs[q + 1] - o == c;
+          for (int k = 0; ok && k < c; k++) ok = d->ggfx_members[o + k] == g[k];
+        }
+      }
+      e0 += nb;
+      m->h_boxes.push_back(t);
+    }
+    if (!ok || e0 != m->nelems) m->h_boxes.clear();
+  }
   // Structured box: enable gather assembly only if every node's GGFX group
   // is exactly the group the box structure implies.
   if (d->box_ne[0] > 0 && !boxunion && d->dim == 3 && d->gtype == GF_GE_REGULAR && m->Niso) {
@@ -1033,11 +1060,14 @@ int gf_mesh_create(gf_ctx *ctx, const gf_mesh_desc *d, gf_mesh **out) {
   }
   // whether the halo's canonical order is GGFX's (gf::box_halo8_ok)
   m->halo8 = m->has_box && m->Niso == 8 && gf::box_halo8_ok(m->box);
-  m->red_cap = gf_red_need(m->nelems);
+  // the CG apply kernels' partials (at most 2056 blocks), the update kernels'
+  // (rho, norm) pairs, and the set-up reductions' pairs
+  m->red_cap = (size_t)GF_RED_MAX_BLOCKS * 8;
   GF_HIP(ctx, hipMalloc((void **)&m->red, m->red_cap * sizeof(double)));
   GF_HIP(ctx, hipMalloc((void **)&m->scal, 64 * sizeof(double)));
   GF_HIP(ctx, hipHostMalloc((void **)&m->hscal, 64 * sizeof(double),
                             hipHostMallocMapped | hipHostMallocCoherent));
+  std::fill(m->hscal, m->hscal + 64, 0.0);
   GF_HIP(ctx, hipHostGetDevicePointer((void **)&m->hscal_dev, m->hscal, 0));
   for (int k = 0; k < 2; k++)
     GF_HIP(ctx, hipEventCreateWithFlags(&m->cg_ev[k], hipEventDisableTiming));
@@ -1144,7 +1174,7 @@ int gf_mesh_destroy(gf_mesh *m) {
   for (int k = 0; k < 6; k++) F(m->G32[k]);
   F(m->mass32);
   if (m->hscal) (void)hipHostFree(m->hscal);
-  F(m->seg_eoff); F(m->seg_boff); F(m->sscal); F(m->dl_I); F(m->dl_wq);
+  F(m->seg_eoff); F(m->seg_boff); F(m->sscal); F(m->seg_topo); F(m->dl_I); F(m->dl_wq);
   if (m->hsscal) (void)hipHostFree(m->hsscal);
   for (int k = 0; k < 2; k++)
     if (m->cg_ev[k]) (void)hipEventDestroy(m->cg_ev[k]);

@@ -19,6 +19,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gf_dtab.hpp"
 
 namespace gf {
@@ -99,6 +101,20 @@ __device__ __forceinline__ void gll_apply(const T (&x)[N], T (&y)[N]) {
   }
 }
 
+// Orders an element's LDS accesses: a workgroup barrier, or, where the
+// element's threads lie in one wave, no more than the wave's program order
+// (its LDS accesses complete in order).
+template <bool WAVE>
+__device__ __forceinline__ void elem_sync() {
+  if constexpr (WAVE) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  } else {
+    __syncthreads();
+  }
+}
+
 template <int N>
 struct Pen3 {
   // Each pass reads D through its own copy (rows contiguous for the gradient,
@@ -134,13 +150,18 @@ struct Pen3 {
 // with HOOK true, hx and hy are carried through LDS to the node's column
 // owner and handed to post (advection-type terms); with HOOK false they are
 // ignored and post receives zeros.
-// All threads of the workgroup must call this (it contains barriers).
-template <int N, typename T, bool HOOK, typename XCB, typename YCB, typename ZCB, typename POST>
+// own false: an idle thread of the workgroup, which reads an element's LDS
+// but writes none (HOOK false only).
+// All threads of the workgroup must call this (it contains barriers; with
+// WAVE true an element's threads lie in one wave and only that wave is
+// ordered, so the workgroup's waves run apart).
+template <int N, typename T, bool HOOK, bool WAVE = false, typename XCB, typename YCB,
+          typename ZCB, typename POST, typename OWN = std::true_type>
 __device__ __forceinline__ void pen_op3(const T (&ru)[N], T *su, T *sd, T *sx, const PenD<T> &Dp,
                                         const T *__restrict__ W, int a, int b, T Wa, T Wb, T jac,
                                         T g0, T g1,
                                         T g2, const T *__restrict__ pe, XCB &&xcb, YCB &&ycb,
-                                        ZCB &&zcb, POST &&post) {
+                                        ZCB &&zcb, POST &&post, OWN own = OWN()) {
   using S = Pen3<N>;
   (void)Dp;
   // even N: the contractions in even/odd form (gll_apply_eo); odd N: the
@@ -153,7 +174,8 @@ __device__ __forceinline__ void pen_op3(const T (&ru)[N], T *su, T *sd, T *sx, c
   // (the factor shared by all of them is formed once)
   const T cab = (Wb * Wa) * jac;
 #pragma unroll
-  for (int k = 0; k < N; k++) su[S::at(a, b, k)] = ru[k];
+  for (int k = 0; k < N; k++)
+    if (own) su[S::at(a, b, k)] = ru[k];
   // z-part on the column, in registers
   T dz[N];
   {
@@ -188,7 +210,7 @@ __device__ __forceinline__ void pen_op3(const T (&ru)[N], T *su, T *sd, T *sx, c
       }
     }
   }
-  __syncthreads();
+  elem_sync<WAVE>();
   // x-part on the x-pencil (j=a, k=b) -> sd
   {
     T xp[N], f[N], uxv[N];
@@ -216,14 +238,15 @@ __device__ __forceinline__ void pen_op3(const T (&ru)[N], T *su, T *sd, T *sx, c
       T sv[N];
       gll_apply_eo<N, true, T>(f, sv);
 #pragma unroll
-      for (int i = 0; i < N; i++) sd[S::at(i, a, b)] = sv[i];
+      for (int i = 0; i < N; i++)
+        if (own) sd[S::at(i, a, b)] = sv[i];
     } else {
 #pragma unroll
       for (int i = 0; i < N; i++) {
         T s = T(0);
 #pragma unroll
         for (int m = 0; m < N; m++) s = fma(dC(i, m), f[m], s);
-        sd[S::at(i, a, b)] = s;
+        if (own) sd[S::at(i, a, b)] = s;
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -265,15 +288,15 @@ __device__ __forceinline__ void pen_op3(const T (&ru)[N], T *su, T *sd, T *sx, c
       }
     }
   }
-  __syncthreads();
+  elem_sync<WAVE>();
   // (x-part + y-part) at the y-pencil's nodes; su is free for hy
 #pragma unroll
   for (int j = 0; j < N; j++) {
     const int q = S::at(a, j, b);
-    sd[q] = sd[q] + dy[j];
+    if (own) sd[q] = sd[q] + dy[j];
     if (HOOK) su[q] = hy[j];
   }
-  __syncthreads();
+  elem_sync<WAVE>();
 #pragma unroll
   for (int k = 0; k < N; k++) {
     const int q = S::at(a, b, k);

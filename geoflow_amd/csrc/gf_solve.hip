@@ -156,14 +156,15 @@ int launch_stage(gf_mesh *m, const StageArgs &a) {
 }
 
 // ---------------------------------------------------------------------------
-// CG kernels (T = double or float).  Scalars live on the device in
-// scal[]: 0 rho, 1 alpha, 2 beta, 3 rnorm, 4 rtol, 5 wq, 6 iter, 7 maxit,
-// 8 done, 9 first, 10 volume, 11 n.
+// CG kernels (T = double or float) of the meshes without pencil kernels; the
+// iteration and its scalars are described at CGCtl.
 // ---------------------------------------------------------------------------
 
 struct CGApplyArgs {
+  CGCtl c;
   const void *r;      // T
   const void *dinv;   // T or NULL
+  void *x;            // T
   void *w;            // T
   void *q;            // T
   const void *D, *W, *edx, *ejac, *qf;  // T
@@ -171,173 +172,132 @@ struct CGApplyArgs {
   const void *mass;  // T lumped mass per node (meshes with node metrics)
   double p;
   double qs;  // mass-term scalar when qf is NULL (0: no mass term)
-  double *scal;
-  double *part;
-  size_t nelems;
 };
 
-// w = beta*w + z (z = Dinv r, or w = z on the first iteration), then
-// q = A w on the element (unassembled) and the partial sum of w*q.  Because
-// w is continuous and zero where masked, sum_j w_j (DSS q)_j imult_j equals
-// sum_j w_j q_j over local nodes, so the dot product of gcg.ipp:307-308 is
-// formed here before the DSS.
-template <int DIM, int N, typename T>
+// The apply of an iteration (CGCtl): x += alpha w, w = z + beta w, q = A w on
+// the element (unassembled) and the partial sums of w q.  GM false: regular
+// elements (DIM 2; 3 without the standard D).  GM true: meshes with per-node
+// metrics (GE_2DEMBEDDED and GE_DEFORMED),
+//   q = p sum_j D_j^T (sum_i G(i,j) D_i w) + q M w
+// in the operation order of embed_prod / def_prod (ghelmholtz.ipp:108-191,
+// 205-290, 494-514), as k_helm_embed and k_helm_def3 form it; 2-D with G00,
+// G01, G11, 3-D with the six vectors G00, G01, G11, G02, G12, G22.  T is the
+// recurrence precision: FP64, or FP32 with FP32 copies of G, the mass and D.
+// Because w is continuous and zero where masked, sum_j w_j (DSS q)_j imult_j
+// equals sum_j w_j q_j over local nodes, so the dot product of
+// gcg.ipp:307-308 is formed here before the DSS.
+template <int DIM, int N, typename T, bool GM>
 __global__ __launch_bounds__(kThreads) void k_cg_apply(CGApplyArgs a) {
   using S = Shape<DIM, N>;
   __shared__ T su[S::NODES];
   __shared__ T sg[DIM][S::NODES];
   __shared__ T sD[N * N];
   __shared__ T sW[N];
-  __shared__ double sred[kThreads / 64];
-  const double *scal = a.scal;
-  if (scal[S_DONE] != 0.0) return;
-  const T *r = (const T *)a.r, *dinv = (const T *)a.dinv;
-  T *w = (T *)a.w, *qv = (T *)a.q;
-  const T *D = (const T *)a.D, *W = (const T *)a.W, *edx = (const T *)a.edx,
-          *ejac = (const T *)a.ejac, *qf = (const T *)a.qf;
-  bool first = scal[S_FIRST] != 0.0;
-  T beta = (T)scal[S_BETA];
-  size_t e0 = (size_t)blockIdx.x * S::EPB;
-  int nel = (int)min((size_t)S::EPB, a.nelems - e0);
-  size_t base = e0 * S::NN;
-  int cnt = nel * S::NN;
-  gf::stage_D(sD, D, N);
-  if (threadIdx.x < N) sW[threadIdx.x] = W[threadIdx.x];
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    size_t g = base + q;
-    T z = dinv ? dinv[g] * r[g] : r[g];
-    T wn = first ? z : beta * w[g] + (T)1 * z;
-    w[g] = wn;
-    su[q] = wn;
-  }
-  __syncthreads();
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    int el = q / S::NN, rr = q - el * S::NN, i, j, k;
-    gf::node_ijk<DIM, N>(rr, i, j, k);
-    size_t e = e0 + el;
-    T M = gf::node_mass<DIM>(sW, i, j, k, ejac[e]);
-#pragma unroll
-    for (int d = 0; d < DIM; d++) {
-      T gd = gf::contract<DIM, N, false>(su + el * S::NN, sD, d, i, j, k);
-      T f = edx[e * DIM + d];
-      sg[d][q] = M * (gd * (f * f));
-    }
-  }
-  __syncthreads();
-  double dot = 0.0;
-  T p = (T)a.p;
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    int el = q / S::NN, rr = q - el * S::NN, i, j, k;
-    gf::node_ijk<DIM, N>(rr, i, j, k);
-    T acc = 0;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) acc += gf::contract<DIM, N, true>(&sg[d][el * S::NN], sD, d, i, j, k);
-    if (p != (T)1) acc *= p;
-    if (qf || a.qs != 0.0) {
-      T M = gf::node_mass<DIM>(sW, i, j, k, ejac[e0 + el]);
-      T t = M * su[q];
-      if (qf) t *= qf[base + q];
-      else if ((T)a.qs != (T)1) t *= (T)a.qs;
-      acc += t;
-    }
-    qv[base + q] = acc;
-    dot += (double)su[q] * (double)acc;
-  }
-  double bsum = gf::block_reduce<false>(dot, sred);
-  if (threadIdx.x == 0) a.part[blockIdx.x] = bsum;
-}
-
-// The same for meshes with per-node metrics (GE_2DEMBEDDED and GE_DEFORMED):
-// q = p sum_j D_j^T (sum_i G(i,j) D_i w) + q M w in the operation order of
-// embed_prod / def_prod (ghelmholtz.ipp:108-191, 205-290, 494-514), as
-// k_helm_embed and k_helm_def3 form it; 2-D with G00, G01, G11, 3-D with the
-// six vectors G00, G01, G11, G02, G12, G22.  T is the recurrence precision:
-// FP64, or FP32 with FP32 copies of G, the mass and D.
-template <int DIM, int N, typename T>
-__global__ __launch_bounds__(kThreads) void k_cg_apply_gm(CGApplyArgs a) {
-  using S = Shape<DIM, N>;
-  __shared__ T su[S::NODES];
-  __shared__ T sg[DIM][S::NODES];
-  __shared__ T sD[N * N];
-  __shared__ double sred[kThreads / 64];
-  const double *scal = a.scal;
-  if (scal[S_DONE] != 0.0) return;
-  const T *r = (const T *)a.r, *dinv = (const T *)a.dinv;
-  T *w = (T *)a.w, *qv = (T *)a.q;
-  const T *qf = (const T *)a.qf, *mass = (const T *)a.mass;
-  const T *G0 = (const T *)a.G[0], *G1 = (const T *)a.G[1], *G2 = (const T *)a.G[2];
-  const bool first = scal[S_FIRST] != 0.0;
-  const T beta = (T)scal[S_BETA];
-  const size_t e0 = (size_t)blockIdx.x * S::EPB;
-  const int nel = (int)min((size_t)S::EPB, a.nelems - e0);
-  const size_t base = e0 * S::NN;
-  const int cnt = nel * S::NN;
+  __shared__ double sred[2 * (kThreads / 64)];
+  const CGBlock b(a.c, (int)xcd_block(), a.c.nbA);
+  if (!b.ok) return;
+  CGHead h(a.c, b);
+  const T *__restrict__ r = (const T *)a.r, *__restrict__ dinv = (const T *)a.dinv;
+  T *__restrict__ x = (T *)a.x, *__restrict__ w = (T *)a.w, *__restrict__ qv = (T *)a.q;
+  const T *__restrict__ edx = (const T *)a.edx, *__restrict__ ejac = (const T *)a.ejac;
+  const T *__restrict__ qf = (const T *)a.qf, *__restrict__ mass = (const T *)a.mass;
+  const T *__restrict__ G0 = (const T *)a.G[0], *__restrict__ G1 = (const T *)a.G[1],
+          *__restrict__ G2 = (const T *)a.G[2], *__restrict__ G3 = (const T *)a.G[3],
+          *__restrict__ G4 = (const T *)a.G[4], *__restrict__ G5 = (const T *)a.G[5];
+  const T p = (T)a.p, qs = (T)a.qs;
   gf::stage_D(sD, (const T *)a.D, N);
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    const size_t g = base + q;
-    const T z = dinv ? dinv[g] * r[g] : r[g];
-    const T wn = first ? z : beta * w[g] + (T)1 * z;
-    w[g] = wn;
-    su[q] = wn;
-  }
-  __syncthreads();
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    int el = q / S::NN, rr = q - el * S::NN, i, j, k;
-    gf::node_ijk<DIM, N>(rr, i, j, k);
-    const size_t g = base + q;
-    const T d0 = gf::contract<DIM, N, false>(su + el * S::NN, sD, 0, i, j, k);
-    const T d1 = gf::contract<DIM, N, false>(su + el * S::NN, sD, 1, i, j, k);
-    if constexpr (DIM == 2) {
-      T g0 = (T)0 + d0 * G0[g];
-      g0 += d1 * G1[g];
-      T g1 = (T)0 + d0 * G1[g];
-      g1 += d1 * G2[g];
-      sg[0][q] = g0;
-      sg[1][q] = g1;
-    } else {
-      const T d2 = gf::contract<DIM, N, false>(su + el * S::NN, sD, 2, i, j, k);
-      const T a00 = G0[g], a01 = G1[g], a11 = G2[g], a02 = ((const T *)a.G[3])[g],
-              a12 = ((const T *)a.G[4])[g], a22 = ((const T *)a.G[5])[g];
-      T g0 = (T)0 + d0 * a00;
-      g0 += d1 * a01;
-      g0 += d2 * a02;
-      T g1 = (T)0 + d0 * a01;
-      g1 += d1 * a11;
-      g1 += d2 * a12;
-      T g2 = (T)0 + d0 * a02;
-      g2 += d1 * a12;
-      g2 += d2 * a22;
-      sg[0][q] = g0;
-      sg[1][q] = g1;
-      sg[DIM - 1][q] = g2;
-    }
-  }
-  __syncthreads();
+  if (!GM && threadIdx.x < N) sW[threadIdx.x] = ((const T *)a.W)[threadIdx.x];
+  h.finish(a.c, b, sred);
+  if (!h.run) return;
+  const T beta = (T)h.beta, alpha = (T)h.alpha;
   double dot = 0.0;
-  for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
-    int el = q / S::NN, rr = q - el * S::NN, i, j, k;
-    gf::node_ijk<DIM, N>(rr, i, j, k);
-    T acc = 0;
-#pragma unroll
-    for (int d = 0; d < DIM; d++) acc += gf::contract<DIM, N, true>(&sg[d][el * S::NN], sD, d, i, j, k);
-    if (a.p != 1.0) acc *= (T)a.p;
-    if (qf || a.qs != 0.0) {
-      T t = mass[base + q] * su[q];
-      if (qf) t *= qf[base + q];
-      else if (a.qs != 1.0) t *= (T)a.qs;
-      acc += t;
+  for (CGWalk wk(a.c, b, S::EPB, false); wk.in(); wk.next()) {
+    const size_t e0 = b.e0 + (size_t)wk.c * S::EPB;
+    const int nel = (int)min((size_t)S::EPB, b.e1 - e0);
+    const size_t base = e0 * S::NN;
+    const int cnt = nel * S::NN;
+    for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
+      const size_t g = base + q;
+      const T wo = h.first ? T(0) : w[g];
+      if (!a.c.init) x[g] = x[g] + alpha * wo;
+      if (h.xonly) continue;
+      const T z = dinv ? dinv[g] * r[g] : r[g];
+      const T wn = h.first ? z : beta * wo + z;
+      w[g] = wn;
+      su[q] = wn;
     }
-    qv[base + q] = acc;
-    dot += (double)su[q] * (double)acc;
+    if (h.xonly) continue;
+    __syncthreads();
+    for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
+      int el = q / S::NN, rr = q - el * S::NN, i, j, k;
+      gf::node_ijk<DIM, N>(rr, i, j, k);
+      const size_t g = base + q;
+      if constexpr (!GM) {
+        const size_t e = e0 + el;
+        const T M = gf::node_mass<DIM>(sW, i, j, k, ejac[e]);
+#pragma unroll
+        for (int d = 0; d < DIM; d++) {
+          T gd = gf::contract<DIM, N, false>(su + el * S::NN, sD, d, i, j, k);
+          T f = edx[e * DIM + d];
+          sg[d][q] = M * (gd * (f * f));
+        }
+      } else {
+        const T d0 = gf::contract<DIM, N, false>(su + el * S::NN, sD, 0, i, j, k);
+        const T d1 = gf::contract<DIM, N, false>(su + el * S::NN, sD, 1, i, j, k);
+        if constexpr (DIM == 2) {
+          T g0 = (T)0 + d0 * G0[g];
+          g0 += d1 * G1[g];
+          T g1 = (T)0 + d0 * G1[g];
+          g1 += d1 * G2[g];
+          sg[0][q] = g0;
+          sg[1][q] = g1;
+        } else {
+          const T d2 = gf::contract<DIM, N, false>(su + el * S::NN, sD, 2, i, j, k);
+          const T a00 = G0[g], a01 = G1[g], a11 = G2[g], a02 = G3[g], a12 = G4[g], a22 = G5[g];
+          T g0 = (T)0 + d0 * a00;
+          g0 += d1 * a01;
+          g0 += d2 * a02;
+          T g1 = (T)0 + d0 * a01;
+          g1 += d1 * a11;
+          g1 += d2 * a12;
+          T g2 = (T)0 + d0 * a02;
+          g2 += d1 * a12;
+          g2 += d2 * a22;
+          sg[0][q] = g0;
+          sg[1][q] = g1;
+          sg[DIM - 1][q] = g2;
+        }
+      }
+    }
+    __syncthreads();
+    for (int q = threadIdx.x; q < cnt; q += blockDim.x) {
+      int el = q / S::NN, rr = q - el * S::NN, i, j, k;
+      gf::node_ijk<DIM, N>(rr, i, j, k);
+      T acc = 0;
+#pragma unroll
+      for (int d = 0; d < DIM; d++)
+        acc += gf::contract<DIM, N, true>(&sg[d][el * S::NN], sD, d, i, j, k);
+      if (p != (T)1) acc *= p;
+      if (qf || a.qs != 0.0) {
+        T t = (GM ? mass[base + q] : gf::node_mass<DIM>(sW, i, j, k, ejac[GM ? 0 : e0 + el])) * su[q];
+        if (qf) t *= qf[base + q];
+        else if (qs != (T)1) t *= qs;
+        acc += t;
+      }
+      qv[base + q] = acc;
+      dot += (double)su[q] * (double)acc;
+    }
+    __syncthreads();  // the next elements reuse the buffers
   }
+  if (h.xonly) return;
   const double bsum = gf::block_reduce<false>(dot, sred);
-  if (threadIdx.x == 0) a.part[blockIdx.x] = bsum;
+  if (threadIdx.x == 0) a.c.partA[b.b0 + b.lb] = bsum;
 }
 
 template <typename T>
 __global__ void k_dss_cg(T *__restrict__ u, const int *__restrict__ goff,
-                         const int *__restrict__ gmem, int ngroups, const double *scal) {
-  if (scal[S_DONE] != 0.0) return;
+                         const int *__restrict__ gmem, int ngroups, const double *done) {
+  if (done && *done != 0.0) return;
   for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < ngroups; g += gridDim.x * blockDim.x) {
     int b = goff[g], e = goff[g + 1];
     if (e - b <= 8) {
@@ -364,91 +324,36 @@ __global__ void k_dss_cg(T *__restrict__ u, const int *__restrict__ goff,
   }
 }
 
-// alpha = rho / (w.q).  One block of 1024 threads reduces the per-block
-// partials of the apply kernel in a fixed order (deterministic).
-constexpr int kRedThreads = 1024;
-__global__ __launch_bounds__(kRedThreads) void k_cg_alpha(double *scal,
-                                                          const double *__restrict__ part, int np) {
-  __shared__ double sred[kRedThreads / 64];
-  if (scal[S_DONE] != 0.0) return;
-  double v0 = 0.0, v1 = 0.0, v2 = 0.0, v3 = 0.0;
-  int i = threadIdx.x;
-  for (; i + 3 * kRedThreads < np; i += 4 * kRedThreads) {
-    v0 += part[i];
-    v1 += part[i + kRedThreads];
-    v2 += part[i + 2 * kRedThreads];
-    v3 += part[i + 3 * kRedThreads];
-  }
-  for (; i < np; i += kRedThreads) v0 += part[i];
-  double v = (v0 + v1) + (v2 + v3);
-  v = gf::wave_sum(v);
-  int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (lane == 0) sred[wid] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double wq = sred[0];
-    for (int w = 1; w < kRedThreads / 64; w++) wq += sred[w];
-    cg_alpha_finish(scal, wq);
-  }
-}
-
-// x += alpha w ; r -= alpha mask q ; partials of r.z.imult and of the norm.
+// CG update where q has been assembled by a DSS pass (CGCtl):
+// r -= alpha mask q ; partials of r.z.imult and of the norm.
 template <typename T, int NORM>
-__global__ void k_cg_update(T *__restrict__ x, const T *__restrict__ w, T *__restrict__ r,
-                            const T *__restrict__ qv, const T *__restrict__ mask,
-                            const T *__restrict__ dinv, const T *__restrict__ imult,
-                            const double *__restrict__ mass, double *scal,
-                            double *__restrict__ part, size_t n) {
-  __shared__ double sred[kThreads / 64];
-  if (scal[S_DONE] != 0.0) return;
-  T alpha = (T)scal[S_ALPHA];
+__global__ void k_cg_update(CGCtl c, T *__restrict__ r, const T *__restrict__ qv,
+                            const T *__restrict__ mask, const T *__restrict__ dinv,
+                            const T *__restrict__ imult, const double *__restrict__ mass,
+                            size_t nn) {
+  __shared__ double sred[2 * (kThreads / 64)];
+  const CGBlock b(c, (int)xcd_block(), c.nbU);
+  if (!b.ok) return;
+  CGAlphaHead h(c, b);
+  double alpha64;
+  if (!h.finish(b, sred, alpha64)) return;
+  const T alpha = (T)alpha64;
   double rho = 0.0, nrm = 0.0;
-  GRID_LOOP(g, n) {
-    const T dv = dinv ? dinv[g] : T(1);
-    const double im = (double)imult[g];
-    T xv = (T)1 * x[g] + alpha * w[g];
-    T qm = mask ? qv[g] * mask[g] : qv[g];
-    T rv = (T)1 * r[g] + (-alpha) * qm;
-    x[g] = xv;
+  const size_t n1 = b.e1 * nn, step = (size_t)b.nb * blockDim.x;
+  for (size_t g = b.e0 * nn + (size_t)b.lb * blockDim.x + threadIdx.x; g < n1; g += step) {
+    const T qm = mask ? qv[g] * mask[g] : qv[g];
+    const T rv = r[g] + (-alpha) * qm;
     r[g] = rv;
-    T z = dinv ? dv * rv : rv;
-    rho += (double)rv * (double)z * (double)im;
-    double rd = (double)rv;
-    if (NORM == GF_NORM_INF) nrm = fmax(nrm, fabs(rd));
-    else if (NORM == GF_NORM_EUC) nrm += rd * rd;
-    else if (NORM == GF_NORM_L2) nrm += mass[g] * rd * rd;
-    else if (NORM == GF_NORM_L1) nrm += mass[g] * fabs(rd);
-    else nrm += rd * rd * (double)im;
+    cg_accum<NORM>((double)rv, dinv ? (double)(dinv[g] * rv) : (double)rv, (double)imult[g], mass, g,
+                   rho, nrm);
   }
-  double a = gf::block_reduce<false>(rho, sred);
-  double b = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
-                                 : gf::block_reduce<false>(nrm, sred);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = a;
-    part[2 * blockIdx.x + 1] = b;
-  }
+  const double ra = gf::block_reduce<false>(rho, sred);
+  const double rb = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
+                                        : gf::block_reduce<false>(nrm, sred);
+  if (threadIdx.x == 0) ((double2 *)c.partU)[b.b0 + b.lb] = make_double2(ra, rb);
 }
 
-// rho_new, beta, rnorm, iteration count and the stopping rule
-// (cg_beta_finish) from the update kernel's (rho, norm) partials.
-__global__ void k_cg_beta(double *scal, const double *__restrict__ part, int np, int normtype,
-                          double *resid, double *hmirror) {
-  __shared__ double sred[kRedThreads / 64];
-  if (scal[S_DONE] != 0.0) return;
-  double v = 0.0, w = 0.0;
-  for (int i = threadIdx.x; i < np; i += blockDim.x) {
-    v += part[2 * i];
-    w = normtype == GF_NORM_INF ? fmax(w, part[2 * i + 1]) : w + part[2 * i + 1];
-  }
-  double rho = gf::block_reduce<false>(v, sred);
-  double nr = normtype == GF_NORM_INF ? gf::block_reduce<true>(w, sred)
-                                      : gf::block_reduce<false>(w, sred);
-  if (threadIdx.x == 0) cg_beta_finish(scal, rho, nr, normtype, resid, hmirror);
-}
-
-// ---- CG on a batched mesh: every member its own scalars ------------------
-// Update blocks are assigned to members in proportion to their size
-// (boff[s] .. boff[s+1]); each block works its member's node range only.
+// System of a block of a batched mesh (boff[s] <= b < boff[s+1]).
 __device__ __forceinline__ int seg_of_block(const int *__restrict__ boff, int nseg, int b) {
   int lo = 0, hi = nseg;
   while (hi - lo > 1) {
@@ -459,110 +364,8 @@ __device__ __forceinline__ int seg_of_block(const int *__restrict__ boff, int ns
   return lo;
 }
 
-template <typename T, int NORM>
-__global__ void k_cg_update_seg(T *__restrict__ x, const T *__restrict__ w, T *__restrict__ r,
-                                const T *__restrict__ qv, const T *__restrict__ mask,
-                                const T *__restrict__ dinv, const T *__restrict__ imult,
-                                const double *__restrict__ mass, const double *sscal,
-                                const int64_t *__restrict__ eoff, const int *__restrict__ boff,
-                                int nseg, size_t nn, double *__restrict__ part) {
-  __shared__ double sred[kThreads / 64];
-  const int s = seg_of_block(boff, nseg, blockIdx.x);
-  const double *scal = sscal + kSegScal * s;
-  double rho = 0.0, nrm = 0.0;
-  if (scal[S_DONE] == 0.0) {
-    const T alpha = (T)scal[S_ALPHA];
-    const size_t n0 = (size_t)eoff[s] * nn, n1 = (size_t)eoff[s + 1] * nn;
-    const size_t lb = blockIdx.x - boff[s], nbs = boff[s + 1] - boff[s];
-    for (size_t g = n0 + lb * blockDim.x + threadIdx.x; g < n1; g += nbs * blockDim.x) {
-      const T dv = dinv ? dinv[g] : T(1);
-      const double im = (double)imult[g];
-      T xv = (T)1 * x[g] + alpha * w[g];
-      T qm = mask ? qv[g] * mask[g] : qv[g];
-      T rv = (T)1 * r[g] + (-alpha) * qm;
-      x[g] = xv;
-      r[g] = rv;
-      T z = dinv ? dv * rv : rv;
-      rho += (double)rv * (double)z * im;
-      double rd = (double)rv;
-      if (NORM == GF_NORM_INF) nrm = fmax(nrm, fabs(rd));
-      else if (NORM == GF_NORM_EUC) nrm += rd * rd;
-      else if (NORM == GF_NORM_L2) nrm += mass[g] * rd * rd;
-      else if (NORM == GF_NORM_L1) nrm += mass[g] * fabs(rd);
-      else nrm += rd * rd * im;
-    }
-  }
-  double a = gf::block_reduce<false>(rho, sred);
-  double b = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
-                                 : gf::block_reduce<false>(nrm, sred);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = a;
-    part[2 * blockIdx.x + 1] = b;
-  }
-}
-
-// alpha of every member: one wave per member, over the member's apply
-// partials (logical blocks eoff[s]/epb .. eoff[s+1]/epb).
-__global__ __launch_bounds__(1024) void k_cg_alpha_seg(double *sscal, const double *__restrict__ part,
-                                                       const int64_t *__restrict__ eoff, int nseg,
-                                                       int epb) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int s = wid; s < nseg; s += nw) {
-    double *sc = sscal + kSegScal * s;
-    if (sc[S_DONE] != 0.0) continue;
-    const int64_t b0 = eoff[s] / epb, b1 = eoff[s + 1] / epb;
-    double v = 0.0;
-    for (int64_t i = b0 + lane; i < b1; i += 64) v += part[i];
-    v = gf::wave_sum(v);
-    if (lane == 0) {
-      sc[S_WQ] = v;
-      sc[S_ALPHA] = sc[S_RHO] / v;
-    }
-  }
-}
-
-// rho, beta, norm, iteration count and stopping test of every member (the
-// rule of k_cg_beta per member), one wave per member; then the batch is
-// done when every member is, which scal[S_DONE] and the host mirror record.
-__global__ __launch_bounds__(1024) void k_cg_beta_seg(double *scal, double *sscal,
-                                                      const double *__restrict__ part,
-                                                      const int *__restrict__ boff, int nseg,
-                                                      int normtype, double *hmirror) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  for (int s = wid; s < nseg; s += nw) {
-    double *sc = sscal + kSegScal * s;
-    if (sc[S_DONE] != 0.0) continue;
-    double v = 0.0, w = 0.0;
-    for (int i = boff[s] + lane; i < boff[s + 1]; i += 64) {
-      v += part[2 * i];
-      w = normtype == GF_NORM_INF ? fmax(w, part[2 * i + 1]) : w + part[2 * i + 1];
-    }
-    v = gf::wave_sum(v);
-    w = normtype == GF_NORM_INF ? gf::wave_max(w) : gf::wave_sum(w);
-    if (lane == 0) {
-      const double rhom = sc[S_RHO];
-      sc[S_RHOM] = rhom;
-      sc[S_RHO] = v;
-      sc[S_BETA] = v / rhom;
-      const double rn = finish_norm(normtype, w, sc);
-      sc[S_RNORM] = rn;
-      const int it = (int)sc[S_ITER] + 1;
-      sc[S_ITER] = it;
-      sc[S_FIRST] = 0.0;
-      if (!(it < (int)sc[S_MAXIT] && rn > sc[S_RTOL])) sc[S_DONE] = 1.0;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    bool all = true;
-    for (int s = 0; s < nseg; s++) all = all && sscal[kSegScal * s + S_DONE] != 0.0;
-    scal[S_DONE] = all ? 1.0 : 0.0;
-    if (hmirror) hmirror[S_DONE] = scal[S_DONE];
-  }
-}
-
 // Set-up reductions per member (rho = sum r z imult and the norm's sum),
-// blocks assigned as in k_cg_update_seg; k_setup_fin_seg finishes them,
+// update blocks in proportion to the members' sizes; k_setup_fin_seg finishes them,
 // out[2s], out[2s+1].
 template <typename T>
 __global__ void k_setup_red_seg(const T *__restrict__ r, const T *__restrict__ z,
@@ -773,14 +576,12 @@ int launch_diag(gf_mesh *m, double p, const double *qf, double qs, double *d) {
 
 template <int DIM, int N, typename T>
 int launch_cg_apply(gf_mesh *m, const CGApplyArgs &a) {
-  using S = Shape<DIM, N>;
-  int nb = (int)((m->nelems + S::EPB - 1) / S::EPB);
-  if (m->gtype != GF_GE_REGULAR) {
-    hipLaunchKernelGGL((k_cg_apply_gm<DIM, N, T>), dim3(nb), dim3(kThreads), 0, m->ctx->stream, a);
-    GF_LAUNCH_CHECK(m->ctx);
-    return GF_OK;
-  }
-  hipLaunchKernelGGL((k_cg_apply<DIM, N, T>), dim3(nb), dim3(kThreads), 0, m->ctx->stream, a);
+  if (m->gtype != GF_GE_REGULAR)
+    hipLaunchKernelGGL((k_cg_apply<DIM, N, T, true>), dim3(a.c.nbA), dim3(kThreads), 0,
+                       m->ctx->stream, a);
+  else
+    hipLaunchKernelGGL((k_cg_apply<DIM, N, T, false>), dim3(a.c.nbA), dim3(kThreads), 0,
+                       m->ctx->stream, a);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
@@ -1599,50 +1400,108 @@ double finish_norm_host(int normtype, double v, gf_mesh *m, double volume) {
 }
 
 template <typename T, int NORM>
-int launch_update_box(gf_mesh *m, CGVecs<T> &v, double *part) {
+int launch_update_box(gf_mesh *m, const CGCtl &c, const CGVecs<T> &v) {
   switch (m->Niso) {
-    case 2: return launch_update_box_n<T, NORM, 2>(m, v, part);
-    case 3: return launch_update_box_n<T, NORM, 3>(m, v, part);
-    case 4: return launch_update_box_n<T, NORM, 4>(m, v, part);
-    case 5: return launch_update_box_n<T, NORM, 5>(m, v, part);
-    case 6: return launch_update_box_n<T, NORM, 6>(m, v, part);
-    case 7: return launch_update_box_n<T, NORM, 7>(m, v, part);
-    case 8: return launch_update_box_n<T, NORM, 8>(m, v, part);
-    case 9: return launch_update_box_n<T, NORM, 9>(m, v, part);
-    case 10: return launch_update_box_n<T, NORM, 10>(m, v, part);
+    case 2: return launch_update_box_n<T, NORM, 2>(m, c, v);
+    case 3: return launch_update_box_n<T, NORM, 3>(m, c, v);
+    case 4: return launch_update_box_n<T, NORM, 4>(m, c, v);
+    case 5: return launch_update_box_n<T, NORM, 5>(m, c, v);
+    case 6: return launch_update_box_n<T, NORM, 6>(m, c, v);
+    case 7: return launch_update_box_n<T, NORM, 7>(m, c, v);
+    case 8: return launch_update_box_n<T, NORM, 8>(m, c, v);
+    case 9: return launch_update_box_n<T, NORM, 9>(m, c, v);
+    case 10: return launch_update_box_n<T, NORM, 10>(m, c, v);
     default: return GF_ERR_UNSUPPORTED;
   }
 }
-
+// Blocks of the 3-D CG kernels on the mesh.
+template <typename T>
+int blocks3(gf_mesh *m) {
+  switch (m->Niso) {
+    case 2: return cg_blocks3<T, 2>(m->nelems);
+    case 3: return cg_blocks3<T, 3>(m->nelems);
+    case 4: return cg_blocks3<T, 4>(m->nelems);
+    case 5: return cg_blocks3<T, 5>(m->nelems);
+    case 6: return cg_blocks3<T, 6>(m->nelems);
+    case 7: return cg_blocks3<T, 7>(m->nelems);
+    case 8: return cg_blocks3<T, 8>(m->nelems);
+    case 9: return cg_blocks3<T, 9>(m->nelems);
+    case 10: return cg_blocks3<T, 10>(m->nelems);
+    default: return kXCD;
+  }
+}
 template <typename T, int NORM>
-void launch_update(gf_mesh *m, CGVecs<T> &v, double *part, bool mask_in_q) {
+int launch_update(gf_mesh *m, const CGCtl &c, const CGVecs<T> &v, bool gather, bool mask_in_q) {
+  if (gather) return launch_update_box<T, NORM>(m, c, v);
   const T *mk = (m->has_mask && !mask_in_q) ? v.mask : nullptr;
-  hipLaunchKernelGGL((k_cg_update<T, NORM>), dim3(kUpdBlocks), dim3(kThreads), 0, m->ctx->stream,
-                     v.x, v.w, v.r, v.q, mk, v.dinv, v.imult, m->mass, m->scal, part, m->ndof);
+  hipLaunchKernelGGL((k_cg_update<T, NORM>), dim3(c.nbU), dim3(kThreads), 0, m->ctx->stream, c, v.r,
+                     v.q, mk, v.dinv, v.imult, m->mass, m->nn);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+template <typename T>
+int launch_update_norm(gf_mesh *m, const CGCtl &c, const CGVecs<T> &v, bool gather,
+                       bool mask_in_q) {
+  switch (c.normtype) {
+    case GF_NORM_INF: return launch_update<T, GF_NORM_INF>(m, c, v, gather, mask_in_q);
+    case GF_NORM_EUC: return launch_update<T, GF_NORM_EUC>(m, c, v, gather, mask_in_q);
+    case GF_NORM_L2: return launch_update<T, GF_NORM_L2>(m, c, v, gather, mask_in_q);
+    case GF_NORM_L1: return launch_update<T, GF_NORM_L1>(m, c, v, gather, mask_in_q);
+    default: return launch_update<T, GF_NORM_ASSEMBLED_L2>(m, c, v, gather, mask_in_q);
+  }
+}
+CGApply3Args apply3_args(gf_mesh *m, const CGCtl &c) {
+  CGApply3Args a;
+  memset(&a, 0, sizeof(a));
+  a.c = c;
+  a.topo = m->box;
+  return a;
 }
 
-// Runs CG iterations from the state prepared in scal (rho, rtol, first=1,
-// iter=0, done) until done.  r holds the masked assembled residual, x the
-// iterate.  Returns iterations performed.
+// Runs CG iterations from the state prepared in the systems' first scalar
+// sets (rho, rtol, first, iter = 0, done) until every system is done; r holds
+// the masked assembled residual, x the iterate.  The final scalars are left
+// in the host mirror (m->hscal, or m->hsscal on a batched mesh).
 template <typename T>
-int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid, int *iters) {
+int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
   hipStream_t s = m->ctx->stream;
+  const int ns = m->nseg, nsys = std::max(ns, 1);
   const bool col = m->dim == 3 && m->dconst;
-  // Structured box: the update assembles q by gather (mask already in q).
-  const bool gather = col && m->has_box;
-  int nbA = 0;
-  if (col) {
-    nbA = col_blocks(m);
+  // Structured boxes: the update assembles q by gather (mask already in q).
+  v.topos = ns > 0 ? m->seg_topo : nullptr;
+  const bool gather = col && (ns > 0 ? m->seg_topo != nullptr : m->has_box);
+  CGCtl c;
+  c.scal = ns > 0 ? m->sscal : m->scal;
+  c.eoff = m->seg_eoff;
+  c.boff = m->seg_boff;
+  c.nseg = ns;
+  c.nelems = m->nelems;
+  if (ns > 0) {
+    c.nbA = c.nbU = xcd_grid(m->h_seg_boff[ns]);
+  } else if (col) {
+    c.nbA = blocks3<T>(m);
+    c.nbU = gather ? c.nbA : loop_blocks((m->ndof + kThreads - 1) / kThreads, kUpdBlocks);
   } else {
-    int NN = (int)m->nn;
-    int epb = NN >= kThreads ? 1 : kThreads / NN;
-    nbA = (int)((m->nelems + epb - 1) / epb);
+    const int NN = (int)m->nn, epb = NN >= kThreads ? 1 : kThreads / NN;
+    c.nbA = loop_blocks((m->nelems + epb - 1) / epb, 2 * kUpdBlocks);
+    c.nbU = loop_blocks((m->ndof + kThreads - 1) / kThreads, kUpdBlocks);
   }
-  double *partA = m->red;
-  double *partU = m->red + (size_t)nbA + 64;
+  c.partA = m->red;
+  c.partU = m->red + (c.nbA + 64) / 2 * 2;  // 16-byte pairs
+  c.normtype = normtype;
+  c.stream = 4 * m->ndof * sizeof(T) > ((size_t)256 << 20);
+  c.resid = d_resid;
+  volatile double *hm = ns > 0 ? m->hsscal : m->hscal;
+  c.mirror = ns > 0 ? m->hsscal_dev : m->hscal_dev;
+  // the done flags carry the solve's number: kernels queued past the end of
+  // an earlier loop may still write theirs
+  c.epoch = ++m->cg_epoch;
   CGApplyArgs a;
+  CGApply3Args a3 = apply3_args(m, c);
+  memset(&a, 0, sizeof(a));
   a.r = v.r;
   a.dinv = v.dinv;
+  a.x = v.x;
   a.w = v.w;
   a.q = v.q;
   a.D = v.D;
@@ -1651,27 +1510,16 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid, int *iters)
   a.ejac = v.ejac;
   a.qf = v.qf;
   a.qs = v.qs;
-  for (int c = 0; c < 6; c++) a.G[c] = v.G[c];
+  for (int k = 0; k < 6; k++) a.G[k] = v.G[k];
   a.mass = v.mass;
   a.p = v.p;
-  a.scal = m->scal;
-  a.part = partA;
-  a.nelems = m->nelems;
-  CGApply3Args a3;
-  a3.seg_eoff = nullptr;
-  a3.nseg = 0;
-  a3.sscal = nullptr;
   a3.r = v.r;
   a3.dinv = v.dinv;
   a3.dtab = v.dtab;
   a3.deq = v.deq;
+  a3.x = v.x;
   a3.w = v.w;
   a3.q = v.q;
-  a3.D = v.D;
-  for (int c = 0; c < 3; c++) {
-    a3.DR[c] = sizeof(T) == 8 ? (const void *)m->pDR[c] : (const void *)m->pDR32[c];
-    a3.DC[c] = sizeof(T) == 8 ? (const void *)m->pDC[c] : (const void *)m->pDC32[c];
-  }
   a3.W = v.W;
   a3.edx = v.edx;
   a3.ejac = v.ejac;
@@ -1679,75 +1527,45 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid, int *iters)
   a3.qs = v.qs;
   // the mask is formed from the box faces when it is known to match them
   a3.tmask = (m->has_mask && v.mask && m->has_box_mask) ? 1 : 0;
-  a3.topo = m->box;
   a3.mask = (m->has_mask && !a3.tmask) ? v.mask : nullptr;
   a3.p = v.p;
-  a3.scal = m->scal;
-  a3.part = partA;
-  a3.nelems = m->nelems;
-  // the host mirror starts from the scalars prepared by the caller (a
-  // solve that is already done queues nothing that would update it)
-  volatile double *hm = m->hscal;
-  GF_HIP(m->ctx, hipMemcpyAsync(m->hscal, m->scal, S_COUNT * sizeof(double),
-                                hipMemcpyDeviceToHost, s));
-  GF_HIP(m->ctx, hipStreamSynchronize(s));
-  if (hm[S_DONE] != 0.0) {
-    *iters = (int)m->hscal[S_ITER];
-    return GF_OK;
-  }
-  int cur = 0, nq = 0;
-  for (;;) {
-    for (int b = 0; b < kBatch; b++) {
-      int rc;
+  auto all_done = [&]() {
+    for (int k = 0; k < nsys; k++)
+      if (hm[(size_t)k * kCGSet + S_DONE] != c.epoch) return false;
+    return true;
+  };
+  // Batches of iterations, one of look-ahead: batch b is queued before the
+  // host waits for batch b - 1, whose apply kernels write the done flags to
+  // the mapped mirror.  Iterations queued after the end return at once.  The
+  // batches grow from 4: a solve of a few iterations queues few too many.
+  int cur = 0, nq = 0, batch = 4;
+  for (int it = 0;;) {
+    for (int k = 0; k < batch; k++, it++) {
+      c.par = it & 1;
+      c.init = it == 0;
+      a.c = a3.c = c;
       if (col)
-        rc = sizeof(T) == 8 ? GF_DISPATCH_N3(m->Niso, cgapply3c_d, m, a3)
-                            : GF_DISPATCH_N3(m->Niso, cgapply3c_f, m, a3);
+        RC(sizeof(T) == 8 ? GF_DISPATCH_N3(m->Niso, cgapply3c_d, m, a3)
+                          : GF_DISPATCH_N3(m->Niso, cgapply3c_f, m, a3));
       else
-        rc = sizeof(T) == 8 ? GF_DISPATCH_N(m->dim, m->Niso, launch_cg_apply_d, m, a)
-                            : GF_DISPATCH_N(m->dim, m->Niso, launch_cg_apply_f, m, a);
-      if (rc) return rc;
+        RC(sizeof(T) == 8 ? GF_DISPATCH_N(m->dim, m->Niso, launch_cg_apply_d, m, a)
+                          : GF_DISPATCH_N(m->dim, m->Niso, launch_cg_apply_f, m, a));
       if (m->ngroups && !gather)
         hipLaunchKernelGGL(k_dss_cg<T>, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
-                           v.q, m->goff, m->gmem, m->ngroups, (const double *)m->scal);
-      hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(kRedThreads), 0, s, m->scal, partA, nbA);
-      if (gather) {
-        switch (normtype) {
-          case GF_NORM_INF: rc = launch_update_box<T, GF_NORM_INF>(m, v, partU); break;
-          case GF_NORM_EUC: rc = launch_update_box<T, GF_NORM_EUC>(m, v, partU); break;
-          case GF_NORM_L2: rc = launch_update_box<T, GF_NORM_L2>(m, v, partU); break;
-          case GF_NORM_L1: rc = launch_update_box<T, GF_NORM_L1>(m, v, partU); break;
-          default: rc = launch_update_box<T, GF_NORM_ASSEMBLED_L2>(m, v, partU); break;
-        }
-        if (rc) return rc;
-      } else {
-        switch (normtype) {
-          case GF_NORM_INF: launch_update<T, GF_NORM_INF>(m, v, partU, col); break;
-          case GF_NORM_EUC: launch_update<T, GF_NORM_EUC>(m, v, partU, col); break;
-          case GF_NORM_L2: launch_update<T, GF_NORM_L2>(m, v, partU, col); break;
-          case GF_NORM_L1: launch_update<T, GF_NORM_L1>(m, v, partU, col); break;
-          default: launch_update<T, GF_NORM_ASSEMBLED_L2>(m, v, partU, col); break;
-        }
-      }
-      hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(kThreads), 0, s, m->scal, partU, kUpdBlocks,
-                         normtype, d_resid, m->hscal_dev);
+                           v.q, m->goff, m->gmem, m->ngroups,
+                           ns > 0 ? (const double *)nullptr
+                                  : (const double *)(m->scal + kCGSet * (c.par ^ 1) + S_DONE));
+      RC(launch_update_norm<T>(m, c, v, gather, col));
     }
     GF_LAUNCH_CHECK(m->ctx);
-    // One batch of look-ahead: batch b is queued before the host waits for
-    // batch b-1, whose last k_cg_beta has written the stopping flag into
-    // the mapped host mirror.  Iterations queued after convergence return
-    // at once (S_DONE).
     GF_HIP(m->ctx, hipEventRecord(m->cg_ev[cur], s));
     if (nq++ > 0) {
       GF_HIP(m->ctx, hipEventSynchronize(m->cg_ev[cur ^ 1]));
-      if (hm[S_DONE] != 0.0) break;
+      if (all_done()) break;
     }
     cur ^= 1;
+    batch = std::min(2 * batch, 32);
   }
-  // the final scalars, after everything queued has run
-  GF_HIP(m->ctx, hipMemcpyAsync(m->hscal, m->scal, S_COUNT * sizeof(double),
-                                hipMemcpyDeviceToHost, s));
-  GF_HIP(m->ctx, hipStreamSynchronize(s));
-  *iters = (int)m->hscal[S_ITER];
   return GF_OK;
 }
 
@@ -1795,89 +1613,6 @@ int seg_red(gf_mesh *m, const T *r, const T *z, const T *imult, int normtype,
   GF_HIP(m->ctx, hipMemcpyAsync(out.data(), dout, 2 * ns * sizeof(double), hipMemcpyDeviceToHost,
                                 m->ctx->stream));
   GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
-  return GF_OK;
-}
-
-// CG iterations of every member of a batched 3-D mesh (pencil apply, CSR
-// assembly) until all members are done; per-member scalars in m->sscal,
-// copied to m->hsscal at the end.
-template <typename T>
-int cg_loop_seg(gf_mesh *m, CGVecs<T> &v, int normtype) {
-  hipStream_t s = m->ctx->stream;
-  const int ns = m->nseg, nbU = m->h_seg_boff[ns];
-  const int nbA = col_blocks(m);
-  double *partA = m->red;  // one partial per element
-  double *partU = m->red + std::max((size_t)nbA, m->nelems) + 64;
-  CGApply3Args a3;
-  a3.r = v.r;
-  a3.dinv = v.dinv;
-  a3.dtab = nullptr;
-  a3.deq = nullptr;
-  a3.w = v.w;
-  a3.q = v.q;
-  a3.D = v.D;
-  for (int c = 0; c < 3; c++) {
-    a3.DR[c] = sizeof(T) == 8 ? (const void *)m->pDR[c] : (const void *)m->pDR32[c];
-    a3.DC[c] = sizeof(T) == 8 ? (const void *)m->pDC[c] : (const void *)m->pDC32[c];
-  }
-  a3.W = v.W;
-  a3.edx = v.edx;
-  a3.ejac = v.ejac;
-  a3.qf = v.qf;
-  a3.qs = v.qs;
-  a3.tmask = 0;
-  a3.topo = m->box;
-  a3.mask = m->has_mask ? v.mask : nullptr;
-  a3.p = v.p;
-  a3.scal = m->scal;
-  a3.part = partA;
-  a3.nelems = m->nelems;
-  a3.seg_eoff = m->seg_eoff;
-  a3.nseg = ns;
-  a3.sscal = m->sscal;
-  volatile double *hm = m->hscal;
-  GF_HIP(m->ctx, hipMemcpyAsync(m->hscal, m->scal, S_COUNT * sizeof(double),
-                                hipMemcpyDeviceToHost, s));
-  GF_HIP(m->ctx, hipStreamSynchronize(s));
-  int cur = 0, nq = 0;
-  while (hm[S_DONE] == 0.0) {
-    for (int bb = 0; bb < kBatch; bb++) {
-      int rc = sizeof(T) == 8 ? GF_DISPATCH_N3(m->Niso, cgapply3c_d, m, a3)
-                              : GF_DISPATCH_N3(m->Niso, cgapply3c_f, m, a3);
-      if (rc) return rc;
-      if (m->ngroups)
-        hipLaunchKernelGGL(k_dss_cg<T>, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
-                           v.q, m->goff, m->gmem, m->ngroups, (const double *)m->scal);
-      hipLaunchKernelGGL(k_cg_alpha_seg, dim3(1), dim3(1024), 0, s, m->sscal, partA, m->seg_eoff,
-                         ns, 1);
-      const T *mk = m->has_mask ? v.mask : nullptr;
-      switch (normtype) {
-#define GF_SEG_UPD(NT)                                                                        \
-  hipLaunchKernelGGL((k_cg_update_seg<T, NT>), dim3(nbU), dim3(kThreads), 0, s, v.x, v.w, v.r, \
-                     v.q, mk, v.dinv, v.imult, m->mass, (const double *)m->sscal, m->seg_eoff,  \
-                     m->seg_boff, ns, m->nn, partU);                                           \
-  break;
-        case GF_NORM_INF: GF_SEG_UPD(GF_NORM_INF)
-        case GF_NORM_EUC: GF_SEG_UPD(GF_NORM_EUC)
-        case GF_NORM_L2: GF_SEG_UPD(GF_NORM_L2)
-        case GF_NORM_L1: GF_SEG_UPD(GF_NORM_L1)
-        default: GF_SEG_UPD(GF_NORM_ASSEMBLED_L2)
-#undef GF_SEG_UPD
-      }
-      hipLaunchKernelGGL(k_cg_beta_seg, dim3(1), dim3(1024), 0, s, m->scal, m->sscal, partU,
-                         m->seg_boff, ns, normtype, m->hscal_dev);
-    }
-    GF_LAUNCH_CHECK(m->ctx);
-    GF_HIP(m->ctx, hipEventRecord(m->cg_ev[cur], s));
-    if (nq++ > 0) {
-      GF_HIP(m->ctx, hipEventSynchronize(m->cg_ev[cur ^ 1]));
-      if (hm[S_DONE] != 0.0) break;
-    }
-    cur ^= 1;
-  }
-  GF_HIP(m->ctx, hipMemcpyAsync(m->hsscal, m->sscal, (size_t)ns * kSegScal * sizeof(double),
-                                hipMemcpyDeviceToHost, s));
-  GF_HIP(m->ctx, hipStreamSynchronize(s));
   return GF_OK;
 }
 
@@ -1940,15 +1675,10 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
     if (bbv) RC(gf_mul_t(m, rr, m->mask, rr));
     return GF_OK;
   };
-  std::vector<double> hs((size_t)ns * kSegScal, 0.0);
+  std::vector<double> hs((size_t)ns * kCGScal, 0.0);
   auto upload = [&]() -> int {
-    bool all = true;
-    for (int k = 0; k < ns; k++) all = all && hs[(size_t)k * kSegScal + S_DONE] != 0.0;
-    double g[S_COUNT] = {0};
-    g[S_DONE] = all ? 1.0 : 0.0;
     GF_HIP(m->ctx, hipMemcpyAsync(m->sscal, hs.data(), hs.size() * sizeof(double),
                                   hipMemcpyHostToDevice, s));
-    GF_HIP(m->ctx, hipMemcpyAsync(m->scal, g, sizeof(g), hipMemcpyHostToDevice, s));
     GF_HIP(m->ctx, hipStreamSynchronize(s));
     return GF_OK;
   };
@@ -1962,7 +1692,7 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
     if (dinv) RC(gf_mul_t(m, dinv, r, z));
     RC(seg_red<double>(m, r, dinv ? z : r, m->imult, normtype, o));
     for (int k = 0; k < ns; k++) {
-      double *h = &hs[(size_t)k * kSegScal];
+      double *h = &hs[(size_t)k * kCGScal];
       h[S_RHO] = o[2 * k];
       h[S_RTOL] = rtol[k];
       h[S_RNORM] = 10.0 * rtol[k];
@@ -1990,9 +1720,9 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
     for (int c = 0; c < 6; c++) v.G[c] = m->G[c];
     v.mass = m->mass;
     v.p = prm->p_scalar;
-    RC(cg_loop_seg<double>(m, v, normtype));
+    RC(cg_loop<double>(m, v, normtype, (double *)nullptr));
     for (int k = 0; k < ns; k++) {
-      const double *h = &m->hsscal[(size_t)k * kSegScal];
+      const double *h = &m->hsscal[(size_t)k * kCGSet];
       m->seg_iters[k] = (int)h[S_ITER];
       m->seg_rnorm[k] = h[S_RNORM];
       if (m->seg_iters[k] >= prm->maxit && h[S_RNORM] > prm->tol) status = GF_ERR_NOCONVERGE;
@@ -2041,8 +1771,8 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
       if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
       RC(seg_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, o));
       for (int k = 0; k < ns; k++) {
-        double *h = &hs[(size_t)k * kSegScal];
-        std::fill(h, h + kSegScal, 0.0);
+        double *h = &hs[(size_t)k * kCGScal];
+        std::fill(h, h + kCGScal, 0.0);
         if (conv[k]) {
           h[S_DONE] = 1.0;
           continue;
@@ -2059,10 +1789,10 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
         h[S_N] = nseg_n[k];
       }
       RC(upload());
-      RC(cg_loop_seg<float>(m, v, normtype));
+      RC(cg_loop<float>(m, v, normtype, (double *)nullptr));
       for (int k = 0; k < ns; k++) {
         if (conv[k]) continue;
-        const double *h = &m->hsscal[(size_t)k * kSegScal];
+        const double *h = &m->hsscal[(size_t)k * kCGSet];
         m->seg_iters[k] += (int)h[S_ITER];
         rhom[k] = h[S_RHOM];
         first[k] = 0;
@@ -2198,12 +1928,15 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
     for (int c = 0; c < 6; c++) v.G[c] = m->G[c];
     v.mass = m->mass;
     v.p = prm->p_scalar;
-    int it = 0;
-    RC(cg_loop<double>(m, v, normtype, d_resid, &it));
+    RC(cg_loop<double>(m, v, normtype, d_resid));
+    const int it = (int)m->hscal[S_ITER];
     total_iters = it;
     rn_final = m->hscal[S_RNORM];
-    if (prm->resid && it > 0)
-      GF_HIP(m->ctx, hipMemcpy(prm->resid, d_resid, it * sizeof(double), hipMemcpyDeviceToHost));
+    if (prm->resid && it > 0) {
+      GF_HIP(m->ctx, hipMemcpyAsync(prm->resid, d_resid, it * sizeof(double),
+                                    hipMemcpyDeviceToHost, s));
+      GF_HIP(m->ctx, hipStreamSynchronize(s));
+    }
     if (it >= prm->maxit && rn_final > prm->tol) status = GF_ERR_NOCONVERGE;
   } else {
     // Mixed precision: the CG recurrences (apply, direction, residual and
@@ -2272,9 +2005,8 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
       hs[S_VOL] = volume;
       hs[S_N] = (double)n;
       GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, sizeof(hs), hipMemcpyHostToDevice, s));
-      int it = 0;
-      RC(cg_loop<float>(m, v, normtype, (double *)nullptr, &it));
-      total_iters += it;
+      RC(cg_loop<float>(m, v, normtype, (double *)nullptr));
+      total_iters += (int)m->hscal[S_ITER];
       first = false;
     }
     if (rn_final > rtol) status = GF_ERR_NOCONVERGE;
@@ -2307,6 +2039,8 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
   (void)hipFree(m->seg_eoff);
   (void)hipFree(m->seg_boff);
   (void)hipFree(m->sscal);
+  (void)hipFree(m->seg_topo);
+  m->seg_topo = nullptr;
   if (m->hsscal) (void)hipHostFree(m->hsscal);
   m->seg_eoff = nullptr;
   m->seg_boff = nullptr;
@@ -2328,13 +2062,12 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
     const double frac = (double)(eoff[k + 1] - eoff[k]) / (double)m->nelems;
     m->h_seg_boff[k + 1] = m->h_seg_boff[k] + std::max(1, (int)(frac * budget + 0.5));
   }
-  // the reduction buffer holds the apply partials (one per logical block),
-  // then the update blocks' pairs, and the set-up pairs plus one pair per
-  // member for the per-member reductions
+  // the reduction buffer holds one apply partial per block and the update
+  // blocks' pairs, or the set-up pairs plus one pair per member
   {
     const int nbU = m->h_seg_boff[nseg];
-    const size_t need = std::max(std::max((size_t)col_blocks(m), m->nelems) + 64 + 2 * (size_t)nbU,
-                                 2 * (size_t)nbU + 64 + 2 * (size_t)nseg) + 64;
+    const size_t nbg = xcd_grid(nbU);
+    const size_t need = std::max(3 * nbg + 128, 2 * nbg + 64 + 2 * (size_t)nseg) + 64;
     if (m->red_cap < need) {
       GF_HIP(m->ctx, hipFree(m->red));
       m->red = nullptr;
@@ -2344,9 +2077,11 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
   }
   GF_HIP(m->ctx, hipMalloc((void **)&m->seg_eoff, (nseg + 1) * sizeof(int64_t)));
   GF_HIP(m->ctx, hipMalloc((void **)&m->seg_boff, (nseg + 1) * sizeof(int)));
-  GF_HIP(m->ctx, hipMalloc((void **)&m->sscal, (size_t)nseg * kSegScal * sizeof(double)));
-  GF_HIP(m->ctx, hipHostMalloc((void **)&m->hsscal, (size_t)nseg * kSegScal * sizeof(double),
-                               hipHostMallocDefault));
+  GF_HIP(m->ctx, hipMalloc((void **)&m->sscal, (size_t)nseg * kCGScal * sizeof(double)));
+  GF_HIP(m->ctx, hipHostMalloc((void **)&m->hsscal, (size_t)nseg * kCGSet * sizeof(double),
+                               hipHostMallocMapped | hipHostMallocCoherent));
+  memset(m->hsscal, 0, (size_t)nseg * kCGSet * sizeof(double));
+  GF_HIP(m->ctx, hipHostGetDevicePointer((void **)&m->hsscal_dev, m->hsscal, 0));
   GF_HIP(m->ctx, hipMemcpy(m->seg_eoff, eoff, (nseg + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
   GF_HIP(m->ctx, hipMemcpy(m->seg_boff, m->h_seg_boff.data(), (nseg + 1) * sizeof(int),
                            hipMemcpyHostToDevice));
@@ -2364,6 +2099,19 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
   if (bad != 0.0) {
     gf_mesh_set_segments(m, 0, nullptr);
     return gf_set_err(m->ctx, GF_ERR_ARG, "segments: a GGFX group joins two members");
+  }
+  // members that are the boxes the mesh was built from (their groups are the
+  // lattice's): the CG update assembles by gather
+  std::vector<gf::BoxTopo> topos;
+  size_t at = 0;
+  for (size_t k = 0; k < m->h_boxes.size() && (int)k < nseg && eoff[k] == (int64_t)at; k++) {
+    topos.push_back(m->h_boxes[k]);
+    at += (size_t)m->h_boxes[k].ne[0] * m->h_boxes[k].ne[1] * m->h_boxes[k].ne[2];
+  }
+  if ((int)topos.size() == nseg && m->h_boxes.size() == topos.size() && at == m->nelems) {
+    GF_HIP(m->ctx, hipMalloc((void **)&m->seg_topo, topos.size() * sizeof(gf::BoxTopo)));
+    GF_HIP(m->ctx, hipMemcpy(m->seg_topo, topos.data(), topos.size() * sizeof(gf::BoxTopo),
+                             hipMemcpyHostToDevice));
   }
   return GF_OK;
 }
@@ -2463,6 +2211,31 @@ __global__ void k_fill_pattern_f(float *a, size_t n, float s) {
 }
 }  // namespace
 
+// Scalars of a running iteration for the timed CG kernels: both sets hold a
+// system that is never done, the partial sums are zero.
+static int timing_scalars(gf_mesh *m, CGCtl &c) {
+  memset(&c, 0, sizeof(c));
+  c.scal = m->scal;
+  c.nelems = m->nelems;
+  c.partA = m->red;
+  c.partU = m->red + 4096;
+  c.normtype = GF_NORM_ASSEMBLED_L2;
+  double hs[kCGScal] = {0};
+  for (int p = 0; p < 2; p++) {
+    double *h = hs + p * kCGSet;
+    h[S_RHO] = 1.0;
+    h[S_RTOL] = -1.0;
+    h[S_MAXIT] = 1e9;
+  }
+  hs[kCGAlpha] = 1e-3;
+  GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, sizeof(hs), hipMemcpyHostToDevice, m->ctx->stream));
+  hipLaunchKernelGGL(k_fill_pattern, dim3(64), dim3(kThreads), 0, m->ctx->stream, m->red,
+                     (size_t)(4096 + 2 * 4096), 0.0);
+  GF_LAUNCH_CHECK(m->ctx);
+  GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
+  return GF_OK;
+}
+
 extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *avg_ms) {
   if (!m || !which || reps < 1 || !avg_ms) return GF_ERR_ARG;
   if (m->gtype != GF_GE_REGULAR || !m->Niso)
@@ -2481,14 +2254,9 @@ extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *a
   GF_LAUNCH_CHECK(m->ctx);
   std::function<int()> launch;
   StageArgs sa;
-  CGApplyArgs ca;
   memset(&sa, 0, sizeof(sa));
-  memset(&ca, 0, sizeof(ca));
   CGApply3Args ca3;
-  ca3.seg_eoff = nullptr;
-  ca3.nseg = 0;
-  ca3.sscal = nullptr;
-  memset(&ca3, 0, sizeof(ca3));
+  CGCtl ctl;
   const bool pencil = w == "burgers_stage" || w == "cg_apply" || w == "cg_apply_f32" ||
                       w == "burgers_stage_box";
   if (pencil && m->dim == 3 && !m->dconst)
@@ -2518,39 +2286,26 @@ extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *a
   } else if (w == "cg_apply" || w == "cg_apply_f32") {
     if (m->dim != 3) return gf_set_err(m->ctx, GF_ERR_UNSUPPORTED, "cg_apply timing: 3-D meshes");
     bool f32 = w == "cg_apply_f32";
-    double hs[12] = {0};
-    hs[S_BETA] = 0.5;
-    hs[S_FIRST] = 0.0;
-    hs[S_DONE] = 0.0;
-    GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, sizeof(hs), hipMemcpyHostToDevice, s));
+    RC(timing_scalars(m, ctl));
+    ctl.nbA = f32 ? blocks3<float>(m) : blocks3<double>(m);
+    ctl.nbU = ctl.nbA;
     if (f32) {
-      for (int k = 0; k < 4; k++)
+      for (int k = 0; k < 5; k++)
         hipLaunchKernelGGL(k_fill_pattern_f, dim3(nblocks(n)), dim3(kThreads), 0, s,
                            (float *)buf[k], n, 0.5f + 0.1f * k);
     }
+    ca3 = apply3_args(m, ctl);
     ca3.r = buf[0];
     ca3.dinv = buf[1];
-    ca3.dtab = nullptr;
-    ca3.deq = nullptr;
     ca3.w = buf[2];
     ca3.q = buf[3];
-    ca3.D = f32 ? (const void *)m->D32 : (const void *)m->D[0];
-    for (int c = 0; c < 3; c++) {
-      ca3.DR[c] = f32 ? (const void *)m->pDR32[c] : (const void *)m->pDR[c];
-      ca3.DC[c] = f32 ? (const void *)m->pDC32[c] : (const void *)m->pDC[c];
-    }
+    ca3.x = buf[4];
     ca3.W = f32 ? (const void *)m->W32 : (const void *)m->W[0];
     ca3.edx = f32 ? (const void *)m->edx32 : (const void *)m->edx;
     ca3.ejac = f32 ? (const void *)m->ejac32 : (const void *)m->ejac;
-    ca3.qf = nullptr;
     ca3.qs = 1.0;
-    ca3.mask = nullptr;
-    ca3.topo = m->box;
     ca3.tmask = (m->has_mask && m->has_box_mask) ? 1 : 0;
     ca3.p = 0.1;
-    ca3.scal = m->scal;
-    ca3.part = m->red;
-    ca3.nelems = m->nelems;
     if (f32)
       launch = [&]() { return GF_DISPATCH_N3(m->Niso, cgapply3c_f, m, ca3); };
     else
@@ -2572,46 +2327,31 @@ extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *a
                             1e-5 / 6.0, 1e-5 / 3.0, 0.02, 1, 1);
     };
   } else if (w == "cg_update" || w == "cg_update_f32") {
-    // CG update with the Jacobi preconditioner: x, w, r, q (the diagonal
-    // formed in the kernel on a uniform box, else read from dinv)
+    // CG update with the Jacobi preconditioner: reads q (gathered), r, dinv;
+    // writes r
     if (m->dim != 3 || !m->has_box)
       return gf_set_err(m->ctx, GF_ERR_UNSUPPORTED, "cg_update timing: structured 3-D boxes");
     bool f32 = w == "cg_update_f32";
-    double hs[S_COUNT] = {0};
-    hs[S_ALPHA] = 1e-3;
-    GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, sizeof(hs), hipMemcpyHostToDevice, s));
+    RC(timing_scalars(m, ctl));
+    ctl.nbA = ctl.nbU = f32 ? blocks3<float>(m) : blocks3<double>(m);
     if (f32) {
       for (int k = 0; k < 5; k++)
         hipLaunchKernelGGL(k_fill_pattern_f, dim3(nblocks(n)), dim3(kThreads), 0, s,
                            (float *)buf[k], n, 0.5f + 0.1f * k);
       launch = [&]() {
         CGVecs<float> v{};
-        v.x = (float *)buf[0];
-        v.w = (float *)buf[1];
         v.r = (float *)buf[2];
         v.q = (float *)buf[3];
         v.dinv = (const float *)buf[4];
-        v.W = m->W32;
-        v.edx = m->edx32;
-        v.ejac = m->ejac32;
-        v.p = 0.1;
-        v.qs = 1.0;
-        return launch_update_box<float, GF_NORM_ASSEMBLED_L2>(m, v, m->red);
+        return launch_update_norm<float>(m, ctl, v, true, true);
       };
     } else {
       launch = [&]() {
         CGVecs<double> v{};
-        v.x = buf[0];
-        v.w = buf[1];
         v.r = buf[2];
         v.q = buf[3];
         v.dinv = buf[4];
-        v.W = m->W[0];
-        v.edx = m->edx;
-        v.ejac = m->ejac;
-        v.p = 0.1;
-        v.qs = 1.0;
-        return launch_update_box<double, GF_NORM_ASSEMBLED_L2>(m, v, m->red);
+        return launch_update_norm<double>(m, ctl, v, true, true);
       };
     }
   } else if (w == "helmholtz") {

@@ -142,14 +142,14 @@ class Mesh:
         if use_mask and getattr(grid, "mask", None) is not None:
             d.mask = host(grid.mask)
         devmaps = getattr(grid, "device_maps", False)
+        bl = getattr(grid, "box_list", None)
+        if bl is not None:
+            arr = (ctypes.c_int * len(bl))(*[int(v) for v in bl])
+            keep.append(arr)
+            d.box_count = len(bl) // 6
+            d.box_list = arr
         if devmaps:
             d.box_device_maps = 1
-            bl = getattr(grid, "box_list", None)
-            if bl is not None:
-                arr = (ctypes.c_int * len(bl))(*[int(v) for v in bl])
-                keep.append(arr)
-                d.box_count = len(bl) // 6
-                d.box_list = arr
         else:
             offs = np.ascontiguousarray(grid.ggfx_offs, dtype=np.int64)
             mem = np.ascontiguousarray(grid.ggfx_members, dtype=np.int64)

@@ -62,8 +62,10 @@ class _UnionGrid:
         self.mask = None
         self.ne = None  # no single box structure: CSR DSS path
         self.device_maps = bool(device_maps)
+        # the boxes in sequence: device-built groups follow from them, host
+        # groups are checked against them
+        self.box_list = [v for g in grids for v in list(g.ne) + list(g.periodic)]
         if self.device_maps:
-            self.box_list = [v for g in grids for v in list(g.ne) + list(g.periodic)]
             self.ggfx_offs = self.ggfx_members = None
             return
         offs, mem, base = [np.zeros(1, dtype=np.int64)], [], 0
