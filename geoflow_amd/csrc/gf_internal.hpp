@@ -101,6 +101,9 @@ struct gf_mesh_s {
   // CG update gathers), and the boxes as given at creation (host)
   gf::BoxTopo *seg_topo = nullptr;
   std::vector<gf::BoxTopo> h_boxes;
+  void *seg_blk = nullptr;          // block table of the CG kernels (device)
+  std::vector<double> seg_vol;      // member volumes (sums of the mass)
+  double volume = -1.0;             // sum of the mass, formed by the first solve
   double cg_epoch = 0.0;            // number of the CG loop (done flags in the mirrors)
   double *sscal = nullptr;          // per-member solver scalars (device)
   double *hsscal = nullptr, *hsscal_dev = nullptr;  // mapped host mirror of sscal

@@ -1174,7 +1174,7 @@ int gf_mesh_destroy(gf_mesh *m) {
   for (int k = 0; k < 6; k++) F(m->G32[k]);
   F(m->mass32);
   if (m->hscal) (void)hipHostFree(m->hscal);
-  F(m->seg_eoff); F(m->seg_boff); F(m->sscal); F(m->seg_topo); F(m->dl_I); F(m->dl_wq);
+  F(m->seg_eoff); F(m->seg_boff); F(m->sscal); F(m->seg_topo); F(m->seg_blk); F(m->dl_I); F(m->dl_wq);
   if (m->hsscal) (void)hipHostFree(m->hsscal);
   for (int k = 0; k < 2; k++)
     if (m->cg_ev[k]) (void)hipEventDestroy(m->cg_ev[k]);

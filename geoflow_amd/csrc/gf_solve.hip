@@ -1280,6 +1280,28 @@ int check_finite(gf_mesh *m, double *const *u, int nev) {
 
 }  // namespace
 
+namespace {
+// Queues the assembled Jacobi diagonal inverse; scal[63] becomes 1 where an
+// entry is not positive: a Jacobi preconditioner needs a positive assembled
+// diagonal; a strongly sheared deformed element (whose doubled off-diagonal
+// metric terms enter it) or p = q = 0 can break that.
+int diag_inv(gf_mesh *m, double p, double qs, const double *qf, double *dinv) {
+  if (!m->Niso) return gf_set_err(m->ctx, GF_ERR_UNSUPPORTED, "Jacobi diagonal: isotropic meshes");
+  RC(GF_DISPATCH_N(m->dim, m->Niso, launch_diag, m, p, qf, qs, dinv));
+  RC(gf_dss_t(m, GF_DSS_SUM, dinv));
+  double *bad = m->scal + 63;
+  GF_HIP(m->ctx, hipMemsetAsync(bad, 0, sizeof(double), m->ctx->stream));
+  hipLaunchKernelGGL(k_recip_pos, dim3(nblocks(m->ndof)), dim3(kThreads), 0, m->ctx->stream, dinv,
+                     bad, m->ndof);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+int diag_status(gf_mesh *m, double bad) {
+  return bad != 0.0 ? gf_set_err(m->ctx, GF_ERR_PRECOND, "Jacobi: assembled diagonal not positive")
+                    : GF_OK;
+}
+}  // namespace
+
 extern "C" {
 
 int gf_burgers_step(gf_mesh *m, int mode, double nu, int order, int nstate, double t, double dt,
@@ -1349,23 +1371,12 @@ int gf_burgers_steps_mixed(gf_mesh *m, int mode, double nu, int order, int nstat
 
 int gf_helmholtz_diag_inv(gf_mesh *m, double p, double qs, const double *qf, double *dinv) {
   if (!m || !dinv) return GF_ERR_ARG;
-  if (!m->Niso) return gf_set_err(m->ctx, GF_ERR_UNSUPPORTED, "Jacobi diagonal: isotropic meshes");
-  RC(GF_DISPATCH_N(m->dim, m->Niso, launch_diag, m, p, qf, qs, dinv));
-  RC(gf_dss_t(m, GF_DSS_SUM, dinv));
-  // a Jacobi preconditioner needs a positive assembled diagonal; a strongly
-  // sheared deformed element (whose doubled off-diagonal metric terms enter
-  // it) or p = q = 0 can break that
-  double *bad = m->scal + 63;
-  GF_HIP(m->ctx, hipMemsetAsync(bad, 0, sizeof(double), m->ctx->stream));
-  hipLaunchKernelGGL(k_recip_pos, dim3(nblocks(m->ndof)), dim3(kThreads), 0, m->ctx->stream, dinv,
-                     bad, m->ndof);
-  GF_LAUNCH_CHECK(m->ctx);
+  RC(diag_inv(m, p, qs, qf, dinv));
   double hb = 0.0;
-  GF_HIP(m->ctx, hipMemcpyAsync(&hb, bad, sizeof(double), hipMemcpyDeviceToHost, m->ctx->stream));
+  GF_HIP(m->ctx, hipMemcpyAsync(&hb, m->scal + 63, sizeof(double), hipMemcpyDeviceToHost,
+                                m->ctx->stream));
   GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
-  if (hb != 0.0)
-    return gf_set_err(m->ctx, GF_ERR_PRECOND, "Jacobi: assembled diagonal not positive");
-  return GF_OK;
+  return diag_status(m, hb);
 }
 
 }  // extern "C"
@@ -1375,16 +1386,24 @@ int gf_helmholtz_diag_inv(gf_mesh *m, double p, double qs, const double *qf, dou
 // ===========================================================================
 namespace {
 
-// Reduce (r.z.imult, norm(r)) at set-up, synchronous; returns both.
+// Set-up scalars of a solve on the device, m->scal: the (r.z.imult, norm)
+// pairs of set-up reductions and the preconditioner's flag, read back together.
+enum { SU_B = 56, SU_R = 58, SU_R32 = 60, SU_BAD = 63, SU_COUNT = 8 };
+
+// Queues the reduction of (r.z.imult, norm(r)) to scal[slot], scal[slot + 1].
 template <typename T>
-int setup_red(gf_mesh *m, const T *r, const T *z, const T *imult, int normtype, double out[2]) {
+int setup_red(gf_mesh *m, const T *r, const T *z, const T *imult, int normtype, int slot) {
   hipLaunchKernelGGL(k_setup_red<T>, dim3(kUpdBlocks), dim3(kThreads), 0, m->ctx->stream, r, z,
                      imult, m->mass, normtype, m->red, m->ndof);
   hipLaunchKernelGGL(k_setup_fin, dim3(1), dim3(kThreads), 0, m->ctx->stream, m->red, kUpdBlocks,
-                     normtype, m->scal + 60);
+                     normtype, m->scal + slot);
   GF_LAUNCH_CHECK(m->ctx);
-  GF_HIP(m->ctx, hipMemcpyAsync(out, m->scal + 60, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                                m->ctx->stream));
+  return GF_OK;
+}
+// Waits and returns the set-up scalars: out[slot - SU_B].
+int setup_get(gf_mesh *m, double (&out)[SU_COUNT]) {
+  GF_HIP(m->ctx, hipMemcpyAsync(out, m->scal + SU_B, SU_COUNT * sizeof(double),
+                                hipMemcpyDeviceToHost, m->ctx->stream));
   GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
   return GF_OK;
 }
@@ -1472,9 +1491,9 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
   const bool gather = col && (ns > 0 ? m->seg_topo != nullptr : m->has_box);
   CGCtl c;
   c.scal = ns > 0 ? m->sscal : m->scal;
-  c.eoff = m->seg_eoff;
-  c.boff = m->seg_boff;
+  c.blk = (const CGSegBlock *)m->seg_blk;
   c.nseg = ns;
+  c.nblk = ns > 0 ? m->h_seg_boff[ns] : 0;
   c.nelems = m->nelems;
   if (ns > 0) {
     c.nbA = c.nbU = xcd_grid(m->h_seg_boff[ns]);
@@ -1536,8 +1555,9 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
   };
   // Batches of iterations, one of look-ahead: batch b is queued before the
   // host waits for batch b - 1, whose apply kernels write the done flags to
-  // the mapped mirror.  Iterations queued after the end return at once.  The
-  // batches grow from 4: a solve of a few iterations queues few too many.
+  // the mapped mirror.  Iterations queued after the end return at once, but
+  // each still costs its launches (5-20 us), so the batches grow slowly, from 4 by
+  // a quarter of the iterations done.
   int cur = 0, nq = 0, batch = 4;
   for (int it = 0;;) {
     for (int k = 0; k < batch; k++, it++) {
@@ -1564,7 +1584,7 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
       if (all_done()) break;
     }
     cur ^= 1;
-    batch = std::min(2 * batch, 32);
+    batch = std::min(std::max(4, it / 4), 32);
   }
   return GF_OK;
 }
@@ -1594,24 +1614,26 @@ int cg_check_args(gf_mesh *m, const gf_cg_params *prm, const double *b, double *
 }
 
 // ---- CG on a batched mesh (members set by gf_mesh_set_segments) -----------
-__global__ void k_fill_d(double *__restrict__ o, double v, size_t n) {
-  GRID_LOOP(g, n) o[g] = v;
-}
 
-// Per-member (rho, norm sum) of r (and z): out[2s], out[2s+1]; synchronous.
+// Queues the per-member (rho, norm sum) of r (and z) to set `at` of the
+// reductions' results.
 template <typename T>
-int seg_red(gf_mesh *m, const T *r, const T *z, const T *imult, int normtype,
-            std::vector<double> &out) {
+int seg_red(gf_mesh *m, const T *r, const T *z, const T *imult, int normtype, int at) {
   const int ns = m->nseg, nbU = m->h_seg_boff[ns];
-  double *dout = m->red + 2 * (size_t)nbU + 64;
   hipLaunchKernelGGL(k_setup_red_seg<T>, dim3(nbU), dim3(kThreads), 0, m->ctx->stream, r, z, imult,
                      m->mass, normtype, m->seg_eoff, m->seg_boff, ns, m->nn, m->red);
   hipLaunchKernelGGL(k_setup_fin_seg, dim3(1), dim3(1024), 0, m->ctx->stream, m->red, m->seg_boff,
-                     ns, normtype, dout);
+                     ns, normtype, m->red + 2 * (size_t)(nbU + at * ns) + 64);
   GF_LAUNCH_CHECK(m->ctx);
-  out.resize(2 * (size_t)ns);
-  GF_HIP(m->ctx, hipMemcpyAsync(out.data(), dout, 2 * ns * sizeof(double), hipMemcpyDeviceToHost,
-                                m->ctx->stream));
+  return GF_OK;
+}
+// Waits and returns the results of sets 0 .. nset-1: out[2 (set ns + s)] (rho)
+// and the norm sum after it.
+int seg_get(gf_mesh *m, int nset, std::vector<double> &out) {
+  const int ns = m->nseg, nbU = m->h_seg_boff[ns];
+  out.resize(2 * (size_t)ns * nset);
+  GF_HIP(m->ctx, hipMemcpyAsync(out.data(), m->red + 2 * (size_t)nbU + 64,
+                                out.size() * sizeof(double), hipMemcpyDeviceToHost, m->ctx->stream));
   GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
   return GF_OK;
 }
@@ -1631,13 +1653,10 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
   const int normtype = prm->normtype;
   double *r = wk.r, *w = wk.w, *q = wk.q, *dinv = wk.dinv;
   const double qs = prm->q_field ? 0.0 : prm->q_scalar;
-  std::vector<double> o, vol(ns), nseg_n(ns), rn0(ns), rtol(ns);
+  std::vector<double> o, nseg_n(ns), rn0(ns), rtol(ns);
+  const std::vector<double> &vol = m->seg_vol;
   for (int k = 0; k < ns; k++)
     nseg_n[k] = (double)((m->h_seg_eoff[k + 1] - m->h_seg_eoff[k]) * (int64_t)m->nn);
-  // member volumes: sum of the mass (the L1 norm of ones)
-  hipLaunchKernelGGL(k_fill_d, dim3(nblocks(n)), dim3(kThreads), 0, s, w, 1.0, n);
-  RC(seg_red<double>(m, w, nullptr, m->imult, GF_NORM_L1, o));
-  for (int k = 0; k < ns; k++) vol[k] = o[2 * k + 1];
   auto fin = [&](int k, double v) {
     switch (normtype) {
       case GF_NORM_INF: return v;
@@ -1647,26 +1666,27 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
       default: return std::sqrt(v);
     }
   };
-  if (prm->precond) RC(gf_helmholtz_diag_inv(m, prm->p_scalar, qs, prm->q_field, dinv));
-  if (bbv) {
-    RC(gf_mul_t(m, x, m->mask, x));
-    RC(gf_axpy_t(m, 1.0, xb, x));
-  }
+  if (prm->precond) RC(diag_inv(m, prm->p_scalar, qs, prm->q_field, dinv));
+  const double *nb = b;  // the stopping test's right-hand side
   if (normtype == GF_NORM_ASSEMBLED_L2) {
     RC(copy(m, q, b));
     RC(gf_dss_t(m, GF_DSS_SUM, q));
     if (bbv) RC(gf_mul_t(m, q, m->mask, q));
-    RC(seg_red<double>(m, q, nullptr, m->imult, normtype, o));
-    for (int k = 0; k < ns; k++) {
-      rn0[k] = fin(k, o[2 * k + 1]);
-      rtol[k] = prm->tol * rn0[k];
-    }
-  } else {
-    RC(seg_red<double>(m, b, nullptr, m->imult, normtype, o));
-    for (int k = 0; k < ns; k++) {
-      rn0[k] = fin(k, o[2 * k + 1]);
-      rtol[k] = rn0[k] < 1.0 ? prm->tol : prm->tol * rn0[k];
-    }
+    nb = q;
+  }
+  RC(seg_red<double>(m, nb, nullptr, m->imult, normtype, 0));
+  double bad = 0.0;
+  if (prm->precond)
+    GF_HIP(m->ctx, hipMemcpyAsync(&bad, m->scal + SU_BAD, sizeof(double), hipMemcpyDeviceToHost, s));
+  RC(seg_get(m, 1, o));
+  RC(diag_status(m, bad));
+  for (int k = 0; k < ns; k++) {
+    rn0[k] = fin(k, o[2 * k + 1]);
+    rtol[k] = prm->tol * (normtype != GF_NORM_ASSEMBLED_L2 && rn0[k] < 1.0 ? 1.0 : rn0[k]);
+  }
+  if (bbv) {
+    RC(gf_mul_t(m, x, m->mask, x));
+    RC(gf_axpy_t(m, 1.0, xb, x));
   }
   auto residual = [&](double *rr) -> int {
     RC(gf_helm_t(m, prm->p_scalar, nullptr, prm->q_field, qs, x, q));
@@ -1679,7 +1699,6 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
   auto upload = [&]() -> int {
     GF_HIP(m->ctx, hipMemcpyAsync(m->sscal, hs.data(), hs.size() * sizeof(double),
                                   hipMemcpyHostToDevice, s));
-    GF_HIP(m->ctx, hipStreamSynchronize(s));
     return GF_OK;
   };
   m->seg_iters.assign(ns, 0);
@@ -1690,7 +1709,8 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
     RC(residual(r));
     double *z = q;
     if (dinv) RC(gf_mul_t(m, dinv, r, z));
-    RC(seg_red<double>(m, r, dinv ? z : r, m->imult, normtype, o));
+    RC(seg_red<double>(m, r, dinv ? z : r, m->imult, normtype, 0));
+    RC(seg_get(m, 1, o));
     for (int k = 0; k < ns; k++) {
       double *h = &hs[(size_t)k * kCGScal];
       h[S_RHO] = o[2 * k];
@@ -1757,7 +1777,14 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
       if (outer > 0)
         hipLaunchKernelGGL(k_add_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, x, x32, 1.0, n);
       RC(residual(r));
-      RC(seg_red<double>(m, r, nullptr, m->imult, normtype, o));
+      // the residual's norm, and rho of the next FP32 cycle (not used when
+      // every member has converged), with one wait
+      RC(seg_red<double>(m, r, nullptr, m->imult, normtype, 0));
+      hipLaunchKernelGGL(k_to_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, r32, r, 1.0, n);
+      float *z32 = q32;
+      if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
+      RC(seg_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, 1));
+      RC(seg_get(m, 2, o));
       bool all = true;
       for (int k = 0; k < ns; k++) {
         m->seg_rnorm[k] = fin(k, o[2 * k + 1]);
@@ -1765,11 +1792,8 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
         all = all && conv[k];
       }
       if (all || outer >= 10000) break;
-      hipLaunchKernelGGL(k_to_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, r32, r, 1.0, n);
       hipLaunchKernelGGL(k_fill_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, x32, 0.0f, n);
-      float *z32 = q32;
-      if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
-      RC(seg_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, o));
+      const double *o32 = o.data() + 2 * ns;
       for (int k = 0; k < ns; k++) {
         double *h = &hs[(size_t)k * kCGScal];
         std::fill(h, h + kCGScal, 0.0);
@@ -1777,9 +1801,9 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
           h[S_DONE] = 1.0;
           continue;
         }
-        const double rn32 = fin(k, o[2 * k + 1]);
-        h[S_RHO] = o[2 * k];
-        h[S_BETA] = first[k] ? 0.0 : o[2 * k] / rhom[k];
+        const double rn32 = fin(k, o32[2 * k + 1]);
+        h[S_RHO] = o32[2 * k];
+        h[S_BETA] = first[k] ? 0.0 : o32[2 * k] / rhom[k];
         h[S_RHOM] = first[k] ? 0.0 : rhom[k];
         h[S_RTOL] = std::max(delta * rn32, 0.5 * rtol[k]);
         h[S_RNORM] = rn32;
@@ -1843,17 +1867,13 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
   bool bbv = xb != nullptr;
   const double *mask = bbv ? m->mask : nullptr;
   double *r = wk.r, *w = wk.w, *q = wk.q, *dinv = wk.dinv, *d_resid = wk.resid;
-  double volume = 0.0;
-  {
-    double *one = w;
-    hipLaunchKernelGGL(k_axpby, dim3(nblocks(n)), dim3(kThreads), 0, s, one, 0.0, b, 0.0, b, n);
-    // integrate(1) = sum of mass
-    RC(gf_dot_t(m, m->mass, nullptr, n, &volume));
-  }
+  // integrate(1) = sum of mass, a constant of the mesh
+  if (m->volume < 0.0) RC(gf_dot_t(m, m->mass, nullptr, n, &m->volume));
+  const double volume = m->volume;
   // mass term: the q field, else the scalar q (GHelmholtz with a one-entry q,
   // ghelmholtz.ipp:184-186, 370-373)
   const double qs = prm->q_field ? 0.0 : prm->q_scalar;
-  if (prm->precond) RC(gf_helmholtz_diag_inv(m, prm->p_scalar, qs, prm->q_field, dinv));
+  if (prm->precond) RC(diag_inv(m, prm->p_scalar, qs, prm->q_field, dinv));
   const bool dtabv = prm->precond && m->deq;
   if (dtabv) {
     hipLaunchKernelGGL(k_dinv_table, dim3((unsigned)std::min<size_t>(m->nelems, 65536)),
@@ -1861,25 +1881,25 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
                        m->deq);
     GF_LAUNCH_CHECK(m->ctx);
   }
-  if (bbv) {  // x = x*mask + xb (gcg.ipp:371-375)
-    RC(gf_mul_t(m, x, m->mask, x));
-    RC(gf_axpy_t(m, 1.0, xb, x));
-  }
   // stopping reference: norm of b (compute_norm(b), gcg.ipp:290-291)
-  double red2[2];
-  double rnorm0, rtol;
-  int normtype = prm->normtype;
+  double su[SU_COUNT];
+  const int normtype = prm->normtype;
+  const double *nb = b;
   if (normtype == GF_NORM_ASSEMBLED_L2) {
     RC(copy(m, q, b));
     RC(gf_dss_t(m, GF_DSS_SUM, q));
     if (bbv) RC(gf_mul_t(m, q, m->mask, q));
-    RC(setup_red<double>(m, q, nullptr, m->imult, normtype, red2));
-    rnorm0 = finish_norm_host(normtype, red2[1], m, volume);
-    rtol = prm->tol * rnorm0;
-  } else {
-    RC(setup_red<double>(m, b, nullptr, m->imult, normtype, red2));
-    rnorm0 = finish_norm_host(normtype, red2[1], m, volume);
-    rtol = rnorm0 < 1.0 ? prm->tol : prm->tol * rnorm0;
+    nb = q;
+  }
+  RC(setup_red<double>(m, nb, nullptr, m->imult, normtype, SU_B));
+  RC(setup_get(m, su));
+  if (prm->precond) RC(diag_status(m, su[SU_BAD - SU_B]));
+  const double rnorm0 = finish_norm_host(normtype, su[1], m, volume);
+  const double rtol =
+      prm->tol * (normtype != GF_NORM_ASSEMBLED_L2 && rnorm0 < 1.0 ? 1.0 : rnorm0);
+  if (bbv) {  // x = x*mask + xb (gcg.ipp:371-375)
+    RC(gf_mul_t(m, x, m->mask, x));
+    RC(gf_axpy_t(m, 1.0, xb, x));
   }
   res->rnorm0 = rnorm0;
   int total_iters = 0, outer = 0, status = GF_OK;
@@ -1897,9 +1917,10 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
     // z = P^-1 r ; w = z (set inside the first apply) ; rho = r.z.imult
     double *z = q;
     if (dinv) RC(gf_mul_t(m, dinv, r, z));
-    RC(setup_red<double>(m, r, dinv ? z : r, m->imult, normtype, red2));
+    RC(setup_red<double>(m, r, dinv ? z : r, m->imult, normtype, SU_R));
+    RC(setup_get(m, su));
     double hs[12] = {0};
-    hs[S_RHO] = red2[0];
+    hs[S_RHO] = su[SU_R - SU_B];
     hs[S_RTOL] = rtol;
     hs[S_RNORM] = 10.0 * rtol;
     hs[S_ITER] = 0;
@@ -1981,20 +2002,24 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
       if (!first)
         hipLaunchKernelGGL(k_add_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, x, x32, 1.0, n);
       RC(residual(r));
-      RC(setup_red<double>(m, r, nullptr, m->imult, normtype, red2));
-      const double rn = finish_norm_host(normtype, red2[1], m, volume);
+      // the residual's norm, and rho of the next FP32 cycle (not used when the
+      // solve has converged), with one wait
+      RC(setup_red<double>(m, r, nullptr, m->imult, normtype, SU_R));
+      hipLaunchKernelGGL(k_to_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, r32, r, 1.0, n);
+      float *z32 = q32;
+      if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
+      RC(setup_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, SU_R32));
+      RC(setup_get(m, su));
+      const double rn = finish_norm_host(normtype, su[SU_R + 1 - SU_B], m, volume);
       rn_final = rn;
       if (prm->resid && hist < prm->maxit) prm->resid[hist++] = rn;
       if (rn <= rtol || total_iters >= prm->maxit || outer >= 10000) break;
-      hipLaunchKernelGGL(k_to_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, r32, r, 1.0, n);
       hipLaunchKernelGGL(k_fill_f32, dim3(nblocks(n)), dim3(kThreads), 0, s, x32, 0.0f, n);
-      float *z32 = q32;
-      if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
-      RC(setup_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, red2));
-      const double rn32 = finish_norm_host(normtype, red2[1], m, volume);
+      const double rho32 = su[SU_R32 - SU_B];
+      const double rn32 = finish_norm_host(normtype, su[SU_R32 + 1 - SU_B], m, volume);
       double hs[S_COUNT] = {0};
-      hs[S_RHO] = red2[0];
-      hs[S_BETA] = first ? 0.0 : red2[0] / m->hscal[S_RHOM];
+      hs[S_RHO] = rho32;
+      hs[S_BETA] = first ? 0.0 : rho32 / m->hscal[S_RHOM];
       hs[S_RHOM] = first ? 0.0 : m->hscal[S_RHOM];
       hs[S_RTOL] = std::max(delta * rn32, 0.5 * rtol);
       hs[S_RNORM] = rn32;
@@ -2040,7 +2065,10 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
   (void)hipFree(m->seg_boff);
   (void)hipFree(m->sscal);
   (void)hipFree(m->seg_topo);
+  (void)hipFree(m->seg_blk);
   m->seg_topo = nullptr;
+  m->seg_blk = nullptr;
+  m->seg_vol.clear();
   if (m->hsscal) (void)hipHostFree(m->hsscal);
   m->seg_eoff = nullptr;
   m->seg_boff = nullptr;
@@ -2063,11 +2091,11 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
     m->h_seg_boff[k + 1] = m->h_seg_boff[k] + std::max(1, (int)(frac * budget + 0.5));
   }
   // the reduction buffer holds one apply partial per block and the update
-  // blocks' pairs, or the set-up pairs plus one pair per member
+  // blocks' pairs, or the set-up pairs plus two pairs per member
   {
     const int nbU = m->h_seg_boff[nseg];
     const size_t nbg = xcd_grid(nbU);
-    const size_t need = std::max(3 * nbg + 128, 2 * nbg + 64 + 2 * (size_t)nseg) + 64;
+    const size_t need = std::max(3 * nbg + 128, 2 * nbg + 64 + 4 * (size_t)nseg) + 64;
     if (m->red_cap < need) {
       GF_HIP(m->ctx, hipFree(m->red));
       m->red = nullptr;
@@ -2085,7 +2113,26 @@ extern "C" int gf_mesh_set_segments(gf_mesh *m, int nseg, const int64_t *eoff) {
   GF_HIP(m->ctx, hipMemcpy(m->seg_eoff, eoff, (nseg + 1) * sizeof(int64_t), hipMemcpyHostToDevice));
   GF_HIP(m->ctx, hipMemcpy(m->seg_boff, m->h_seg_boff.data(), (nseg + 1) * sizeof(int),
                            hipMemcpyHostToDevice));
+  std::vector<CGSegBlock> blk;
+  for (int k = 0; k < nseg; k++) {
+    const int b0 = m->h_seg_boff[k], nb = m->h_seg_boff[k + 1] - b0;
+    for (int l = 0; l < nb; l++) blk.push_back({k, l, nb, b0, eoff[k], eoff[k + 1]});
+  }
+  GF_HIP(m->ctx, hipMalloc(&m->seg_blk, blk.size() * sizeof(CGSegBlock)));
+  GF_HIP(m->ctx, hipMemcpy(m->seg_blk, blk.data(), blk.size() * sizeof(CGSegBlock),
+                           hipMemcpyHostToDevice));
   m->nseg = nseg;
+  // member volumes: sums of the mass
+  {
+    std::vector<double> mass(m->ndof);
+    GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
+    GF_HIP(m->ctx, hipMemcpy(mass.data(), m->mass, m->ndof * sizeof(double), hipMemcpyDeviceToHost));
+    for (int k = 0; k < nseg; k++) {
+      double v = 0.0;
+      for (size_t q = (size_t)eoff[k] * m->nn; q < (size_t)eoff[k + 1] * m->nn; q++) v += mass[q];
+      m->seg_vol.push_back(v);
+    }
+  }
   // no GGFX group may join two members
   double bad = 0.0;
   double *dbad = m->scal + 63;

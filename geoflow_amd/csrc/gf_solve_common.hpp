@@ -131,11 +131,17 @@ struct ColIdx {
 // one-block reduction kernel runs between the two, and the system's first
 // block stores the results.  x is advanced in the apply, which reads w
 // anyway: 9 passes over the fields an iteration instead of 10.
+// Place of a block of a batched mesh: its system s (elements e0 .. e1, blocks
+// b0 .. b0 + nb) and its number lb there.
+struct CGSegBlock {
+  int s, lb, nb, b0;
+  int64_t e0, e1;
+};
+
 struct CGCtl {
-  double *scal;          // kCGScal doubles per system
-  const int64_t *eoff;   // batched mesh (nseg > 0): elements of system s are
-  const int *boff;       // eoff[s] .. eoff[s+1], its blocks boff[s] .. boff[s+1]
-  int nseg;
+  double *scal;           // kCGScal doubles per system
+  const CGSegBlock *blk;  // batched mesh (nseg > 0): nblk blocks
+  int nseg, nblk;
   size_t nelems;
   int nbA, nbU;          // blocks of the apply and update kernels (nseg == 0)
   double *partA, *partU; // w.q per apply block; (r.z, norm) per update block
@@ -267,19 +273,14 @@ struct CGBlock {
     e1 = c.nelems;
     ok = true;
     if (c.nseg > 0) {
-      ok = b < c.boff[c.nseg];
-      int lo = 0, hi = c.nseg;
-      while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (c.boff[mid] <= b) lo = mid;
-        else hi = mid;
-      }
-      s = lo;
-      b0 = c.boff[s];
-      lb = b - b0;
-      nb = c.boff[s + 1] - b0;
-      e0 = (size_t)c.eoff[s];
-      e1 = (size_t)c.eoff[s + 1];
+      ok = b < c.nblk;
+      const CGSegBlock v = c.blk[ok ? b : 0];
+      s = v.s;
+      lb = v.lb;
+      nb = v.nb;
+      b0 = v.b0;
+      e0 = (size_t)v.e0;
+      e1 = (size_t)v.e1;
     }
     st = c.scal + (size_t)s * kCGScal;
   }

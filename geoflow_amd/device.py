@@ -180,6 +180,10 @@ class Mesh:
     def new(self, dtype=torch.float64):
         return torch.zeros(self.ndof, dtype=dtype, device="cuda")
 
+    def _out(self, dtype=torch.float64):
+        # an operator's result, written whole by it
+        return torch.empty(self.ndof, dtype=dtype, device="cuda")
+
     def get(self, which):
         out = np.zeros(self.ndof)
         self._c(lib().gf_mesh_get(self.h, which.encode(), _hp(out)))
@@ -187,40 +191,40 @@ class Mesh:
 
     # -- operators (mirror GGrid / GMTK / GMass / GHelmholtz / GGFX) -------
     def grefderiv(self, u, idir, dotrans=False, out=None):
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         self._c(lib().gf_grefderiv(self.h, idir, int(dotrans), _ptr(u), _ptr(out)))
         return out
 
     def grefderivs(self, u, dotrans=False):
-        outs = [self.new() for _ in range(self.dim)]
+        outs = [self._out() for _ in range(self.dim)]
         self._c(lib().gf_grefderivs(self.h, int(dotrans), _ptr(u), _ptrs(outs)))
         return outs
 
     def grefdiv(self, us, dotrans=True, out=None):
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         us = list(us) + [None] * (3 - len(us))
         self._c(lib().gf_grefdiv(self.h, int(dotrans), _ptrs(us), _ptr(out)))
         return out
 
     def deriv(self, u, idir, out=None):
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         self._c(lib().gf_deriv(self.h, idir, _ptr(u), _ptr(out)))
         return out
 
     def grad(self, u):
         # embedded 2-D meshes return all three Cartesian derivatives
         ncomp = 3 if self.gtype == GF_GE_2DEMBEDDED else self.dim
-        outs = [self.new() for _ in range(ncomp)]
+        outs = [self._out() for _ in range(ncomp)]
         self._c(lib().gf_grad(self.h, _ptr(u), _ptrs(outs)))
         return outs
 
     def mass_apply(self, u, out=None):
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         self._c(lib().gf_mass_apply(self.h, _ptr(u), _ptr(out)))
         return out
 
     def imass_apply(self, u, out=None):
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         self._c(lib().gf_imass_apply(self.h, _ptr(u), _ptr(out)))
         return out
 
@@ -232,7 +236,7 @@ class Mesh:
     def helmholtz(self, u, p=1.0, q=None, out=None):
         """uo = p L u + q M u; p and q may be scalars or per-node fields, q None
         for the pure Laplacian."""
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         pf = p if torch.is_tensor(p) else None
         ps = 1.0 if pf is not None else float(p)
         qf, qs = _q_args(q)
@@ -240,14 +244,14 @@ class Mesh:
         return out
 
     def helmholtz_f32(self, u, p=1.0, q=None, out=None):
-        out = self.new(torch.float32) if out is None else out
+        out = self._out(torch.float32) if out is None else out
         qf, qs = _q_args(q)
         self._c(lib().gf_helmholtz_apply_f32(self.h, float(p), qs, _ptr(qf), _ptr(u), _ptr(out)))
         return out
 
     def dealias(self, v1, v2, pq, out=None):
         """GGrid::dealias: v1 v2 through the order-pq GLL grid."""
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         self._c(lib().gf_dealias(self.h, int(pq), _ptr(v1), _ptr(v2), _ptr(out)))
         return out
 
@@ -257,12 +261,12 @@ class Mesh:
         return u
 
     def imult(self):
-        out = self.new()
+        out = self._out()
         self._c(lib().gf_imult(self.h, _ptr(out)))
         return out
 
     def advect(self, p, us, out=None):
-        out = self.new() if out is None else out
+        out = self._out() if out is None else out
         self._c(lib().gf_advect(self.h, _ptr(p), len(us), _ptrs(us), _ptr(out)))
         return out
 
@@ -270,7 +274,7 @@ class Mesh:
         # one output per component for the nonlinear (0) and heat (2) modes,
         # a single output for pure advection (1)
         nout = 1 if mode == 1 else len(us)
-        outs = [self.new() for _ in range(nout)]
+        outs = [self._out() for _ in range(nout)]
         self._c(lib().gf_burgers_rhs(self.h, mode, nu, len(us), _ptrs(us), _ptrs(outs)))
         return outs
 
@@ -347,7 +351,7 @@ class Mesh:
         self._c(lib().gf_mesh_reserve(self.h, int(what), ctypes.byref(prm)))
 
     def helmholtz_diag_inv(self, p=1.0, q=None):
-        out = self.new()
+        out = self._out()
         qf, qs = _q_args(q)
         self._c(lib().gf_helmholtz_diag_inv(self.h, float(p), qs, _ptr(qf), _ptr(out)))
         return out
