@@ -90,9 +90,32 @@ int deriv_T(gf_mesh *m, int j, const double *v, double *out, double *t1, double 
   return gf_axpy_t(m, 1.0, t2, out);
 }
 
+Adj3Args adj3_args(gf_mesh *m, double nu) {
+  Adj3Args a;
+  memset(&a, 0, sizeof(a));
+  a.imass = m->imass_el ? m->imass_el : m->imass;
+  a.imstride = m->imass_el ? 0 : m->nn;
+  a.W = m->W[0];
+  a.edx = m->edx;
+  a.ejac = m->ejac;
+  a.nu = nu;
+  a.topo = m->box;
+  a.nelems = m->nelems;
+  return a;
+}
+
 // lam[k] += (dF/du)^T w  at the state u (nonlinear Burgers, n_c = nvel).
 int rhs_adjoint(gf_mesh *m, double nu, const double *const *u, const double *const *w,
                 double *const *lam) {
+  if (m->dim == 3 && m->dconst) {
+    Adj3Args a = adj3_args(m, nu);
+    for (int k = 0; k < 3; k++) {
+      a.u[k] = u[k];
+      a.y[k] = w[k];
+      a.yo[k] = lam[k];
+    }
+    return GF_DISPATCH_N3(m->Niso, launch_adj3, m, a, 0);
+  }
   const size_t bytes = m->ndof * sizeof(double);
   double *z = (double *)gf_ws(m, WS_ADJ_TMP + 0, bytes);
   double *mz = (double *)gf_ws(m, WS_ADJ_TMP + 1, bytes);
@@ -162,9 +185,67 @@ int stage_states(gf_mesh *m, double nu, int order, double h, const double *const
   return GF_OK;
 }
 
+// Whether the step and its adjoint run in the fused box kernels.
+bool box_path(const gf_mesh *m, int order) {
+  return m->dim == 3 && m->dconst && m->has_box && order >= 2;
+}
+
+// step_adjoint on a structured box: the stage states by the RK stage kernels,
+// then one kernel per stage in reverse (k_burgers_adj3).  cont: un is
+// continuous bit for bit.
+int step_adjoint_box(gf_mesh *m, double nu, int order, double h, const double *const *un,
+                     double *const *lam, bool cont) {
+  const size_t bytes = m->ndof * sizeof(double);
+  double beta[16], c[4];
+  butcher_tab(order, beta, c);
+  double *us[4][3] = {}, *K[2][3], *abar[3], *lin[3], *y[2][3];
+  int slot = WS_ADJ_BEGIN;
+  bool ok = true;
+  auto ws = [&](double *&p) {
+    p = (double *)gf_ws(m, slot++, bytes);
+    ok = ok && p;
+  };
+  for (int k = 0; k < 3; k++) {
+    us[0][k] = const_cast<double *>(un[k]);
+    for (int s = 1; s < order; s++) ws(us[s][k]);
+    ws(abar[k]);
+    ws(y[0][k]);
+    ws(y[1][k]);
+    ws(K[0][k]);
+    K[1][k] = lin[k] = nullptr;
+    if (order > 2) ws(K[1][k]);
+    if (order > 2) ws(lin[k]);
+  }
+  if (!ok) return gf_set_err(m->ctx, GF_ERR_ALLOC, "adjoint workspace");
+  double *const *none = nullptr;
+  RCA(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, us[0], none, none, K[0], 0.0, 0.0, 0.0, nu, 0, 0));
+  for (int s = 1; s < order - 1; s++)
+    RCA(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, us[0], K[(s - 1) % 2], us[s], K[s % 2],
+                       beta[s * 4 + (s - 1)] * h, 0.0, 0.0, nu, 1, 4));
+  const int l = order - 1;
+  RCA(GF_DISPATCH_N3(m->Niso, launch_stage_input, m, un, K[(l - 1) % 2], us[l],
+                     beta[l * 4 + (l - 1)] * h, cont ? 1 : 0));
+  Adj3Args a = adj3_args(m, nu);
+  for (int s = l; s >= 0; s--) {
+    for (int k = 0; k < 3; k++) {
+      a.u[k] = us[s][k];
+      a.y[k] = s == l ? lam[k] : y[(s + 1) % 2][k];
+      a.abar[k] = abar[k];
+      a.lin[k] = lin[k];
+      a.yo[k] = s == 0 ? lam[k] : y[s % 2][k];
+    }
+    a.hc = h * c[s];
+    a.hb = s < l ? h * beta[(s + 1) * 4 + s] : 0.0;
+    const int mode = s == l ? 1 : (s == 0 ? (l == 1 ? 5 : 4) : (s == l - 1 ? 2 : 3));
+    RCA(GF_DISPATCH_N3(m->Niso, launch_adj3, m, a, mode));
+  }
+  return GF_OK;
+}
+
 // lam: in dJ/du_{n+1}, out dJ/du_n, for one step from un.
 int step_adjoint(gf_mesh *m, double nu, int order, double h, const double *const *un,
-                 double *const *lam) {
+                 double *const *lam, bool cont) {
+  if (box_path(m, order)) return step_adjoint_box(m, nu, order, h, un, lam, cont);
   const int nv = nvel_of(m);
   const size_t bytes = m->ndof * sizeof(double);
   double beta[16], c[4];
@@ -219,6 +300,29 @@ int step_adjoint(gf_mesh *m, double nu, int order, double h, const double *const
   return GF_OK;
 }
 
+// nsteps steps from src to dst (other buffers); cont as in gf_rk_steps_box.
+int advance(gf_mesh *m, double nu, int order, int nstate, double t, double dt, int nsteps,
+            const double *const *src, double *const *dst, bool cont) {
+  if (nsteps > 0 && box_path(m, order))
+    return gf_rk_steps_box(m, nu, order, dt, nsteps, src, dst, cont);
+  for (int k = 0; k < nstate; k++) RCA(copyd(m, dst[k], src[k]));
+  return gf_burgers_steps(m, 0, nu, order, nstate, t, dt, nsteps, dst);
+}
+
+// Reverse sweep over the steps s0 .. s1 - 1 from the state st0 at s0; seg(i),
+// i >= 1, are the buffers of the states after it.
+template <typename SEG>
+int reverse_segment(gf_mesh *m, double nu, int order, int nstate, double dt, int s0, int s1,
+                    double *const *st0, SEG &&seg, double *const *lam) {
+  auto state = [&](int i) { return i == 0 ? st0 : seg(i); };
+  for (int s = s0 + 1; s < s1; s++)  // state at step s from the one before
+    RCA(advance(m, nu, order, nstate, (s - 1) * dt, dt, 1, state(s - s0 - 1), state(s - s0),
+                s - 1 > 0));
+  for (int s = s1 - 1; s >= s0; s--)
+    RCA(step_adjoint(m, nu, order, dt, state(s - s0), lam, s > 0));
+  return GF_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -242,7 +346,7 @@ int gf_burgers_step_adjoint(gf_mesh *m, double nu, int order, int nstate, double
   if (nstate != nvel_of(m)) return gf_set_err(m->ctx, GF_ERR_ARG, "adjoint: nonlinear mode needs nstate == velocity components");
   for (int k = 0; k < nstate; k++)
     if (!un[k] || !lam[k]) return GF_ERR_ARG;
-  return step_adjoint(m, nu, order, dt, un, lam);
+  return step_adjoint(m, nu, order, dt, un, lam, false);
 }
 
 int gf_burgers_adjoint(gf_mesh *m, double nu, int order, int nstate, double dt, int nsteps,
@@ -263,36 +367,22 @@ int gf_burgers_adjoint(gf_mesh *m, double nu, int order, int nstate, double dt, 
   auto cp = [&](int i) { return &store[(size_t)i * nstate]; };
   auto seg = [&](int i) { return &store[(size_t)(ncp + i) * nstate]; };
   auto run = [&]() -> int {
-    // forward sweep, checkpointing every ckpt steps
-    double *cur[3] = {nullptr, nullptr, nullptr};
-    for (int k = 0; k < nstate; k++) {
-      cur[k] = seg(0)[k];
-      RCA(copyd(m, cur[k], u0[k]));
-    }
-    for (int s = 0; s < nsteps; s++) {
-      if (s % ckpt == 0)
-        for (int k = 0; k < nstate; k++) RCA(copyd(m, cp(s / ckpt)[k], cur[k]));
-      RCA(gf_burgers_step(m, 0, nu, order, nstate, s * dt, dt, cur, 0));
-    }
-    if (uT)
+    // forward sweep: each checkpoint from the one before; the steps after the
+    // last one serve only uT
+    for (int k = 0; ncp > 0 && k < nstate; k++) RCA(copyd(m, cp(0)[k], u0[k]));
+    for (int c = 1; c < ncp; c++)
+      RCA(advance(m, nu, order, nstate, (c - 1) * ckpt * dt, dt, ckpt, cp(c - 1), cp(c), c > 1));
+    if (uT) {
+      const int s0 = ncp > 0 ? (ncp - 1) * ckpt : 0;
+      const double *const *from = ncp > 0 ? (const double *const *)cp(ncp - 1) : u0;
+      RCA(advance(m, nu, order, nstate, s0 * dt, dt, nsteps - s0, from, seg(0), s0 > 0));
       for (int k = 0; k < nstate; k++)
-        if (uT[k]) RCA(copyd(m, uT[k], cur[k]));
-    // reverse sweep: recompute each segment's states from its checkpoint
-    for (int c = ncp - 1; c >= 0; c--) {
-      const int s0 = c * ckpt, s1 = std::min(nsteps, s0 + ckpt);
-      for (int k = 0; k < nstate; k++) RCA(copyd(m, seg(0)[k], cp(c)[k]));
-      for (int s = s0 + 1; s < s1; s++) {  // state at step s from the one before
-        for (int k = 0; k < nstate; k++) RCA(copyd(m, seg(s - s0)[k], seg(s - s0 - 1)[k]));
-        double *st[3] = {seg(s - s0)[0], nstate > 1 ? seg(s - s0)[1] : nullptr,
-                         nstate > 2 ? seg(s - s0)[2] : nullptr};
-        RCA(gf_burgers_step(m, 0, nu, order, nstate, (s - 1) * dt, dt, st, 0));
-      }
-      for (int s = s1 - 1; s >= s0; s--) {
-        const double *un[3] = {seg(s - s0)[0], nstate > 1 ? seg(s - s0)[1] : nullptr,
-                               nstate > 2 ? seg(s - s0)[2] : nullptr};
-        RCA(step_adjoint(m, nu, order, dt, un, lam));
-      }
+        if (uT[k]) RCA(copyd(m, uT[k], seg(0)[k]));
     }
+    // reverse sweep: recompute each segment's states from its checkpoint
+    for (int c = ncp - 1; c >= 0; c--)
+      RCA(reverse_segment(m, nu, order, nstate, dt, c * ckpt, std::min(nsteps, (c + 1) * ckpt),
+                          cp(c), seg, lam));
     GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
     return GF_OK;
   };
@@ -355,32 +445,24 @@ int gf_burgers_adjoint_gio(gf_mesh *m, double nu, int order, int nstate, double 
       GF_HIP(m->ctx, hipMemcpyAsync(st[k], hf[k], bytes, hipMemcpyHostToDevice, m->ctx->stream));
     return GF_OK;
   };
-  double *cur[3] = {nullptr, nullptr, nullptr};
-  for (int k = 0; k < nstate; k++) {
-    cur[k] = seg(0)[k];
-    RCA(copyd(m, cur[k], u0[k]));
-  }
-  for (int s = 0; s < nsteps; s++) {
-    if (s % ckpt == 0) RCA(save(s / ckpt, s, cur));
-    RCA(gf_burgers_step(m, 0, nu, order, nstate, s * dt, dt, cur, 0));
+  // forward sweep in two alternating buffers, checkpointing every ckpt steps;
+  // the steps after the last checkpoint serve only uT
+  double *const *cur = seg(0), *const *next = seg(1);
+  for (int k = 0; k < nstate; k++) RCA(copyd(m, cur[k], u0[k]));
+  for (int c = 0; c < ncp; c++) {
+    RCA(save(c, c * ckpt, cur));
+    const int len = std::min(nsteps - c * ckpt, ckpt);
+    if (c == ncp - 1 && !uT) break;
+    RCA(advance(m, nu, order, nstate, c * ckpt * dt, dt, len, cur, next, c > 0));
+    std::swap(cur, next);
   }
   if (uT)
     for (int k = 0; k < nstate; k++)
       if (uT[k]) RCA(copyd(m, uT[k], cur[k]));
   for (int c = ncp - 1; c >= 0; c--) {
-    const int s0 = c * ckpt, s1 = std::min(nsteps, s0 + ckpt);
-    RCA(load(c, s0, seg(0)));
-    for (int s = s0 + 1; s < s1; s++) {
-      for (int k = 0; k < nstate; k++) RCA(copyd(m, seg(s - s0)[k], seg(s - s0 - 1)[k]));
-      double *st[3] = {seg(s - s0)[0], nstate > 1 ? seg(s - s0)[1] : nullptr,
-                       nstate > 2 ? seg(s - s0)[2] : nullptr};
-      RCA(gf_burgers_step(m, 0, nu, order, nstate, (s - 1) * dt, dt, st, 0));
-    }
-    for (int s = s1 - 1; s >= s0; s--) {
-      const double *un[3] = {seg(s - s0)[0], nstate > 1 ? seg(s - s0)[1] : nullptr,
-                             nstate > 2 ? seg(s - s0)[2] : nullptr};
-      RCA(step_adjoint(m, nu, order, dt, un, lam));
-    }
+    RCA(load(c, c * ckpt, seg(0)));
+    RCA(reverse_segment(m, nu, order, nstate, dt, c * ckpt, std::min(nsteps, (c + 1) * ckpt),
+                        seg(0), seg, lam));
   }
   GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
   return GF_OK;

@@ -141,6 +141,11 @@ int gf_grefderiv_t(gf_mesh *m, int idir, int trans, const double *u, double *du,
 int gf_mul_t(gf_mesh *m, const double *a, const double *b, double *out);
 int gf_dot_t(gf_mesh *m, const double *a, const double *b, size_t n, double *result);
 int gf_axpy_t(gf_mesh *m, double a, const double *x, double *y);
+// nsteps RK steps (order >= 2) on a structured box (has_box, dconst), from src
+// to u (which may be src); cont: src is continuous bit for bit, as any step's
+// output is.
+int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,
+                    const double *const *src, double *const *u, bool cont);
 int gf_grad3c(gf_mesh *m, const double *u, double *const *du, const double *edx);
 int gf_helm3c(gf_mesh *m, double p, const double *pf, const double *qf, double qs,
               const double *u, double *uo);

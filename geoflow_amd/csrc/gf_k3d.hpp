@@ -358,6 +358,7 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 //     1  acc = uin + ca kp + cb K       K -> kout
 //     2  acc = uin + ca kp + cb K       (last stage: K is not stored)
 //     3  acc = acc + ca kp + cb K       (last stage)
+//     4  acc = v                        K -> kout  (stage states of the adjoint)
 // Group sums are pairwise (x, then y, then z), exact for equal members of
 // groups of 2, 4 and 8, so S leaves a continuous state as it is and IN 1 and
 // IN 2 agree bit for bit on it.
@@ -403,7 +404,8 @@ void k_burgers_stage3b(
   double im[N];
 #pragma unroll
   for (int k = 0; k < N; k++) im[k] = imass[t.e * imstride + t.r + (size_t)k * S::N2];
-  double ru[3][N], ra[ACC ? 3 : 1][ACC ? N : 1];
+  constexpr bool RA = ACC >= 1 && ACC <= 3;  // accumulates after the operator
+  double ru[3][N], ra[RA ? 3 : 1][RA ? N : 1];
   if constexpr (KP) {
     int ec[3];
     gf::box_elem_coords(topo, t.e, ec);
@@ -477,6 +479,9 @@ void k_burgers_stage3b(
         // interleaves the sums of many nodes and keeps their operands live
         // (354 registers instead of 154 at N = 8, IN 1, ACC 0)
         asm volatile("" : "+v"(v));
+        if constexpr (ACC == 4) {
+          if (t.active) acc[c][col + (size_t)k * S::N2] = v;
+        }
         ru[c][k] = v;
       });
     });
@@ -508,8 +513,8 @@ void k_burgers_stage3b(
       if (nu != 1.0) L *= nu;
       const double urhs = fma(-po, M, -L);
       const double K = im[k] * urhs;
-      if (ACC < 2) ko[g] = K;
-      if (ACC) ac[g] = fma(cb, K, ra[ACC ? c : 0][ACC ? k : 0]);
+      if (ACC < 2 || ACC == 4) ko[g] = K;
+      if (RA) ac[g] = fma(cb, K, ra[RA ? c : 0][RA ? k : 0]);
     };
     gf::pen_op3<N, double, true>(ru[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,
                                  rz * rz, (const double *)nullptr, xcb, ycb, zcb, post);
@@ -594,6 +599,7 @@ int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *co
   GF_STAGE(1, 1);
   GF_STAGE(1, 2);
   GF_STAGE(1, 3);
+  GF_STAGE(1, 4);
   GF_STAGE(2, 2);
   GF_STAGE(2, 3);
 #undef GF_STAGE
@@ -606,6 +612,277 @@ int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc) {
   hipLaunchKernelGGL(k_rk_out_halo<N>, dim3(xcd_grid((m->nelems + S::EPB - 1) / S::EPB)),
                      dim3(S::THREADS), 0, m->ctx->stream, u[0], u[1], u[2], acc[0], acc[1], acc[2],
                      m->box, m->nelems);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+
+// ---------------------------------------------------------------------------
+// Adjoint of the Burgers right-hand side on regular 3-D elements, and of the
+// RK step's stages on structured boxes.  With z_c = Minv w_c,
+//   y_j = -( sum_d D_d^T [ M (nu r_d^2 D_d z_j + r_d u_d z_j) ]
+//            + sum_c (r_j D_j u_c) M z_c )
+// is (dF/du)^T w (see gf_adjoint.hip): the viscous term and the transported
+// quantity share one transposed contraction per direction, and the element's
+// three components are worked together.  On a box the Smooths of the step's
+// adjoint are formed by gather, as in k_burgers_stage3b:
+//   MODE
+//     0  w = y; lam (`yo`) += (dF/du)^T w
+//     1  last stage: abar = S(y), y = dJ/du_{n+1}; w = hc abar; yo = y_s
+//     2  after it: w = hc abar + hb S(y); lin = abar + S(y) (the final-stage
+//        input is smoothed); yo = y_s
+//     3  w as in 2; lin += y; yo = y_s
+//     4  first stage: w as in 2; yo = lin + y + y_0 = dJ/du_n
+//     5  first stage of two: w as in 2; yo = abar + S(y) + y_0
+// abar is smooth, so S(hc abar + hb y) is hc abar + hb S(y).  Bound by memory
+// and latency like the forward stage: 9-18 fields a stage.  12^3, p = 6: a
+// step's adjoint takes 193 us with its stage states; composed (a
+// derivative, a product and an update for every pair of components, a DSS
+// pass for every smoothed field) 1750.
+// ---------------------------------------------------------------------------
+template <int N, int MODE>
+__global__ __launch_bounds__(gf::Pen3<N>::THREADS) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))
+void k_burgers_adj3(Adj3Args a) {
+  using S = gf::Pen3<N>;
+  using H = gf::Halo<N>;
+  constexpr bool G = MODE != 0, FIN = MODE >= 4;
+  constexpr int NSL = G && H::SIZE > 5 * S::SZ ? H::SIZE : 5 * S::SZ;
+  __shared__ double sl[S::EPB * NSL];
+  ColIdx<N> t(a.nelems);
+  const size_t col = t.e * S::NN + t.r;
+  const int64_t ebase = (int64_t)t.e * S::NN;
+  double *hk = sl + t.el * NSL;
+  double rz[3][N], rl[FIN ? 3 : 1][FIN ? N : 1];
+  {
+    double im[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) im[k] = a.imass[t.e * a.imstride + t.r + (size_t)k * S::N2];
+    if constexpr (G) {
+      int ec[3];
+      gf::box_elem_coords(a.topo, t.e, ec);
+      const gf::BoxElemDeltas de = gf::box_elem_deltas(a.topo, N, ec);
+      const gf::HaloCol<N> hc(de, t.i, t.j);
+      gf::static_for<0, 3>([&](auto cc) {
+        constexpr int c = decltype(cc)::value;
+        const double *__restrict__ y = a.y[c];
+        __syncthreads();  // the previous component's sums have read LDS
+        double yo[N], ab[N], li[N];
+#pragma unroll
+        for (int k = 0; k < N; k++) yo[k] = y[col + (size_t)k * S::N2];
+        gf::HaloRim<N, double> L;
+        L.issue(y, de, ebase, t.r);
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+          if (MODE >= 2) ab[k] = a.abar[c][col + (size_t)k * S::N2];
+          if (MODE == 3 || MODE == 4) li[k] = a.lin[c][col + (size_t)k * S::N2];
+        }
+#pragma unroll
+        for (int k = 0; k < N; k++) hk[t.r + S::N2 * k] = yo[k];
+        L.store(hk, t.r);
+        __syncthreads();
+        gf::static_for<0, N>([&](auto kc) {
+          constexpr int k = decltype(kc)::value;
+          const size_t g = col + (size_t)k * S::N2;
+          int ad[8];
+          const int cnt = gf::halo_order<N, k>(hc, de, ad);
+          double s = (hk[ad[0]] + hk[ad[1]]) + (hk[ad[2]] + hk[ad[3]]);
+          if (k == 0 || k == N - 1) s = s + ((hk[ad[4]] + hk[ad[5]]) + (hk[ad[6]] + hk[ad[7]]));
+          s *= gf::box_inv(cnt);
+          asm volatile("" : "+v"(s));  // node by node (see k_burgers_stage3b)
+          double w;
+          if constexpr (MODE == 1) {
+            if (t.active) a.abar[c][g] = s;
+            w = a.hc * s;
+          } else {
+            w = fma(a.hb, s, a.hc * ab[k]);
+            if constexpr (MODE == 2) {
+              if (t.active) a.lin[c][g] = ab[k] + s;
+            }
+            if constexpr (MODE == 3) {
+              if (t.active) a.lin[c][g] = li[k] + yo[k];
+            }
+            if constexpr (MODE == 4) rl[c][k] = li[k] + yo[k];
+            if constexpr (MODE == 5) rl[c][k] = ab[k] + s;
+          }
+          rz[c][k] = im[k] * w;
+        });
+      });
+      __syncthreads();  // the element buffers below reuse the halo
+    } else {
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int k = 0; k < N; k++) rz[c][k] = im[k] * a.y[c][col + (size_t)k * S::N2];
+    }
+  }
+  // element buffers: u_0, u_1, u_2, and two for the passes
+  double *U[3] = {hk, hk + S::SZ, hk + 2 * S::SZ}, *su = hk + 3 * S::SZ, *sd = hk + 4 * S::SZ;
+  const double cab = (a.W[t.j] * a.W[t.i]) * a.ejac[t.e];  // M = W[k] cab on the thread's pencils
+  const double r_[3] = {a.edx[t.e * 3], a.edx[t.e * 3 + 1], a.edx[t.e * 3 + 2]};
+#pragma unroll
+  for (int c = 0; c < 3; c++)
+#pragma unroll
+    for (int k = 0; k < N; k++) U[c][S::at(t.i, t.j, k)] = a.u[c][col + (size_t)k * S::N2];
+  // element (pencil node m) of the thread's pencil along direction d
+  auto at = [&](int d, int m) {
+    return d == 0 ? S::at(m, t.i, t.j) : (d == 1 ? S::at(t.i, m, t.j) : S::at(t.i, t.j, m));
+  };
+  gf::static_for<0, 3>([&](auto jc) {
+    constexpr int j = decltype(jc)::value;
+    // T = sum_c (r_j D_j u_c) M z_c at the column's nodes: the derivatives on
+    // the pencils of direction j, through sd to the column
+    double T[N], p[N], d[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) su[S::at(t.i, t.j, k)] = rz[j][k];
+    gf::static_for<0, 3>([&](auto cc) {
+      constexpr int c = decltype(cc)::value;
+      if (c == 0 || j != 2) __syncthreads();  // U and su are written; sd has been read
+#pragma unroll
+      for (int m = 0; m < N; m++) p[m] = U[c][at(j, m)];
+      gf::gll_apply<N, false>(p, d);
+      if constexpr (j != 2) {
+#pragma unroll
+        for (int m = 0; m < N; m++) sd[at(j, m)] = d[m];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < N; k++) d[k] = sd[S::at(t.i, t.j, k)];
+      }
+#pragma unroll
+      for (int k = 0; k < N; k++) {
+        const double v = (a.W[k] * cab) * rz[c][k];
+        T[k] = c == 0 ? d[k] * v : fma(d[k], v, T[k]);
+        asm volatile("" : "+v"(T[k]));
+      }
+    });
+#pragma unroll
+    for (int k = 0; k < N; k++) T[k] *= r_[j];
+    if (j != 2) __syncthreads();  // sd has been read
+    // sum_d D_d^T [ M (nu r_d^2 D_d z_j + r_d u_d z_j) ]: z on the column,
+    // x and y on their pencils
+    gf::static_for<0, 3>([&](auto dc) {
+      constexpr int dd = 2 - decltype(dc)::value;  // z, y, x
+      double f[N];
+      const double nr = a.nu * (r_[dd] * r_[dd]);
+#pragma unroll
+      for (int m = 0; m < N; m++) p[m] = dd == 2 ? rz[j][m] : su[at(dd, m)];
+      gf::gll_apply<N, false>(p, f);
+#pragma unroll
+      for (int m = 0; m < N; m++)
+        f[m] = (a.W[m] * cab) * fma(nr, f[m], (r_[dd] * U[dd][at(dd, m)]) * p[m]);
+      gf::gll_apply<N, true>(f, d);
+      if constexpr (dd == 2) {
+#pragma unroll
+        for (int k = 0; k < N; k++) {
+          T[k] += d[k];
+          asm volatile("" : "+v"(T[k]));
+        }
+      } else if constexpr (dd == 1) {
+#pragma unroll
+        for (int m = 0; m < N; m++) sd[at(1, m)] = d[m];
+        __syncthreads();
+      } else {
+#pragma unroll
+        for (int m = 0; m < N; m++) sd[at(0, m)] += d[m];
+        __syncthreads();
+      }
+    });
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      const size_t g = col + (size_t)k * S::N2;
+      const double y = -(sd[S::at(t.i, t.j, k)] + T[k]);
+      if (t.active) {
+        if (MODE == 0) a.yo[j][g] += y;
+        else if (FIN) a.yo[j][g] = rl[FIN ? j : 0][FIN ? k : 0] + y;
+        else a.yo[j][g] = y;
+      }
+    }
+  });
+}
+
+// The final-stage input of a step on a structured box: v = S(u + bh S(k)), or
+// u + bh S(k) on a continuous u (SM false), where the two agree bit for bit.
+template <int N, bool SM>
+__global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_stage_input_halo(
+    const double *__restrict__ u0, const double *__restrict__ u1, const double *__restrict__ u2,
+    const double *__restrict__ k0, const double *__restrict__ k1, const double *__restrict__ k2,
+    double *__restrict__ v0, double *__restrict__ v1, double *__restrict__ v2, double bh,
+    gf::BoxTopo topo, size_t nelems) {
+  using S = gf::Pen3<N>;
+  using H = gf::Halo<N>;
+  __shared__ double sl[S::EPB * (SM ? 2 : 1) * H::SIZE];
+  const double *u[3] = {u0, u1, u2}, *kf[3] = {k0, k1, k2};
+  double *v[3] = {v0, v1, v2};
+  ColIdx<N> t(nelems);
+  double *hk = sl + t.el * (SM ? 2 : 1) * H::SIZE, *hu = hk + H::SIZE;
+  const int64_t ebase = (int64_t)t.e * S::NN;
+  int ec[3];
+  gf::box_elem_coords(topo, t.e, ec);
+  const gf::BoxElemDeltas de = gf::box_elem_deltas(topo, N, ec);
+  const gf::HaloCol<N> hc(de, t.i, t.j);
+  gf::static_for<0, 3>([&](auto cc) {
+    constexpr int c = decltype(cc)::value;
+    __syncthreads();  // the previous component's sums have read LDS
+    double ko[N], uo[N];
+    gf::HaloRim<N, double> Lk, Lu;
+#pragma unroll
+    for (int k = 0; k < N; k++) ko[k] = kf[c][ebase + t.r + S::N2 * k];
+#pragma unroll
+    for (int k = 0; k < N; k++) uo[k] = u[c][ebase + t.r + S::N2 * k];
+    Lk.issue(kf[c], de, ebase, t.r);
+    if (SM) Lu.issue(u[c], de, ebase, t.r);
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+      hk[t.r + S::N2 * k] = ko[k];
+      if (SM) hu[t.r + S::N2 * k] = uo[k];
+    }
+    Lk.store(hk, t.r);
+    if (SM) Lu.store(hu, t.r);
+    __syncthreads();
+    gf::static_for<0, N>([&](auto kc) {
+      constexpr int k = decltype(kc)::value;
+      constexpr bool ZF = k == 0 || k == N - 1;
+      int ad[8];
+      const int cnt = gf::halo_order<N, k>(hc, de, ad);
+      const double inv = gf::box_inv(cnt);
+      auto sum = [&](auto &&val) {
+        double s = (val(ad[0]) + val(ad[1])) + (val(ad[2]) + val(ad[3]));
+        if (ZF) s = s + ((val(ad[4]) + val(ad[5])) + (val(ad[6]) + val(ad[7])));
+        return s * inv;
+      };
+      const double ks = sum([&](int q) { return hk[q]; });
+      double r = fma(bh, ks, uo[k]);
+      if (SM) r = sum([&](int q) { return q == H::ZERO ? 0.0 : fma(bh, ks, hu[q]); });
+      asm volatile("" : "+v"(r));  // node by node (see k_burgers_stage3b)
+      if (t.active) v[c][ebase + t.r + S::N2 * k] = r;
+    });
+  });
+}
+
+template <int N>
+int launch_adj3(gf_mesh *m, const Adj3Args &a, int mode) {
+  using S = gf::Pen3<N>;
+  const dim3 nb(xcd_grid((m->nelems + S::EPB - 1) / S::EPB)), nt(S::THREADS);
+  switch (mode) {
+    case 0: hipLaunchKernelGGL((k_burgers_adj3<N, 0>), nb, nt, 0, m->ctx->stream, a); break;
+    case 1: hipLaunchKernelGGL((k_burgers_adj3<N, 1>), nb, nt, 0, m->ctx->stream, a); break;
+    case 2: hipLaunchKernelGGL((k_burgers_adj3<N, 2>), nb, nt, 0, m->ctx->stream, a); break;
+    case 3: hipLaunchKernelGGL((k_burgers_adj3<N, 3>), nb, nt, 0, m->ctx->stream, a); break;
+    case 4: hipLaunchKernelGGL((k_burgers_adj3<N, 4>), nb, nt, 0, m->ctx->stream, a); break;
+    default: hipLaunchKernelGGL((k_burgers_adj3<N, 5>), nb, nt, 0, m->ctx->stream, a); break;
+  }
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+template <int N>
+int launch_stage_input(gf_mesh *m, const double *const *u, double *const *k, double *const *v,
+                       double bh, int cont) {
+  using S = gf::Pen3<N>;
+  const dim3 nb(xcd_grid((m->nelems + S::EPB - 1) / S::EPB)), nt(S::THREADS);
+  if (cont)
+    hipLaunchKernelGGL((k_stage_input_halo<N, false>), nb, nt, 0, m->ctx->stream, u[0], u[1], u[2],
+                       k[0], k[1], k[2], v[0], v[1], v[2], bh, m->box, m->nelems);
+  else
+    hipLaunchKernelGGL((k_stage_input_halo<N, true>), nb, nt, 0, m->ctx->stream, u[0], u[1], u[2],
+                       k[0], k[1], k[2], v[0], v[1], v[2], bh, m->box, m->nelems);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
@@ -767,6 +1044,9 @@ int launch_update_box_n(gf_mesh *m, const CGCtl &c, const CGVecs<T> &v) {
   template int launch_stage3b<N>(gf_mesh *, double *const *, double *const *, double *const *, \
                                  double *const *, double, double, double, double, int, int); \
   template int launch_rk_out_box<N>(gf_mesh *, double *const *, double *const *);             \
+  template int launch_adj3<N>(gf_mesh *, const Adj3Args &, int);                             \
+  template int launch_stage_input<N>(gf_mesh *, const double *const *, double *const *,      \
+                                     double *const *, double, int);                          \
   template int helm3c_d<N>(gf_mesh *, double, const double *, const double *, double,         \
                            const double *, double *);                                        \
   template int helm3c_f<N>(gf_mesh *, float, const float *, float, const float *, float *);   \

@@ -924,8 +924,12 @@ int rk_step_fused(gf_mesh *m, double nu, int order, double dt, double *const *u)
 // operations, so n steps give the same bits as n single steps.  The state
 // the caller passes may be discontinuous, so the first step smooths its
 // final-stage input as step_b does; from then on the state is continuous,
-// that Smooth is the identity bit for bit and is not formed.
-int rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps, double *const *u) {
+// that Smooth is the identity bit for bit and is not formed (cont: nor for the
+// first step).
+}  // namespace
+
+int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,
+                    const double *const *src, double *const *u, bool cont) {
   size_t bytes = m->ndof * sizeof(double);
   double alpha[4], beta[16], c[4];
   butcher(order, alpha, beta, c);
@@ -938,11 +942,14 @@ int rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps, double
   const double h = dt;
   const int ns = order;
   double *const *none = nullptr;
+  double *from[3];
+  for (int k = 0; k < 3; k++) from[k] = const_cast<double *>(src[k]);
   for (int n = 0; n < nsteps; n++) {
+    double *const *ui = n == 0 ? from : u;
     // stage 0: from the state, or from the previous step's accumulator
     // (whose Smooth is stored as the state)
     if (n == 0)
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, u, none, none, K[0], 0.0, 0.0, 0.0, nu, 0, 0));
+      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, ui, none, none, K[0], 0.0, 0.0, 0.0, nu, 0, 0));
     else
       RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, none, acc, u, K[0], 0.0, 0.0, 0.0, nu, 3, 0));
     for (int s = 1; s < ns; s++) {
@@ -950,14 +957,16 @@ int rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps, double
       // accumulate K_{s-1} and K_s at odd s; a last stage at even s adds K_s
       const bool odd = s % 2 == 1;
       const int accm = last ? (s == 1 ? 2 : 3) : (s == 1 ? 1 : 0);
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, u, K[(s - 1) % 2], acc, K[s % 2],
+      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, ui, K[(s - 1) % 2], acc, K[s % 2],
                         beta[s * 4 + (s - 1)] * h, odd ? c[s - 1] * h : 0.0, c[s] * h, nu,
-                        last && n == 0 ? 2 : 1, accm));
+                        last && n == 0 && !cont ? 2 : 1, accm));
     }
   }
   if (nsteps > 0) RC(GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, u, acc));
   return GF_OK;
 }
+
+namespace {
 
 // ---- pure-advection stage on 2-D embedded (sphere) elements ----------------
 // One kernel per RK stage computes, per element,
@@ -1315,7 +1324,7 @@ int gf_burgers_step(gf_mesh *m, int mode, double nu, int order, int nstate, doub
   int rc;
   const bool embed_adv = mode == 1 && m->gtype == GF_GE_2DEMBEDDED && m->Niso && nstate == 4;
   if (fused && m->has_box && order >= 2)
-    rc = rk_steps_box(m, nu, order, dt, 1, u);
+    rc = gf_rk_steps_box(m, nu, order, dt, 1, u, u, false);
   else if (fused)
     rc = rk_step_fused(m, nu, order, dt, u);
   else if (embed_adv)
@@ -1334,7 +1343,7 @@ int gf_burgers_steps(gf_mesh *m, int mode, double nu, int order, int nstate, dou
       m->dconst && m->has_box && nstate == 3 && order >= 2 && order <= 4) {
     for (int k = 0; k < nstate; k++)
       if (!u[k]) return GF_ERR_ARG;
-    return rk_steps_box(m, nu, order, dt, nsteps, u);
+    return gf_rk_steps_box(m, nu, order, dt, nsteps, u, u, false);
   }
   if (mode == 1 && m->gtype == GF_GE_2DEMBEDDED && m->Niso && nstate == 4 && order >= 1 &&
       order <= 4) {

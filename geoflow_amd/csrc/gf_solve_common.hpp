@@ -52,6 +52,16 @@ struct StageArgs {
   size_t nelems;
 };
 
+// Arguments of the adjoint stage kernel (k_burgers_adj3).
+struct Adj3Args {
+  const double *u[3], *y[3];
+  double *abar[3], *lin[3], *yo[3];
+  const double *imass, *W, *edx, *ejac;
+  double hc, hb, nu;
+  gf::BoxTopo topo;
+  size_t nelems, imstride;
+};
+
 inline gf::PenD<double> pend_d(gf_mesh *m) {
   gf::PenD<double> p;
   for (int c = 0; c < 3; c++) {
@@ -497,6 +507,11 @@ int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *co
                    int accm);
 template <int N>
 int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc);
+template <int N>
+int launch_adj3(gf_mesh *m, const Adj3Args &a, int mode);
+template <int N>
+int launch_stage_input(gf_mesh *m, const double *const *u, double *const *k, double *const *v,
+                       double bh, int cont);
 template <int N>
 int helm3c_d(gf_mesh *m, double p, const double *pf, const double *qf, double qs, const double *u,
              double *uo);

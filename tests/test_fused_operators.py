@@ -59,3 +59,30 @@ def test_fused_operators(dim, p, ne):
         assert _rel(out, og.advect(q, [z, us[1], z])) <= TOL
         # fewer components than directions
         assert _rel(m.advect(dq, dus[:2]), og.advect(q, us[:2] + [z])) <= TOL
+
+
+@pytest.mark.parametrize("p,ne,bdy", [(1, [3, 2, 1], 0), (2, [5, 1, 3], 6), (3, [2, 3, 2], 0),
+                                      (4, [3, 1, 1], 6), (5, [1, 1, 1], 6), (6, [3, 2, 1], 6),
+                                      (7, [2, 1, 3], 0), (8, [2, 2, 1], 6), (9, [1, 2, 1], 0)])
+def test_fused_adjoint(p, ne, bdy):
+    """The adjoint kernels at every element order: the right-hand side's
+    adjoint added to a cotangent, and the step's adjoint of orders 2-4 on the
+    box path from a discontinuous state, against the oracle."""
+    from geoflow_amd.device import Context, Mesh
+    bg, og = ga.BoxGrid(3, p, ne, bdy=[bdy] * 6), oracle.Grid.box(3, p, ne, bdy=[bdy] * 6)
+    m = Mesh(Context(0), bg)
+    rng = np.random.default_rng(40 + p)
+    f = lambda: [rng.standard_normal(bg.ndof) for _ in range(3)]  # noqa: E731
+    u, w, l0 = f(), f(), f()
+    ref = og.burgers_rhs_adjoint(u, w, [a.copy() for a in l0], 0.03)
+    got = m.burgers_rhs_adjoint([_dev(a) for a in u], [_dev(a) for a in w],
+                                [_dev(a) for a in l0], 0.03)
+    for a, b in zip(got, ref):
+        assert _rel(a, b) <= TOL
+    for order in (2, 3, 4):
+        dt = 1e-3 / (p + 1) ** 4
+        ref = og.burgers_step_adjoint(u, [a.copy() for a in w], 0.04, dt, order=order)
+        got = m.burgers_step_adjoint([_dev(a) for a in u], [_dev(a) for a in w], 0.04, dt,
+                                     order=order)
+        for a, b in zip(got, ref):
+            assert _rel(a, b) <= TOL, order
