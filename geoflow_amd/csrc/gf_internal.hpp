@@ -70,6 +70,9 @@ struct gf_mesh_s {
   int *goff = nullptr;
   int *gmem = nullptr;
   int maxgrp = 1;
+  // 2-D regular isotropic meshes with groups of at most 4: the members of every
+  // node's group, ascending, -1 past the group (the RK stages gather with it)
+  int4 *mem4 = nullptr;
   // Structured box: when has_box, the groups above are exactly those of
   // gf::box_group for `box`, and fused kernels may assemble by gather.
   gf::BoxTopo box = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0, 0, 0, 0}};
@@ -141,7 +144,7 @@ int gf_grefderiv_t(gf_mesh *m, int idir, int trans, const double *u, double *du,
 int gf_mul_t(gf_mesh *m, const double *a, const double *b, double *out);
 int gf_dot_t(gf_mesh *m, const double *a, const double *b, size_t n, double *result);
 int gf_axpy_t(gf_mesh *m, double a, const double *x, double *y);
-// nsteps RK steps (order >= 2) on a structured box (has_box, dconst), from src
+// nsteps RK steps (order >= 2) in the gather stages (structured boxes, 2-D), from src
 // to u (which may be src); cont: src is continuous bit for bit, as any step's
 // output is.
 int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,

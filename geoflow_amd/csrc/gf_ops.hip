@@ -581,6 +581,22 @@ __global__ void k_imult_groups(double *__restrict__ imult, const int *__restrict
   }
 }
 
+// Members of every node's group, ascending, -1 past the group.
+__global__ void k_mem4_self(int4 *__restrict__ mem4, size_t n) {
+  for (size_t g = blockIdx.x * (size_t)blockDim.x + threadIdx.x; g < n;
+       g += (size_t)gridDim.x * blockDim.x)
+    mem4[g] = make_int4((int)g, -1, -1, -1);
+}
+__global__ void k_mem4_groups(int4 *__restrict__ mem4, const int *__restrict__ goff,
+                              const int *__restrict__ gmem, int ngroups) {
+  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < ngroups; g += gridDim.x * blockDim.x) {
+    const int b = goff[g], e = goff[g + 1];
+    const int4 v = make_int4(gmem[b], gmem[b + 1], b + 2 < e ? gmem[b + 2] : -1,
+                             b + 3 < e ? gmem[b + 3] : -1);
+    for (int s = b; s < e; s++) mem4[gmem[s]] = v;
+  }
+}
+
 // Deterministic two-stage sum: per-block partials then one block in order.
 __global__ void k_partial_dot(const double *__restrict__ a, const double *__restrict__ b,
                               double *__restrict__ part, size_t n) {
@@ -1106,6 +1122,13 @@ int gf_mesh_create(gf_ctx *ctx, const gf_mesh_desc *d, gf_mesh **out) {
   if (m->ngroups)
     hipLaunchKernelGGL(k_imult_groups, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
                        m->imult, m->goff, m->gmem, m->ngroups);
+  if (m->dim == 2 && d->gtype == GF_GE_REGULAR && m->Niso && m->maxgrp <= 4) {
+    GF_HIP(ctx, hipMalloc((void **)&m->mem4, n * sizeof(int4)));
+    hipLaunchKernelGGL(k_mem4_self, dim3(nblocks(n)), dim3(kThreads), 0, s, m->mem4, n);
+    if (m->ngroups)
+      hipLaunchKernelGGL(k_mem4_groups, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
+                         m->mem4, m->goff, m->gmem, m->ngroups);
+  }
   GF_HIP(ctx, hipStreamSynchronize(s));
   {
     std::vector<double> im(n);
@@ -1170,7 +1193,7 @@ int gf_mesh_destroy(gf_mesh *m) {
   F(m->mask); F(m->mass); F(m->imass); F(m->imass_el); F(m->dtab); F(m->dtab32); F(m->deq);
   F(m->imult); F(m->mask32);
   F(m->imult32);
-  F(m->goff); F(m->gmem); F(m->red); F(m->scal);
+  F(m->goff); F(m->gmem); F(m->mem4); F(m->red); F(m->scal);
   for (int k = 0; k < 6; k++) F(m->G32[k]);
   F(m->mass32);
   if (m->hscal) (void)hipHostFree(m->hscal);

@@ -146,6 +146,175 @@ __global__ void k_final_input(double *__restrict__ u3, const double *__restrict_
   }
 }
 
+// ---------------------------------------------------------------------------
+// Burgers RK on 2-D regular meshes: k_burgers_stage3b's scheme (the same IN and
+// ACC forms, one gathered Smooth per step output), the group members of each
+// node read from mem4 (ascending, -1 past the group).  One node per thread.
+// A 2-D mesh is small and a step is bound by the number of its launches: order
+// stage kernels and, per call, one output kernel (16x16 elements, p = 4, RK4:
+// 17 us a step against 81 of the 20 launches with DSS passes).
+// ---------------------------------------------------------------------------
+struct Stage2Args {
+  const double *uin[2], *kp[2];
+  double *acc[2], *kout[2];
+  const int4 *mem4;
+  const double *D, *W, *edx, *ejac, *imass;
+  double bh, ca, cb, nu;
+  size_t nelems;
+};
+
+// Smooth of a group's values, v[m] in GGFX order: Sum / count.  Equal members
+// return their value, so a continuous field is left as it is (for counts 1, 2
+// and 4 the quotient is that value anyway).
+__device__ __forceinline__ double smooth4(const double (&v)[4], int cnt) {
+  double s = 0.0;
+  bool eq = true;
+#pragma unroll
+  for (int k = 0; k < 4; k++)
+    if (k < cnt) {
+      s = s + v[k];
+      eq = eq && v[k] == v[0];
+    }
+  return eq ? v[0] : s / (double)cnt;
+}
+__device__ __forceinline__ int group4(const int4 &m, int (&id)[4]) {
+  id[0] = m.x;
+  id[1] = m.y;
+  id[2] = m.z;
+  id[3] = m.w;
+  return 1 + (m.y >= 0) + (m.z >= 0) + (m.w >= 0);
+}
+__device__ __forceinline__ void load4(const double *__restrict__ u, const int (&id)[4],
+                                      double (&v)[4]) {
+#pragma unroll
+  for (int k = 0; k < 4; k++) v[k] = id[k] >= 0 ? u[id[k]] : 0.0;
+}
+
+template <int N, int IN, int ACC>
+__global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
+  using S = Shape<2, N>;
+  static_assert(S::NODES <= kThreads, "one node per thread");
+  __shared__ double su[2][S::NODES], sg[2][2][S::NODES], sD[N * N], sW[N];
+  const size_t e0 = xcd_block() * S::EPB;
+  const int nel = e0 < a.nelems ? (int)min((size_t)S::EPB, a.nelems - e0) : 0;
+  const int q = threadIdx.x;
+  const bool act = q < nel * S::NN;
+  const size_t g = e0 * S::NN + q;
+  gf::stage_D(sD, a.D, N);
+  if (q < N) sW[q] = a.W[q];
+  double ra[2] = {0.0, 0.0}, im = 0.0;
+  if (act) {
+    im = a.imass[g];
+    int id[4];
+    int cnt = 1;
+    if (IN) cnt = group4(a.mem4[g], id);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const double u = IN != 3 ? a.uin[c][g] : 0.0;
+      double v = u;
+      if constexpr (IN != 0) {
+        double kv[4];
+        load4(a.kp[c], id, kv);
+        const double ks = smooth4(kv, cnt);
+        if constexpr (IN == 3) {
+          v = ks;
+          a.acc[c][g] = v;
+        } else {
+          v = fma(a.bh, ks, u);
+          if constexpr (IN == 2) {
+            double uv[4];
+            load4(a.uin[c], id, uv);
+#pragma unroll
+            for (int k = 0; k < 4; k++) uv[k] = fma(a.bh, ks, uv[k]);
+            v = smooth4(uv, cnt);
+          }
+          if constexpr (ACC != 0) {
+            double ko = kv[0];
+#pragma unroll
+            for (int k = 1; k < 4; k++) ko = id[k] == (int)g ? kv[k] : ko;
+            ra[c] = fma(a.ca, ko, ACC == 3 ? a.acc[c][g] : u);
+          }
+        }
+      }
+      su[c][q] = v;
+    }
+  }
+  __syncthreads();
+  const int el = q / S::NN, r = q - el * S::NN;
+  int i, j, k;
+  gf::node_ijk<2, N>(r, i, j, k);
+  double M = 0.0, ad[2] = {0.0, 0.0};
+  if (act) {
+    const size_t e = e0 + el;
+    const double f0 = a.edx[e * 2], f1 = a.edx[e * 2 + 1];
+    M = gf::node_mass<2>(sW, i, j, k, a.ejac[e]);
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      const double *se = &su[c][el * S::NN];
+      const double g0 = gf::contract<2, N, false>(se, sD, 0, i, j, k);
+      const double g1 = gf::contract<2, N, false>(se, sD, 1, i, j, k);
+      ad[c] = fma(g1 * f1, su[1][q], (g0 * f0) * su[0][q]);
+      sg[c][0][q] = M * (g0 * (f0 * f0));
+      sg[c][1][q] = M * (g1 * (f1 * f1));
+    }
+  }
+  __syncthreads();
+  if (act) {
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+      double L = gf::contract<2, N, true>(&sg[c][0][el * S::NN], sD, 0, i, j, k);
+      L += gf::contract<2, N, true>(&sg[c][1][el * S::NN], sD, 1, i, j, k);
+      if (a.nu != 1.0) L *= a.nu;
+      const double K = im * fma(-ad[c], M, -L);
+      if (ACC < 2) a.kout[c][g] = K;
+      if (ACC) a.acc[c][g] = fma(a.cb, K, ra[c]);
+    }
+  }
+}
+
+// Step output: u = S(acc), as the fused form (IN 3).
+__global__ __launch_bounds__(kThreads) void k_rk_out2(double *__restrict__ u0,
+                                                      double *__restrict__ u1,
+                                                      const double *__restrict__ a0,
+                                                      const double *__restrict__ a1,
+                                                      const int4 *__restrict__ mem4, size_t n) {
+  GRID_LOOP(g, n) {
+    int id[4];
+    const int cnt = group4(mem4[g], id);
+    double v0[4], v1[4];
+    load4(a0, id, v0);
+    load4(a1, id, v1);
+    u0[g] = smooth4(v0, cnt);
+    u1[g] = smooth4(v1, cnt);
+  }
+}
+
+template <int N, int IN, int ACC>
+int launch_stage2_h(gf_mesh *m, const Stage2Args &a) {
+  using S = Shape<2, N>;
+  hipLaunchKernelGGL((k_burgers_stage2<N, IN, ACC>), dim3(xcd_grid((m->nelems + S::EPB - 1) / S::EPB)),
+                     dim3(kThreads), 0, m->ctx->stream, a);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+template <int DIM, int N>
+int launch_stage2(gf_mesh *m, const Stage2Args &a, int in, int accm) {
+  if constexpr (DIM == 2) {
+#define GF_STAGE(I, A) \
+  if (in == I && accm == A) return launch_stage2_h<N, I, A>(m, a)
+    GF_STAGE(0, 0);
+    GF_STAGE(3, 0);
+    GF_STAGE(1, 0);
+    GF_STAGE(1, 1);
+    GF_STAGE(1, 2);
+    GF_STAGE(1, 3);
+    GF_STAGE(2, 2);
+    GF_STAGE(2, 3);
+#undef GF_STAGE
+  }
+  return gf_set_err(m->ctx, GF_ERR_ARG, "stage2: unsupported stage form");
+}
+
 template <int DIM, int N>
 int launch_stage(gf_mesh *m, const StageArgs &a) {
   using S = Shape<DIM, N>;
@@ -915,7 +1084,7 @@ int rk_step_fused(gf_mesh *m, double nu, int order, double dt, double *const *u)
   return GF_OK;
 }
 
-// RK steps on a structured box (order >= 2): step_b with every Smooth formed
+// RK steps on a structured box or a 2-D mesh (order >= 2): step_b with every Smooth formed
 // by gather inside the stage kernels (k_burgers_stage3b) and the output
 // kernel, no DSS passes.  The accumulator uin + sum_s c_s h K_s is advanced
 // by two stage derivatives at a time, in the stages 1, 3 (and the last one);
@@ -926,6 +1095,45 @@ int rk_step_fused(gf_mesh *m, double nu, int order, double dt, double *const *u)
 // final-stage input as step_b does; from then on the state is continuous,
 // that Smooth is the identity bit for bit and is not formed (cont: nor for the
 // first step).
+// One stage (IN, ACC forms of k_burgers_stage3b) and the step output, in 3-D on
+// structured boxes and in 2-D with the groups' member lists.
+int gather_stage(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
+                 double *const *kout, double bh, double ca, double cb, double nu, int in, int accm) {
+  if (m->dim == 3)
+    return GF_DISPATCH_N3(m->Niso, launch_stage3b, m, uin, kp, acc, kout, bh, ca, cb, nu, in, accm);
+  Stage2Args a;
+  for (int k = 0; k < 2; k++) {
+    a.uin[k] = uin ? uin[k] : nullptr;
+    a.kp[k] = kp ? kp[k] : nullptr;
+    a.acc[k] = acc ? acc[k] : nullptr;
+    a.kout[k] = kout ? kout[k] : nullptr;
+  }
+  a.mem4 = m->mem4;
+  a.D = m->D[0];
+  a.W = m->W[0];
+  a.edx = m->edx;
+  a.ejac = m->ejac;
+  a.imass = m->imass;
+  a.bh = bh;
+  a.ca = ca;
+  a.cb = cb;
+  a.nu = nu;
+  a.nelems = m->nelems;
+  return GF_DISPATCH_N(m->dim, m->Niso, launch_stage2, m, a, in, accm);
+}
+int gather_out(gf_mesh *m, double *const *u, double *const *acc) {
+  if (m->dim == 3) return GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, u, acc);
+  hipLaunchKernelGGL(k_rk_out2, dim3(nblocks(m->ndof)), dim3(kThreads), 0, m->ctx->stream, u[0], u[1],
+                     acc[0], acc[1], m->mem4, m->ndof);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+// Whether the nonlinear RK steps of order >= 2 run in the gather stages.
+bool gather_steps(const gf_mesh *m) {
+  return m->gtype == GF_GE_REGULAR && m->Niso &&
+         (m->dim == 2 ? m->mem4 != nullptr : m->dconst && m->has_box);
+}
+
 }  // namespace
 
 int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,
@@ -934,7 +1142,8 @@ int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,
   double alpha[4], beta[16], c[4];
   butcher(order, alpha, beta, c);
   double *acc[3], *K[2][3];
-  for (int k = 0; k < 3; k++) {
+  const int nc = m->dim;
+  for (int k = 0; k < nc; k++) {
     acc[k] = (double *)gf_ws(m, WS_RK_BEGIN + k, bytes);
     for (int s = 0; s < 2; s++) K[s][k] = (double *)gf_ws(m, WS_RK_BEGIN + 6 + 3 * s + k, bytes);
     if (!acc[k] || !K[0][k] || !K[1][k]) return gf_set_err(m->ctx, GF_ERR_ALLOC, "workspace");
@@ -943,26 +1152,25 @@ int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,
   const int ns = order;
   double *const *none = nullptr;
   double *from[3];
-  for (int k = 0; k < 3; k++) from[k] = const_cast<double *>(src[k]);
+  for (int k = 0; k < nc; k++) from[k] = const_cast<double *>(src[k]);
   for (int n = 0; n < nsteps; n++) {
     double *const *ui = n == 0 ? from : u;
     // stage 0: from the state, or from the previous step's accumulator
     // (whose Smooth is stored as the state)
     if (n == 0)
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, ui, none, none, K[0], 0.0, 0.0, 0.0, nu, 0, 0));
+      RC(gather_stage(m, ui, none, none, K[0], 0.0, 0.0, 0.0, nu, 0, 0));
     else
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, none, acc, u, K[0], 0.0, 0.0, 0.0, nu, 3, 0));
+      RC(gather_stage(m, none, acc, u, K[0], 0.0, 0.0, 0.0, nu, 3, 0));
     for (int s = 1; s < ns; s++) {
       const bool last = s == ns - 1;
       // accumulate K_{s-1} and K_s at odd s; a last stage at even s adds K_s
       const bool odd = s % 2 == 1;
       const int accm = last ? (s == 1 ? 2 : 3) : (s == 1 ? 1 : 0);
-      RC(GF_DISPATCH_N3(m->Niso, launch_stage3b, m, ui, K[(s - 1) % 2], acc, K[s % 2],
-                        beta[s * 4 + (s - 1)] * h, odd ? c[s - 1] * h : 0.0, c[s] * h, nu,
-                        last && n == 0 && !cont ? 2 : 1, accm));
+      RC(gather_stage(m, ui, K[(s - 1) % 2], acc, K[s % 2], beta[s * 4 + (s - 1)] * h,
+                      odd ? c[s - 1] * h : 0.0, c[s] * h, nu, last && n == 0 && !cont ? 2 : 1, accm));
     }
   }
-  if (nsteps > 0) RC(GF_DISPATCH_N3(m->Niso, launch_rk_out_box, m, u, acc));
+  if (nsteps > 0) RC(gather_out(m, u, acc));
   return GF_OK;
 }
 
@@ -1323,7 +1531,7 @@ int gf_burgers_step(gf_mesh *m, int mode, double nu, int order, int nstate, doub
                (m->dim == 2 || m->dconst);
   int rc;
   const bool embed_adv = mode == 1 && m->gtype == GF_GE_2DEMBEDDED && m->Niso && nstate == 4;
-  if (fused && m->has_box && order >= 2)
+  if (fused && gather_steps(m) && order >= 2)
     rc = gf_rk_steps_box(m, nu, order, dt, 1, u, u, false);
   else if (fused)
     rc = rk_step_fused(m, nu, order, dt, u);
@@ -1339,8 +1547,7 @@ int gf_burgers_step(gf_mesh *m, int mode, double nu, int order, int nstate, doub
 int gf_burgers_steps(gf_mesh *m, int mode, double nu, int order, int nstate, double t, double dt,
                      int nsteps, double *const *u) {
   if (!m || !u || nsteps < 0) return GF_ERR_ARG;
-  if (nsteps > 1 && mode == 0 && m->gtype == GF_GE_REGULAR && m->Niso && m->dim == 3 &&
-      m->dconst && m->has_box && nstate == 3 && order >= 2 && order <= 4) {
+  if (nsteps > 1 && mode == 0 && gather_steps(m) && nstate == m->dim && order >= 2 && order <= 4) {
     for (int k = 0; k < nstate; k++)
       if (!u[k]) return GF_ERR_ARG;
     return gf_rk_steps_box(m, nu, order, dt, nsteps, u, u, false);

@@ -86,3 +86,30 @@ def test_fused_adjoint(p, ne, bdy):
                                      order=order)
         for a, b in zip(got, ref):
             assert _rel(a, b) <= TOL, order
+
+
+@pytest.mark.parametrize("order", [2, 3, 4])
+@pytest.mark.parametrize("p,ne,bdy", [(1, [5, 3], [6] * 4), (2, [1, 1], [6] * 4),
+                                      (4, [7, 3], [0] * 4), (5, [3, 2], [6, 6, 0, 0]),
+                                      (7, [2, 5], [6] * 4), (11, [3, 1], [0] * 4)])
+def test_steps_2d(p, ne, bdy, order):
+    """2-D steps from a state whose copies of a node disagree against the
+    oracle, n steps in a call equal to n calls bit for bit, and the state
+    continuous afterwards; boxes of both kinds of direction too."""
+    from geoflow_amd.device import Context, Mesh
+    bg, og = ga.BoxGrid(2, p, ne, bdy=bdy), oracle.Grid.box(2, p, ne, bdy=bdy)
+    m = Mesh(Context(0), bg)
+    rng = np.random.default_rng(7 * p + order)
+    us = [np.cos(2 * np.pi * (bg.xyz[0] + c * bg.xyz[1])) + 0.1 * rng.standard_normal(bg.ndof)
+          for c in range(2)]
+    dt = 1e-3 / (p + 1) ** 4
+    ref, one = [u.copy() for u in us], [_dev(u) for u in us]
+    for n in range(1, 4):
+        og.burgers_step(ref, 0.02, dt, order=order)
+        m.burgers_step(one, 0.02, dt, order=order)
+        many = [_dev(u) for u in us]
+        m.burgers_steps(many, 0.02, dt, n, order=order)
+        for c in range(2):
+            assert _rel(many[c], ref[c]) <= TOL, (n, c)
+            assert torch.equal(many[c], one[c]), (n, c)
+            assert torch.equal(m.dss(many[c].clone(), "max"), many[c]), (n, c)
