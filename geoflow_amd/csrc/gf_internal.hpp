@@ -137,6 +137,9 @@ int gf_box_groups_device(gf_mesh *m, int nbox, const int *ne, const int *periodi
 // order-pq weights, gf_setup.cpp.
 int gf_dealias_matrix(int p, int pq, double *I, double *wq);
 int gf_dss_f32(gf_mesh *m, int op, float *u);
+// Smooth that is the identity, bit for bit, on a continuous field.
+int gf_dss_keep(gf_mesh *m, double *u);
+int gf_dss_keep(gf_mesh *m, float *u);
 int gf_helm_t(gf_mesh *m, double p, const double *pf, const double *qf, double qs,
               const double *u, double *uo);
 int gf_grefderiv_t(gf_mesh *m, int idir, int trans, const double *u, double *du,

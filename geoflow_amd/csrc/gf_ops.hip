@@ -510,6 +510,10 @@ __global__ void k_narrow_f32(float *__restrict__ o, const double *__restrict__ a
 // The grid is a multiple of 8 and its blocks are renumbered so that each of
 // the 8 XCDs (each with its own L2) walks one contiguous range of groups:
 // groups of neighbouring indices share elements, and so cache lines.
+// kDssKeep: Smooth that leaves a group of equal members as it is (a sum of 3,
+// 5 or 6 equal values over their count may round away from them), so that it
+// is the identity on a continuous field.
+constexpr int kDssKeep = 16;
 template <int OP, typename T>
 __global__ void k_dss(T *__restrict__ u, const int *__restrict__ goff,
                       const int *__restrict__ gmem, int ngroups) {
@@ -528,12 +532,19 @@ __global__ void k_dss(T *__restrict__ u, const int *__restrict__ goff,
 #pragma unroll
       for (int k = 0; k < 8; k++) v[k] = k < cnt ? u[id[k]] : T(0);
       T r;
-      if (OP == GF_DSS_SUM || OP == GF_DSS_SMOOTH) {
+      if (OP == kDssKeep) {
+        bool eq = true;
+#pragma unroll
+        for (int k = 1; k < 8; k++)
+          if (k < cnt) eq = eq && v[k] == v[0];
+        if (eq) continue;
+      }
+      if (OP == GF_DSS_SUM || OP == GF_DSS_SMOOTH || OP == kDssKeep) {
         r = T(0);
 #pragma unroll
         for (int k = 0; k < 8; k++)
           if (k < cnt) r = r + v[k];
-        if (OP == GF_DSS_SMOOTH) r = r / (T)cnt;
+        if (OP != GF_DSS_SUM) r = r / (T)cnt;
       } else if (OP == GF_DSS_MAX) {
         r = std::numeric_limits<T>::lowest();
 #pragma unroll
@@ -551,10 +562,15 @@ __global__ void k_dss(T *__restrict__ u, const int *__restrict__ goff,
       continue;
     }
     T r;
-    if (OP == GF_DSS_SUM || OP == GF_DSS_SMOOTH) {
+    if (OP == kDssKeep) {
+      bool eq = true;
+      for (int s = b + 1; s < e; s++) eq = eq && u[gmem[s]] == u[gmem[b]];
+      if (eq) continue;
+    }
+    if (OP == GF_DSS_SUM || OP == GF_DSS_SMOOTH || OP == kDssKeep) {
       r = T(0);
       for (int s = b; s < e; s++) r = r + u[gmem[s]];
-      if (OP == GF_DSS_SMOOTH) r = r / (T)(e - b);
+      if (OP != GF_DSS_SUM) r = r / (T)(e - b);
     } else if (OP == GF_DSS_MAX) {
       r = std::numeric_limits<T>::lowest();
       for (int s = b; s < e; s++) r = fmax(r, u[gmem[s]]);
@@ -728,6 +744,18 @@ int gf_dss_f32(gf_mesh *m, int op, float *u) {
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
+
+template <typename T>
+static int dss_keep(gf_mesh *m, T *u) {
+  if (m->ngroups == 0) return GF_OK;
+  const int nb = (nblocks((size_t)m->ngroups) + 7) / 8 * 8;
+  hipLaunchKernelGGL((k_dss<kDssKeep, T>), dim3(nb), dim3(kThreads), 0, m->ctx->stream, u, m->goff,
+                     m->gmem, m->ngroups);
+  GF_LAUNCH_CHECK(m->ctx);
+  return GF_OK;
+}
+int gf_dss_keep(gf_mesh *m, double *u) { return dss_keep(m, u); }
+int gf_dss_keep(gf_mesh *m, float *u) { return dss_keep(m, u); }
 
 int gf_helm_t(gf_mesh *m, double p, const double *pf, const double *qf, double qs,
               const double *u, double *uo) {
