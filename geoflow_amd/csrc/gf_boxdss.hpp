@@ -266,7 +266,8 @@ __device__ __forceinline__ T box_sum8z(const T (&v)[8], int n) {
 //                    pair pd (0: xy, 1: xz, 2: yz) with sides s1, s2, r the
 //                    node's third index
 //   corners          CORNER + sx + 2 sy + 4 sz
-//   zero             ZERO: +0, read for absent partners
+//   zeros            [ZERO, SIZE): +0, read for absent partners; as many as
+//                    the stride of a column's face slots spans
 // A halo slot holds the value at the partner node across that face, edge
 // or corner (the offsets of box_elem_deltas added up); where the element has
 // no partner the offset is 0, the slot holds an own value and is never read.
@@ -274,7 +275,8 @@ __device__ __forceinline__ T box_sum8z(const T (&v)[8], int n) {
 template <int N>
 struct Halo {
   static constexpr int N2 = N * N, FACE = N * N * N, EDGE = FACE + 6 * N2,
-                       CORNER = EDGE + 12 * N, ZERO = CORNER + 8, SIZE = ZERO + 1;
+                       CORNER = EDGE + 12 * N, ZERO = CORNER + 8, NZ = N * (N - 1) + 1,
+                       SIZE = ZERO + NZ;
   static constexpr int ER = (12 * N + N2 - 1) / N2;  // edge rounds per thread
   static constexpr int CR = (8 + N2 - 1) / N2;       // corner rounds
   static constexpr int RQ = 6 + ER + CR;             // partner loads per thread
@@ -354,7 +356,7 @@ struct HaloRim {
 #pragma unroll
     for (int q = 0; q < RQ; q++)
       if (slot[q] >= 0) hl[slot[q]] = hv[q];
-    if (l == 0) hl[Halo<N>::ZERO] = T(0);
+    if (l < Halo<N>::NZ) hl[Halo<N>::ZERO + l] = T(0);
   }
 };
 
@@ -407,7 +409,8 @@ struct HaloCol {
   }
 };
 
-// The group of node (i, j, K) as halo addresses in canonical order -- lower
+// The group of node (i, j, K) as halo addresses in canonical order (the layout's
+// statement in GGFX's terms; the kernels sum with HaloSum) -- lower
 // side first in z, then in y, then in x, the lower side of a direction being
 // the copy with the smaller global index -- over the 2 x 2 (x 2 on the z
 // faces) crossings, an absent partner's terms reading the zero slot, which
@@ -450,6 +453,64 @@ __device__ __forceinline__ int halo_order(const HaloCol<N> &c, const BoxElemDelt
   }
   return (1 + c.xon) * (1 + c.yon) * (1 + zon);
 }
+
+// Group sums of a column (i, j, .) from the halo:
+//   (own + X) + (Y + XY)  [+ ((Z + XZ) + (YZ + XYZ)) on the z faces],
+// X the x partner's value and so on, zeros where there is none.  Each copy of
+// a node has the same pairs, at most exchanged, so all copies get the same
+// sum bit for bit whatever the partners' order; the sums of 2, 4 and 8 equal
+// values are exact.  A column's slots lie at fixed strides from one address
+// per partner kind (absent partners: the zeros), so no address is formed per
+// node.  Choosing the members' slots in GGFX order node by node instead took
+// more instructions than the operator at small orders: RK3 on 19x14x11, p = 5
+// 75 us a step against 66, FP32 CG at 20^3, p = 6 41 us an iteration against 37.
+template <int N>
+struct HaloSum {
+  using H = Halo<N>;
+  int x, y, xy, z[2], xz[2], yz[2], xyz[2];
+  bool xon, yon, zon[2];
+  double inv;  // 1 / (group size) off the z faces
+  __device__ __forceinline__ HaloSum(const BoxElemDeltas &de, int i, int j) {
+    const int sx = i == N - 1, sy = j == N - 1;
+    xon = (i == 0 && de.lo[0] != 0) || (sx && de.hi[0] != 0);
+    yon = (j == 0 && de.lo[1] != 0) || (sy && de.hi[1] != 0);
+    const bool both = xon && yon;
+    x = xon ? H::FACE + H::N2 * sx + j : H::ZERO;
+    y = yon ? H::FACE + H::N2 * (2 + sy) + i : H::ZERO;
+    xy = both ? H::EDGE + N * (2 * sx + sy) : H::ZERO;
+#pragma unroll
+    for (int s = 0; s < 2; s++) {
+      zon[s] = (s ? de.hi[2] : de.lo[2]) != 0;
+      z[s] = zon[s] ? H::FACE + H::N2 * (4 + s) + i + N * j : H::ZERO;
+      xz[s] = zon[s] && xon ? H::EDGE + N * (4 + 2 * sx + s) + j : H::ZERO;
+      yz[s] = zon[s] && yon ? H::EDGE + N * (8 + 2 * sy + s) + i : H::ZERO;
+      xyz[s] = zon[s] && both ? H::CORNER + sx + 2 * sy + 4 * s : H::ZERO;
+    }
+    inv = (xon ? 0.5 : 1.0) * (yon ? 0.5 : 1.0);
+  }
+  // 1 / (group size) of node K, exact
+  template <int K>
+  __device__ __forceinline__ double inv_k() const {
+    if (K == 0 || K == N - 1) return zon[K != 0] ? 0.5 * inv : inv;
+    return inv;
+  }
+  // sum over the group of node K of f(value, present)
+  template <int K, typename T, typename F>
+  __device__ __forceinline__ T sum(const T *h, T own, F &&f) const {
+    T s = (f(own, true) + f(h[x + K * N], xon)) +
+          (f(h[y + K * N], yon) + f(h[xy + K], xon && yon));
+    if constexpr (K == 0 || K == N - 1) {
+      constexpr int e = K != 0;
+      s = s + ((f(h[z[e]], zon[e]) + f(h[xz[e]], zon[e] && xon)) +
+               (f(h[yz[e]], zon[e] && yon) + f(h[xyz[e]], zon[e] && xon && yon)));
+    }
+    return s;
+  }
+  template <int K, typename T>
+  __device__ __forceinline__ T sum(const T *h, T own) const {
+    return sum<K>(h, own, [](T v, bool) { return v; });
+  }
+};
 
 // The N = 8 instances under their own names.
 constexpr int kHalo8 = Halo<8>::SIZE;

@@ -414,7 +414,7 @@ void k_burgers_stage3b(
     const int64_t ebase = (int64_t)t.e * S::NN;
     double *hu = hk + UOFF;
     double *ha = hk + (GU ? 2 * H::SIZE : AOFF);
-    const gf::HaloCol<N> hc(de, t.i, t.j);
+    const gf::HaloSum<N> hs(de, t.i, t.j);
     gf::static_for<0, 3>([&](auto cc) {
       constexpr int c = decltype(cc)::value;
       __syncthreads();  // the previous component's group sums have read LDS
@@ -451,18 +451,10 @@ void k_burgers_stage3b(
       __syncthreads();
       gf::static_for<0, N>([&](auto kc) {
         constexpr int k = decltype(kc)::value;
-        constexpr bool ZF = k == 0 || k == N - 1;  // groups of up to 8, else 4
         const int own = l + S::N2 * k;
-        int ad[8];
-        const int cnt = gf::halo_order<N, k>(hc, de, ad);
-        const double inv = gf::box_inv(cnt);  // Smooth: Sum / count, exact
-        auto sum = [&](auto &&val) {
-          double s = (val(ad[0]) + val(ad[1])) + (val(ad[2]) + val(ad[3]));
-          if (ZF) s = s + ((val(ad[4]) + val(ad[5])) + (val(ad[6]) + val(ad[7])));
-          return s * inv;
-        };
+        const double inv = hs.template inv_k<k>();  // Smooth: Sum / count, exact
         const double kown = L8 ? hk[own] : ko[k];
-        const double ks = sum([&](int q) { return hk[q]; });
+        const double ks = hs.template sum<k>(hk, kown) * inv;
         double v;
         if constexpr (IN == 3) {
           v = ks;
@@ -470,8 +462,11 @@ void k_burgers_stage3b(
         } else {
           const double u = L8 ? hu[own] : uo[k];
           v = fma(bh, ks, u);
-          // the members only: an absent partner's zero slot would add bh ks
-          if (GU) v = sum([&](int q) { return q == H::ZERO ? 0.0 : fma(bh, ks, hu[q]); });
+          // the members only: an absent partner's zero would add bh ks
+          if (GU)
+            v = hs.template sum<k>(hu, u, [&](double w, bool on) {
+              return on ? fma(bh, ks, w) : 0.0;
+            }) * inv;
           if constexpr (ACC == 1 || ACC == 2) ra[c][k] = fma(ca, kown, u);
           if constexpr (ACC == 3) ra[c][k] = fma(ca, kown, L8 ? ha[own] : ao[k]);
         }
@@ -541,7 +536,7 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_rk_out_halo(
   int ec[3];
   gf::box_elem_coords(topo, t.e, ec);
   const gf::BoxElemDeltas de = gf::box_elem_deltas(topo, N, ec);
-  const gf::HaloCol<N> hc(de, t.i, t.j);
+  const gf::HaloSum<N> hs(de, t.i, t.j);
   gf::static_for<0, 3>([&](auto cc) {
     constexpr int c = decltype(cc)::value;
     __syncthreads();  // the previous component's sums have read LDS
@@ -561,12 +556,8 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_rk_out_halo(
     __syncthreads();
     gf::static_for<0, N>([&](auto kc) {
       constexpr int k = decltype(kc)::value;
-      constexpr bool ZF = k == 0 || k == N - 1;
-      int ad[8];
-      const int cnt = gf::halo_order<N, k>(hc, de, ad);
-      double s = (hk[ad[0]] + hk[ad[1]]) + (hk[ad[2]] + hk[ad[3]]);
-      if (ZF) s = s + ((hk[ad[4]] + hk[ad[5]]) + (hk[ad[6]] + hk[ad[7]]));
-      if (t.active) u[c][ebase + l + S::N2 * k] = s * gf::box_inv(cnt);
+      const double s = hs.template sum<k>(hk, hk[l + S::N2 * k]);
+      if (t.active) u[c][ebase + l + S::N2 * k] = s * hs.template inv_k<k>();
     });
   });
 }
@@ -660,7 +651,7 @@ void k_burgers_adj3(Adj3Args a) {
       int ec[3];
       gf::box_elem_coords(a.topo, t.e, ec);
       const gf::BoxElemDeltas de = gf::box_elem_deltas(a.topo, N, ec);
-      const gf::HaloCol<N> hc(de, t.i, t.j);
+      const gf::HaloSum<N> hs(de, t.i, t.j);
       gf::static_for<0, 3>([&](auto cc) {
         constexpr int c = decltype(cc)::value;
         const double *__restrict__ y = a.y[c];
@@ -682,11 +673,7 @@ void k_burgers_adj3(Adj3Args a) {
         gf::static_for<0, N>([&](auto kc) {
           constexpr int k = decltype(kc)::value;
           const size_t g = col + (size_t)k * S::N2;
-          int ad[8];
-          const int cnt = gf::halo_order<N, k>(hc, de, ad);
-          double s = (hk[ad[0]] + hk[ad[1]]) + (hk[ad[2]] + hk[ad[3]]);
-          if (k == 0 || k == N - 1) s = s + ((hk[ad[4]] + hk[ad[5]]) + (hk[ad[6]] + hk[ad[7]]));
-          s *= gf::box_inv(cnt);
+          double s = hs.template sum<k>(hk, yo[k]) * hs.template inv_k<k>();
           asm volatile("" : "+v"(s));  // node by node (see k_burgers_stage3b)
           double w;
           if constexpr (MODE == 1) {
@@ -817,7 +804,7 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_stage_input_halo(
   int ec[3];
   gf::box_elem_coords(topo, t.e, ec);
   const gf::BoxElemDeltas de = gf::box_elem_deltas(topo, N, ec);
-  const gf::HaloCol<N> hc(de, t.i, t.j);
+  const gf::HaloSum<N> hs(de, t.i, t.j);
   gf::static_for<0, 3>([&](auto cc) {
     constexpr int c = decltype(cc)::value;
     __syncthreads();  // the previous component's sums have read LDS
@@ -839,18 +826,13 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_stage_input_halo(
     __syncthreads();
     gf::static_for<0, N>([&](auto kc) {
       constexpr int k = decltype(kc)::value;
-      constexpr bool ZF = k == 0 || k == N - 1;
-      int ad[8];
-      const int cnt = gf::halo_order<N, k>(hc, de, ad);
-      const double inv = gf::box_inv(cnt);
-      auto sum = [&](auto &&val) {
-        double s = (val(ad[0]) + val(ad[1])) + (val(ad[2]) + val(ad[3]));
-        if (ZF) s = s + ((val(ad[4]) + val(ad[5])) + (val(ad[6]) + val(ad[7])));
-        return s * inv;
-      };
-      const double ks = sum([&](int q) { return hk[q]; });
+      const double inv = hs.template inv_k<k>();
+      const double ks = hs.template sum<k>(hk, ko[k]) * inv;
       double r = fma(bh, ks, uo[k]);
-      if (SM) r = sum([&](int q) { return q == H::ZERO ? 0.0 : fma(bh, ks, hu[q]); });
+      if (SM)
+        r = hs.template sum<k>(hu, uo[k], [&](double w, bool on) {
+          return on ? fma(bh, ks, w) : 0.0;
+        }) * inv;
       asm volatile("" : "+v"(r));  // node by node (see k_burgers_stage3b)
       if (t.active) v[c][ebase + t.r + S::N2 * k] = r;
     });
@@ -994,19 +976,16 @@ __global__ __launch_bounds__(kThreads) void k_cg_update_halo(
       if (t.own()) hl[t.r + S::N2 * q] = qo[q];
     if (t.own()) L.store(hl, t.r);
     gf::elem_sync<C::WAVE>();
-    const gf::HaloCol<N> hc(de, t.i, t.j);
+    const gf::HaloSum<N> hs(de, t.i, t.j);
     gf::static_for<0, N>([&](auto kc) {
       constexpr int q = decltype(kc)::value;
-      int ad[8];
-      const int cnt = gf::halo_order<N, q>(hc, de, ad);
-      T s = (hl[ad[0]] + hl[ad[1]]) + (hl[ad[2]] + hl[ad[3]]);
-      if (q == 0 || q == N - 1) s = s + ((hl[ad[4]] + hl[ad[5]]) + (hl[ad[6]] + hl[ad[7]]));
+      const T s = hs.template sum<q>(hl, qo[q]);
       T rn = ro[q] + (-alpha) * s;
       asm volatile("" : "+v"(rn));  // node by node (see k_burgers_stage3b)
       const size_t g = col + q * S::N2;
       if (act) {
         r[g] = rn;
-        cg_accum<NORM>((double)rn, dinv ? (double)(dv[q] * rn) : (double)rn, gf::box_inv(cnt), mass,
+        cg_accum<NORM>((double)rn, dinv ? (double)(dv[q] * rn) : (double)rn, hs.template inv_k<q>(), mass,
                        g, rho, nrm);
       }
     });

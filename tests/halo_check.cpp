@@ -3,19 +3,74 @@
 // (own values, HaloRim), and for every node the slots of halo_order, absent
 // partners skipped, must be the members of box_group, in an order that every
 // copy of the node shares and that is ascending wherever box_halo_ok says so;
-// only the z faces may use the last four terms.  Exit status 0 when
+// only the z faces may use the last four terms.  With random values in place of
+// the indices, HaloSum's group sums must be the same bit for bit at every copy
+// of a node and equal the members' sum to rounding, eight equal members must
+// average to themselves, and inv_k must be 1 / (group size).  Exit status 0 when
 // everything holds.
 #define __host__
 #define __device__
 #define __forceinline__ inline
 #define HIP_INCLUDE_HIP_HIP_RUNTIME_H
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <map>
 #include <vector>
 
 #include "gf_boxdss.hpp"
+
+template <int N>
+size_t check_sums(const gf::BoxTopo &t) {
+  using H = gf::Halo<N>;
+  const size_t nel = (size_t)t.ne[0] * t.ne[1] * t.ne[2], nn = (size_t)N * N * N, n = nel * nn;
+  std::vector<double> u(n), hl(H::SIZE), ones(H::SIZE);
+  unsigned r = 12345;
+  for (double &v : u) {
+    r = r * 1664525u + 1013904223u;
+    v = (double)r / 4294967296.0 - 0.5;
+  }
+  size_t wrong = 0;
+  std::map<size_t, double> sums;
+  for (size_t e = 0; e < nel; e++) {
+    int ec[3];
+    gf::box_elem_coords(t, e, ec);
+    const gf::BoxElemDeltas de = gf::box_elem_deltas(t, N, ec);
+    for (size_t q = 0; q < nn; q++) hl[q] = u[e * nn + q];
+    for (int l = 0; l < N * N; l++) {
+      gf::HaloRim<N, double> L;
+      L.issue(u.data(), de, (int64_t)(e * nn), l);
+      L.store(hl.data(), l);
+    }
+    for (size_t q = 0; q < H::SIZE; q++) ones[q] = (int)q < H::ZERO ? u[0] : 0.0;
+    for (int l = 0; l < N * N; l++) {
+      const int i = l % N, j = l / N;
+      const gf::HaloSum<N> hs(de, i, j);
+      gf::static_for<0, N>([&](auto kc) {
+        constexpr int k = decltype(kc)::value;
+        const size_t q = e * nn + i + N * j + (size_t)N * N * k;
+        size_t g[8];
+        const int cnt = gf::box_group(t, N, ec, q, i, j, k, g);
+        double ref = 0.0;
+        for (int s = 0; s < cnt; s++) ref += u[g[s]];
+        const double v = hs.template sum<k>(hl.data(), u[q]);
+        int np = 0;
+        hs.template sum<k>(hl.data(), u[q], [&](double w, bool on) {
+          np += on;
+          return on ? w : 0.0;
+        });
+        auto it = sums.find(g[0]);
+        if (it == sums.end()) sums[g[0]] = v;
+        else wrong += !(it->second == v);
+        wrong += !(std::fabs(v - ref) <= 1e-15) || np != cnt ||
+                 hs.template inv_k<k>() != 1.0 / cnt ||
+                 hs.template sum<k>(ones.data(), u[0]) * hs.template inv_k<k>() != u[0];
+      });
+    }
+  }
+  return wrong;
+}
 
 template <int N>
 size_t check(const gf::BoxTopo &t) {
@@ -71,7 +126,7 @@ size_t check(const gf::BoxTopo &t) {
       });
     }
   }
-  return wrong;
+  return wrong + check_sums<N>(t);
 }
 
 int main() {
