@@ -363,6 +363,10 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 // groups of 2, 4 and 8, so S leaves a continuous state as it is and IN 1 and
 // IN 2 agree bit for bit on it.
 //
+// Stages that do not accumulate (every second one of RK4) walk the elements
+// backwards and start with what the stage before left in the Infinity Cache
+// (32^3, p = 5 817 -> 791 us a step, p = 7 1402 -> 1389).
+//
 // Bound by memory: at 32^3, p = 7 an RK4 step moves 42 fields of 134 MB; the
 // form whose every stage smoothed into the accumulator moved 54 and gathered
 // uin too in the last one.  Stages (IN, ACC) = (3,0) 358, (1,1) 424, (1,0)
@@ -371,7 +375,7 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 // 39 + 41 + 27, where the members were loaded node by node.
 // ---------------------------------------------------------------------------
 template <int N, int IN, int ACC>
-__global__ __launch_bounds__(gf::Pen3<N>::THREADS) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))
+__global__ __launch_bounds__(gf::PenS<N>::THREADS) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))
 void k_burgers_stage3b(
     const double *__restrict__ ui0, const double *__restrict__ ui1, const double *__restrict__ ui2,
     const double *__restrict__ kp0, const double *__restrict__ kp1, const double *__restrict__ kp2,
@@ -379,7 +383,7 @@ void k_burgers_stage3b(
     double *__restrict__ ko2, const double *__restrict__ imass, const double *__restrict__ W,
     const double *__restrict__ edx, const double *__restrict__ ejac, gf::PenD<double> Dp,
     double bh, double ca, double cb, double nu, gf::BoxTopo topo, size_t nelems, size_t imstride) {
-  using S = gf::Pen3<N>;
+  using S = gf::PenS<N>;
   using H = gf::Halo<N>;
   constexpr bool KP = IN != 0, GU = IN == 2, UIN = IN != 3;
   static_assert(KP || ACC == 0, "the first stage accumulates nothing");
@@ -398,7 +402,7 @@ void k_burgers_stage3b(
   const double *kp[3] = {kp0, kp1, kp2};
   double *acc[3] = {ac0, ac1, ac2};
   double *kout[3] = {ko0, ko1, ko2};
-  ColIdx<N> t(nelems);
+  ColIdx<N, gf::PenS<N>> t(nelems, ACC == 0);
   const size_t col = t.e * S::NN + t.r;
   double *hk = sl + t.el * NSL;
   double im[N];
@@ -509,7 +513,7 @@ void k_burgers_stage3b(
       const double urhs = fma(-po, M, -L);
       const double K = im[k] * urhs;
       if (ACC < 2 || ACC == 4) ko[g] = K;
-      if (RA) ac[g] = fma(cb, K, ra[RA ? c : 0][RA ? k : 0]);
+      if constexpr (RA) ac[g] = fma(cb, K, ra[c][k]);
     };
     gf::pen_op3<N, double, true>(ru[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,
                                  rz * rz, (const double *)nullptr, xcb, ycb, zcb, post);
@@ -520,16 +524,16 @@ void k_burgers_stage3b(
 // Step output on a structured box: u = S(acc), the Smooth by gather through
 // the LDS halo, with the operations of the fused form (IN 3 above).
 template <int N>
-__global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_rk_out_halo(
+__global__ __launch_bounds__(gf::PenS<N>::THREADS) void k_rk_out_halo(
     double *__restrict__ u0, double *__restrict__ u1, double *__restrict__ u2,
     const double *__restrict__ a0, const double *__restrict__ a1, const double *__restrict__ a2,
     gf::BoxTopo topo, size_t nelems) {
-  using S = gf::Pen3<N>;
+  using S = gf::PenS<N>;
   using H = gf::Halo<N>;
   __shared__ double sl[S::EPB * H::SIZE];
   double *u[3] = {u0, u1, u2};
   const double *acc[3] = {a0, a1, a2};
-  ColIdx<N> t(nelems);
+  ColIdx<N, gf::PenS<N>> t(nelems);
   double *hk = sl + t.el * H::SIZE;
   const int l = t.r;
   const int64_t ebase = (int64_t)t.e * S::NN;
@@ -565,7 +569,7 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_rk_out_halo(
 template <int N, int IN, int ACC>
 int launch_stage3b_h(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
                      double *const *kout, double bh, double ca, double cb, double nu) {
-  using S = gf::Pen3<N>;
+  using S = gf::PenS<N>;
   const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
   auto at = [](double *const *p, int c) { return p ? p[c] : nullptr; };
   hipLaunchKernelGGL((k_burgers_stage3b<N, IN, ACC>), dim3(nb), dim3(S::THREADS), 0,
@@ -599,7 +603,7 @@ int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *co
 
 template <int N>
 int launch_rk_out_box(gf_mesh *m, double *const *u, double *const *acc) {
-  using S = gf::Pen3<N>;
+  using S = gf::PenS<N>;
   hipLaunchKernelGGL(k_rk_out_halo<N>, dim3(xcd_grid((m->nelems + S::EPB - 1) / S::EPB)),
                      dim3(S::THREADS), 0, m->ctx->stream, u[0], u[1], u[2], acc[0], acc[1], acc[2],
                      m->box, m->nelems);

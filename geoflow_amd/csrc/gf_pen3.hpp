@@ -130,6 +130,16 @@ struct Pen3 {
   __device__ static constexpr int at(int i, int j, int k) { return i + j * P + k * SK; }
 };
 
+// Workgroups of the box RK stages: where one element leaves a wave's lanes idle
+// (36 of 64 at N = 6, 81 of 128 at N = 9) three elements share a workgroup.
+// RK4 steps: 32^3, p = 5 791 -> 721 us, 20^3, p = 8 755 -> 641.  At N = 5 and 7
+// packing five elements gained nothing (24^3, p = 6 533 -> 535).
+template <int N>
+struct PenS : Pen3<N> {
+  static constexpr int EPB = (N == 6 || N == 9) ? 3 : Pen3<N>::EPB;
+  static constexpr int THREADS = EPB * N * N;
+};
+
 // Computes, for the column (i=a, j=b) owned by the calling thread,
 //   post(k, Lu_k, M_k, hx_k, hy_k),   Lu = ((x-part + y-part) + z-part)
 // where each part is D_d^T (M * ((D_d u) * G_d) [* p]), the operations of

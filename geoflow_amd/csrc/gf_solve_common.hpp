@@ -86,9 +86,10 @@ inline gf::PenD<float> pend_f(gf_mesh *m) {
 // run on the same XCD close together in time.
 constexpr int kXCD = 8;
 inline int xcd_grid(size_t nblocks) { return (int)((nblocks + kXCD - 1) / kXCD * kXCD); }
-__device__ __forceinline__ size_t xcd_block() {
-  const size_t per = gridDim.x / kXCD;
-  return (size_t)(blockIdx.x % kXCD) * per + blockIdx.x / kXCD;
+// rev: each XCD walks its range from the end.
+__device__ __forceinline__ size_t xcd_block(bool rev = false) {
+  const size_t per = gridDim.x / kXCD, at = blockIdx.x / kXCD;
+  return (size_t)(blockIdx.x % kXCD) * per + (rev ? per - 1 - at : at);
 }
 
 // Copies the 512 doubles at g (an element, 4 KB) to LDS at l with four
@@ -112,18 +113,18 @@ __device__ __forceinline__ void lds_copy512(const double *__restrict__ g, double
        g += (size_t)gridDim.x * blockDim.x)
 
 // Thread/element mapping shared by the 3-D element kernels.
-template <int N>
+template <int N, typename P = gf::Pen3<N>>
 struct ColIdx {
   int el, i, j, r;
   size_t e;
   bool active;
-  __device__ __forceinline__ ColIdx(size_t nelems) {
-    using C = gf::Pen3<N>;
+  __device__ __forceinline__ ColIdx(size_t nelems, bool rev = false) {
+    using C = P;
     el = threadIdx.x / C::N2;
     r = threadIdx.x - el * C::N2;
     i = r % N;
     j = r / N;
-    size_t eg = xcd_block() * C::EPB + el;
+    size_t eg = xcd_block(rev) * C::EPB + el;
     active = el < C::EPB && eg < nelems;
     e = active ? eg : (nelems - 1);
   }
