@@ -24,6 +24,13 @@ struct gf_ctx_s {
 // Reduction slot layout on the device (see gf_reduce.hpp).
 #define GF_RED_MAX_BLOCKS 4096
 
+// Up to this many nodes the CG update gathers each group from its list
+// (gf_mesh_s::nref) instead of a DSS pass ahead of it, which is then mostly
+// launch.  us an iteration FP64 / FP32, list against pass: terrain 185 k nodes
+// 16.7 against 21 (FP64), 516 k 27.2 / 19.8 against 29.1 / 21.2, sphere 753 k
+// 31.7 / 23.2 against 32.4 / 22.6, 1.5 M 50.6 / 40.5 against 50.3 / 38.3.
+constexpr size_t kNrefMax = (size_t)3 << 18;
+
 struct gf_mesh_s {
   gf_ctx *ctx = nullptr;
   int dim = 3, gtype = 0;
@@ -73,6 +80,10 @@ struct gf_mesh_s {
   // 2-D regular isotropic meshes with groups of at most 4: the members of every
   // node's group, ascending, -1 past the group (the RK stages gather with it)
   int4 *mem4 = nullptr;
+  // Meshes of up to kNrefMax nodes without a box structure: per node the offset
+  // of its group in gmem and the group's size (1: no group), for the CG
+  // update's gather
+  int2 *nref = nullptr;
   // Structured box: when has_box, the groups above are exactly those of
   // gf::box_group for `box`, and fused kernels may assemble by gather.
   gf::BoxTopo box = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0, 0, 0, 0}};

@@ -613,6 +613,20 @@ __global__ void k_mem4_groups(int4 *__restrict__ mem4, const int *__restrict__ g
   }
 }
 
+// Offset of every node's group in gmem and its size.
+__global__ void k_nref_self(int2 *__restrict__ nref, size_t n) {
+  for (size_t g = blockIdx.x * (size_t)blockDim.x + threadIdx.x; g < n;
+       g += (size_t)gridDim.x * blockDim.x)
+    nref[g] = make_int2(0, 1);
+}
+__global__ void k_nref_groups(int2 *__restrict__ nref, const int *__restrict__ goff,
+                              const int *__restrict__ gmem, int ngroups) {
+  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g < ngroups; g += gridDim.x * blockDim.x) {
+    const int b = goff[g], e = goff[g + 1];
+    for (int s = b; s < e; s++) nref[gmem[s]] = make_int2(b, e - b);
+  }
+}
+
 // Deterministic two-stage sum: per-block partials then one block in order.
 __global__ void k_partial_dot(const double *__restrict__ a, const double *__restrict__ b,
                               double *__restrict__ part, size_t n) {
@@ -1150,6 +1164,13 @@ int gf_mesh_create(gf_ctx *ctx, const gf_mesh_desc *d, gf_mesh **out) {
   if (m->ngroups)
     hipLaunchKernelGGL(k_imult_groups, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
                        m->imult, m->goff, m->gmem, m->ngroups);
+  if (m->Niso && !(m->has_box && m->dconst) && n <= kNrefMax) {
+    GF_HIP(ctx, hipMalloc((void **)&m->nref, n * sizeof(int2)));
+    hipLaunchKernelGGL(k_nref_self, dim3(nblocks(n)), dim3(kThreads), 0, s, m->nref, n);
+    if (m->ngroups)
+      hipLaunchKernelGGL(k_nref_groups, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
+                         m->nref, m->goff, m->gmem, m->ngroups);
+  }
   if (m->dim == 2 && d->gtype == GF_GE_REGULAR && m->Niso && m->maxgrp <= 4) {
     GF_HIP(ctx, hipMalloc((void **)&m->mem4, n * sizeof(int4)));
     hipLaunchKernelGGL(k_mem4_self, dim3(nblocks(n)), dim3(kThreads), 0, s, m->mem4, n);
@@ -1221,7 +1242,7 @@ int gf_mesh_destroy(gf_mesh *m) {
   F(m->mask); F(m->mass); F(m->imass); F(m->imass_el); F(m->dtab); F(m->dtab32); F(m->deq);
   F(m->imult); F(m->mask32);
   F(m->imult32);
-  F(m->goff); F(m->gmem); F(m->mem4); F(m->red); F(m->scal);
+  F(m->goff); F(m->gmem); F(m->mem4); F(m->nref); F(m->red); F(m->scal);
   for (int k = 0; k < 6; k++) F(m->G32[k]);
   F(m->mass32);
   if (m->hscal) (void)hipHostFree(m->hscal);

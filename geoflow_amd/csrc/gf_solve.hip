@@ -493,28 +493,61 @@ __global__ void k_dss_cg(T *__restrict__ u, const int *__restrict__ goff,
   }
 }
 
-// CG update where q has been assembled by a DSS pass (CGCtl):
-// r -= alpha mask q ; partials of r.z.imult and of the norm.
-template <typename T, int NORM>
+// CG update on meshes without a box structure (CGCtl): r -= alpha mask DSS(q);
+// partials of r.z.imult and of the norm.  G: q is assembled here from the
+// node's group list (members ascending, the sum of k_dss), else by a DSS pass
+// that ran before.
+template <typename T, int NORM, bool G>
 __global__ void k_cg_update(CGCtl c, T *__restrict__ r, const T *__restrict__ qv,
                             const T *__restrict__ mask, const T *__restrict__ dinv,
                             const T *__restrict__ imult, const double *__restrict__ mass,
-                            size_t nn) {
+                            size_t nn, const int2 *__restrict__ nref,
+                            const int *__restrict__ gmem) {
   __shared__ double sred[2 * (kThreads / 64)];
   const CGBlock b(c, (int)xcd_block(), c.nbU);
   if (!b.ok) return;
   CGAlphaHead h(c, b);
+  const size_t n1 = b.e1 * nn, step = (size_t)b.nb * blockDim.x;
+  size_t g = b.e0 * nn + (size_t)b.lb * blockDim.x + threadIdx.x;
+  T q = T(0), rv = T(0), dv = T(1), mk = T(1), im = T(0);
+  auto load = [&]() {
+    if constexpr (G) {
+      const int2 f = nref[g];
+      if (f.y == 1) {
+        q = qv[g];
+      } else {
+        int id[8];
+        T v[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) id[k] = k < f.y ? gmem[f.x + k] : 0;
+#pragma unroll
+        for (int k = 0; k < 8; k++) v[k] = k < f.y ? qv[id[k]] : T(0);
+        q = T(0);
+#pragma unroll
+        for (int k = 0; k < 8; k++)
+          if (k < f.y) q = q + v[k];
+        for (int k = 8; k < f.y; k++) q = q + qv[gmem[f.x + k]];
+      }
+    } else {
+      q = qv[g];
+    }
+    rv = r[g];
+    if (dinv) dv = dinv[g];
+    if (mask) mk = mask[g];
+    im = imult[g];
+  };
+  if (g < n1) load();  // in flight with the scalars' loads
   double alpha64;
   if (!h.finish(b, sred, alpha64)) return;
   const T alpha = (T)alpha64;
   double rho = 0.0, nrm = 0.0;
-  const size_t n1 = b.e1 * nn, step = (size_t)b.nb * blockDim.x;
-  for (size_t g = b.e0 * nn + (size_t)b.lb * blockDim.x + threadIdx.x; g < n1; g += step) {
-    const T qm = mask ? qv[g] * mask[g] : qv[g];
-    const T rv = r[g] + (-alpha) * qm;
-    r[g] = rv;
-    cg_accum<NORM>((double)rv, dinv ? (double)(dinv[g] * rv) : (double)rv, (double)imult[g], mass, g,
-                   rho, nrm);
+  while (g < n1) {
+    const T qm = mask ? q * mk : q;
+    const T rn = rv + (-alpha) * qm;
+    r[g] = rn;
+    cg_accum<NORM>((double)rn, dinv ? (double)(dv * rn) : (double)rn, (double)im, mass, g, rho, nrm);
+    g += step;
+    if (g < n1) load();
   }
   const double ra = gf::block_reduce<false>(rho, sred);
   const double rb = NORM == GF_NORM_INF ? gf::block_reduce<true>(nrm, sred)
@@ -1694,8 +1727,13 @@ template <typename T, int NORM>
 int launch_update(gf_mesh *m, const CGCtl &c, const CGVecs<T> &v, bool gather, bool mask_in_q) {
   if (gather) return launch_update_box<T, NORM>(m, c, v);
   const T *mk = (m->has_mask && !mask_in_q) ? v.mask : nullptr;
-  hipLaunchKernelGGL((k_cg_update<T, NORM>), dim3(c.nbU), dim3(kThreads), 0, m->ctx->stream, c, v.r,
-                     v.q, mk, v.dinv, v.imult, m->mass, m->nn);
+  if (m->nref)
+    hipLaunchKernelGGL((k_cg_update<T, NORM, true>), dim3(c.nbU), dim3(kThreads), 0, m->ctx->stream,
+                       c, v.r, v.q, mk, v.dinv, v.imult, m->mass, m->nn, m->nref, m->gmem);
+  else
+    hipLaunchKernelGGL((k_cg_update<T, NORM, false>), dim3(c.nbU), dim3(kThreads), 0,
+                       m->ctx->stream, c, v.r, v.q, mk, v.dinv, v.imult, m->mass, m->nn,
+                       (const int2 *)nullptr, (const int *)nullptr);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
@@ -1811,7 +1849,7 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
       else
         RC(sizeof(T) == 8 ? GF_DISPATCH_N(m->dim, m->Niso, launch_cg_apply_d, m, a)
                           : GF_DISPATCH_N(m->dim, m->Niso, launch_cg_apply_f, m, a));
-      if (m->ngroups && !gather)
+      if (m->ngroups && !gather && !m->nref)
         hipLaunchKernelGGL(k_dss_cg<T>, dim3(nblocks((size_t)m->ngroups)), dim3(kThreads), 0, s,
                            v.q, m->goff, m->gmem, m->ngroups,
                            ns > 0 ? (const double *)nullptr
