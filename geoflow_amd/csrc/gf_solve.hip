@@ -1212,8 +1212,8 @@ namespace {
 // ---- pure-advection stage on 2-D embedded (sphere) elements ----------------
 // One kernel per RK stage computes, per element,
 //   us   = uin + bh Kprev            (stage input; Kprev already smoothed)
-//   ust  = ust + ch Kprev            (the step_b accumulation of Kprev)
 //   K    = imass * ( -nu L us - M (c . grad us) )
+//   acc  = base + ch Kprev + cn K    (the step_b accumulation, every second stage)
 // with the advection of GAdvect::apply on an embedded grid (gadvect.ipp:57-99,
 // deriv(p,j) = (D1 p) dXidX(0,j) + (D2 p) dXidX(1,j), ggrid.ipp:1179-1200) and
 // the Laplacian of embed_prod (ghelmholtz.ipp:205-290).  The advection is
@@ -1225,15 +1225,12 @@ namespace {
 // The regrouping changes rounding only (relative 1e-16 per term).
 template <typename T>
 struct EmbAdvArgs {
-  const T *uin;         // stage input base (state at s = 0, step-start copy after)
+  const T *uin;         // stage input base
   const T *kprev;       // smoothed K of the previous stage, or null
-  T *ust;               // state, advanced by ch * kprev when kprev is set
-  T *ucopy;             // step-start copy: receives uin when kprev is null, else (the
-                        // previous step's output fused with this step's first stage)
-                        // uin + bh kprev, which ust receives too and which is the
-                        // stage's input
-  int acc_from_uin;     // the accumulation of kprev starts from the stage's uin
-                        // value instead of ust (the step's first accumulation)
+  const T *base;        // accumulation base, null: the uin value
+  T *acc;               // receives the accumulation, or null (node by node, so
+                        // that it may be uin or base)
+  double cn;
   double bh, ch, nu;
   const double *c[3];   // velocity (read when wform is set)
   const double *ndx[6]; // dXi_i/dX_j at [i*3+j]
@@ -1242,7 +1239,7 @@ struct EmbAdvArgs {
   const T *D;
   double *w[2];         // imass M chat_i: written when wform is set, else read
   int wform;
-  T *kout;
+  T *kout;              // K, or null
   size_t nelems;
 };
 
@@ -1264,20 +1261,12 @@ __global__ __launch_bounds__(kThreads) void k_adv_stage_embed(EmbAdvArgs<T> a) {
   const int q = threadIdx.x;
   const bool act = q < nel * S::NN;
   const size_t g = base + q;
+  T ra = T(0);
   if (act) {
     T v = a.uin[g];
-    if (a.kprev && a.ucopy) {
-      v = fma((T)a.bh, a.kprev[g], v);
-      a.ust[g] = v;
-      a.ucopy[g] = v;
-    } else if (a.kprev) {
-      const T kp = a.kprev[g];
-      const T base = a.acc_from_uin ? v : a.ust[g];
-      a.ust[g] = fma((T)a.ch, kp, base);
-      v = fma((T)a.bh, kp, v);
-    } else if (a.ucopy) {
-      a.ucopy[g] = v;
-    }
+    const T kp = a.kprev ? a.kprev[g] : T(0);
+    if (a.acc) ra = fma((T)a.ch, kp, a.base ? a.base[g] : v);
+    if (a.kprev) v = fma((T)a.bh, kp, v);
     su[q] = v;
   }
   __syncthreads();
@@ -1318,7 +1307,9 @@ __global__ __launch_bounds__(kThreads) void k_adv_stage_embed(EmbAdvArgs<T> a) {
     lt += gf::contract<2, N, true>(&sg[1][el * S::NN], sD, 1, i, j, k);
     double lap = lt;
     if (a.nu != 1.0) lap *= a.nu;
-    a.kout[g] = (T)(im * (-lap) - po);
+    const T kn = (T)(im * (-lap) - po);
+    if (a.kout) a.kout[g] = kn;
+    if (a.acc) a.acc[g] = fma((T)a.cn, kn, ra);
   }
 }
 
@@ -1349,6 +1340,7 @@ int launch_adv_stage_embed_t(gf_mesh *m, const EmbAdvArgs<float> &a) {
   return GF_DISPATCH_N(2, m->Niso, launch_adv_stage_embed_f, m, a);
 }
 
+// u3 = uin + bh k; acc += ch k
 template <typename T>
 __global__ void k_final_input_t(T *__restrict__ u3, const T *__restrict__ uin,
                                 const T *__restrict__ k, T bh, T *acc, const T *accsrc, T ch,
@@ -1359,11 +1351,6 @@ __global__ void k_final_input_t(T *__restrict__ u3, const T *__restrict__ uin,
     if (acc) acc[g] = fma(ch, kv, accsrc[g]);
   }
 }
-// z += b y
-template <typename T>
-__global__ void k_add_t(T *z, T b, const T *__restrict__ y, size_t n) {
-  XCD_GRID_LOOP(g, n) z[g] = fma(b, y[g], z[g]);
-}
 int dss_smooth(gf_mesh *m, double *u) { return gf_dss_t(m, GF_DSS_SMOOTH, u); }
 int dss_smooth(gf_mesh *m, float *u) { return gf_dss_f32(m, GF_DSS_SMOOTH, u); }
 
@@ -1371,14 +1358,20 @@ int dss_smooth(gf_mesh *m, float *u) { return gf_dss_f32(m, GF_DSS_SMOOTH, u); }
 // components (mode 1, nstate 4): the arithmetic of rk_step_general with each
 // stage's RHS, stage input and state accumulation fused into one element
 // kernel.  Stage sequence (step_b, gexrk_stepper.ipp:251-341):
-//   s < ns-1:  K_s = F(uin + b_{s,s-1} h K_{s-1});  Smooth K_s;  ust += c_s h K_s
-//   last:      us = uin + b h K_{ns-2};  Smooth us;  K = F(us);  Smooth K;
-//              ust += c h K;  Smooth ust
-// (from the second step on without the last two Smooths, see below: level 5,
-// p = 5, a step takes 170 us against 234 with six DSS passes and the
-// pointwise kernels)
-// where the ust accumulation of K_{s-1} is done by stage s's kernel, the
-// first one from the step-start copy of uin (equal to ust at that point).
+//   s < ns-1:  K_s = F(u + b_{s,s-1} h K_{s-1});  Smooth K_s
+//   last:      us = u + b h K_{ns-2};  Smooth us;  K = F(us)
+//   u = Smooth(u + sum_s c_s h K_s)
+// The accumulation takes the last K, and at odd s the K the kernel has just
+// formed, before their Smooth: Smooth is linear and the sum is smoothed in the
+// end.  So it runs at every second stage, the last K is never stored, and u
+// stays as it is until the last stage overwrites it: 36 fields a step of order
+// 4 where a sum advanced at each stage and a copy of u move 43.  The state
+// passed in may be discontinuous; from the second step on u is continuous, the
+// Smooth of us is the identity, and the last stage's kernel forms us as the
+// others do.  Level 5, p = 5, order 4 (2.2 M nodes), a step: 234 us with six
+// DSS passes and pointwise kernels, 172 with four and no pointwise kernel, 156
+// with the fewer fields; a stage kernel moves 8 to 10 fields at 6.8 TB/s, a DSS
+// pass takes 13 us.
 // The Butcher tables of orders 1-4 have only sub-diagonal b, so the
 // reference's isum = sum_j b_{sj} h K_j equals b_{s,s-1} h K_{s-1} exactly.
 // (Forming the Smooths by gather in the reading kernels instead of the DSS
@@ -1394,12 +1387,12 @@ int rk_steps_embed_adv_t(gf_mesh *m, double nu, int order, double dt, T *ust0,
   butcher(order, alpha, beta, c);
   const int ns = order;
   const double h = dt;
-  T *ucopy = (T *)gf_ws(m, WS_RK_BEGIN + 0, bytes);
+  T *acc = (T *)gf_ws(m, WS_RK_BEGIN + 0, bytes);
   T *us = (T *)gf_ws(m, WS_RK_BEGIN + 3, bytes);
   T *K[2] = {(T *)gf_ws(m, WS_RK_BEGIN + 6, bytes), (T *)gf_ws(m, WS_RK_BEGIN + 9, bytes)};
   double *w0 = (double *)gf_ws(m, WS_RK_BEGIN + 1, dbytes);
   double *w1 = (double *)gf_ws(m, WS_RK_BEGIN + 2, dbytes);
-  if (!ucopy || !us || !K[0] || !K[1] || !w0 || !w1)
+  if (!acc || !us || !K[0] || !K[1] || !w0 || !w1)
     return gf_set_err(m->ctx, GF_ERR_ALLOC, "workspace");
   EmbAdvArgs<T> a;
   memset(&a, 0, sizeof(a));
@@ -1413,60 +1406,39 @@ int rk_steps_embed_adv_t(gf_mesh *m, double nu, int order, double dt, T *ust0,
   a.w[0] = w0;
   a.w[1] = w1;
   a.nelems = m->nelems;
-  T *kl = K[(ns - 1) % 2];
-  const T cl = (T)(c[ns - 1] * h);
-  // ust += c h K_last, and its Smooth (keep: the identity on a continuous one)
-  auto output = [&](bool smooth) -> int {
-    hipLaunchKernelGGL(k_add_t<T>, dim3(xcd_grid(nblocks(n))), dim3(kThreads), 0, m->ctx->stream,
-                       ust0, cl, kl, n);
-    GF_LAUNCH_CHECK(m->ctx);
-    return smooth ? gf_dss_keep(m, ust0) : GF_OK;
-  };
   for (int step = 0; step < nsteps; step++) {
-    // The state passed in may be discontinuous; after the first step it is
-    // continuous, and then the Smooths of the final-stage input and of the
-    // output are the identity: the former is formed in the last stage's
-    // kernel, the latter in the next step's first stage.  The velocity is
-    // constant in a call: w_i is formed once.
-    const bool cont = step > 0 && ns > 1;
-    for (int s = 0; s < (cont ? ns : ns - 1); s++) {
-      a.wform = step == 0 && s == 0;
-      a.uin = s == 0 ? ust0 : ucopy;
-      a.acc_from_uin = s == 1;
-      a.ust = ust0;
-      a.ucopy = s == 0 ? ucopy : nullptr;
-      a.kprev = s == 0 ? (step > 1 ? kl : nullptr) : K[(s - 1) % 2];
-      a.bh = s == 0 ? (double)cl : beta[s * 4 + (s - 1)] * h;
-      a.ch = s == 0 ? 0.0 : c[s - 1] * h;
-      a.kout = K[s % 2];
+    for (int s = 0; s < ns; s++) {
+      const bool last = s == ns - 1, odd = s % 2 == 1;
+      const T *kp = s > 0 ? K[(s - 1) % 2] : nullptr;
+      const T *base = s > 1 ? acc : ust0;
+      a.wform = step == 0 && s == 0;  // the velocity is constant in a call
+      a.uin = ust0;
+      a.kprev = kp;
+      a.bh = s > 0 ? beta[s * 4 + (s - 1)] * h : 0.0;
+      a.base = s > 1 ? acc : nullptr;
+      a.ch = odd ? c[s - 1] * h : 0.0;
+      a.cn = c[s] * h;
+      a.acc = last ? ust0 : odd ? acc : nullptr;
+      a.kout = last ? nullptr : K[s % 2];
+      if (last && (step == 0 || ns == 1)) {
+        // the state may be discontinuous
+        if (s > 0) {
+          hipLaunchKernelGGL(k_final_input_t<T>, dim3(xcd_grid(nblocks(n))), dim3(kThreads), 0,
+                             m->ctx->stream, us, ust0, kp, (T)a.bh, odd ? acc : nullptr, base,
+                             (T)a.ch, n);
+          GF_LAUNCH_CHECK(m->ctx);
+          a.base = acc;
+        } else {
+          GF_HIP(m->ctx, hipMemcpyAsync(us, ust0, bytes, hipMemcpyDeviceToDevice, m->ctx->stream));
+          a.base = ust0;
+        }
+        RC(gf_dss_keep(m, us));
+        a.uin = us;
+        a.kprev = nullptr;
+      }
       RC(launch_adv_stage_embed_t(m, a));
-      RC(dss_smooth(m, K[s % 2]));
+      RC(last ? gf_dss_keep(m, ust0) : dss_smooth(m, K[s % 2]));
     }
-    if (cont) {
-      if (step == nsteps - 1) RC(output(false));
-      continue;
-    }
-    if (ns >= 2) {
-      // order 2: the step's first accumulation, from the step-start copy
-      hipLaunchKernelGGL(k_final_input_t<T>, dim3(xcd_grid(nblocks(n))), dim3(kThreads), 0,
-                         m->ctx->stream, us, ucopy, K[(ns - 2) % 2],
-                         (T)(beta[(ns - 1) * 4 + (ns - 2)] * h), ust0, ns == 2 ? ucopy : ust0,
-                         (T)(c[ns - 2] * h), n);
-      GF_LAUNCH_CHECK(m->ctx);
-    } else {
-      GF_HIP(m->ctx, hipMemcpyAsync(us, ust0, bytes, hipMemcpyDeviceToDevice, m->ctx->stream));
-    }
-    RC(gf_dss_keep(m, us));
-    a.uin = us;
-    a.acc_from_uin = 0;
-    a.kprev = nullptr;
-    a.ucopy = nullptr;
-    a.wform = ns == 1 && step == 0;
-    a.bh = a.ch = 0.0;
-    a.kout = kl;
-    RC(launch_adv_stage_embed_t(m, a));
-    RC(dss_smooth(m, kl));
-    RC(output(true));
   }
   return GF_OK;
 }
