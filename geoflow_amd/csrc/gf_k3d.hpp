@@ -359,6 +359,9 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 //     2  acc = uin + ca kp + cb K       (last stage: K is not stored)
 //     3  acc = acc + ca kp + cb K       (last stage)
 //     4  acc = v                        K -> kout  (stage states of the adjoint)
+//   SP  a third of the workgroup's threads to each component, which exchange
+//       the stage input through LDS; else a thread does all three in turn.
+//       The same operations (stage_split_max says which runs)
 // Group sums are pairwise (x, then y, then z), exact for equal members of
 // groups of 2, 4 and 8, so S leaves a continuous state as it is and IN 1 and
 // IN 2 agree bit for bit on it.
@@ -371,11 +374,10 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 // form whose every stage smoothed into the accumulator moved 54 and gathered
 // uin too in the last one.  Stages (IN, ACC) = (3,0) 358, (1,1) 424, (1,0)
 // 338, (1,3) 399 us, 3.6-3.8 TB/s where a copy of this size has 4.7; before,
-// 392 + 543 + 459 + 601 us.  19x14x11, p = 5 (RK3): 27 + 27 + 22 us against
-// 39 + 41 + 27, where the members were loaded node by node.
+// 392 + 543 + 459 + 601 us.
 // ---------------------------------------------------------------------------
-template <int N, int IN, int ACC>
-__global__ __launch_bounds__(gf::PenS<N>::THREADS) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))
+template <int N, int IN, int ACC, bool SP>
+__global__ __launch_bounds__((gf::PenStage<N, SP>::THREADS)) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))
 void k_burgers_stage3b(
     const double *__restrict__ ui0, const double *__restrict__ ui1, const double *__restrict__ ui2,
     const double *__restrict__ kp0, const double *__restrict__ kp1, const double *__restrict__ kp2,
@@ -383,33 +385,37 @@ void k_burgers_stage3b(
     double *__restrict__ ko2, const double *__restrict__ imass, const double *__restrict__ W,
     const double *__restrict__ edx, const double *__restrict__ ejac, gf::PenD<double> Dp,
     double bh, double ca, double cb, double nu, gf::BoxTopo topo, size_t nelems, size_t imstride) {
-  using S = gf::PenS<N>;
+  using S = gf::PenStage<N, SP>;
   using H = gf::Halo<N>;
   constexpr bool KP = IN != 0, GU = IN == 2, UIN = IN != 3;
   static_assert(KP || ACC == 0, "the first stage accumulates nothing");
   static_assert(IN != 3 || ACC == 0, "an output stage is a first stage");
   // N = 8: an element is one wave and its own values go straight to LDS
   // (lds_copy512), behind kp's halo; else they pass through registers
-  constexpr bool L8 = N == 8;
+  constexpr bool L8 = N == 8 && !SP;
   constexpr int UOFF = H::SIZE, AOFF = UOFF + 512;
   constexpr int HL = !KP ? 0
                          : (GU ? 2 * H::SIZE
                                : H::SIZE + (L8 && UIN ? 512 : 0)) + (L8 && ACC == 3 ? 512 : 0);
   // per element: the halos, then (the same memory) the three element buffers
   constexpr int NSL = HL > 3 * S::SZ ? HL : 3 * S::SZ;
-  __shared__ double sl[S::EPB * NSL];
+  constexpr int NC = SP ? 3 : 1, TPC = S::EPB * S::N2;
+  __shared__ double sl[NC * S::EPB * NSL];
   const double *uin[3] = {ui0, ui1, ui2};
   const double *kp[3] = {kp0, kp1, kp2};
   double *acc[3] = {ac0, ac1, ac2};
   double *kout[3] = {ko0, ko1, ko2};
-  ColIdx<N, gf::PenS<N>> t(nelems, ACC == 0);
+  const int cs = SP ? (int)threadIdx.x / TPC : 0;
+  ColIdx<N, S> t(nelems, ACC == 0, SP ? (int)threadIdx.x - cs * TPC : (int)threadIdx.x);
   const size_t col = t.e * S::NN + t.r;
-  double *hk = sl + t.el * NSL;
+  double *hk = sl + (cs * S::EPB + t.el) * NSL;
   double im[N];
 #pragma unroll
   for (int k = 0; k < N; k++) im[k] = imass[t.e * imstride + t.r + (size_t)k * S::N2];
   constexpr bool RA = ACC >= 1 && ACC <= 3;  // accumulates after the operator
-  double ru[3][N], ra[RA ? 3 : 1][RA ? N : 1];
+  // SP: this thread's component, else all three
+  double rv[SP ? 1 : 3][N], ra[RA && !SP ? 3 : 1][RA ? N : 1];
+  auto pick = [&](auto *const (&p)[3]) { return cs == 0 ? p[0] : (cs == 1 ? p[1] : p[2]); };
   if constexpr (KP) {
     int ec[3];
     gf::box_elem_coords(topo, t.e, ec);
@@ -419,30 +425,32 @@ void k_burgers_stage3b(
     double *hu = hk + UOFF;
     double *ha = hk + (GU ? 2 * H::SIZE : AOFF);
     const gf::HaloSum<N> hs(de, t.i, t.j);
-    gf::static_for<0, 3>([&](auto cc) {
+    gf::static_for<0, SP ? 1 : 3>([&](auto cc) {
       constexpr int c = decltype(cc)::value;
-      __syncthreads();  // the previous component's group sums have read LDS
+      const double *kpc = SP ? pick(kp) : kp[c], *uic = SP ? pick(uin) : uin[c];
+      double *acl = SP ? pick(acc) : acc[c];
+      if (c > 0) __syncthreads();  // the previous component's group sums have read LDS
       // every load of the component is issued before the first LDS store
       double ko[N], uo[N], ao[N];
       if constexpr (L8) {
-        lds_copy512(kp[c] + ebase, hk, l);
-        if (UIN) lds_copy512(uin[c] + ebase, hu, l);
-        if (ACC == 3) lds_copy512(acc[c] + ebase, ha, l);
+        lds_copy512(kpc + ebase, hk, l);
+        if (UIN) lds_copy512(uic + ebase, hu, l);
+        if (ACC == 3) lds_copy512(acl + ebase, ha, l);
       } else {
 #pragma unroll
-        for (int k = 0; k < N; k++) ko[k] = kp[c][col + (size_t)k * S::N2];
+        for (int k = 0; k < N; k++) ko[k] = kpc[col + (size_t)k * S::N2];
         if (UIN) {
 #pragma unroll
-          for (int k = 0; k < N; k++) uo[k] = uin[c][col + (size_t)k * S::N2];
+          for (int k = 0; k < N; k++) uo[k] = uic[col + (size_t)k * S::N2];
         }
         if (ACC == 3) {
 #pragma unroll
-          for (int k = 0; k < N; k++) ao[k] = acc[c][col + (size_t)k * S::N2];
+          for (int k = 0; k < N; k++) ao[k] = acl[col + (size_t)k * S::N2];
         }
       }
       gf::HaloRim<N, double> Lk, Lu;
-      Lk.issue(kp[c], de, ebase, l);
-      if (GU) Lu.issue(uin[c], de, ebase, l);
+      Lk.issue(kpc, de, ebase, l);
+      if (GU) Lu.issue(uic, de, ebase, l);
       Lk.store(hk, l);
       if (GU) Lu.store(hu, l);
       if constexpr (!L8) {
@@ -462,7 +470,7 @@ void k_burgers_stage3b(
         double v;
         if constexpr (IN == 3) {
           v = ks;
-          if (t.active) acc[c][col + (size_t)k * S::N2] = v;
+          if (t.active) acl[col + (size_t)k * S::N2] = v;
         } else {
           const double u = L8 ? hu[own] : uo[k];
           v = fma(bh, ks, u);
@@ -479,45 +487,60 @@ void k_burgers_stage3b(
         // (354 registers instead of 154 at N = 8, IN 1, ACC 0)
         asm volatile("" : "+v"(v));
         if constexpr (ACC == 4) {
-          if (t.active) acc[c][col + (size_t)k * S::N2] = v;
+          if (t.active) acl[col + (size_t)k * S::N2] = v;
         }
-        ru[c][k] = v;
+        rv[c][k] = v;
       });
     });
     __syncthreads();  // the element buffers below reuse the halo area
   } else {
 #pragma unroll
+    for (int c = 0; c < (SP ? 1 : 3); c++) {
+      const double *uic = SP ? pick(uin) : uin[c];
+#pragma unroll
+      for (int k = 0; k < N; k++) rv[c][k] = uic[col + (size_t)k * S::N2];
+    }
+  }
+  // the velocity of the column
+  double va[SP ? 3 : 1][N];
+  if constexpr (SP) {
+#pragma unroll
+    for (int k = 0; k < N; k++) hk[t.r + S::N2 * k] = rv[0][k];
+    __syncthreads();
+#pragma unroll
     for (int c = 0; c < 3; c++)
 #pragma unroll
-      for (int k = 0; k < N; k++) ru[c][k] = uin[c][col + (size_t)k * S::N2];
+      for (int k = 0; k < N; k++) va[c][k] = sl[(c * S::EPB + t.el) * NSL + t.r + S::N2 * k];
+    __syncthreads();
   }
+  auto vel = [&](int c, int k) { return SP ? va[SP ? c : 0][k] : rv[SP ? 0 : c][k]; };
   double *su = hk, *sd = hk + S::SZ, *sx = hk + 2 * S::SZ;
   const double jac = ejac[t.e];
   const double wa = W[t.i], wb = W[t.j];
   const double rx = edx[t.e * 3], ry = edx[t.e * 3 + 1], rz = edx[t.e * 3 + 2];
 #pragma unroll
-  for (int c = 0; c < 3; c++) {
+  for (int c = 0; c < (SP ? 1 : 3); c++) {
     // the z pass's derivatives, kept for the advection term
     double uzs[N];
     auto zcb = [&](int k, double uz, double) { uzs[k] = uz; };
     auto xcb = [&](int, double ux, double) { return ux * rx; };
     auto ycb = [&](int, double uy, double) { return uy * ry; };
-    double *ko = kout[c], *ac = acc[c];
+    double *ko = SP ? pick(kout) : kout[c], *ac = SP ? pick(acc) : acc[c];
     auto post = [&](int k, double L, double M, double hx, double hy) {
       if (!t.active) return;
       const size_t g = col + k * S::N2;
       // contractions written out: every form of the stage rounds alike
       const double po =
-          fma(uzs[k] * rz, ru[2][k], fma(hy, ru[1][k], hx * ru[0][k]));
+          fma(uzs[k] * rz, vel(2, k), fma(hy, vel(1, k), hx * vel(0, k)));
       if (nu != 1.0) L *= nu;
       const double urhs = fma(-po, M, -L);
       const double K = im[k] * urhs;
       if (ACC < 2 || ACC == 4) ko[g] = K;
       if constexpr (RA) ac[g] = fma(cb, K, ra[c][k]);
     };
-    gf::pen_op3<N, double, true>(ru[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,
+    gf::pen_op3<N, double, true>(rv[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,
                                  rz * rz, (const double *)nullptr, xcb, ycb, zcb, post);
-    __syncthreads();  // the next component reuses the LDS buffers
+    if (!SP) __syncthreads();  // the next component reuses the LDS buffers
   }
 }
 
@@ -566,13 +589,13 @@ __global__ __launch_bounds__(gf::PenS<N>::THREADS) void k_rk_out_halo(
   });
 }
 
-template <int N, int IN, int ACC>
+template <int N, int IN, int ACC, bool SP>
 int launch_stage3b_h(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
                      double *const *kout, double bh, double ca, double cb, double nu) {
-  using S = gf::PenS<N>;
+  using S = gf::PenStage<N, SP>;
   const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
   auto at = [](double *const *p, int c) { return p ? p[c] : nullptr; };
-  hipLaunchKernelGGL((k_burgers_stage3b<N, IN, ACC>), dim3(nb), dim3(S::THREADS), 0,
+  hipLaunchKernelGGL((k_burgers_stage3b<N, IN, ACC, SP>), dim3(nb), dim3(S::THREADS), 0,
                      m->ctx->stream, at(uin, 0), at(uin, 1), at(uin, 2), at(kp, 0), at(kp, 1),
                      at(kp, 2), at(acc, 0), at(acc, 1), at(acc, 2), at(kout, 0), at(kout, 1),
                      at(kout, 2), m->imass_el ? m->imass_el : m->imass, m->W[0], m->edx, m->ejac,
@@ -582,12 +605,32 @@ int launch_stage3b_h(gf_mesh *m, double *const *uin, double *const *kp, double *
   return GF_OK;
 }
 
+// Up to this many elements a stage is bound by the latency of one element's
+// chain of loads, group sums and contractions, three components long, and a
+// component to each third of the workgroup (SP) shortens it; beyond it the
+// chip is full either way.  The line lies low where a wave is one element
+// without idle lanes (N = 8) and where three components' LDS leaves one or two
+// workgroups to a CU (N = 10), high at N = 6, where SP needs fewer registers
+// and so has more waves.  RK4 steps, us, all three in a thread against SP:
+//   p = 1  20^3 25 / 22              p = 5  7^3 42 / 28, 16^3 100 / 91,
+//   p = 3  7^3 30 / 21, 16^3 40 / 37        20^3 162 / 148, 24^3 295 / 311
+//   p = 4  7^3 36 / 24, 14^3 59 / 57, 16^3 66 / 71
+//   p = 6  7^3 48 / 37, 13^3 110 / 97, 16^3 148 / 152
+//   p = 7  7^3 49 / 37, 10^3 70 / 64, 12^3 93 / 96, 16^3 165 / 177
+//   p = 8  7^3 84 / 50, 12^3 179 / 157, 14^3 229 / 222, 20^3 635 / 659
+//   p = 9  7^3 86 / 83, 8^3 93 / 89, 9^3 115 / 128
+constexpr size_t stage_split_max(int N) {
+  return N == 6 ? 8192 : (N == 8 ? 1024 : (N == 10 ? 512 : 3072));
+}
 template <int N>
 int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
                    double *const *kout, double bh, double ca, double cb, double nu, int in,
                    int accm) {
-#define GF_STAGE(I, A) \
-  if (in == I && accm == A) return launch_stage3b_h<N, I, A>(m, uin, kp, acc, kout, bh, ca, cb, nu)
+  const bool sp = m->nelems <= stage_split_max(N);
+#define GF_STAGE(I, A)                                                                         \
+  if (in == I && accm == A)                                                                    \
+  return sp ? launch_stage3b_h<N, I, A, true>(m, uin, kp, acc, kout, bh, ca, cb, nu)           \
+            : launch_stage3b_h<N, I, A, false>(m, uin, kp, acc, kout, bh, ca, cb, nu)
   GF_STAGE(0, 0);
   GF_STAGE(3, 0);
   GF_STAGE(1, 0);

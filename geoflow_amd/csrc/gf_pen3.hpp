@@ -140,6 +140,14 @@ struct PenS : Pen3<N> {
   static constexpr int THREADS = EPB * N * N;
 };
 
+// SP: the box RK stages with a component to each third of the workgroup.
+template <int N, bool SP>
+struct PenStage : PenS<N> {};
+template <int N>
+struct PenStage<N, true> : Pen3<N> {
+  static constexpr int THREADS = 3 * Pen3<N>::THREADS;
+};
+
 // Computes, for the column (i=a, j=b) owned by the calling thread,
 //   post(k, Lu_k, M_k, hx_k, hy_k),   Lu = ((x-part + y-part) + z-part)
 // where each part is D_d^T (M * ((D_d u) * G_d) [* p]), the operations of

@@ -118,10 +118,12 @@ struct ColIdx {
   int el, i, j, r;
   size_t e;
   bool active;
-  __device__ __forceinline__ ColIdx(size_t nelems, bool rev = false) {
+  __device__ __forceinline__ ColIdx(size_t nelems, bool rev = false)
+      : ColIdx(nelems, rev, (int)threadIdx.x) {}
+  __device__ __forceinline__ ColIdx(size_t nelems, bool rev, int tid) {
     using C = P;
-    el = threadIdx.x / C::N2;
-    r = threadIdx.x - el * C::N2;
+    el = tid / C::N2;
+    r = tid - el * C::N2;
     i = r % N;
     j = r / N;
     size_t eg = xcd_block(rev) * C::EPB + el;
