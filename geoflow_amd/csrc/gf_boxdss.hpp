@@ -215,42 +215,6 @@ __host__ __device__ __forceinline__ int box_members(const BoxElemDeltas &d, int 
   return box_members_own<I>(d, N, gself, i, j, k, g, &own);
 }
 
-// 1/count for a box group (count 1, 2, 4 or 8): exact, so x * box_inv(n)
-// equals x / n bit for bit and no division is needed.
-__host__ __device__ __forceinline__ double box_inv(int n) {
-  return n == 1 ? 1.0 : (n == 2 ? 0.5 : (n == 4 ? 0.25 : 0.125));
-}
-
-// Loads u at the member slots of a group; absent slots are not read (their
-// lanes are masked off and the slot is set to 0), which saves address and
-// cache work when most nodes of a wave have small groups.  Slot 0 (the
-// smallest member) is always read.
-template <typename I, typename T>
-__device__ __forceinline__ void box_load8m(const T *__restrict__ u, const I (&g)[8], int n,
-                                           T (&v)[8]) {
-  v[0] = u[g[0]];
-#pragma unroll
-  for (int m = 1; m < 8; m++) {
-    T t = T(0);
-    if (m < n) t = u[g[m]];
-    v[m] = t;
-  }
-}
-
-// 0 + v[0] + v[1] + ... over the members in that order (n == 1 returns v[0]
-// unchanged: singleton groups are not reduced), for slots filled by box_load8m.
-// Absent slots hold +0 and adding them changes nothing, because a sum that
-// starts from +0 is never -0 (in
-// round-to-nearest x + y is -0 only when both are -0), and s + (+0) == s for
-// every other s.  Same result bit for bit, without a select per slot.
-template <typename T>
-__device__ __forceinline__ T box_sum8z(const T (&v)[8], int n) {
-  T s = T(0);
-#pragma unroll
-  for (int m = 0; m < 8; m++) s = s + v[m];
-  return n == 1 ? v[0] : s;
-}
-
 // ---------------------------------------------------------------------------
 // Element halo in LDS for a gather Smooth (N^2 threads per element, thread
 // l = a + N b owning the column (a, b, .)).  Instead of each node loading its
@@ -414,7 +378,7 @@ struct HaloCol {
 // side first in z, then in y, then in x, the lower side of a direction being
 // the copy with the smaller global index -- over the 2 x 2 (x 2 on the z
 // faces) crossings, an absent partner's terms reading the zero slot, which
-// adds +0 and leaves every sum as it is (box_sum8z).  Every copy of a node
+// adds +0 and leaves every sum as it is.  Every copy of a node
 // has the same order.  Where box_halo_ok holds it is ascending global index,
 // GGFX's order.  Returns the count of the group.
 template <int N, int K>

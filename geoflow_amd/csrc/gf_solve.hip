@@ -26,9 +26,6 @@ __global__ void k_axpby(double *__restrict__ z, double a, const double *__restri
 __global__ void k_axpy(double *y, double a, const double *__restrict__ x, size_t n) {
   GRID_LOOP(g, n) y[g] = y[g] + a * x[g];
 }
-__global__ void k_copy(double *__restrict__ y, const double *__restrict__ x, size_t n) {
-  GRID_LOOP(g, n) y[g] = x[g];
-}
 __global__ void k_zero(double *__restrict__ y, size_t n) {
   GRID_LOOP(g, n) y[g] = 0.0;
 }

@@ -490,8 +490,10 @@ int gf_helmholtz_diag_inv(gf_mesh *mesh, double p_scalar, double q_scalar, const
  * Average duration in ms of `reps` back-to-back launches of one kernel of the
  * path on scratch data of the mesh's size, timed with HIP events on the
  * context stream.  which: "burgers_stage" (fused RK stage, the stage 2-3
- * form), "cg_apply" / "cg_apply_f32" (CG direction update + Helmholtz apply),
- * "helmholtz".  No reference counterpart (the reference's timers are never
+ * form), "burgers_stage_box" / "rk_out_box" (structured box: the second stage
+ * and the step output), "cg_apply" / "cg_apply_f32" (CG step of x, direction
+ * update and Helmholtz apply), "cg_update" / "cg_update_f32" (structured box:
+ * step of r), "helmholtz".  No reference counterpart (the reference's timers are never
  * set, src/apps/hackathon_driver.cpp:91,258-259).  Synchronous. */
 int gf_time_kernel(gf_mesh *mesh, const char *which, int reps, double *avg_ms);
 
