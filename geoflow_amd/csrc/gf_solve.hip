@@ -1725,6 +1725,12 @@ CGApply3Args apply3_args(gf_mesh *m, const CGCtl &c) {
   return a;
 }
 
+// The vectors exceed the Infinity Cache (CGCtl::stream).
+template <typename T>
+bool cg_streams(const gf_mesh *m) {
+  return 4 * m->ndof * sizeof(T) > ((size_t)256 << 20);
+}
+
 // Runs CG iterations from the state prepared in the systems' first scalar
 // sets (rho, rtol, first, iter = 0, done) until every system is done; r holds
 // the masked assembled residual, x the iterate.  The final scalars are left
@@ -1756,7 +1762,7 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
   c.partA = m->red;
   c.partU = m->red + (c.nbA + 64) / 2 * 2;  // 16-byte pairs
   c.normtype = normtype;
-  c.stream = 4 * m->ndof * sizeof(T) > ((size_t)256 << 20);
+  c.stream = cg_streams<T>(m);
   c.resid = d_resid;
   volatile double *hm = ns > 0 ? m->hsscal : m->hscal;
   c.mirror = ns > 0 ? m->hsscal_dev : m->hscal_dev;
@@ -2584,6 +2590,7 @@ extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *a
     RC(timing_scalars(m, ctl));
     ctl.nbA = f32 ? blocks3<float>(m) : blocks3<double>(m);
     ctl.nbU = ctl.nbA;
+    ctl.stream = f32 ? cg_streams<float>(m) : cg_streams<double>(m);
     if (f32) {
       for (int k = 0; k < 5; k++)
         hipLaunchKernelGGL(k_fill_pattern_f, dim3(nblocks(n)), dim3(kThreads), 0, s,
