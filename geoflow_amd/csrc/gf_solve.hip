@@ -1733,8 +1733,11 @@ bool cg_streams(const gf_mesh *m) {
 
 // Runs CG iterations from the state prepared in the systems' first scalar
 // sets (rho, rtol, first, iter = 0, done) until every system is done; r holds
-// the masked assembled residual, x the iterate.  The final scalars are left
-// in the host mirror (m->hscal, or m->hsscal on a batched mesh).
+// the masked assembled residual, x the iterate.  Returns on sight of the done
+// flags, which the kernels that set them, still running, may show ahead of
+// the scalars beside them: the caller reads the final scalars, in the host
+// mirror (m->hscal, or m->hsscal on a batched mesh), after its next wait for
+// the stream.
 template <typename T>
 int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
   hipStream_t s = m->ctx->stream;
@@ -1999,12 +2002,6 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
     v.mass = m->mass;
     v.p = prm->p_scalar;
     RC(cg_loop<double>(m, v, normtype, (double *)nullptr));
-    for (int k = 0; k < ns; k++) {
-      const double *h = &m->hsscal[(size_t)k * kCGSet];
-      m->seg_iters[k] = (int)h[S_ITER];
-      m->seg_rnorm[k] = h[S_RNORM];
-      if (m->seg_iters[k] >= prm->maxit && h[S_RNORM] > prm->tol) status = GF_ERR_NOCONVERGE;
-    }
   } else {
     float *r32 = wk.r32, *w32 = wk.w32, *q32 = wk.q32, *x32 = wk.x32;
     float *dinv32 = dinv ? wk.dinv32 : nullptr;
@@ -2043,6 +2040,14 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
       if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
       RC(seg_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, 1));
       RC(seg_get(m, 2, o));
+      // the cycle's scalars, complete after this wait
+      for (int k = 0; outer > 0 && k < ns; k++) {
+        if (conv[k]) continue;
+        const double *h = &m->hsscal[(size_t)k * kCGSet];
+        m->seg_iters[k] += (int)h[S_ITER];
+        rhom[k] = h[S_RHOM];
+        first[k] = 0;
+      }
       bool all = true;
       for (int k = 0; k < ns; k++) {
         m->seg_rnorm[k] = fin(k, o[2 * k + 1]);
@@ -2072,13 +2077,6 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
       }
       RC(upload());
       RC(cg_loop<float>(m, v, normtype, (double *)nullptr));
-      for (int k = 0; k < ns; k++) {
-        if (conv[k]) continue;
-        const double *h = &m->hsscal[(size_t)k * kCGSet];
-        m->seg_iters[k] += (int)h[S_ITER];
-        rhom[k] = h[S_RHOM];
-        first[k] = 0;
-      }
     }
     for (int k = 0; k < ns; k++)
       if (m->seg_rnorm[k] > rtol[k]) status = GF_ERR_NOCONVERGE;
@@ -2088,6 +2086,13 @@ int cg_solve_seg(gf_mesh *m, const gf_cg_params *prm, const double *b, const dou
     RC(gf_axpy_t(m, 1.0, xb, x));
   }
   GF_HIP(m->ctx, hipStreamSynchronize(s));
+  if (prm->precision == 0)
+    for (int k = 0; k < ns; k++) {
+      const double *h = &m->hsscal[(size_t)k * kCGSet];
+      m->seg_iters[k] = (int)h[S_ITER];
+      m->seg_rnorm[k] = h[S_RNORM];
+      if (m->seg_iters[k] >= prm->maxit && h[S_RNORM] > prm->tol) status = GF_ERR_NOCONVERGE;
+    }
   res->status = status;
   res->iters = *std::max_element(m->seg_iters.begin(), m->seg_iters.end());
   res->outer = outer;
@@ -2208,15 +2213,6 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
     v.mass = m->mass;
     v.p = prm->p_scalar;
     RC(cg_loop<double>(m, v, normtype, d_resid));
-    const int it = (int)m->hscal[S_ITER];
-    total_iters = it;
-    rn_final = m->hscal[S_RNORM];
-    if (prm->resid && it > 0) {
-      GF_HIP(m->ctx, hipMemcpyAsync(prm->resid, d_resid, it * sizeof(double),
-                                    hipMemcpyDeviceToHost, s));
-      GF_HIP(m->ctx, hipStreamSynchronize(s));
-    }
-    if (it >= prm->maxit && rn_final > prm->tol) status = GF_ERR_NOCONVERGE;
   } else {
     // Mixed precision: the CG recurrences (apply, direction, residual and
     // iterate increments) run in FP32 with FP64 reductions; whenever the
@@ -2268,6 +2264,8 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
       if (dinv32) hipLaunchKernelGGL(k_mul_t<float>, dim3(nblocks(n)), dim3(kThreads), 0, s, dinv32, r32, z32, n);
       RC(setup_red<float>(m, r32, dinv32 ? z32 : r32, m->imult32, normtype, SU_R32));
       RC(setup_get(m, su));
+      // the cycle's scalars, complete after this wait
+      if (!first) total_iters += (int)m->hscal[S_ITER];
       const double rn = finish_norm_host(normtype, su[SU_R + 1 - SU_B], m, volume);
       rn_final = rn;
       if (prm->resid && hist < prm->maxit) prm->resid[hist++] = rn;
@@ -2289,7 +2287,6 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
       hs[S_N] = (double)n;
       GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, sizeof(hs), hipMemcpyHostToDevice, s));
       RC(cg_loop<float>(m, v, normtype, (double *)nullptr));
-      total_iters += (int)m->hscal[S_ITER];
       first = false;
     }
     if (rn_final > rtol) status = GF_ERR_NOCONVERGE;
@@ -2299,6 +2296,16 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
     RC(gf_axpy_t(m, 1.0, xb, x));
   }
   GF_HIP(m->ctx, hipStreamSynchronize(s));
+  if (prm->precision == 0) {
+    total_iters = (int)m->hscal[S_ITER];
+    rn_final = m->hscal[S_RNORM];
+    if (prm->resid && total_iters > 0) {
+      GF_HIP(m->ctx, hipMemcpyAsync(prm->resid, d_resid, total_iters * sizeof(double),
+                                    hipMemcpyDeviceToHost, s));
+      GF_HIP(m->ctx, hipStreamSynchronize(s));
+    }
+    if (total_iters >= prm->maxit && rn_final > prm->tol) status = GF_ERR_NOCONVERGE;
+  }
   res->status = status;
   res->iters = total_iters;
   res->outer = outer;
