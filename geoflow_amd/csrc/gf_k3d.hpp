@@ -231,7 +231,8 @@ void k_burgers_stage3p(
 //   ADV false  o0, o1, o2 = d_x p, d_y p, d_z p (GMTK::grad, gmtk.ipp:2883-2892;
 //              edx NULL: reference-space derivatives, compute_grefderivs)
 //   ADV true   o0 = M (((d_x p) v0 + (d_y p) v1) + (d_z p) v2), GAdvect::apply
-//              (gadvect.ipp:57-99); a missing velocity component is zero
+//              (gadvect.ipp:57-99); the term of a missing velocity component is
+//              left out (its derivative may be infinite or NaN)
 // Memory bound: four fields for the gradient, five for the advection (the
 // composed advection moved 23).  At 24^3, p = 7: gradient 34 us against 43 of
 // the LDS form k_grad, advection 41.5 us (6.8 TB/s) against 242 composed; at
@@ -287,9 +288,9 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_grad3p(
 #pragma unroll
     for (int k = 0; k < N; k++) {
       const int q = S::at(t.i, t.j, k);
-      double a = (d[q] * rx) * vx[k];
-      a += (u[q] * ry) * vy[k];
-      a += (dz[k] * rz) * vz[k];
+      double a = v0 ? (d[q] * rx) * vx[k] : 0.0;
+      if (v1) a += (u[q] * ry) * vy[k];
+      if (v2) a += (dz[k] * rz) * vz[k];
       o0[col + k * S::N2] = a * (((W[k] * wj) * wi) * jac);
     }
   } else {
