@@ -347,6 +347,15 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 // unsmoothed own K_s, and one gather at the end serves the whole sum.  A
 // stage has its own K_s in registers and the previous one in its halo, so
 // the accumulator is touched in every second stage only.
+//
+// Copies of a node differ in the accumulator, so its Smooth rounds where
+// step_b's, of equal copies, is exact.  RK4 has no more error for it: four
+// additions to the state in either order (rms against extended precision, 4
+// steps at 4x3x3, p = 7: 1.67e-16 of the field, 1.75e-16 in step_b's order).  At
+// orders 2 and 3, with two additions, it would have (1.31e-16 against 1.25e-16): they
+// accumulate the increments alone (ACC 5) and add the state once, in the last
+// stage (ACC 2 and 6: 1.09e-16).  RK4 that way would read the state once more in
+// its last stage, 5.66 -> 5.75 ms for 4 steps at 32^3, p = 7.
 //   IN  stage input
 //     0  v = uin                        (first stage from a state)
 //     1  v = uin + bh S(kp)
@@ -357,9 +366,11 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 //   ACC  accumulation after the operator
 //     0  none                           K -> kout
 //     1  acc = uin + ca kp + cb K       K -> kout
-//     2  acc = uin + ca kp + cb K       (last stage: K is not stored)
+//     2  acc = uin + (ca kp + cb K)     (last stage: K is not stored)
 //     3  acc = acc + ca kp + cb K       (last stage)
 //     4  acc = v                        K -> kout  (stage states of the adjoint)
+//     5  acc = ca kp + cb K             K -> kout
+//     6  acc = uin + (acc + ca kp + cb K)  (last stage)
 //   SP  a third of the workgroup's threads to each component, which exchange
 //       the stage input through LDS; else a thread does all three in turn.
 //       The same operations (stage_split_max says which runs)
@@ -389,6 +400,7 @@ void k_burgers_stage3b(
   using S = gf::PenStage<N, SP>;
   using H = gf::Halo<N>;
   constexpr bool KP = IN != 0, GU = IN == 2, UIN = IN != 3;
+  constexpr bool RDA = ACC == 3 || ACC == 6, LAST = ACC == 2 || RDA;
   static_assert(KP || ACC == 0, "the first stage accumulates nothing");
   static_assert(IN != 3 || ACC == 0, "an output stage is a first stage");
   // N = 8: an element is one wave and its own values go straight to LDS
@@ -397,7 +409,7 @@ void k_burgers_stage3b(
   constexpr int UOFF = H::SIZE, AOFF = UOFF + 512;
   constexpr int HL = !KP ? 0
                          : (GU ? 2 * H::SIZE
-                               : H::SIZE + (L8 && UIN ? 512 : 0)) + (L8 && ACC == 3 ? 512 : 0);
+                               : H::SIZE + (L8 && UIN ? 512 : 0)) + (L8 && RDA ? 512 : 0);
   // per element: the halos, then (the same memory) the three element buffers
   constexpr int NSL = HL > 3 * S::SZ ? HL : 3 * S::SZ;
   constexpr int NC = SP ? 3 : 1, TPC = S::EPB * S::N2;
@@ -413,9 +425,13 @@ void k_burgers_stage3b(
   double im[N];
 #pragma unroll
   for (int k = 0; k < N; k++) im[k] = imass[t.e * imstride + t.r + (size_t)k * S::N2];
-  constexpr bool RA = ACC >= 1 && ACC <= 3;  // accumulates after the operator
+  constexpr bool RA = ACC != 0 && ACC != 4;  // accumulates after the operator
   // SP: this thread's component, else all three
   double rv[SP ? 1 : 3][N], ra[RA && !SP ? 3 : 1][RA ? N : 1];
+  // the state for the last stage's sum: SP keeps it (read again, RK3 on 19x14x11,
+  // p = 5 takes 60 us a step against 58), three components have no registers left
+  constexpr bool AU = ACC == 2 || ACC == 6;
+  double ru[AU && SP ? N : 1];
   auto pick = [&](auto *const (&p)[3]) { return cs == 0 ? p[0] : (cs == 1 ? p[1] : p[2]); };
   if constexpr (KP) {
     int ec[3];
@@ -436,7 +452,7 @@ void k_burgers_stage3b(
       if constexpr (L8) {
         lds_copy512(kpc + ebase, hk, l);
         if (UIN) lds_copy512(uic + ebase, hu, l);
-        if (ACC == 3) lds_copy512(acl + ebase, ha, l);
+        if (RDA) lds_copy512(acl + ebase, ha, l);
       } else {
 #pragma unroll
         for (int k = 0; k < N; k++) ko[k] = kpc[col + (size_t)k * S::N2];
@@ -444,7 +460,7 @@ void k_burgers_stage3b(
 #pragma unroll
           for (int k = 0; k < N; k++) uo[k] = uic[col + (size_t)k * S::N2];
         }
-        if (ACC == 3) {
+        if (RDA) {
 #pragma unroll
           for (int k = 0; k < N; k++) ao[k] = acl[col + (size_t)k * S::N2];
         }
@@ -480,8 +496,10 @@ void k_burgers_stage3b(
             v = hs.template sum<k>(hu, u, [&](double w, bool on) {
               return on ? fma(bh, ks, w) : 0.0;
             }) * inv;
-          if constexpr (ACC == 1 || ACC == 2) ra[c][k] = fma(ca, kown, u);
-          if constexpr (ACC == 3) ra[c][k] = fma(ca, kown, L8 ? ha[own] : ao[k]);
+          if constexpr (ACC == 1) ra[c][k] = fma(ca, kown, u);
+          if constexpr (ACC == 2 || ACC == 5) ra[c][k] = ca * kown;
+          if constexpr (RDA) ra[c][k] = fma(ca, kown, L8 ? ha[own] : ao[k]);
+          if constexpr (AU && SP) ru[k] = u;
         }
         // the value is formed here, node by node: without this the compiler
         // interleaves the sums of many nodes and keeps their operands live
@@ -527,6 +545,7 @@ void k_burgers_stage3b(
     auto xcb = [&](int, double ux, double) { return ux * rx; };
     auto ycb = [&](int, double uy, double) { return uy * ry; };
     double *ko = SP ? pick(kout) : kout[c], *ac = SP ? pick(acc) : acc[c];
+    const double *uic = uin[c];
     auto post = [&](int k, double L, double M, double hx, double hy) {
       if (!t.active) return;
       const size_t g = col + k * S::N2;
@@ -536,8 +555,12 @@ void k_burgers_stage3b(
       if (nu != 1.0) L *= nu;
       const double urhs = fma(-po, M, -L);
       const double K = im[k] * urhs;
-      if (ACC < 2 || ACC == 4) ko[g] = K;
-      if constexpr (RA) ac[g] = fma(cb, K, ra[c][k]);
+      if (!LAST) ko[g] = K;
+      if constexpr (RA) {
+        double a = fma(cb, K, ra[c][k]);
+        if constexpr (AU) a = (SP ? ru[SP ? k : 0] : uic[g]) + a;
+        ac[g] = a;
+      }
     };
     gf::pen_op3<N, double, true>(rv[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,
                                  rz * rz, (const double *)nullptr, xcb, ycb, zcb, post);
@@ -639,8 +662,11 @@ int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *co
   GF_STAGE(1, 2);
   GF_STAGE(1, 3);
   GF_STAGE(1, 4);
+  GF_STAGE(1, 5);
+  GF_STAGE(1, 6);
   GF_STAGE(2, 2);
   GF_STAGE(2, 3);
+  GF_STAGE(2, 6);
 #undef GF_STAGE
   return gf_set_err(m->ctx, GF_ERR_ARG, "stage3b: unsupported stage form");
 }

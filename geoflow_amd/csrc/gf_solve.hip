@@ -199,7 +199,8 @@ __global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
   const size_t g = e0 * S::NN + q;
   gf::stage_D(sD, a.D, N);
   if (q < N) sW[q] = a.W[q];
-  double ra[2] = {0.0, 0.0}, im = 0.0;
+  constexpr bool RDA = ACC == 3 || ACC == 6, LAST = ACC == 2 || RDA;
+  double ra[2] = {0.0, 0.0}, ru[2] = {0.0, 0.0}, im = 0.0;
   if (act) {
     im = a.imass[g];
     int id[4];
@@ -229,7 +230,8 @@ __global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
             double ko = kv[0];
 #pragma unroll
             for (int k = 1; k < 4; k++) ko = id[k] == (int)g ? kv[k] : ko;
-            ra[c] = fma(a.ca, ko, ACC == 3 ? a.acc[c][g] : u);
+            ra[c] = fma(a.ca, ko, RDA ? a.acc[c][g] : (ACC == 1 ? u : 0.0));
+            if (ACC == 2 || ACC == 6) ru[c] = u;
           }
         }
       }
@@ -263,8 +265,11 @@ __global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
       L += gf::contract<2, N, true>(&sg[c][1][el * S::NN], sD, 1, i, j, k);
       if (a.nu != 1.0) L *= a.nu;
       const double K = im * fma(-ad[c], M, -L);
-      if (ACC < 2) a.kout[c][g] = K;
-      if (ACC) a.acc[c][g] = fma(a.cb, K, ra[c]);
+      if (!LAST) a.kout[c][g] = K;
+      if (ACC) {
+        const double v = fma(a.cb, K, ra[c]);
+        a.acc[c][g] = ACC == 2 || ACC == 6 ? ru[c] + v : v;
+      }
     }
   }
 }
@@ -305,8 +310,11 @@ int launch_stage2(gf_mesh *m, const Stage2Args &a, int in, int accm) {
     GF_STAGE(1, 1);
     GF_STAGE(1, 2);
     GF_STAGE(1, 3);
+    GF_STAGE(1, 5);
+    GF_STAGE(1, 6);
     GF_STAGE(2, 2);
     GF_STAGE(2, 3);
+    GF_STAGE(2, 6);
 #undef GF_STAGE
   }
   return gf_set_err(m->ctx, GF_ERR_ARG, "stage2: unsupported stage form");
@@ -1116,7 +1124,8 @@ int rk_step_fused(gf_mesh *m, double nu, int order, double dt, double *const *u)
 
 // RK steps on a structured box or a 2-D mesh (order >= 2): step_b with every Smooth formed
 // by gather inside the stage kernels (k_burgers_stage3b) and the output
-// kernel, no DSS passes.  The accumulator uin + sum_s c_s h K_s is advanced
+// kernel, no DSS passes.  The accumulator uin + sum_s c_s h K_s (uin added in
+// the last stage at orders 2 and 3) is advanced
 // by two stage derivatives at a time, in the stages 1, 3 (and the last one);
 // its Smooth, the step output, is formed by the output kernel or, between
 // consecutive steps, by the next step's first stage with the same
@@ -1195,7 +1204,7 @@ int gf_rk_steps_box(gf_mesh *m, double nu, int order, double dt, int nsteps,
       const bool last = s == ns - 1;
       // accumulate K_{s-1} and K_s at odd s; a last stage at even s adds K_s
       const bool odd = s % 2 == 1;
-      const int accm = last ? (s == 1 ? 2 : 3) : (s == 1 ? 1 : 0);
+      const int accm = last ? (s == 1 ? 2 : (ns == 3 ? 6 : 3)) : (s == 1 ? (ns == 3 ? 5 : 1) : 0);
       RC(gather_stage(m, ui, K[(s - 1) % 2], acc, K[s % 2], beta[s * 4 + (s - 1)] * h,
                       odd ? c[s - 1] * h : 0.0, c[s] * h, nu, last && n == 0 && !cont ? 2 : 1, accm));
     }
