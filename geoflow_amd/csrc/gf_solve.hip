@@ -1412,12 +1412,17 @@ int rk_steps_embed_adv_t(gf_mesh *m, double nu, int order, double dt, T *ust0,
   a.w[0] = w0;
   a.w[1] = w1;
   a.nelems = m->nelems;
+  // a velocity component in the state's own memory moves with it
+  bool moves = false;
+  for (int k = 0; k < 3; k++)
+    moves = moves || ((const char *)vel[k] < (const char *)ust0 + bytes &&
+                      (const char *)ust0 < (const char *)vel[k] + dbytes);
   for (int step = 0; step < nsteps; step++) {
     for (int s = 0; s < ns; s++) {
       const bool last = s == ns - 1, odd = s % 2 == 1;
       const T *kp = s > 0 ? K[(s - 1) % 2] : nullptr;
       const T *base = s > 1 ? acc : ust0;
-      a.wform = step == 0 && s == 0;  // the velocity is constant in a call
+      a.wform = s == 0 && (step == 0 || moves);
       a.uin = ust0;
       a.kprev = kp;
       a.bh = s > 0 ? beta[s * 4 + (s - 1)] * h : 0.0;
