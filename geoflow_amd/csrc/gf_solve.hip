@@ -1234,8 +1234,10 @@ struct EmbAdvArgs {
   const T *uin;         // stage input base
   const T *kprev;       // smoothed K of the previous stage, or null
   const T *base;        // accumulation base, null: the uin value
+  const T *state;       // added to the accumulation last, or null
+  int nobase;           // the accumulation starts from nothing
   T *acc;               // receives the accumulation, or null (node by node, so
-                        // that it may be uin or base)
+                        // that it may be uin, base or state)
   double cn;
   double bh, ch, nu;
   const double *c[3];   // velocity (read when wform is set)
@@ -1267,11 +1269,12 @@ __global__ __launch_bounds__(kThreads) void k_adv_stage_embed(EmbAdvArgs<T> a) {
   const int q = threadIdx.x;
   const bool act = q < nel * S::NN;
   const size_t g = base + q;
-  T ra = T(0);
+  T ra = T(0), st = T(0);
   if (act) {
     T v = a.uin[g];
     const T kp = a.kprev ? a.kprev[g] : T(0);
-    if (a.acc) ra = fma((T)a.ch, kp, a.base ? a.base[g] : v);
+    if (a.acc) ra = fma((T)a.ch, kp, a.base ? a.base[g] : (a.nobase ? T(0) : v));
+    if (a.state) st = a.state[g];
     if (a.kprev) v = fma((T)a.bh, kp, v);
     su[q] = v;
   }
@@ -1315,7 +1318,10 @@ __global__ __launch_bounds__(kThreads) void k_adv_stage_embed(EmbAdvArgs<T> a) {
     if (a.nu != 1.0) lap *= a.nu;
     const T kn = (T)(im * (-lap) - po);
     if (a.kout) a.kout[g] = kn;
-    if (a.acc) a.acc[g] = fma((T)a.cn, kn, ra);
+    if (a.acc) {
+      const T r = fma((T)a.cn, kn, ra);
+      a.acc[g] = a.state ? st + r : r;
+    }
   }
 }
 
@@ -1346,9 +1352,9 @@ int launch_adv_stage_embed_t(gf_mesh *m, const EmbAdvArgs<float> &a) {
   return GF_DISPATCH_N(2, m->Niso, launch_adv_stage_embed_f, m, a);
 }
 
-// u3 = uin + bh k; acc += ch k
+// u3 = uin + bh k (u3 may be uin); acc += ch k
 template <typename T>
-__global__ void k_final_input_t(T *__restrict__ u3, const T *__restrict__ uin,
+__global__ void k_final_input_t(T *u3, const T *uin,
                                 const T *__restrict__ k, T bh, T *acc, const T *accsrc, T ch,
                                 size_t n) {
   XCD_GRID_LOOP(g, n) {
@@ -1371,7 +1377,11 @@ int dss_smooth(gf_mesh *m, float *u) { return gf_dss_f32(m, GF_DSS_SMOOTH, u); }
 // formed, before their Smooth: Smooth is linear and the sum is smoothed in the
 // end.  So it runs at every second stage, the last K is never stored, and u
 // stays as it is until the last stage overwrites it: 36 fields a step of order
-// 4 where a sum advanced at each stage and a copy of u move 43.  The state
+// 4 where a sum advanced at each stage and a copy of u move 43.  The Smooth of
+// the sum's unequal copies rounds, which at order 1 would be the larger part of
+// the error: there K is smoothed first.  Order 3 makes up for it by adding u to
+// the sum once, in the last stage; orders 2 and 4 have no more error than step_b's
+// order of operations gives.  The state
 // passed in may be discontinuous; from the second step on u is continuous, the
 // Smooth of us is the identity, and the last stage's kernel forms us as the
 // others do.  Level 5, p = 5, order 4 (2.2 M nodes), a step: 234 us with six
@@ -1427,10 +1437,12 @@ int rk_steps_embed_adv_t(gf_mesh *m, double nu, int order, double dt, T *ust0,
       a.kprev = kp;
       a.bh = s > 0 ? beta[s * 4 + (s - 1)] * h : 0.0;
       a.base = s > 1 ? acc : nullptr;
+      a.nobase = ns == 3;
+      a.state = ns == 3 && last ? ust0 : nullptr;
       a.ch = odd ? c[s - 1] * h : 0.0;
       a.cn = c[s] * h;
-      a.acc = last ? ust0 : odd ? acc : nullptr;
-      a.kout = last ? nullptr : K[s % 2];
+      a.acc = ns == 1 ? nullptr : last ? ust0 : odd ? acc : nullptr;
+      a.kout = last && ns > 1 ? nullptr : K[s % 2];
       if (last && (step == 0 || ns == 1)) {
         // the state may be discontinuous
         if (s > 0) {
@@ -1441,14 +1453,20 @@ int rk_steps_embed_adv_t(gf_mesh *m, double nu, int order, double dt, T *ust0,
           a.base = acc;
         } else {
           GF_HIP(m->ctx, hipMemcpyAsync(us, ust0, bytes, hipMemcpyDeviceToDevice, m->ctx->stream));
-          a.base = ust0;
         }
         RC(gf_dss_keep(m, us));
         a.uin = us;
         a.kprev = nullptr;
       }
       RC(launch_adv_stage_embed_t(m, a));
-      RC(last ? gf_dss_keep(m, ust0) : dss_smooth(m, K[s % 2]));
+      if (!last || ns == 1) RC(dss_smooth(m, K[s % 2]));
+      if (ns == 1) {
+        hipLaunchKernelGGL(k_final_input_t<T>, dim3(xcd_grid(nblocks(n))), dim3(kThreads), 0,
+                           m->ctx->stream, ust0, ust0, K[0], (T)a.cn, (T *)nullptr,
+                           (const T *)nullptr, (T)0, n);
+        GF_LAUNCH_CHECK(m->ctx);
+      }
+      if (last) RC(gf_dss_keep(m, ust0));
     }
   }
   return GF_OK;
