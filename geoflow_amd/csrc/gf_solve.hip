@@ -29,7 +29,8 @@ __global__ void k_axpy(double *y, double a, const double *__restrict__ x, size_t
 __global__ void k_zero(double *__restrict__ y, size_t n) {
   GRID_LOOP(g, n) y[g] = 0.0;
 }
-__global__ void k_nonfinite(const double *__restrict__ x, size_t n, double *flag) {
+template <typename T>
+__global__ void k_nonfinite(const T *__restrict__ x, size_t n, double *flag) {
   bool bad = false;
   GRID_LOOP(g, n) bad |= !isfinite(x[g]);
   if (bad) *flag = 1.0;
@@ -1544,7 +1545,7 @@ int rk_step_general(gf_mesh *m, int mode, double nu, int order, int nstate, doub
 int check_finite(gf_mesh *m, double *const *u, int nev) {
   GF_HIP(m->ctx, hipMemsetAsync(m->scal + 62, 0, sizeof(double), m->ctx->stream));
   for (int k = 0; k < nev; k++)
-    hipLaunchKernelGGL(k_nonfinite, dim3(nblocks(m->ndof)), dim3(kThreads), 0, m->ctx->stream,
+    hipLaunchKernelGGL(k_nonfinite<double>, dim3(nblocks(m->ndof)), dim3(kThreads), 0, m->ctx->stream,
                        u[k], m->ndof, m->scal + 62);
   GF_LAUNCH_CHECK(m->ctx);
   double f = 0;
@@ -2556,7 +2557,8 @@ __global__ void k_fill_pattern_f(float *a, size_t n, float s) {
 }  // namespace
 
 // Scalars of a running iteration for the timed CG kernels: both sets hold a
-// system that is never done, the partial sums are zero.
+// system that is never done, the partial sums of w.q add up to 1000, so that
+// alpha is 1e-3, and those of the update are zero (beta = 0).
 static int timing_scalars(gf_mesh *m, CGCtl &c) {
   memset(&c, 0, sizeof(c));
   c.scal = m->scal;
@@ -2576,6 +2578,8 @@ static int timing_scalars(gf_mesh *m, CGCtl &c) {
   hipLaunchKernelGGL(k_fill_pattern, dim3(64), dim3(kThreads), 0, m->ctx->stream, m->red,
                      (size_t)(4096 + 2 * 4096), 0.0);
   GF_LAUNCH_CHECK(m->ctx);
+  const double wq = 1e3;
+  GF_HIP(m->ctx, hipMemcpyAsync(m->red, &wq, sizeof(double), hipMemcpyHostToDevice, m->ctx->stream));
   GF_HIP(m->ctx, hipStreamSynchronize(m->ctx->stream));
   return GF_OK;
 }
@@ -2717,5 +2721,19 @@ extern "C" int gf_time_kernel(gf_mesh *m, const char *which, int reps, double *a
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   *avg_ms = (double)ms / reps;
-  return GF_OK;
+  // a time on infinities or NaN would be another kernel's
+  double bad = 0.0;
+  GF_HIP(m->ctx, hipMemsetAsync(m->scal + 62, 0, sizeof(double), s));
+  for (int k = 0; k < nbuf; k++) {
+    if (w == "cg_apply_f32" || w == "cg_update_f32")
+      hipLaunchKernelGGL(k_nonfinite<float>, dim3(nblocks(n)), dim3(kThreads), 0, s,
+                         (const float *)buf[k], k < 5 ? n : 0, m->scal + 62);
+    else
+      hipLaunchKernelGGL(k_nonfinite<double>, dim3(nblocks(n)), dim3(kThreads), 0, s, buf[k], n,
+                         m->scal + 62);
+  }
+  GF_LAUNCH_CHECK(m->ctx);
+  GF_HIP(m->ctx, hipMemcpyAsync(&bad, m->scal + 62, sizeof(double), hipMemcpyDeviceToHost, s));
+  GF_HIP(m->ctx, hipStreamSynchronize(s));
+  return bad != 0.0 ? gf_set_err(m->ctx, GF_ERR_NONFINITE, "timing: fields not finite") : GF_OK;
 }

@@ -493,8 +493,11 @@ int gf_helmholtz_diag_inv(gf_mesh *mesh, double p_scalar, double q_scalar, const
  * form), "burgers_stage_box" / "rk_out_box" (structured box: the second stage
  * and the step output), "cg_apply" / "cg_apply_f32" (CG step of x, direction
  * update and Helmholtz apply), "cg_update" / "cg_update_f32" (structured box:
- * step of r), "helmholtz".  No reference counterpart (the reference's timers are never
- * set, src/apps/hackathon_driver.cpp:91,258-259).  Synchronous. */
+ * step of r), "helmholtz".  The CG kernels read the Jacobi diagonal in full (a
+ * solve reads it from one element's table where the elements' are equal).
+ * GF_ERR_NONFINITE if a field is not finite afterwards.  No reference
+ * counterpart (the reference's timers are never set,
+ * src/apps/hackathon_driver.cpp:91,258-259).  Synchronous. */
 int gf_time_kernel(gf_mesh *mesh, const char *which, int reps, double *avg_ms);
 
 #ifdef __cplusplus
