@@ -629,23 +629,6 @@ int launch_stage3b_h(gf_mesh *m, double *const *uin, double *const *kp, double *
   return GF_OK;
 }
 
-// Up to this many elements a stage is bound by the latency of one element's
-// chain of loads, group sums and contractions, three components long, and a
-// component to each third of the workgroup (SP) shortens it; beyond it the
-// chip is full either way.  The line lies low where a wave is one element
-// without idle lanes (N = 8) and where three components' LDS leaves one or two
-// workgroups to a CU (N = 10), high at N = 6, where SP needs fewer registers
-// and so has more waves.  RK4 steps, us, all three in a thread against SP:
-//   p = 1  20^3 25 / 22              p = 5  7^3 42 / 28, 16^3 100 / 91,
-//   p = 3  7^3 30 / 21, 16^3 40 / 37        20^3 162 / 148, 24^3 295 / 311
-//   p = 4  7^3 36 / 24, 14^3 59 / 57, 16^3 66 / 71
-//   p = 6  7^3 48 / 37, 13^3 110 / 97, 16^3 148 / 152
-//   p = 7  7^3 49 / 37, 10^3 70 / 64, 12^3 93 / 96, 16^3 165 / 177
-//   p = 8  7^3 84 / 50, 12^3 179 / 157, 14^3 229 / 222, 20^3 635 / 659
-//   p = 9  7^3 86 / 83, 8^3 93 / 89, 9^3 115 / 128
-constexpr size_t stage_split_max(int N) {
-  return N == 6 ? 8192 : (N == 8 ? 1024 : (N == 10 ? 512 : 3072));
-}
 template <int N>
 int launch_stage3b(gf_mesh *m, double *const *uin, double *const *kp, double *const *acc,
                    double *const *kout, double bh, double ca, double cb, double nu, int in,
