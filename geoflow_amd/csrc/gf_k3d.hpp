@@ -228,16 +228,19 @@ void k_burgers_stage3p(
 // First derivatives of a field on regular 3-D elements in one pass, the
 // element in the pencil layout of pen_op3 (z derivative in the column's
 // registers, x and y through LDS):
-//   ADV false  o0, o1, o2 = d_x p, d_y p, d_z p (GMTK::grad, gmtk.ipp:2883-2892;
-//              edx NULL: reference-space derivatives, compute_grefderivs)
-//   ADV true   o0 = M (((d_x p) v0 + (d_y p) v1) + (d_z p) v2), GAdvect::apply
-//              (gadvect.ipp:57-99); the term of a missing velocity component is
-//              left out (its derivative may be infinite or NaN)
+//   ADV 0  o0, o1, o2 = d_x p, d_y p, d_z p (GMTK::grad, gmtk.ipp:2883-2892;
+//          edx NULL: reference-space derivatives, compute_grefderivs)
+//   ADV 1  o0 = M (((d_x p) v0 + (d_y p) v1) + (d_z p) v2), GAdvect::apply
+//          (gadvect.ipp:57-99)
+//   ADV 2  the same, where a velocity component may be missing (NULL): its term
+//          is left out, for its derivative may be infinite or NaN (a form of its
+//          own: with the tests in every call the operators of 21x17x13, p = 5
+//          took 40.6 us together against 39.3)
 // Memory bound: four fields for the gradient, five for the advection (the
 // composed advection moved 23).  At 24^3, p = 7: gradient 34 us against 43 of
 // the LDS form k_grad, advection 41.5 us (6.8 TB/s) against 242 composed; at
 // 21x17x13, p = 5: 8.1 against 9.7 us and 8.5 against 51 us.
-template <int N, bool ADV>
+template <int N, int ADV>
 __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_grad3p(
     const double *__restrict__ p, const double *__restrict__ v0, const double *__restrict__ v1,
     const double *__restrict__ v2, double *__restrict__ o0, double *__restrict__ o1,
@@ -245,6 +248,7 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_grad3p(
     const double *__restrict__ ejac, size_t nelems) {
   using S = gf::Pen3<N>;
   constexpr int NV = ADV ? N : 1;
+  const bool h0 = ADV != 2 || v0, h1 = ADV != 2 || v1, h2 = ADV != 2 || v2;
   __shared__ double su[S::EPB][S::SZ], sd[S::EPB][S::SZ];
   ColIdx<N> t(nelems);
   const size_t col = t.e * S::NN + t.r;
@@ -252,13 +256,13 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_grad3p(
 #pragma unroll
   for (int k = 0; k < N; k++) rp[k] = p[col + k * S::N2];
   // the velocities' loads are in flight while p is differentiated
-  if constexpr (ADV) {
+  if constexpr (ADV != 0) {
 #pragma unroll
     for (int k = 0; k < N; k++) {
       const size_t g = col + k * S::N2;
-      vx[k] = v0 ? v0[g] : 0.0;
-      vy[k] = v1 ? v1[g] : 0.0;
-      vz[k] = v2 ? v2[g] : 0.0;
+      vx[k] = h0 ? v0[g] : 0.0;
+      vy[k] = h1 ? v1[g] : 0.0;
+      vz[k] = h2 ? v2[g] : 0.0;
     }
   }
   const double rx = edx ? edx[t.e * 3] : 1.0, ry = edx ? edx[t.e * 3 + 1] : 1.0,
@@ -283,14 +287,14 @@ __global__ __launch_bounds__(gf::Pen3<N>::THREADS) void k_grad3p(
   for (int m = 0; m < N; m++) u[S::at(t.i, m, t.j)] = y[m];
   __syncthreads();
   if (!t.active) return;
-  if constexpr (ADV) {
+  if constexpr (ADV != 0) {
     const double jac = ejac[t.e], wi = W[t.i], wj = W[t.j];
 #pragma unroll
     for (int k = 0; k < N; k++) {
       const int q = S::at(t.i, t.j, k);
-      double a = v0 ? (d[q] * rx) * vx[k] : 0.0;
-      if (v1) a += (u[q] * ry) * vy[k];
-      if (v2) a += (dz[k] * rz) * vz[k];
+      double a = h0 ? (d[q] * rx) * vx[k] : 0.0;
+      if (h1) a += (u[q] * ry) * vy[k];
+      if (h2) a += (dz[k] * rz) * vz[k];
       o0[col + k * S::N2] = a * (((W[k] * wj) * wi) * jac);
     }
   } else {
@@ -309,9 +313,9 @@ template <int N>
 int launch_advect3p(gf_mesh *m, const double *p, const double *const *v, double *po) {
   using S = gf::Pen3<N>;
   const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
-  hipLaunchKernelGGL((k_grad3p<N, true>), dim3(nb), dim3(S::THREADS), 0, m->ctx->stream, p, v[0],
-                     v[1], v[2], po, (double *)nullptr, (double *)nullptr, m->W[0], m->edx, m->ejac,
-                     m->nelems);
+  auto *k = v[0] && v[1] && v[2] ? k_grad3p<N, 1> : k_grad3p<N, 2>;
+  hipLaunchKernelGGL(k, dim3(nb), dim3(S::THREADS), 0, m->ctx->stream, p, v[0], v[1], v[2], po,
+                     (double *)nullptr, (double *)nullptr, m->W[0], m->edx, m->ejac, m->nelems);
   GF_LAUNCH_CHECK(m->ctx);
   return GF_OK;
 }
@@ -319,7 +323,7 @@ template <int N>
 int launch_grad3p(gf_mesh *m, const double *p, double *const *o, const double *edx) {
   using S = gf::Pen3<N>;
   const int nb = xcd_grid((m->nelems + S::EPB - 1) / S::EPB);
-  hipLaunchKernelGGL((k_grad3p<N, false>), dim3(nb), dim3(S::THREADS), 0, m->ctx->stream, p,
+  hipLaunchKernelGGL((k_grad3p<N, 0>), dim3(nb), dim3(S::THREADS), 0, m->ctx->stream, p,
                      (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, o[0],
                      o[1], o[2], m->W[0], edx, m->ejac, m->nelems);
   GF_LAUNCH_CHECK(m->ctx);
