@@ -8,12 +8,13 @@
 // periodic).  The group is the product of these per-direction choices, at
 // most 8 nodes.  A consumer kernel can therefore assemble a local vector on
 // the fly ("gather"): every copy of a shared node reads all members of its
-// group and sums them in ascending global index, which is the order in which
-// GGFX::doOp accumulates a group (std::accumulate from 0 over the sorted
-// members, src/cdg/comm/ggfx.hpp:346-443).  All copies compute the same sum,
-// so the result stays continuous, and no separate DSS pass or index array is
-// needed.  gf_mesh_create enables this only after checking on the host that
-// the groups it produces equal the GGFX groups of the mesh.
+// group, through a halo of its element in LDS, and sums them in pairs along x,
+// then y, then z (HaloSum).  GGFX::doOp accumulates a group in ascending
+// global index (std::accumulate from 0 over the sorted members,
+// src/cdg/comm/ggfx.hpp:346-443), so the two agree to rounding.  All copies
+// compute the same sum, so the result stays continuous, and no separate DSS
+// pass or index array is needed.  gf_mesh_create enables this only after checking
+// on the host that the groups it produces equal the GGFX groups of the mesh.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -476,7 +477,9 @@ struct HaloSum {
   }
 };
 
-// The N = 8 instances under their own names.
+// HaloCol, halo_order and box_halo_ok state the halo's layout in GGFX's terms,
+// and are run by the CPU checks of the halo; no kernel uses them.  The N = 8
+// instances under their own names.
 constexpr int kHalo8 = Halo<8>::SIZE;
 constexpr int kHalo8Zero = Halo<8>::ZERO;
 template <typename T>

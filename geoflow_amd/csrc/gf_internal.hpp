@@ -32,19 +32,23 @@ struct gf_ctx_s {
 constexpr size_t kNrefMax = (size_t)3 << 18;
 
 // 3-D box RK stages (gfs::k_burgers_stage3b): up to this many elements a stage is
-// bound by the latency of one element's
-// chain of loads, group sums and contractions, three components long, and a
-// component to each third of the workgroup (SP) shortens it; beyond it the
-// chip is full either way.  The line lies low where a wave is one element
-// without idle lanes (N = 8) and where three components' LDS leaves one or two
-// workgroups to a CU (N = 10), high at N = 6, where SP needs fewer registers
-// and so has more waves.  RK4 steps, us, all three in a thread against SP:
-//   p = 1  20^3 25 / 22              p = 5  7^3 42 / 28, 16^3 100 / 91,
-//   p = 3  7^3 30 / 21, 16^3 40 / 37        20^3 162 / 148, 24^3 295 / 311
-//   p = 4  7^3 36 / 24, 14^3 59 / 57, 16^3 66 / 71
-//   p = 6  7^3 48 / 37, 13^3 110 / 97, 16^3 148 / 152
+// bound by the latency of one element's chain of loads, group sums and
+// contractions, three components long, and a component to each third of the
+// workgroup (SP) shortens it; beyond it the chip is full either way.  The line
+// lies low where a wave is one element without idle lanes (N = 8) and where
+// three components' LDS leaves one or two workgroups to a CU (N = 10), high at
+// N = 6, where SP needs fewer registers and so has more waves.  The other orders
+// share the line of N = 5 and 7, which cross between 15^3 = 3375 and 16^3 elements;
+// N = 2, 3, 4 and 9 cross only at 8000 to 20000 elements and have up to a fifth
+// (N = 2) left above the line.  RK4 steps, us, all three in a thread against SP:
+//   p = 1  15^3 23 / 19, 16^3 23 / 19, 20^3 26 / 22, 24^3 30 / 29, 32^3 41 / 43
+//   p = 2  7^3 29 / 21, 15^3 34 / 28, 16^3 36 / 34, 20^3 45 / 45, 24^3 55 / 59
+//   p = 3  7^3 30 / 21, 15^3 40 / 36, 16^3 39 / 37, 20^3 57 / 57, 24^3 87 / 84
+//   p = 4  7^3 36 / 24, 14^3 57 / 55, 15^3 62 / 61, 16^3 66 / 70
+//   p = 5  7^3 42 / 28, 16^3 100 / 91, 20^3 162 / 148, 24^3 295 / 311
+//   p = 6  7^3 48 / 37, 14^3 118 / 113, 15^3 144 / 133, 16^3 149 / 152
 //   p = 7  7^3 49 / 37, 10^3 70 / 64, 12^3 93 / 96, 16^3 165 / 177
-//   p = 8  7^3 84 / 50, 12^3 179 / 157, 14^3 229 / 222, 20^3 635 / 659
+//   p = 8  7^3 84 / 50, 10^3 119 / 94, 14^3 225 / 216, 16^3 328 / 314, 20^3 635 / 659
 //   p = 9  7^3 86 / 83, 8^3 93 / 89, 9^3 115 / 128
 constexpr size_t stage_split_max(int N) {
   return N == 6 ? 8192 : (N == 8 ? 1024 : (N == 10 ? 512 : 3072));

@@ -388,9 +388,9 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 //
 // Bound by memory: at 32^3, p = 7 an RK4 step moves 42 fields of 134 MB; the
 // form whose every stage smoothed into the accumulator moved 54 and gathered
-// uin too in the last one.  Stages (IN, ACC) = (3,0) 358, (1,1) 424, (1,0)
-// 338, (1,3) 399 us, 3.6-3.8 TB/s where a copy of this size has 4.7; before,
-// 392 + 543 + 459 + 601 us.
+// uin too in the last one.  Stages (IN, ACC) = (3,0) 346, (1,1) 420, (1,0)
+// 312, (1,3) 373 us, 3.5-4.3 TB/s where copies beyond the Infinity Cache have
+// 4.6-5.3; before, 392 + 543 + 459 + 601 us.
 // ---------------------------------------------------------------------------
 template <int N, int IN, int ACC, bool SP>
 __global__ __launch_bounds__((gf::PenStage<N, SP>::THREADS)) __attribute__((amdgpu_waves_per_eu(N <= 8 ? 2 : 1)))

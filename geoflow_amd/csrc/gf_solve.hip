@@ -1849,8 +1849,8 @@ int cg_loop(gf_mesh *m, CGVecs<T> &v, int normtype, double *d_resid) {
   // each still costs its launches (5-20 us), so the batches grow slowly, by a
   // quarter of the iterations done.  They start from 2; from 4 where an
   // iteration is hardly longer than the host needs to queue it and to notice
-  // its end.  Eight ensemble members, 9 solves of 5-6 iterations: 5.62 against
-  // 6.08 ms a step from 4; 60 elements, p = 4, 144 iterations: 2.49 against 2.41.
+  // its end.  Eight ensemble members, 9 solves of 5-6 iterations: 5.82 against
+  // 6.28 ms a step from 4; 60 elements, p = 4, 144 iterations: 2.52 against 2.48.
   const int batch0 = m->ndof > ((size_t)1 << 17) ? 2 : 4;
   int cur = 0, nq = 0, batch = batch0;
   for (int it = 0;;) {
@@ -2215,7 +2215,7 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
     if (dinv) RC(gf_mul_t(m, dinv, r, z));
     RC(setup_red<double>(m, r, dinv ? z : r, m->imult, normtype, SU_R));
     RC(setup_get(m, su));
-    double hs[12] = {0};
+    double hs[S_COUNT] = {0};
     hs[S_RHO] = su[SU_R - SU_B];
     hs[S_RTOL] = rtol;
     hs[S_RNORM] = 10.0 * rtol;
@@ -2225,7 +2225,7 @@ int cg_solve_impl(gf_mesh *m, const gf_cg_params *prm, const double *b, const do
     hs[S_FIRST] = 1.0;
     hs[S_VOL] = volume;
     hs[S_N] = (double)n;
-    GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, 12 * sizeof(double), hipMemcpyHostToDevice, s));
+    GF_HIP(m->ctx, hipMemcpyAsync(m->scal, hs, sizeof(hs), hipMemcpyHostToDevice, s));
     CGVecs<double> v{};
     v.x = x;
     v.r = r;
