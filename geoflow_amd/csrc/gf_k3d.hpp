@@ -358,8 +358,10 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 // steps at 4x3x3, p = 7: 1.67e-16 of the field, 1.75e-16 in step_b's order).  At
 // orders 2 and 3, with two additions, it would have (1.31e-16 against 1.25e-16): they
 // accumulate the increments alone (ACC 5) and add the state once, in the last
-// stage (ACC 2 and 6: 1.09e-16).  RK4 that way would read the state once more in
-// its last stage, 5.66 -> 5.75 ms for 4 steps at 32^3, p = 7.
+// stage (ACC 2 and 6: 1.09e-16).  It is read once more for that where a thread
+// does all three components: at 32^3, p = 7 RK2 665 -> 694 us a step, RK3 1115 ->
+// 1137 (RK4 that way 1415 -> 1438).  A Smooth corrected to one rounding instead
+// left 1.28e-16 and cost 2-4 % at all sizes.
 //   IN  stage input
 //     0  v = uin                        (first stage from a state)
 //     1  v = uin + bh S(kp)
