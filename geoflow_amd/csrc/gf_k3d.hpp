@@ -358,10 +358,9 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 // steps at 4x3x3, p = 7: 1.67e-16 of the field, 1.75e-16 in step_b's order).  At
 // orders 2 and 3, with two additions, it would have (1.31e-16 against 1.25e-16): they
 // accumulate the increments alone (ACC 5) and add the state once, in the last
-// stage (ACC 2 and 6: 1.09e-16).  It is read once more for that where a thread
-// does all three components: at 32^3, p = 7 RK2 665 -> 694 us a step, RK3 1115 ->
-// 1137 (RK4 that way 1415 -> 1438).  A Smooth corrected to one rounding instead
-// left 1.28e-16 and cost 2-4 % at all sizes.
+// stage (ACC 2 and 6: 1.09e-16).  It is read once more for that: at 32^3, p = 7
+// RK2 652 -> 676 us a step, RK3 1102 -> 1115 (RK4 that way 1415 -> 1438).  A Smooth
+// corrected to one rounding instead left 1.28e-16 and cost 2-4 % at all sizes.
 //   IN  stage input
 //     0  v = uin                        (first stage from a state)
 //     1  v = uin + bh S(kp)
@@ -375,8 +374,9 @@ int launch_stage3p(gf_mesh *m, const StageArgs &a) {
 //     2  acc = uin + (ca kp + cb K)     (last stage: K is not stored)
 //     3  acc = acc + ca kp + cb K       (last stage)
 //     4  acc = v                        K -> kout  (stage states of the adjoint)
-//     5  acc = ca kp + cb K             K -> kout
-//     6  acc = uin + (acc + ca kp + cb K)  (last stage)
+//     5  acc = ca kp                    K -> kout
+//     6  acc = uin + (acc + cb K)       (last stage)
+//        (RK3, whose second stage has no weight)
 //   SP  a third of the workgroup's threads to each component, which exchange
 //       the stage input through LDS; else a thread does all three in turn.
 //       The same operations (stage_split_max says which runs)
@@ -406,7 +406,7 @@ void k_burgers_stage3b(
   using S = gf::PenStage<N, SP>;
   using H = gf::Halo<N>;
   constexpr bool KP = IN != 0, GU = IN == 2, UIN = IN != 3;
-  constexpr bool RDA = ACC == 3 || ACC == 6, LAST = ACC == 2 || RDA;
+  constexpr bool LAST = ACC == 2 || ACC == 3 || ACC == 6;
   static_assert(KP || ACC == 0, "the first stage accumulates nothing");
   static_assert(IN != 3 || ACC == 0, "an output stage is a first stage");
   // N = 8: an element is one wave and its own values go straight to LDS
@@ -415,7 +415,7 @@ void k_burgers_stage3b(
   constexpr int UOFF = H::SIZE, AOFF = UOFF + 512;
   constexpr int HL = !KP ? 0
                          : (GU ? 2 * H::SIZE
-                               : H::SIZE + (L8 && UIN ? 512 : 0)) + (L8 && RDA ? 512 : 0);
+                               : H::SIZE + (L8 && UIN ? 512 : 0)) + (L8 && ACC == 3 ? 512 : 0);
   // per element: the halos, then (the same memory) the three element buffers
   constexpr int NSL = HL > 3 * S::SZ ? HL : 3 * S::SZ;
   constexpr int NC = SP ? 3 : 1, TPC = S::EPB * S::N2;
@@ -431,13 +431,12 @@ void k_burgers_stage3b(
   double im[N];
 #pragma unroll
   for (int k = 0; k < N; k++) im[k] = imass[t.e * imstride + t.r + (size_t)k * S::N2];
-  constexpr bool RA = ACC != 0 && ACC != 4;  // accumulates after the operator
+  // KR: kp is read again for the sum, where to keep it costs a wave (RK2 at 9^3,
+  // p = 7 25.0 us a step against 26.6, p = 9 51.6 against 63)
+  constexpr bool KR = ACC == 2 && N == (SP ? 8 : 10), RA = ACC >= 1 && ACC <= 3 && !KR;
   // SP: this thread's component, else all three
   double rv[SP ? 1 : 3][N], ra[RA && !SP ? 3 : 1][RA ? N : 1];
-  // the state for the last stage's sum: SP keeps it (read again, RK3 on 19x14x11,
-  // p = 5 takes 60 us a step against 58), three components have no registers left
-  constexpr bool AU = ACC == 2 || ACC == 6;
-  double ru[AU && SP ? N : 1];
+  constexpr bool AU = ACC == 2 || ACC == 6;  // the state is added in the end
   auto pick = [&](auto *const (&p)[3]) { return cs == 0 ? p[0] : (cs == 1 ? p[1] : p[2]); };
   if constexpr (KP) {
     int ec[3];
@@ -458,7 +457,7 @@ void k_burgers_stage3b(
       if constexpr (L8) {
         lds_copy512(kpc + ebase, hk, l);
         if (UIN) lds_copy512(uic + ebase, hu, l);
-        if (RDA) lds_copy512(acl + ebase, ha, l);
+        if (ACC == 3) lds_copy512(acl + ebase, ha, l);
       } else {
 #pragma unroll
         for (int k = 0; k < N; k++) ko[k] = kpc[col + (size_t)k * S::N2];
@@ -466,7 +465,7 @@ void k_burgers_stage3b(
 #pragma unroll
           for (int k = 0; k < N; k++) uo[k] = uic[col + (size_t)k * S::N2];
         }
-        if (RDA) {
+        if (ACC == 3) {
 #pragma unroll
           for (int k = 0; k < N; k++) ao[k] = acl[col + (size_t)k * S::N2];
         }
@@ -503,9 +502,11 @@ void k_burgers_stage3b(
               return on ? fma(bh, ks, w) : 0.0;
             }) * inv;
           if constexpr (ACC == 1) ra[c][k] = fma(ca, kown, u);
-          if constexpr (ACC == 2 || ACC == 5) ra[c][k] = ca * kown;
-          if constexpr (RDA) ra[c][k] = fma(ca, kown, L8 ? ha[own] : ao[k]);
-          if constexpr (AU && SP) ru[k] = u;
+          if constexpr (ACC == 2 && RA) ra[c][k] = ca * kown;
+          if constexpr (ACC == 3) ra[c][k] = fma(ca, kown, L8 ? ha[own] : ao[k]);
+          if constexpr (ACC == 5) {
+            if (t.active) acl[col + (size_t)k * S::N2] = ca * kown;
+          }
         }
         // the value is formed here, node by node: without this the compiler
         // interleaves the sums of many nodes and keeps their operands live
@@ -549,9 +550,18 @@ void k_burgers_stage3b(
     double uzs[N];
     auto zcb = [&](int k, double uz, double) { uzs[k] = uz; };
     auto xcb = [&](int, double ux, double) { return ux * rx; };
-    auto ycb = [&](int, double uy, double) { return uy * ry; };
     double *ko = SP ? pick(kout) : kout[c], *ac = SP ? pick(acc) : acc[c];
-    const double *uic = uin[c];
+    const double *uic = SP ? pick(uin) : uin[c];
+    // operands of the sum, read again (kept over the operator, the state and the
+    // accumulator cost N = 9 a wave: RK3 at 16^3 317 us a step against 253) and on
+    // their way while the y pencil is worked
+    const double *kpc = SP ? pick(kp) : kp[c];
+    double us[AU ? N : 1], as[ACC == 6 || KR ? N : 1];
+    auto ycb = [&](int j, double uy, double) {
+      if constexpr (AU) us[j] = uic[col + (size_t)j * S::N2];
+      if constexpr (ACC == 6 || KR) as[j] = (KR ? kpc : ac)[col + (size_t)j * S::N2];
+      return uy * ry;
+    };
     auto post = [&](int k, double L, double M, double hx, double hy) {
       if (!t.active) return;
       const size_t g = col + k * S::N2;
@@ -562,10 +572,12 @@ void k_burgers_stage3b(
       const double urhs = fma(-po, M, -L);
       const double K = im[k] * urhs;
       if (!LAST) ko[g] = K;
-      if constexpr (RA) {
-        double a = fma(cb, K, ra[c][k]);
-        if constexpr (AU) a = (SP ? ru[SP ? k : 0] : uic[g]) + a;
-        ac[g] = a;
+      if constexpr (ACC == 1 || ACC == 3) ac[g] = fma(cb, K, ra[c][k]);
+      if constexpr (AU) {
+        double a;
+        if constexpr (RA) a = ra[c][k];
+        else a = ACC == 6 ? as[k] : ca * as[k];
+        ac[g] = us[k] + fma(cb, K, a);
       }
     };
     gf::pen_op3<N, double, true>(rv[c], su, sd, sx, Dp, W, t.i, t.j, wa, wb, jac, rx * rx, ry * ry,

@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
   const size_t g = e0 * S::NN + q;
   gf::stage_D(sD, a.D, N);
   if (q < N) sW[q] = a.W[q];
-  constexpr bool RDA = ACC == 3 || ACC == 6, LAST = ACC == 2 || RDA;
+  constexpr bool LAST = ACC == 2 || ACC == 3 || ACC == 6;
   double ra[2] = {0.0, 0.0}, ru[2] = {0.0, 0.0}, im = 0.0;
   if (act) {
     im = a.imass[g];
@@ -231,7 +231,8 @@ __global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
             double ko = kv[0];
 #pragma unroll
             for (int k = 1; k < 4; k++) ko = id[k] == (int)g ? kv[k] : ko;
-            ra[c] = fma(a.ca, ko, RDA ? a.acc[c][g] : (ACC == 1 ? u : 0.0));
+            if (ACC == 6) ra[c] = a.acc[c][g];
+            else ra[c] = fma(a.ca, ko, ACC == 3 ? a.acc[c][g] : (ACC == 1 ? u : 0.0));
             if (ACC == 2 || ACC == 6) ru[c] = u;
           }
         }
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(kThreads) void k_burgers_stage2(Stage2Args a) {
       const double K = im * fma(-ad[c], M, -L);
       if (!LAST) a.kout[c][g] = K;
       if (ACC) {
-        const double v = fma(a.cb, K, ra[c]);
+        const double v = ACC == 5 ? ra[c] : fma(a.cb, K, ra[c]);
         a.acc[c][g] = ACC == 2 || ACC == 6 ? ru[c] + v : v;
       }
     }
